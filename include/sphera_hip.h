@@ -53,12 +53,8 @@ typedef struct sph_params {
                             momentum pass, and the others where theirs is 0 */
     int32_t chunk_v, chunk_c, chunk_p; /* the same for velocity smoothing, continuity,
                                           pressure smoothing (0 = chunk) */
-    int32_t nb_shape;    /* neighbour-search workgroup size x LDS candidate tile:
-                            0 = 256 x 4096 in FP16 (default), 1 = 256 x 3072 in FP32,
-                            2 = 128 x 1536 in FP32, 3 = 256 x 2816 in FP16 with 64
-                            registers (8 waves per SIMD), 4 = 256 x 4096 in 16-bit
-                            fixed point over the cell.  The lists are the same in
-                            every shape (FP64 decides near the cut-off). */
+    int32_t nb_shape;    /* 0 to 4, accepted for callers that set it: the neighbour search has
+                            one launch shape, and the lists never depended on it */
     int32_t options;     /* SPH_OPT_* flags of the deck (below) */
 } sph_params;
 

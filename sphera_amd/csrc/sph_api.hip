@@ -53,8 +53,8 @@ struct sph_ctx {
     std::vector<DP> segs;
     Seg S{};
     DP* d_P = nullptr;
-    int *d_pblk = nullptr, *d_kblk = nullptr, *d_rseg = nullptr, *d_adj = nullptr;
-    int nkeys = 1, nrows = 1;  // cell keys (cells + out-of-grid bucket per segment), cell rows
+    int *d_pblk = nullptr, *d_kblk = nullptr, *d_adj = nullptr;
+    int nkeys = 1;             // cell keys (cells + out-of-grid bucket per segment)
     int nb_stride_max = 1;     // largest NMAXPARTJ of the segments (list capacity)
     std::vector<int> staged;   // segments uploaded since the last commit
     int precision = SPH_FP64;
@@ -84,10 +84,7 @@ struct sph_ctx {
     int *cell = nullptr, *key = nullptr, *slot = nullptr, *cnt = nullptr, *start = nullptr,
         *perm = nullptr, *pid = nullptr, *bsum = nullptr;
     int *work = nullptr, *nwork = nullptr;  // (particle, face) pairs of the boundary table
-    int* rowblk = nullptr;                  // first neighbour-search block of each cell row
     int *idslot = nullptr, *rmids = nullptr;  // id -> slot, ids removed by a sort
-    int nb_grid = 8;                        // persistent workgroups of the neighbour search
-    int nb_shape = 0;                       // its launch shape (index into NB_SHAPES)
     int wg = 256, grid = 1, bt_grid = 1024;  // launch shape of the particle kernels
     int chunk = 8;                            // list entries gathered per step of the FP32 walks
     int chunk_v = 8, chunk_c = 8, chunk_p = 8;  // the same for smoothing, continuity, pressure smoothing
@@ -99,7 +96,7 @@ struct sph_ctx {
     double* scal = nullptr;
     int* iscal = nullptr;
     unsigned long long* dtmin = nullptr;
-    unsigned long long* pairs = nullptr;  // running pair-interaction count
+    unsigned long long* pairs = nullptr;  // running pair-interaction count, NBC_PAIRS partial counters
     // DB-SPH walls: the wall-element tables (w0, w1, w2, cell lists), their
     // density, pressure and wet flags; per particle Gamma and dShep (two
     // buffers each: the sort gathers [0] into [1]), sigma, rhoSPH_new, FS,
@@ -258,31 +255,10 @@ int run_sort(sph_ctx* c) {
     return 0;
 }
 
-// the tiled search in launch shape `shape` of NB_SHAPES
-#define NB_KERNEL(SG, k) \
-    k_neighbours<SG, NB_SHAPES[k].wg, NB_SHAPES[k].tile, NB_SHAPES[k].tk, NB_SHAPES[k].minb>
-
-template <bool SG>
-void launch_nb(sph_ctx* c) {
-    const int wg = NB_SHAPES[c->nb_shape].wg;
-    auto go = [&](auto kern) {
-        kern<<<c->nb_grid, wg, 0, c->stream>>>(c->P, c->S, c->xm[0], c->xmf, c->cell, c->start, c->rowblk,
-                                               c->nbr, c->nnb, c->iscal, c->pairs);
-    };
-    switch (c->nb_shape) {
-        case 1: go(NB_KERNEL(SG, 1)); break;
-        case 2: go(NB_KERNEL(SG, 2)); break;
-        case 3: go(NB_KERNEL(SG, 3)); break;
-        case 4: go(NB_KERNEL(SG, 4)); break;
-        default: go(NB_KERNEL(SG, 0)); break;
-    }
-}
-
 int run_neighbours(sph_ctx* c) {
     KTime t(c, "neighbours");
-    SEGL(k_nb_rowblocks, 1, 1024, c->start, c->rowblk, NB_SHAPES[c->nb_shape].wg);
-    if (c->nseg > 1) launch_nb<true>(c);
-    else launch_nb<false>(c);
+    SEGL(k_neighbours, nblk(c->P.cap, 4 * NBC_SLOTS), 256, c->xm[0], c->xmf, c->cell, c->start, c->nbr, c->nnb,
+         c->iscal, c->pairs);
     return 0;
 }
 
@@ -466,7 +442,7 @@ sph_ctx::~sph_ctx() {
         if (p) hipFree(p);
     };
     F(d_faces); F(d_edges); F(d_gcount); F(d_gstart); F(d_gvec); F(d_kt); F(d_bit); F(d_btf);
-    F(d_P); F(d_pblk); F(d_kblk); F(d_rseg); F(d_adj);
+    F(d_P); F(d_pblk); F(d_kblk); F(d_adj);
     for (auto p : xm) F(p);
     for (auto p : vel) F(p);
     for (auto p : acc) F(p);
@@ -475,7 +451,7 @@ sph_ctx::~sph_ctx() {
     F(xmf); F(xrf);
     for (auto p : rec) F(p);
     for (auto p : rpf) F(p);
-    F(dden); F(vpres); F(dden2); F(vpres2); F(gone); F(rowblk); F(idslot); F(rmids); F(cell); F(key); F(slot); F(cnt); F(start); F(perm); F(pid); F(bsum);
+    F(dden); F(vpres); F(dden2); F(vpres2); F(gone); F(idslot); F(rmids); F(cell); F(key); F(slot); F(cnt); F(start); F(perm); F(pid); F(bsum);
     F(work); F(nwork);
     F(nbr); F(nnb); F(bn); F(bt); F(scal); F(iscal); F(dtmin); F(pairs);
     F(mon_icont); F(mon_pts); F(mon_out);
@@ -516,7 +492,6 @@ int sph_ctx::alloc() {
     HIPC(da(&cnt, m));
     HIPC(da(&start, m + 1));
     HIPC(da(&bsum, (m + 1023) / 1024 + 1));
-    HIPC(da(&rowblk, (size_t)nrows + 1));
     HIPC(da(&idslot, N));
     HIPC(da(&rmids, RM_CAP * ns));
     HIPC(da(&nbr, N * (size_t)nb_stride(nb_stride_max)));
@@ -526,9 +501,9 @@ int sph_ctx::alloc() {
     HIPC(da(&scal, SC_COUNT * ns));
     HIPC(da(&iscal, IS_COUNT * ns));
     HIPC(da(&dtmin, ns));
-    HIPC(da(&pairs, 1));
+    HIPC(da(&pairs, NBC_PAIRS * NBC_PSTRIDE));
     if (dry) return 0;
-    HIPC(hipMemset(pairs, 0, sizeof(unsigned long long)));
+    HIPC(hipMemset(pairs, 0, sizeof(unsigned long long) * NBC_PAIRS * NBC_PSTRIDE));
     HIPC(hipMemset(acc[0], 0, sizeof(double4) * N));
     HIPC(hipMemset(acc[1], 0, sizeof(double4) * N));
     HIPC(hipMemset(lam[0], 0, sizeof(int) * N));
@@ -668,15 +643,15 @@ int fill_dp(const sph_params* p, const sph_faces* f, DP& P, bool dry = false) {
 
 inline int round256(long long v) { return (int)((v + 255) / 256 * 256); }
 
-// Places nseg solves in one context: slots, keys and rows of segment s follow
+// Places nseg solves in one context: slots and keys of segment s follow
 // those of segment s-1 (slots and keys in whole 256-blocks).  One solve keeps
 // its own sizes.  Fills c->P (segment 0 with the context capacity), c->segs,
-// nkeys, nrows, nseg and the list stride; allocates nothing.
+// nkeys, nseg and the list stride; allocates nothing.
 int layout_segments(sph_ctx* c, int nseg, const sph_params* p, const sph_faces* const* f = nullptr,
                     bool dry = false) {
     c->nseg = nseg;
     c->segs.assign(nseg, DP{});
-    long long slots = 0, keys = 0, rows = 0, faces = 0, edges = 0;
+    long long slots = 0, keys = 0, faces = 0, edges = 0;
     int nmaxpartj = 0;
     for (int s = 0; s < nseg; ++s) {
         const sph_faces* fs = f ? f[s] : nullptr;
@@ -688,7 +663,6 @@ int layout_segments(sph_ctx* c, int nseg, const sph_params* p, const sph_faces* 
         P.seg = s;
         P.base = (int)slots;
         P.koff = (int)keys;
-        P.roff = (int)rows;
         P.foff = (int)faces;
         P.eoff = (int)edges;
         if (nseg == 1) {
@@ -698,7 +672,6 @@ int layout_segments(sph_ctx* c, int nseg, const sph_params* p, const sph_faces* 
             slots += round256(P.scap);
             keys += round256((long long)P.nmax + 1);
         }
-        rows += (long long)P.ncd[1] * P.ncd[2];
         faces += P.nf;
         edges += P.ne;
         nmaxpartj = std::max(nmaxpartj, P.nmaxpartj);
@@ -708,7 +681,6 @@ int layout_segments(sph_ctx* c, int nseg, const sph_params* p, const sph_faces* 
     for (auto& P : c->segs) P.cap = (int)slots;
     c->P = c->segs[0];
     c->nkeys = (int)keys;
-    c->nrows = (int)rows;
     c->nb_stride_max = nmaxpartj;
     return 0;
 }
@@ -733,26 +705,7 @@ int setup_launch(sph_ctx* c, const sph_params* p) {
     if (c->nseg > 1)  // the segmented pair passes are built for whole-group walks
         c->chunk = c->chunk_v = c->chunk_c = c->chunk_p = 8;
     c->bt_grid = 4 * ncu;
-    // persistent neighbour-search workgroups: as many as fit a CU (LDS
-    // tile), times the CUs, a multiple of the 8 XCDs
-    c->nb_shape = p->nb_shape;
-    if (c->nb_shape < 0 || c->nb_shape >= NB_NSHAPES) return fail(2, "nb_shape must be 0 to 4");
-    if (NB_SHAPES[c->nb_shape].tk == NB_T16)  // FP16 keeps its relative precision for cells of 1e-4..1e4 m
-        for (const auto& Q : c->segs)
-            for (int d = 0; d < 3; ++d)
-                if (!(Q.dcd[d] >= 1.0e-4 && Q.dcd[d] <= 1.0e4)) c->nb_shape = 1;
-    int per_cu = 0;
-    hipError_t oe;
-    const int nwg = NB_SHAPES[c->nb_shape].wg;
-    switch (c->nb_shape) {
-        case 1: oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, NB_KERNEL(false, 1), nwg, 0); break;
-        case 2: oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, NB_KERNEL(false, 2), nwg, 0); break;
-        case 3: oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, NB_KERNEL(false, 3), nwg, 0); break;
-        case 4: oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, NB_KERNEL(false, 4), nwg, 0); break;
-        default: oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, NB_KERNEL(false, 0), nwg, 0); break;
-    }
-    if (oe != hipSuccess || per_cu <= 0) per_cu = 3;
-    c->nb_grid = (per_cu * ncu + 7) / 8 * 8;
+    if (p->nb_shape < 0 || p->nb_shape > 4) return fail(2, "nb_shape must be 0 to 4");
     return 0;
 }
 
@@ -863,17 +816,16 @@ int upload_tables(sph_ctx* c, const sph_faces* const* f) {
 }
 
 // Segment maps of a segmented context: per-segment constants, segment of
-// every 256-slot block, 256-key block and cell row.
+// every 256-slot block and 256-key block.
 int upload_segment_maps(sph_ctx* c) {
     if (c->nseg == 1) return 0;
-    std::vector<int> pblk(c->P.cap / 256), kblk(c->nkeys / 256), rseg(c->nrows);
+    std::vector<int> pblk(c->P.cap / 256), kblk(c->nkeys / 256);
     for (int s = 0; s < c->nseg; ++s) {
         const DP& P = c->segs[s];
         const int sb = (s + 1 < c->nseg ? c->segs[s + 1].base : c->P.cap);
         for (int b = P.base / 256; b < sb / 256; ++b) pblk[b] = s;
         const int ke = (s + 1 < c->nseg ? c->segs[s + 1].koff : c->nkeys);
         for (int b = P.koff / 256; b < ke / 256; ++b) kblk[b] = s;
-        for (int r = 0; r < P.ncd[1] * P.ncd[2]; ++r) rseg[P.roff + r] = s;
     }
     bool ok = hipMalloc(&c->d_P, sizeof(DP) * c->nseg) == hipSuccess &&
               hipMemcpy(c->d_P, c->segs.data(), sizeof(DP) * c->nseg, hipMemcpyHostToDevice) == hipSuccess &&
@@ -881,11 +833,9 @@ int upload_segment_maps(sph_ctx* c) {
               hipMemcpy(c->d_pblk, pblk.data(), sizeof(int) * pblk.size(), hipMemcpyHostToDevice) == hipSuccess &&
               hipMalloc(&c->d_kblk, sizeof(int) * kblk.size()) == hipSuccess &&
               hipMemcpy(c->d_kblk, kblk.data(), sizeof(int) * kblk.size(), hipMemcpyHostToDevice) == hipSuccess &&
-              hipMalloc(&c->d_rseg, sizeof(int) * rseg.size()) == hipSuccess &&
-              hipMemcpy(c->d_rseg, rseg.data(), sizeof(int) * rseg.size(), hipMemcpyHostToDevice) == hipSuccess &&
               hipMalloc(&c->d_adj, sizeof(int) * c->nseg) == hipSuccess;
     if (!ok) return fail(102, "device allocation/copy of the segment maps failed");
-    c->S = Seg{c->d_P, c->d_pblk, c->d_kblk, c->d_rseg, c->nseg, c->nrows};
+    c->S = Seg{c->d_P, c->d_pblk, c->d_kblk, c->nseg};
     return 0;
 }
 
@@ -1511,7 +1461,10 @@ int sph_free_surface(sph_ctx* c, double* pelolib, double* zlft) {
 int sph_pair_counter(sph_ctx* c, unsigned long long* total) {
     if (!c || !total) return fail(1, "null argument");
     HIPC(hipStreamSynchronize(c->stream));
-    HIPC(hipMemcpy(total, c->pairs, sizeof(unsigned long long), hipMemcpyDeviceToHost));
+    unsigned long long part[NBC_PAIRS * NBC_PSTRIDE];
+    HIPC(hipMemcpy(part, c->pairs, sizeof(part), hipMemcpyDeviceToHost));
+    *total = 0;
+    for (int q = 0; q < NBC_PAIRS; ++q) *total += part[q * NBC_PSTRIDE];
     return 0;
 }
 

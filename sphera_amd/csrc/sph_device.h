@@ -70,7 +70,6 @@ struct DP {
     int scap;  // slots reserved for the segment
     int koff;  // first cell key: keys koff .. koff+nmax-1 are the cells, koff+nmax the
                // particles out of the grid (a multiple of 256)
-    int roff;  // first cell row (fixed j, k) of the segment in the context's row list
     int foff;  // first frontier face of the segment in the context's face array
     int eoff;  // first convex edge of the segment in the context's edge array
     int ne;    // its convex edges (NumBEdges)
@@ -82,15 +81,13 @@ struct DP {
 };
 
 // Segment maps of a segmented context, passed by value to the kernels that
-// take a segmented form.  Slots, keys and rows are partitioned in whole
-// 256-blocks (slots, keys) or whole rows, so a workgroup of a particle or key
-// kernel lies in one segment.
+// take a segmented form.  Slots and keys are partitioned in whole 256-blocks,
+// so a workgroup of a particle or key kernel lies in one segment.
 struct Seg {
     const DP* P;        // per-segment constants
     const int* pblk;    // segment of each 256-slot block
     const int* kblk;    // segment of each 256-key block
-    const int* rseg;    // segment of each cell row
-    int nseg, nrows;
+    int nseg;
 };
 
 // one convex frontier edge (BoundaryConvexEdge, FindBoundaryConvexEdges3D.f90):

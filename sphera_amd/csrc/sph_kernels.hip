@@ -17,7 +17,6 @@
 // FP64 kernels are compiled with -ffp-contract=off and evaluate every
 // expression in the order of the cited reference line, so sums over a list in
 // the reference's order reproduce the reference's values.
-#include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -539,37 +538,16 @@ __global__ void k_gather(DP P0, Seg S, const int* __restrict__ perm, const int* 
 // |x - corner| <= dcd, so the FP32 separation is within ~5e-7 dcd per axis and
 // the FP32 r^2 within ~1.5e-6 relative of (2h)^2 near the cut-off.)
 // ----------------------------------------------------------------------------
-// List writer of one lane.  SPH_NB_BUF = 4 (default) or 8: the entries are
-// collected in a shift register of that many registers and stored as one
-// 16-byte (two for 8) vector store per full run, so the lane's list reaches
-// L2 in whole 16/32-byte pieces instead of one 4-byte store per entry; flush()
-// stores the last, partial run (its unused tail slots are past the count and
-// never read).  A run is stored only while it lies inside the particle's
-// list capacity (nb_stride(NMAXPARTJ)); the count keeps running, so the first
-// NMAXPARTJ entries are the stored ones, as in the reference.  SPH_NB_BUF = 0:
-// one 4-byte store per entry.
-#ifndef SPH_NB_BUF
-#define SPH_NB_BUF 4
-#endif
-#if SPH_NB_BUF == 0
+// List writer of one lane (cells too dense for the wavefront form below): the
+// entries are collected in a shift register of four and stored as one 16-byte
+// vector per full run; flush() stores the last, partial run (its unused tail
+// slots are past the count and never read).  A run is stored only while it
+// lies inside the particle's list capacity (nb_stride(NMAXPARTJ)); the count
+// keeps running, so the first NMAXPARTJ entries are the stored ones, as in
+// the reference.
+static_assert(NB_G == 8, "the list writer stores runs inside 8-entry groups");
 struct NbOut {
-    uint32_t* wp;
-    int cnt;
-    size_t jump;  // N*NB_G - (NB_G-1): from the last entry of a group to the first of the next
-    __device__ __forceinline__ NbOut(uint32_t* nbr, size_t N, int p, int)
-        : wp(nbr + nb_index(N, p, 0)), cnt(0), jump(N * NB_G - (NB_G - 1)) {}
-    __device__ __forceinline__ void push(uint32_t e, int mj) {
-        if (cnt < mj) *wp = e;
-        ++cnt;
-        wp += ((cnt & (NB_G - 1)) == 0) ? jump : (size_t)1;
-    }
-    __device__ __forceinline__ void flush() {}
-};
-#else
-static_assert(SPH_NB_BUF == 4 || SPH_NB_BUF == 8, "SPH_NB_BUF is 0, 4 or 8");
-static_assert(NB_G == 8, "the buffered list writer stores runs inside 8-entry groups");
-struct NbOut {
-    static constexpr int B = SPH_NB_BUF;
+    static constexpr int B = 4;
     uint32_t* wp;  // first slot of the current run
     int cnt;
     int lim;       // list capacity: runs ending past it are not stored
@@ -583,7 +561,6 @@ struct NbOut {
     __device__ __forceinline__ void store_run() {
         uint4* q = reinterpret_cast<uint4*>(wp);
         q[0] = make_uint4(b[0], b[1], b[2], b[3]);
-        if constexpr (B == 8) q[1] = make_uint4(b[4], b[5], b[6], b[7]);
     }
     __device__ __forceinline__ void push(uint32_t e, int) {
 #pragma unroll
@@ -613,7 +590,6 @@ struct NbOut {
         store_run();
     }
 };
-#endif
 
 // The neighbour test of one candidate and the list append: FP32 on
 // cell-relative positions, and the reference's FP64 expression on the FP64
@@ -624,22 +600,10 @@ struct NbOut {
 // exact one, far inside the 4e-5 band.  Every accepted candidate is counted;
 // the first NMAXPARTJ are stored (the reference keeps the first NMAXPARTJ of
 // its list, CalcVarLength.f90:200-207), so the loops have no early exit.
-// Q: xj holds the candidate's 16-bit fixed-point coordinates (0..65535 over
-// the cell), decoded with the per-axis step sc in one fused multiply-add.
-template <bool Q = false>
 __device__ __forceinline__ void nb_test(const DP& P, const double4* __restrict__ xm, double4 xi64,
                                         float4 xo, float4 xj, int m, uint32_t ctag, float lo, float hi,
-                                        NbOut& w, int mj, float4 sc = float4{}) {
-    float r0, r1, r2;
-    if constexpr (Q) {
-        r0 = __builtin_fmaf(xj.x, -sc.x, xo.x);
-        r1 = __builtin_fmaf(xj.y, -sc.y, xo.y);
-        r2 = __builtin_fmaf(xj.z, -sc.z, xo.z);
-    } else {
-        r0 = xo.x - xj.x;
-        r1 = xo.y - xj.y;
-        r2 = xo.z - xj.z;
-    }
+                                        NbOut& w, int mj) {
+    const float r0 = xo.x - xj.x, r1 = xo.y - xj.y, r2 = xo.z - xj.z;
     const float r2f = __builtin_fmaf(r0, r0, __builtin_fmaf(r1, r1, r2 * r2));
     if (r2f <= hi) {
         bool acc = r2f < lo;
@@ -656,22 +620,21 @@ __device__ __forceinline__ void nb_test(const DP& P, const double4* __restrict__
 }
 
 // Candidates [b,e) of one stencil cell, four loads ahead: load(x) gives the
-// FP32 position of slot x, gl + x its sorted index.
-template <bool Q = false, class Load>
+// FP32 position of slot x.
+template <class Load>
 __device__ __forceinline__ void nb_cell(const DP& P, const double4* __restrict__ xm, double4 xi64,
-                                        float4 xi, float4 o, uint32_t ctag, int b, int e, int gl,
-                                        Load&& load, float lo, float hi, NbOut& w, int mj,
-                                        float4 sc = float4{}) {
+                                        float4 xi, float4 o, uint32_t ctag, int b, int e,
+                                        Load&& load, float lo, float hi, NbOut& w, int mj) {
     const float4 xo = make_float4(xi.x - o.x, xi.y - o.y, xi.z - o.z, 0.0f);
     int x = b;
     for (; x + 4 <= e; x += 4) {
         const float4 q0 = load(x), q1 = load(x + 1), q2 = load(x + 2), q3 = load(x + 3);
-        nb_test<Q>(P, xm, xi64, xo, q0, gl + x, ctag, lo, hi, w, mj, sc);
-        nb_test<Q>(P, xm, xi64, xo, q1, gl + x + 1, ctag, lo, hi, w, mj, sc);
-        nb_test<Q>(P, xm, xi64, xo, q2, gl + x + 2, ctag, lo, hi, w, mj, sc);
-        nb_test<Q>(P, xm, xi64, xo, q3, gl + x + 3, ctag, lo, hi, w, mj, sc);
+        nb_test(P, xm, xi64, xo, q0, x, ctag, lo, hi, w, mj);
+        nb_test(P, xm, xi64, xo, q1, x + 1, ctag, lo, hi, w, mj);
+        nb_test(P, xm, xi64, xo, q2, x + 2, ctag, lo, hi, w, mj);
+        nb_test(P, xm, xi64, xo, q3, x + 3, ctag, lo, hi, w, mj);
     }
-    for (; x < e; ++x) nb_test<Q>(P, xm, xi64, xo, load(x), gl + x, ctag, lo, hi, w, mj, sc);
+    for (; x < e; ++x) nb_test(P, xm, xi64, xo, load(x), x, ctag, lo, hi, w, mj);
 }
 
 // List of particle p from global memory (candidates gathered through L1/L2).
@@ -700,7 +663,7 @@ __device__ int nb_particle_global(const DP& P, int p, const double4* __restrict_
                 const int cn = ((kk - 1) * nj + (jj - 1)) * ni + ii;
                 const int code = (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1);
                 nb_cell(P, xm, xi64, xi, g_soff[code], (uint32_t)code << NB_SHIFT, start[P.koff + cn - 1],
-                        start[P.koff + cn], 0, load, lo, hi, w, mj);
+                        start[P.koff + cn], load, lo, hi, w, mj);
             }
         }
     }
@@ -709,275 +672,223 @@ __device__ int nb_particle_global(const DP& P, int p, const double4* __restrict_
     return min(w.cnt, mj);
 }
 
-// Tiled form.  The particles of one row of cells (fixed j,k; cells i are
-// contiguous in the sorted order, hence in memory) are cut into blocks of at
-// most NB_WG.  For a block over cells ia..ib the FP32 positions of the 9
-// neighbouring row segments (rows j+-1, k+-1 over cells ia-1..ib+1) are staged
-// in LDS once, and every lane walks its 27 stencil cells in the reference's
-// order out of LDS.  A block over more than NB_MAXC cells or with more than
-// NB_TILE candidates takes the global path above.  Persistent workgroups take
-// the blocks of one contiguous range per XCD.
-// Launch shapes of the tiled search (workgroup size, candidate tile, FP16
-// tile, register bound): the default 256 x 4096 FP16 (26 KB of LDS, 6 waves
-// per SIMD, registers held to 80 so that 6 fit) and three the autotuner may
-// pick instead: 256 x 3072 FP32 (36 KB,
-// 4 waves), 128 x 1536 FP32, and 256 x 2816 FP16 held to 64 registers for 8
-// waves per SIMD.
-constexpr int NB_WG = 256;
-constexpr int NB_MAXC = 48;
-constexpr int NB_TILE = 3072;
-// tk: tile coordinates in FP32 (NB_T32), FP16 (NB_T16) or 16-bit fixed point
-// over the cell (NB_TQ16); minb: workgroups per CU the registers must allow
-enum { NB_T32 = 0, NB_T16 = 1, NB_TQ16 = 2 };
-struct NbShape { int wg, tile; int tk; int minb; };
-constexpr int NB_NSHAPES = 5;
-constexpr NbShape NB_SHAPES[NB_NSHAPES] = {{256, 4096, NB_T16, 6},  {256, 3072, NB_T32, 1},
-                                           {128, 1536, NB_T32, 1},  {256, 2816, NB_T16, 8},
-                                           {256, 4096, NB_TQ16, 6}};
+// One wavefront per cell.  All particles of a cell share the candidates of its
+// 27 stencil cells (475 at 17.6 particles per cell), in the same order: the
+// lanes hold them in registers (candidate 64 q + lane in chunk q), relative
+// to the cell's corner, and the particles of the cell are taken one after the
+// other.  With c = |xj|^2 kept per candidate, the test
+// c - 2 xi.xj <= (2h)^2 - |xi|^2 is three fused multiply-adds and a compare
+// for 64 candidates; the hits of a chunk are a lane mask, so a hit's place in
+// the list is the count of mask bits below it, and the list is built in LDS
+// and stored in 16-byte pieces.  VALU issue bounds it: 8 instructions per 64
+// candidates, against 19 per candidate and lane (with the append in the
+// divergent branch of every test) for one lane per particle.
+// 576,000 particles: 219 -> 171 us; a batch of eight solves, 536,000: 334 -> 159;
+// 1,440 particles (one lane's 475 serial tests were the time): 71 -> 17 us.
+//
+// The FP32 test: a candidate's coordinates are within 2 dcd of the corner, so
+// with the rounding of the sums r^2 is within 3.5e-6 dcd^2; the guard band
+// 4e-5 (2h)^2 (wider for cells larger than 2h) goes to the FP64 test.
+// A wavefront takes the cells whose first particle lies in its NBC_SLOTS
+// sorted slots: about one cell, so small solves spread over the chip.
+// Cells with more candidates than the registers hold (denser than 1.35 times
+// water) take one lane per particle from global memory.
+constexpr int NBC_CH = 10;             // chunks of 64 candidates in registers
+constexpr int NBC_MAX = 64 * NBC_CH;
+constexpr int NBC_SLOTS = 16;          // sorted slots per wavefront
+constexpr int NBC_PAIRS = 64;          // pair counters, one 128-byte line each
+constexpr int NBC_PSTRIDE = 16;
 
-// rowblk[r] = first block of row r (exclusive scan of ceil(count_r / bw), bw
-// the search's workgroup size),
-// rowblk[R] = number of blocks.  One workgroup.  Segmented contexts: the rows
-// of all segments, each row read with its segment's grid.
-template <bool SG>
-__global__ __launch_bounds__(1024) void k_nb_rowblocks(DP P0, Seg S, const int* __restrict__ start,
-                                                       int* __restrict__ rowblk, int bw) {
-    __shared__ int wsum[16];
-    __shared__ int carry;
-    const int R = SG ? S.nrows : P0.ncd[1] * P0.ncd[2];
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int base = 0; base < R; base += 1024) {
-        const int r = base + threadIdx.x;
-        int v = 0;
-        if (r < R) {
-            const DP& P = SG ? S.P[S.rseg[r]] : P0;
-            const int ni = P.ncd[0];
-            const int rl = r - P.roff;
-            const int k0 = P.koff + rl * ni;
-            v = (start[k0 + ni] - start[k0] + bw - 1) / bw;
-        }
-        const int incl = wave_incl_scan(v);
-        const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        if (lane == 63) wsum[wid] = incl;
-        __syncthreads();
-        int woff = 0;
-        for (int w = 0; w < wid; ++w) woff += wsum[w];
-        const int c0 = carry;
-        if (r < R) rowblk[r] = c0 + woff + incl - v;
-        __syncthreads();
-        if (threadIdx.x == 1023) carry = c0 + woff + incl;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) rowblk[R] = carry;
+__device__ __forceinline__ float readlane_f(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// TK = NB_T16: the tile holds the candidates' cell-relative positions in FP16
-// (6 bytes each: more workgroups per CU).  A coordinate in [0, dcd] rounds by
-// at most 2^-11 dcd, so the FP32 r^2 from it is within ~2e-3 relative of the
-// exact one near (2h)^2; the FP64 guard band is widened to 5e-3 to keep the
-// lists exactly the reference's.  TK = NB_TQ16: 16-bit fixed point over the
-// cell instead (q = rint(x 65535 / dcd), also 6 bytes): a coordinate rounds
-// by at most 2^-17 dcd, the FP32 r^2 is within ~2.8e-5 (dcd / 2h) relative of
-// the exact one near (2h)^2 (dcd / 2h < 1.5 on the reference's grid), and the
-// guard band is 2e-4, so the FP64 test runs 25 times less often.
-template <bool SG, int WG = NB_WG, int TILE = NB_TILE, int TK = NB_T32, int MINB = 1>
-__global__ __launch_bounds__(WG, MINB) void k_neighbours(DP P0, Seg S, const double4* __restrict__ xm,
-                                                      const float4* __restrict__ xmf,
-                                                      const int* __restrict__ cell,
-                                                      const int* __restrict__ start,
-                                                      const int* __restrict__ rowblk,
-                                                      uint32_t* __restrict__ nbr, int* __restrict__ nnb,
-                                                      int* iscal, unsigned long long* pairs) {
-    using TXY = typename std::conditional<TK == NB_T16, __half2,
-                                          typename std::conditional<TK == NB_TQ16, uint32_t, float2>::type>::type;
-    using TZ = typename std::conditional<TK == NB_T16, __half,
-                                         typename std::conditional<TK == NB_TQ16, uint16_t, float>::type>::type;
-    constexpr bool Q = TK == NB_TQ16;
-    __shared__ TXY tile_xy[TILE];  // staged candidates: (x, y) and z, 12 (FP16: 6) bytes each
-    __shared__ TZ tile_z[TILE];
-    __shared__ int bnd[9][NB_MAXC + 4];  // LDS offset of the start of cell ia-1+u of row t
-    __shared__ int seg_g[9];             // sorted index of a segment's first particle
-    __shared__ int seg_l[9];             // its LDS offset
-    __shared__ int seg_n[9];
-    __shared__ int s_row, s_ia, s_ib, s_p0, s_p1, s_global, s_seg;
-    if (!SG) stencil_offsets(P0);
-    int cur_seg = -1;
-    const int R = SG ? S.nrows : P0.ncd[1] * P0.ncd[2];
-    const int nblocks = rowblk[R];
-    const int per_xcd = gridDim.x >> 3;  // gridDim.x is a multiple of 8
-    const int xcd = blockIdx.x & 7;
-    const int b_lo = (int)((long long)nblocks * xcd / 8), b_hi = (int)((long long)nblocks * (xcd + 1) / 8);
-    unsigned long long mypairs = 0;
-    for (int blk = b_lo + (blockIdx.x >> 3); blk < b_hi; blk += per_xcd) {
-        if (threadIdx.x == 0) {
-            // row of the block: last r with rowblk[r] <= blk
-            int a = 0, b = R;  // rowblk[a] <= blk < rowblk[b]
-            while (b - a > 1) {
-                const int m = (a + b) >> 1;
-                if (rowblk[m] <= blk) a = m;
-                else b = m;
-            }
-            const int r = a;
-            const int sg0 = SG ? S.rseg[r] : 0;
-            const DP& Q = SG ? S.P[sg0] : P0;
-            const int rl = r - Q.roff;  // the row in its segment's grid
-            const int qi = Q.ncd[0];
-            const int p0 = start[Q.koff + rl * qi] + (blk - rowblk[r]) * WG;
-            const int p1 = min(p0 + WG, start[Q.koff + (rl + 1) * qi]);
-            const int ia = cell[p0] - rl * qi, ib = cell[p1 - 1] - rl * qi;
-            s_seg = sg0;
-            s_row = rl;
-            s_ia = ia;
-            s_ib = ib;
-            s_p0 = p0;
-            s_p1 = p1;
-            s_global = ib - ia + 1 > NB_MAXC;
-        }
-        __syncthreads();
-        const int sg = SG ? __builtin_amdgcn_readfirstlane(s_seg) : 0;
-        const DP& P = SG ? S.P[sg] : P0;
-        if (SG && sg != cur_seg) {  // the stencil offsets of this segment's grid
-            stencil_offsets(P);
-            cur_seg = sg;
-        }
-        const int ni = P.ncd[0], nj = P.ncd[1], nk = P.ncd[2];
-        const float sq = (float)P.square_doubleh;
-        const float lo = sq * (1.0f - 4.0e-5f), hi = sq * (1.0f + 4.0e-5f);
-        const float band = TK == NB_T16 ? 5.0e-3f : (Q ? 2.0e-4f : 4.0e-5f);  // guard band of the tiled test
-        // fixed-point step per axis (NB_TQ16) and its inverse for the staging
-        const float4 qs = make_float4(P.f_dcd[0] * (1.0f / 65535.0f), P.f_dcd[1] * (1.0f / 65535.0f),
-                                      P.f_dcd[2] * (1.0f / 65535.0f), 0.0f);
-        const float4 qi = make_float4(65535.0f / P.f_dcd[0], 65535.0f / P.f_dcd[1], 65535.0f / P.f_dcd[2], 0.0f);
-        const float tlo = sq * (1.0f - band), thi = sq * (1.0f + band);
-        const int mj = P.nmaxpartj;
-        const size_t N = P.cap;
-        const int r = s_row, ia = s_ia, ib = s_ib, p0 = s_p0, p1 = s_p1;
-        const int jc = r % nj + 1, kc = r / nj + 1;
-        const int ca = max(ia - 1, 1), cb = min(ib + 1, ni);
-        if (!s_global) {
-            if (threadIdx.x < 9) {
-                const int t = threadIdx.x;
-                const int jj = jc + t / 3 - 1, kk = kc + t % 3 - 1;
-                int g0 = 0, g1 = 0;
-                if (jj >= 1 && jj <= nj && kk >= 1 && kk <= nk) {
-                    const int rb = P.koff + ((kk - 1) * nj + (jj - 1)) * ni;
-                    g0 = start[rb + ca - 1];
-                    g1 = start[rb + cb];
-                }
-                seg_g[t] = g0;
-                seg_n[t] = g1 - g0;
-            }
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                int off = 0;
-                for (int t = 0; t < 9; ++t) {
-                    seg_l[t] = off;
-                    off += seg_n[t];
-                }
-                s_global = off > TILE;
-            }
-            __syncthreads();
-        }
-        const int p = p0 + threadIdx.x;
-        if (!s_global) {
-            // cell boundaries inside the tile: u = 0 .. ib-ia+3 is the start of cell
-            // ia-1+u (cells ia-1 .. ib+1, and the end of ib+1)
-            const int nu = ib - ia + 4;
-            for (int x = threadIdx.x; x < 9 * nu; x += WG) {
-                const int t = x / nu, u = x % nu;
-                const int jj = jc + t / 3 - 1, kk = kc + t % 3 - 1;
-                const int ii = ia - 1 + u;
-                int v;
-                if (jj < 1 || jj > nj || kk < 1 || kk > nk || ii < ca) v = seg_l[t];
-                else if (ii > cb) v = seg_l[t] + seg_n[t];
-                else v = seg_l[t] + start[P.koff + ((kk - 1) * nj + (jj - 1)) * ni + ii - 1] - seg_g[t];
-                bnd[t][u] = v;
-            }
-            // stage the candidates' FP32 positions, four loads in flight per thread
-            {
-                const int total = seg_l[8] + seg_n[8];
-                for (int e0 = threadIdx.x; e0 < total; e0 += 4 * WG) {
-                    float4 v[4];
-                    int dst[4];
+// The cell's particles hb .. hb+hc-1 against its `total` candidates, NCH chunks
+// of 64 (64 (NCH-1) < total <= 64 NCH).  A lane without a hit writes to the
+// slot past the list, so a chunk's append has no branch.  Returns the sum of
+// the list lengths without the particles themselves; over counts truncated lists.
+template <int NCH>
+__device__ __forceinline__ int nb_cell_lists(const DP& P, const double4* __restrict__ xm,
+                                             const float4* __restrict__ xmf, const uint32_t* cand,
+                                             uint32_t* list, int total, int hb, int hc, float lo, float hi,
+                                             uint32_t* __restrict__ nbr, int* __restrict__ nnb, int& over) {
+    const int lane = threadIdx.x & 63;
+    const int mj = P.nmaxpartj, stride = nb_stride(mj);
+    const size_t N = P.cap;
+    float cx[NCH], cy[NCH], cz[NCH], cq[NCH];
+    uint32_t ce[NCH];
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const int e = e0 + u * WG;
-                        dst[u] = -1;
-                        if (e < total) {
-                            int t = 0;
+    for (int q = 0; q < NCH; ++q) {
+        const int f = 64 * q + lane;
+        ce[q] = f < total ? cand[f] : (uint32_t)hb;
+    }
 #pragma unroll
-                            for (int q = 1; q < 9; ++q) t += e >= seg_l[q];
-                            v[u] = xmf[seg_g[t] + (e - seg_l[t])];
-                            dst[u] = e;
-                        }
+    for (int q = 0; q < NCH; ++q) {
+        const float4 x = xmf[ce[q] & NB_MASK];
+        const float4 o = g_soff[ce[q] >> NB_SHIFT];
+        cx[q] = x.x + o.x;
+        cy[q] = x.y + o.y;
+        cz[q] = x.z + o.z;
+        const float r2 = __builtin_fmaf(cx[q], cx[q], __builtin_fmaf(cy[q], cy[q], cz[q] * cz[q]));
+        cq[q] = 64 * q + lane < total ? r2 : 3.0e38f;
+    }
+    int pairs = 0;
+    for (int h0 = 0; h0 < hc; h0 += 64) {
+        // the lane's own particle of the cell, as it enters the test
+        float mx = 0.f, my = 0.f, mz = 0.f, tl = 0.f, th = 0.f;
+        if (h0 + lane < hc) {
+            const float4 x = xmf[hb + h0 + lane];
+            const float r2 = __builtin_fmaf(x.x, x.x, __builtin_fmaf(x.y, x.y, x.z * x.z));
+            mx = -2.0f * x.x;
+            my = -2.0f * x.y;
+            mz = -2.0f * x.z;
+            tl = lo - r2;
+            th = hi - r2;
+        }
+        const int hn = min(64, hc - h0);
+        int mine = 0;  // list length of the lane's own particle
+        for (int u = 0; u < hn; ++u) {
+            const int p = hb + h0 + u;
+            const float ax = readlane_f(mx, u), ay = readlane_f(my, u), az = readlane_f(mz, u);
+            const float al = readlane_f(tl, u), ah = readlane_f(th, u);
+            auto r2of = [&](int q) {
+                return __builtin_fmaf(ax, cx[q], __builtin_fmaf(ay, cy[q], __builtin_fmaf(az, cz[q], cq[q])));
+            };
+            unsigned long long guard = 0ull;
+            int k = 0;
+            auto append = [&](int q, bool in) {
+                const unsigned long long m = __ballot(in);
+                const int at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)m, k));
+                list[in ? at : NBC_MAX] = ce[q];
+                k += __popcll(m);
+                return m;
+            };
+#pragma unroll
+            for (int q = 0; q < NCH; ++q) {
+                const float r2 = r2of(q);
+                guard |= __ballot(r2 <= ah) ^ append(q, r2 < al);
+            }
+            if (guard) {  // candidates in the guard band (1 particle in 100): the reference's FP64 test
+                const double4 xi = xm[p];
+                k = 0;
+#pragma unroll
+                for (int q = 0; q < NCH; ++q) {
+                    const float r2 = r2of(q);
+                    bool in = r2 < al;
+                    if (!in && r2 <= ah) {
+                        const double4 xj = xm[ce[q] & NB_MASK];
+                        const double d0 = xi.x - xj.x;
+                        const double d1 = xi.y - xj.y;
+                        const double d2 = xi.z - xj.z;
+                        in = !(d0 * d0 + d1 * d1 + d2 * d2 > P.square_doubleh);
                     }
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        if (dst[u] >= 0) {
-                            if constexpr (TK == NB_T16) {
-                                tile_xy[dst[u]] = __floats2half2_rn(v[u].x, v[u].y);
-                                tile_z[dst[u]] = __float2half_rn(v[u].z);
-                            } else if constexpr (Q) {
-                                auto q16 = [](float a) {  // 0 <= a <= 65535 (+ rounding)
-                                    return (uint32_t)__float2uint_rn(fminf(fmaxf(a, 0.0f), 65535.0f));
-                                };
-                                tile_xy[dst[u]] = q16(v[u].x * qi.x) | (q16(v[u].y * qi.y) << 16);
-                                tile_z[dst[u]] = (uint16_t)q16(v[u].z * qi.z);
-                            } else {
-                                tile_xy[dst[u]] = make_float2(v[u].x, v[u].y);
-                                tile_z[dst[u]] = v[u].z;
-                            }
-                        }
+                    append(q, in);
                 }
             }
-            __syncthreads();
-            if (p < p1) {
-                const int ucell = cell[p] - r * ni - ia + 1;  // u index of the own cell
-                const float4 xi = xmf[p];
-                const double4 xi64 = xm[p];
-                NbOut w(nbr, N, p, nb_stride(mj));
-                auto load = [&](int x) {
-                    if constexpr (TK == NB_T16) {
-                        const float2 a = __half22float2(tile_xy[x]);
-                        return make_float4(a.x, a.y, __half2float(tile_z[x]), 0.0f);
-                    } else if constexpr (Q) {
-                        const uint32_t a = tile_xy[x];
-                        return make_float4((float)(a & 0xFFFFu), (float)(a >> 16), (float)tile_z[x], 0.0f);
-                    } else {
-                        const float2 a = tile_xy[x];
-                        return make_float4(a.x, a.y, tile_z[x], 0.0f);
-                    }
-                };
-                for (int dy = 0; dy < 3; ++dy)
-                    for (int dx = 0; dx < 3; ++dx)
-                        for (int dz = 0; dz < 3; ++dz) {
-                            const int t = 3 * dy + dz;
-                            const int code = dx + 3 * dy + 9 * dz;
-                            nb_cell<Q>(P, xm, xi64, xi, g_soff[code], (uint32_t)code << NB_SHIFT,
-                                       bnd[t][ucell + dx - 1], bnd[t][ucell + dx], seg_g[t] - seg_l[t], load,
-                                       tlo, thi, w, mj, qs);
-                        }
-                w.flush();
-                const bool ov = w.cnt > mj;
-                const int cnt = min(w.cnt, mj);
-                nnb[p] = cnt;
-                mypairs += (unsigned long long)(cnt - 1);
-                if (ov) atomicAdd(&iscal[sg * IS_COUNT + IS_NB_OVERFLOW], 1);
-            }
-        } else if (p < p1) {
-            bool ov;
-            const int cnt = nb_particle_global(P, p, xm, xmf, cell, start, nbr, lo, hi, ov);
-            nnb[p] = cnt;
-            mypairs += (unsigned long long)(cnt - 1);
-            if (ov) atomicAdd(&iscal[sg * IS_COUNT + IS_NB_OVERFLOW], 1);
+            __builtin_amdgcn_wave_barrier();
+            for (int e = 4 * lane, ke = min(k, stride); e < ke; e += 256)
+                *reinterpret_cast<uint4*>(nbr + nb_index(N, p, e)) = *reinterpret_cast<const uint4*>(list + e);
+            __builtin_amdgcn_wave_barrier();
+            const int kn = min(k, mj);
+            mine = lane == u ? kn : mine;
+            pairs += kn - 1;
+            over += k > mj;
         }
-        __syncthreads();  // the tile and the block descriptors are reused
+        if (lane < hn) nnb[hb + h0 + lane] = mine;
+    }
+    return pairs;
+}
+
+template <bool SG>
+__global__ __launch_bounds__(256, 4) void k_neighbours(DP P0, Seg S, const double4* __restrict__ xm,
+                                                    const float4* __restrict__ xmf,
+                                                    const int* __restrict__ cell,
+                                                    const int* __restrict__ start,
+                                                    uint32_t* __restrict__ nbr, int* __restrict__ nnb,
+                                                    int* iscal, unsigned long long* pairs) {
+    __shared__ uint32_t s_cand[4][NBC_MAX];                // a wave's candidates: sorted index | stencil code
+    __shared__ __align__(16) uint32_t s_list[4][NBC_MAX + 4];  // the list of its current particle
+    __shared__ int s_pairs[4];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int vb = xcd_block(gridDim.x);
+    const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * 4 * NBC_SLOTS) >> 8]) : 0;
+    const DP& P = SG ? S.P[sg] : P0;
+    iscal += sg * IS_COUNT;
+    const int n = iscal[IS_N];
+    if (vb * 4 * NBC_SLOTS - P.base >= n) return;
+    stencil_offsets(P);
+    const int ni = P.ncd[0], nj = P.ncd[1], nk = P.ncd[2];
+    const float sq = (float)P.square_doubleh;
+    const float dm = fmaxf(P.f_dcd[0], fmaxf(P.f_dcd[1], P.f_dcd[2]));
+    const float band = 4.0e-5f * fmaxf(1.0f, dm * dm / sq);
+    const float lo = sq * (1.0f - band), hi = sq * (1.0f + band);
+    const int s0 = (vb * 4 + wid) * NBC_SLOTS;
+    uint32_t* cand = s_cand[wid];
+    uint32_t* list = s_list[wid];
+    int mypairs = 0, over = 0;
+    int cl = 0;
+    bool first = false;  // the lane's slot starts a cell
+    if (lane < NBC_SLOTS && s0 + lane - P.base < n) {
+        cl = cell[s0 + lane];
+        first = s0 + lane == P.base || cell[s0 + lane - 1] != cl;
+    }
+    unsigned long long todo = __ballot(first);
+    while (todo) {
+        const int l = __ffsll((long long)todo) - 1;
+        todo &= todo - 1ull;
+        int ic, jc, kc;
+        d_cell_indices(P, __builtin_amdgcn_readlane(cl, l), ic, jc, kc);
+        // lane t: the t-th stencil cell in the order dy, dx, dz
+        int b = 0, cnt = 0;
+        uint32_t tag = 0u;
+        if (lane < 27) {
+            const int dy = lane / 9 - 1, dx = (lane / 3) % 3 - 1, dz = lane % 3 - 1;
+            const int ii = ic + dx, jj = jc + dy, kk = kc + dz;
+            if (ii >= 1 && ii <= ni && jj >= 1 && jj <= nj && kk >= 1 && kk <= nk) {
+                const int key = P.koff + ((kk - 1) * nj + (jj - 1)) * ni + ii - 1;
+                b = start[key];
+                cnt = start[key + 1] - b;
+                tag = (uint32_t)((dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)) << NB_SHIFT;
+            }
+        }
+        const int incl = wave_incl_scan(cnt);
+        const int total = __builtin_amdgcn_readlane(incl, 63);
+        const int hb = __builtin_amdgcn_readlane(b, 13), hc = __builtin_amdgcn_readlane(cnt, 13);
+        if (total > NBC_MAX) {
+            for (int q = lane; q < hc; q += 64) {
+                bool ov;
+                const int k = nb_particle_global(P, hb + q, xm, xmf, cell, start, nbr, lo, hi, ov);
+                nnb[hb + q] = k;
+                if (ov) atomicAdd(&iscal[IS_NB_OVERFLOW], 1);
+                atomicAdd(&pairs[(vb % NBC_PAIRS) * NBC_PSTRIDE], (unsigned long long)(k - 1));
+            }
+            continue;
+        }
+        for (int u = 0, pre = incl - cnt; u < cnt; ++u) cand[pre + u] = (uint32_t)(b + u) | tag;
+        __builtin_amdgcn_wave_barrier();
+        switch ((total + 63) >> 6) {
+            case 1: mypairs += nb_cell_lists<1>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+            case 2: mypairs += nb_cell_lists<2>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+            case 3: mypairs += nb_cell_lists<3>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+            case 4: mypairs += nb_cell_lists<4>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+            case 5: mypairs += nb_cell_lists<5>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+            case 6: mypairs += nb_cell_lists<6>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+            case 7: mypairs += nb_cell_lists<7>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+            case 8: mypairs += nb_cell_lists<8>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+            case 9: mypairs += nb_cell_lists<9>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+            case 10: mypairs += nb_cell_lists<10>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+        }
     }
     // pair-interaction counter: sum_i (nPartIntorno(i) - 1), self excluded
-    unsigned long long v = mypairs;
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((threadIdx.x & 63) == 0 && v) atomicAdd(pairs, v);
+    if (lane == 0) {
+        s_pairs[wid] = mypairs;
+        if (over) atomicAdd(&iscal[IS_NB_OVERFLOW], over);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+        atomicAdd(&pairs[(vb % NBC_PAIRS) * NBC_PSTRIDE],
+                  (unsigned long long)((long long)s_pairs[0] + s_pairs[1] + s_pairs[2] + s_pairs[3]));
 }
 
 // ----------------------------------------------------------------------------
