@@ -48,11 +48,9 @@ typedef struct sph_params {
     int32_t semi;        /* 1: SA-SPH frontiers active (Domain%tipo=="semi") */
     /* launch tunables of the particle kernels (0 = default; the autotuner in
      * sphera_amd/autotune.py picks them per case) */
-    int32_t wg_size;     /* threads per workgroup: 64 (default), 128, 192 or 256 */
-    int32_t chunk;       /* list entries gathered per step of the FP32 walks: 4 or 8 (default);
-                            momentum pass, and the others where theirs is 0 */
-    int32_t chunk_v, chunk_c, chunk_p; /* the same for velocity smoothing, continuity,
-                                          pressure smoothing (0 = chunk) */
+    int32_t wg_size;     /* threads per workgroup of the FP64 pair passes: 64 (default), 128, 192 or 256 */
+    int32_t chunk;       /* 4 or 8 (default), accepted for callers that set it, as are the next three: */
+    int32_t chunk_v, chunk_c, chunk_p; /* the list walks have one form each */
     int32_t nb_shape;    /* 0 to 4, accepted for callers that set it: the neighbour search has
                             one launch shape, and the lists never depended on it */
     int32_t options;     /* SPH_OPT_* flags of the deck (below) */

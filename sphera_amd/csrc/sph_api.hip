@@ -53,7 +53,7 @@ struct sph_ctx {
     std::vector<DP> segs;
     Seg S{};
     DP* d_P = nullptr;
-    int *d_pblk = nullptr, *d_kblk = nullptr, *d_adj = nullptr;
+    int *d_pblk = nullptr, *d_kblk = nullptr, *d_tblk = nullptr, *d_adj = nullptr;
     int nkeys = 1;             // cell keys (cells + out-of-grid bucket per segment)
     int nb_stride_max = 1;     // largest NMAXPARTJ of the segments (list capacity)
     std::vector<int> staged;   // segments uploaded since the last commit
@@ -71,18 +71,20 @@ struct sph_ctx {
     double4 *xm[2] = {}, *vel[3] = {}, *acc[2] = {};
     double2* rp[3] = {};
     int* lam[2] = {};
-    float4* xmf = nullptr;  // FP32 cell-relative positions (x, y, z, mass)
-    float4* xrf = nullptr;  // FP32 (x, y, z, rho - den0) after continuity, for the pressure smoothing
-    // FP32 record buffers, (position, velocity) float4 pairs per particle:
-    // [0] read by momentum and continuity, [1] by velocity smoothing
-    float4* rec[2] = {};
-    float2* rpf[3] = {};
+    int4* xq = nullptr;     // integer positions (x, y, z in P.lsb, mass as float bits)
+    float* dr = nullptr;    // FP32 rho - den0 after continuity, for the pressure smoothing
+    // FP32 (vx, vy, vz, rho - den0): [0] read by momentum and continuity, [1]
+    // (written by momentum) by velocity smoothing
+    float4* vf[2] = {};
     double *dden = nullptr, *vpres = nullptr;
     // explicit RK1: dden and vpres in the order after the step's closing sort
     double *dden2 = nullptr, *vpres2 = nullptr;
     int* gone = nullptr;  // 1: the last trajectory step left through an open face
     int *cell = nullptr, *key = nullptr, *slot = nullptr, *cnt = nullptr, *start = nullptr,
         *perm = nullptr, *pid = nullptr, *bsum = nullptr;
+    int *tlist = nullptr, *ntile = nullptr;  // the tiles that hold particles, their number
+    int ntiles = 0;                          // tile ids of all segments (whole 256-blocks)
+    int tile_cap = 0, tile_grid = 8, tile_wg = 64, tile_g = 1;  // slots of the pair passes' LDS form, their launch shape
     int *work = nullptr, *nwork = nullptr;  // (particle, face) pairs of the boundary table
     int *idslot = nullptr, *rmids = nullptr;  // id -> slot, ids removed by a sort
     int wg = 256, grid = 1, bt_grid = 1024;  // launch shape of the particle kernels
@@ -189,11 +191,6 @@ int collect_timing(sph_ctx* c) {
 }
 
 // ---- device steps --------------------------------------------------------
-// position / velocity halves of FP32 record buffer k
-inline F4In XF(const sph_ctx* c, int k) { return F4In{c->rec[k]}; }
-inline F4In VF(const sph_ctx* c, int k) { return F4In{c->rec[k] + 1}; }
-inline F4Out XFo(const sph_ctx* c, int k) { return F4Out{c->rec[k]}; }
-inline F4Out VFo(const sph_ctx* c, int k) { return F4Out{c->rec[k] + 1}; }
 void scan_ints(sph_ctx* c, const int* in, int* out, int* bs, int m, int* total) {
     const int nb = (m + 1023) / 1024;
     k_scan_local<<<nb, 256, 0, c->stream>>>(in, out, bs, m);
@@ -204,8 +201,8 @@ void scan_ints(sph_ctx* c, const int* in, int* out, int* bs, int m, int* total) 
 // Launches kernel K in its one-solve (<false>) or segmented (<true>) form.
 #define SEGL(K, G, B, ...)                                                                 \
     do {                                                                                   \
-        if (c->nseg > 1) K<true><<<(G), (B), 0, c->stream>>>(c->P, c->S, __VA_ARGS__);      \
-        else K<false><<<(G), (B), 0, c->stream>>>(c->P, c->S, __VA_ARGS__);                 \
+        if (c->nseg > 1) K<true><<<(G), (B), 0, c->stream>>>(c->S, __VA_ARGS__);      \
+        else K<false><<<(G), (B), 0, c->stream>>>(c->S, __VA_ARGS__);                 \
     } while (0)
 
 __global__ void k_fill_strided(int* p, int stride, int v, int m) {
@@ -228,7 +225,7 @@ int run_sort(sph_ctx* c) {
         k_fill_int<<<nblk(m), 256, 0, c->stream>>>(c->cnt, 0, m);
         k_fill_strided<<<nblk(ns, 64), 64, 0, c->stream>>>(c->iscal + IS_NRM, IS_COUNT, 0, ns);
         SEGL(k_cell_count, nblk(cap), 256, c->xm[1], c->vel[2], c->key, c->slot, c->cnt, c->idslot, c->rmids,
-             c->iscal, c->gone);
+             c->iscal, c->gone, c->ntile);
         SEGL(k_renumber, nblk(ns, 64), 64, c->rmids, c->idslot, c->vel[2], c->iscal);
     }
     {
@@ -241,14 +238,14 @@ int run_sort(sph_ctx* c) {
     }
     {
         KTime t(c, "sort_scatter");
-        SEGL(k_scatter, nblk(cap), 256, c->key, c->slot, c->start, c->vel[2], c->perm, c->pid, c->iscal);
+        SEGL(k_scatter, nblk(cap) + c->ntiles / 256, 256, c->key, c->slot, c->start, c->vel[2], c->perm, c->pid,
+             c->iscal, nblk(cap), c->tlist, c->ntile);
         SEGL(k_cell_sort, ns > 1 ? m / 256 : (c->P.nmax + 255) / 256, 256, c->start, c->perm, c->pid);
     }
     {
         KTime t(c, "sort_gather");
         SEGL(k_gather, nblk(cap), 256, c->perm, c->key, c->xm[1], c->vel[2], c->rp[0], c->lam[0], c->acc[1],
-             c->xm[0], c->vel[0], c->rp[1], c->lam[1], c->acc[0], c->cell, c->xmf, XFo(c, 0), XFo(c, 1),
-             VFo(c, 0), c->rpf[1], c->start, c->iscal, c->P.rk1 ? c->dden : nullptr, c->dden2,
+             c->xm[0], c->vel[0], c->rp[1], c->lam[1], c->acc[0], c->cell, c->xq, c->vf[0], c->start, c->iscal, c->P.rk1 ? c->dden : nullptr, c->dden2,
              c->P.rk1 ? c->vpres : nullptr, c->vpres2, c->P.dbsph ? c->gam[0] : nullptr, c->gam[1],
              c->dsh[0], c->dsh[1]);
     }
@@ -257,8 +254,9 @@ int run_sort(sph_ctx* c) {
 
 int run_neighbours(sph_ctx* c) {
     KTime t(c, "neighbours");
-    SEGL(k_neighbours, nblk(c->P.cap, 4 * NBC_SLOTS), 256, c->xm[0], c->xmf, c->cell, c->start, c->nbr, c->nnb,
-         c->iscal, c->pairs);
+    const int slots = c->P.cap < NBC_LARGE ? NBC_SLOTS : NBC_SLOTS_L;
+    SEGL(k_neighbours, nblk(c->P.cap, 4 * slots), 256, c->xm[0], c->xq, c->cell, c->start, c->nbr, c->nnb,
+         c->iscal, c->pairs, slots);
     return 0;
 }
 
@@ -269,7 +267,7 @@ int run_btab(sph_ctx* c) {
     }
     if (c->P.dim == 2) {  // ComputeBoundaryDataTab_2D
         KTime t(c, "boundary_2d");
-        k_boundary_2d<<<nblk(c->P.cap), 256, 0, c->stream>>>(c->P, c->d_faces, c->d_bit, c->xm[0], c->cell,
+        k_boundary_2d<<<nblk(c->P.cap), 256, 0, c->stream>>>(c->S.P, c->d_faces, c->d_bit, c->xm[0], c->cell,
                                                             c->bn, c->bt, c->iscal);
         return 0;
     }
@@ -294,49 +292,86 @@ int run_dt(sph_ctx* c, int advance, bool reduce) {
     return 0;
 }
 
-// The pair passes: FP32-mixed with the list-walk chunk of the pass (4 or 8;
-// segmented contexts use 8), or FP64; one-solve or segmented form.
-#define PAIRL(K, CHV, ...)                                                                          \
-    do {                                                                                            \
-        if (c->P.f32) {                                                                             \
-            if (c->nseg > 1) K<true, 8, true><<<c->grid, c->wg, 0, c->stream>>>(c->P, c->S, __VA_ARGS__); \
-            else if ((CHV) == 4) K<true, 4, false><<<c->grid, c->wg, 0, c->stream>>>(c->P, c->S, __VA_ARGS__); \
-            else K<true, 8, false><<<c->grid, c->wg, 0, c->stream>>>(c->P, c->S, __VA_ARGS__);        \
-        } else {                                                                                    \
-            if (c->nseg > 1) K<false, 4, true><<<c->grid, c->wg, 0, c->stream>>>(c->P, c->S, __VA_ARGS__); \
-            else K<false, 4, false><<<c->grid, c->wg, 0, c->stream>>>(c->P, c->S, __VA_ARGS__);      \
-        }                                                                                           \
+// The pair passes in FP64: one lane per particle, one-solve or segmented form.
+#define PAIR64(K, ...)                                                                            \
+    do {                                                                                          \
+        if (c->nseg > 1) K<true><<<c->grid, c->wg, 0, c->stream>>>(c->S, __VA_ARGS__);      \
+        else K<false><<<c->grid, c->wg, 0, c->stream>>>(c->S, __VA_ARGS__);                 \
     } while (0)
+
+// The pair passes in FP32-mixed form: launch(CAP, SG, G) of the context's tile
+// form (more than one lane per particle only with the smallest tiles).
+template <int V>
+using IntC = std::integral_constant<int, V>;
+template <class Launch>
+void tile_dispatch(sph_ctx* c, Launch&& launch) {
+    auto form = [&](auto sg) {
+        if (c->tile_cap == TILE_CAP_L) launch(IntC<TILE_CAP_L>{}, sg, IntC<1>{});
+        else if (c->tile_cap == TILE_CAP_M) launch(IntC<TILE_CAP_M>{}, sg, IntC<1>{});
+        else if (c->tile_g == 1) launch(IntC<TILE_CAP_S>{}, sg, IntC<1>{});
+        else launch(IntC<TILE_CAP_S>{}, sg, IntC<2>{});
+    };
+    if (c->nseg > 1) form(std::true_type{});
+    else form(std::false_type{});
+}
+#define TILE_RUN(...) \
+    <<<c->tile_grid, c->tile_wg, 0, c->stream>>>(c->S, Tiles{c->tlist, c->ntile}, c->start, __VA_ARGS__)
 
 int run_momentum(sph_ctx* c) {
     KTime t(c, "momentum");
-    PAIRL(k_momentum, c->chunk, c->d_faces, c->d_edges, c->bn, c->bt, c->xm[0], c->vel[0], c->rp[cur_rp(c)], XF(c, 0),
-          VF(c, 0), c->rpf[cur_rp(c)], c->lam[1], c->lam[0], c->nbr, c->nnb, c->acc[1], c->vel[1], VFo(c, 1), c->scal, c->iscal);
+    if (!c->P.f32) {
+        PAIR64(k_momentum64, c->d_faces, c->d_edges, c->bn, c->bt, c->xm[0], c->vel[0], c->rp[cur_rp(c)], c->lam[1],
+               c->lam[0], c->nbr, c->nnb, c->acc[1], c->vel[1], c->scal, c->iscal);
+        return 0;
+    }
+    bool um = c->nseg == 1 ? c->P.umass != 0 : true;
+    for (int s = 0; c->nseg > 1 && s < c->nseg; ++s) um = um && c->segs[s].umass;
+#define MOM_ARGS c->d_faces, c->d_edges, c->bn, c->bt, c->xm[0], c->vel[0], c->rp[cur_rp(c)], c->xq, c->vf[0],   \
+        c->lam[1], c->lam[0], c->nbr, c->nnb, c->acc[1], c->vel[1], c->vf[1], c->scal, c->iscal
+    tile_dispatch(c, [&](auto cap, auto sg, auto g) {
+        if (um) k_momentum<cap.value, sg.value, g.value, true> TILE_RUN(MOM_ARGS);
+        else k_momentum<cap.value, sg.value, g.value, false> TILE_RUN(MOM_ARGS);
+    });
+#undef MOM_ARGS
     return 0;
 }
 
 int run_vsmooth(sph_ctx* c) {
     KTime t(c, "velocity_smoothing");
-    PAIRL(k_vsmooth, c->chunk_v, c->d_faces, c->bn, c->bt, c->xm[0], c->vel[1], c->rp[cur_rp(c)], XF(c, 1),
-          VF(c, 1), c->nbr, c->nnb, c->vel[2], c->xm[1], c->scal, c->dtmin, c->iscal, c->dden, c->rp[2],
-          c->rpf[2], c->xrf, c->gone);
+    if (!c->P.f32)
+        PAIR64(k_vsmooth64, c->d_faces, c->bn, c->bt, c->xm[0], c->vel[1], c->rp[cur_rp(c)], c->nbr, c->nnb, c->vel[2],
+               c->xm[1], c->scal, c->dtmin, c->iscal, c->dden, c->rp[2], c->gone);
+    else
+        tile_dispatch(c, [&](auto cap, auto sg, auto g) {
+            k_vsmooth<cap.value, sg.value, g.value> TILE_RUN(c->d_faces, c->bn, c->bt, c->xm[0], c->vel[1], c->rp[cur_rp(c)], c->xq, c->vf[1],
+              c->nbr, c->nnb, c->vel[2], c->xm[1], c->scal, c->dtmin, c->iscal, c->dden, c->rp[2], c->dr, c->gone);
+        });
     return 0;
 }
 
 int run_continuity(sph_ctx* c) {
     KTime t(c, "continuity");
-    PAIRL(k_continuity, c->chunk_c, c->d_faces, c->bn, c->bt, c->xm[0], c->vel[0],
-          c->P.dbsph ? c->rp[0] : c->rp[1], XF(c, 0),
-          VF(c, 0), c->nbr, c->nnb, c->dden, c->rp[2], c->rpf[2], c->xrf, c->scal, c->iscal);
+    if (!c->P.f32)
+        PAIR64(k_continuity64, c->d_faces, c->bn, c->bt, c->xm[0], c->vel[0], c->P.dbsph ? c->rp[0] : c->rp[1], c->nbr,
+               c->nnb, c->dden, c->rp[2], c->scal, c->iscal);
+    else
+        tile_dispatch(c, [&](auto cap, auto sg, auto g) {
+            k_continuity<cap.value, sg.value, g.value> TILE_RUN(c->d_faces, c->bn, c->bt, c->vel[0], c->rp[1], c->xq, c->vf[0], c->nbr, c->nnb,
+              c->dden, c->rp[2], c->dr, c->scal, c->iscal);
+        });
     return 0;
 }
 
 int run_psmooth(sph_ctx* c) {
     KTime t(c, "pressure_smoothing");
-    // w of the velocity half of FP32 record buffer 0 (read by the next momentum pass)
-    float* velw = c->P.f32 ? reinterpret_cast<float*>(c->rec[0] + 1) + 3 : nullptr;
-    PAIRL(k_psmooth, c->chunk_p, c->d_faces, c->bn, c->bt, c->xm[0], c->rp[2], c->xmf, c->rpf[2], c->xrf,
-          c->nbr, c->nnb, c->vpres, c->rp[0], c->rpf[0], velw, c->scal, c->iscal);
+    if (!c->P.f32)
+        PAIR64(k_psmooth64, c->d_faces, c->bn, c->bt, c->xm[0], c->rp[2], c->nbr, c->nnb, c->vpres, c->rp[0], c->scal,
+               c->iscal);
+    else
+        tile_dispatch(c, [&](auto cap, auto sg, auto g) {
+            k_psmooth<cap.value, sg.value, g.value> TILE_RUN(c->d_faces, c->bn, c->bt, c->rp[2], c->xq, c->dr, c->nbr, c->nnb, c->vpres,
+              c->rp[0], c->vf[0], c->scal);
+        });
     return 0;
 }
 
@@ -349,17 +384,17 @@ int run_dbsph_lists(sph_ctx* c, int mode) {
     KTime t(c, "dbsph_lists");
     const int cap = c->P.cap;
     if (mode == 0)
-        k_dbsph_lists<0><<<nblk(DB_G * cap), 256, 0, c->stream>>>(c->P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->cell,
+        k_dbsph_lists<0><<<nblk(DB_G * cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->cell,
                                                            c->nbr, c->nnb, c->gam[0], c->dsh[0], c->gam[0], c->dsh[0],
                                                            c->sig, c->rsph, c->fsf, c->nfw, c->fwl, c->d_wwet,
                                                            c->dden2, c->rp[2], c->scal, c->iscal);
     else if (mode == 1)
-        k_dbsph_lists<1><<<nblk(DB_G * cap), 256, 0, c->stream>>>(c->P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->cell,
+        k_dbsph_lists<1><<<nblk(DB_G * cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->cell,
                                                            c->nbr, c->nnb, c->gam[0], c->dsh[0], c->gam[0], c->dsh[0],
                                                            c->sig, c->rsph, c->fsf, c->nfw, c->fwl, c->d_wwet,
                                                            c->dden2, c->rp[2], c->scal, c->iscal);
     else
-        k_dbsph_lists<2><<<nblk(DB_G * cap), 256, 0, c->stream>>>(c->P, dwall(c), c->xm[0], c->vel[0], c->rp[1], c->cell,
+        k_dbsph_lists<2><<<nblk(DB_G * cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[1], c->cell,
                                                            c->nbr, c->nnb, c->gam[1], c->dsh[1], c->gam[0], c->dsh[0],
                                                            c->sig, c->rsph, c->fsf, c->nfw, c->fwl, c->d_wwet,
                                                            c->dden2, c->rp[2], c->scal, c->iscal);
@@ -368,7 +403,7 @@ int run_dbsph_lists(sph_ctx* c, int mode) {
 
 int run_momentum_dbsph(sph_ctx* c) {
     KTime t(c, "momentum");
-    k_momentum_dbsph<<<nblk(DB_G * c->P.cap), 256, 0, c->stream>>>(c->P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->nbr,
+    k_momentum_dbsph<<<nblk(DB_G * c->P.cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->nbr,
                                                             c->nnb, c->nfw, c->fwl, c->gam[0], c->d_wdens,
                                                             c->d_wpres, c->lam[0], c->acc[1], c->vel[1], c->scal,
                                                             c->iscal);
@@ -378,15 +413,15 @@ int run_momentum_dbsph(sph_ctx* c) {
 // PressureSmoothing_3D.f90 for bsph on the new lists: rp[2] -> rp[0]
 int run_psmooth_dbsph(sph_ctx* c) {
     KTime t(c, "pressure_smoothing");
-    PAIRL(k_psmooth, c->chunk_p, c->d_faces, c->bn, c->bt, c->xm[0], c->rp[2], c->xmf, c->rpf[2], c->xrf,
-          c->nbr, c->nnb, c->vpres2, c->rp[0], c->rpf[0], nullptr, c->scal, c->iscal);
+    PAIR64(k_psmooth64, c->d_faces, c->bn, c->bt, c->xm[0], c->rp[2], c->nbr, c->nnb, c->vpres2, c->rp[0], c->scal,
+           c->iscal);
     return 0;
 }
 
 // the wall elements' velocity and position in Euler, after the particles'
 int run_dbsph_kinematics(sph_ctx* c) {
     KTime t(c, "dbsph_kinematics");
-    k_dbsph_kinematics<<<nblk(c->P.nw), 256, 0, c->stream>>>(c->P, c->d_kin, c->d_wids, c->d_w0, c->d_w2,
+    k_dbsph_kinematics<<<nblk(c->P.nw), 256, 0, c->stream>>>(c->S.P, c->d_kin, c->d_wids, c->d_w0, c->d_w2,
                                                              c->d_wpos, c->scal);
     return 0;
 }
@@ -394,10 +429,10 @@ int run_dbsph_kinematics(sph_ctx* c) {
 // Gradients_to_MUSCL and BC_wall_elements on the step's final state
 int run_dbsph_walls(sph_ctx* c) {
     KTime t(c, "dbsph_walls");
-    k_dbsph_muscl<<<nblk(c->P.cap), 256, 0, c->stream>>>(c->P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->nbr,
+    k_dbsph_muscl<<<nblk(c->P.cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->nbr,
                                                          c->nnb, c->nfw, c->fwl, c->sig, c->d_wdens, c->drho,
                                                          c->dvelg, c->iscal);
-    k_dbsph_walls<<<(c->P.nw + DB_WPB - 1) / DB_WPB, 256, 0, c->stream>>>(c->P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->start,
+    k_dbsph_walls<<<(c->P.nw + DB_WPB - 1) / DB_WPB, 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->start,
                                                         c->drho, c->dvelg, c->d_wdens, c->d_wpres, c->iscal);
     return 0;
 }
@@ -442,15 +477,14 @@ sph_ctx::~sph_ctx() {
         if (p) hipFree(p);
     };
     F(d_faces); F(d_edges); F(d_gcount); F(d_gstart); F(d_gvec); F(d_kt); F(d_bit); F(d_btf);
-    F(d_P); F(d_pblk); F(d_kblk); F(d_adj);
+    F(d_P); F(d_pblk); F(d_kblk); F(d_tblk); F(d_adj);
     for (auto p : xm) F(p);
     for (auto p : vel) F(p);
     for (auto p : acc) F(p);
     for (auto p : rp) F(p);
     for (auto p : lam) F(p);
-    F(xmf); F(xrf);
-    for (auto p : rec) F(p);
-    for (auto p : rpf) F(p);
+    F(xq); F(dr); F(tlist); F(ntile);
+    for (auto p : vf) F(p);
     F(dden); F(vpres); F(dden2); F(vpres2); F(gone); F(idslot); F(rmids); F(cell); F(key); F(slot); F(cnt); F(start); F(perm); F(pid); F(bsum);
     F(work); F(nwork);
     F(nbr); F(nnb); F(bn); F(bt); F(scal); F(iscal); F(dtmin); F(pairs);
@@ -473,10 +507,11 @@ int sph_ctx::alloc() {
     for (auto& p : acc) HIPC(da(&p, N));
     for (auto& p : rp) HIPC(da(&p, N));
     for (auto& p : lam) HIPC(da(&p, N));
-    HIPC(da(&xmf, N));
-    HIPC(da(&xrf, P.f32 ? N : 1));
-    for (auto& r : rec) HIPC(da(&r, P.f32 ? 2 * N : 1));
-    for (auto& p : rpf) HIPC(da(&p, P.f32 ? N : 1));
+    HIPC(da(&xq, N));
+    HIPC(da(&dr, P.f32 ? N : 1));
+    for (auto& p : vf) HIPC(da(&p, P.f32 ? N : 1));
+    HIPC(da(&tlist, ntiles ? (size_t)ntiles : 1));
+    HIPC(da(&ntile, 1));
     HIPC(da(&dden, N));
     HIPC(da(&vpres, N));
     HIPC(da(&dden2, P.rk1 ? N : 1));
@@ -514,6 +549,7 @@ int sph_ctx::alloc() {
         HIPC(hipMemset(dden2, 0, sizeof(double) * N));
         HIPC(hipMemset(vpres2, 0, sizeof(double) * N));
     }
+    HIPC(hipMemset(ntile, 0, sizeof(int)));
     HIPC(hipMemset(nnb, 0, sizeof(int) * N));
     HIPC(hipMemset(gone, 0, sizeof(int) * N));
     HIPC(hipMemset(bn, 0, sizeof(int) * N));
@@ -599,6 +635,8 @@ int fill_dp(const sph_params* p, const sph_faces* f, DP& P, bool dry = false) {
         P.dcd[d] = p->dcd[d];
         P.grav[d] = p->grav[d];
     }
+    P.inv_nij = 1.0 / ((double)P.ncd[0] * P.ncd[1]);
+    P.inv_ni = 1.0 / P.ncd[0];
     P.h = p->h;
     P.dx = p->dx;
     P.coefke = p->coefke;
@@ -623,17 +661,12 @@ int fill_dp(const sph_params* p, const sph_faces* f, DP& P, bool dry = false) {
     P.pesodt = p->pesodt;
     P.tetap = p->tetap;
     P.tetav = p->tetav;
-    P.f_h = (float)P.h;
-    P.f_unosuh = (float)(1.0 / P.h);
-    P.f_unosusquareh = (float)(1.0 / P.squareh);
-    P.f_eta = (float)P.eta;
-    P.f_eta2 = (float)P.eta2;
-    P.f_ke_coef = (float)P.ke_coef;
-    P.f_kacl_coef = (float)P.kacl_coef;
-    P.f_coefke = (float)P.coefke;
+    P.lsb = std::max(P.dcd[0], std::max(P.dcd[1], P.dcd[2])) * 0x1p-28;
+    P.inv_lsb = 1.0 / P.lsb;
+    P.f_q = (float)(P.lsb / P.h);
+    P.f_etal = (float)(P.eta * P.inv_lsb);
+    P.f_eta2l = (float)(P.eta2 * P.inv_lsb * P.inv_lsb);
     for (int d = 0; d < 3; ++d) P.f_dcd[d] = (float)P.dcd[d];
-    P.f_alfamon = (float)P.alfamon;
-    P.f_celerita = (float)P.celerita;
     P.f_kin_visc = (float)P.kin_visc;
     P.f_den0 = (float)P.den0;
     P.f_eosk = (float)(P.eps / P.den0);
@@ -642,6 +675,62 @@ int fill_dp(const sph_params* p, const sph_faces* f, DP& P, bool dry = false) {
 }
 
 inline int round256(long long v) { return (int)((v + 255) / 256 * 256); }
+
+// The tile of the FP32-mixed pair passes, one for all segments: the largest
+// box of cells of the ladder that cuts the solve's water into TILE_MIN tiles
+// (2D: TILE_MIN2) - fewer leave CUs idle, smaller ones read more halo - and whose
+// cells with their halo, an eighth denser than water, fit the largest LDS
+// form.  The first box of a ladder fills a workgroup of 512 threads, two a CU:
+// it needs TILE_MIN_L.  Step times, us: 576,000 particles 3x3x3 677, 3x3x2 788,
+// 4x3x2 740; 250,000 409, 439; 185,000 (390 tiles) 3x3x3 446, 3x3x2 377,
+// 3x2x1 411; 103,000 3x3x2 294, 3x2x2 334, 3x3x3 396; 72,000 3x2x2 229, 3x3x2
+// 245, 3x1x1 292; 2D 61,000 7x6 182, 6x5 185, 4x4 189.
+void choose_tile(sph_ctx* c) {
+    const int L3[][3] = {{3, 3, 3}, {3, 3, 2}, {3, 2, 2}, {3, 2, 1}, {3, 1, 1}, {2, 1, 1}, {1, 1, 1}};
+    const int L2[][3] = {{8, 1, 8}, {7, 1, 6}, {6, 1, 5}, {4, 1, 4}, {3, 1, 3}, {2, 1, 2}, {1, 1, 1}};
+    const DP& A = c->segs[0];
+    const bool flat = A.ncd[1] == 1;
+    double ppc = 0.0;  // particles of a water cell
+    for (const DP& Q : c->segs) {
+        const double n = Q.dcd[0] / Q.dx * (flat ? 1.0 : Q.dcd[1] / Q.dx) * (Q.dcd[2] / Q.dx);
+        if (n > ppc) ppc = n;
+    }
+    if (!(ppc >= 1.0 && ppc <= 1.0e4)) ppc = 1.0e4;
+    const int* best = flat ? L2[6] : L3[6];
+    double need = 0.0, home = 0.0;
+    for (int k = 0; k < 7; ++k) {
+        best = flat ? L2[k] : L3[k];
+        home = ppc * best[0] * best[1] * best[2];
+        need = 1.125 * ppc * (best[0] + 2) * (flat ? 1 : best[1] + 2) * (best[2] + 2);
+        if (need <= TILE_CAP_L && A.cap >= (k == 0 ? TILE_MIN_L : flat ? TILE_MIN2 : TILE_MIN) * home) break;
+    }
+    c->tile_cap = need <= TILE_CAP_S ? TILE_CAP_S : need <= TILE_CAP_M ? TILE_CAP_M : TILE_CAP_L;
+    c->tile_g = c->tile_cap != TILE_CAP_S ? 1 : A.cap < TILE_G2 ? 2 : 1;
+    // threads for the most particles a tile of lattice water holds
+    double most = c->tile_g;
+    for (int d = 0; d < 3; d += flat ? 2 : 1) most *= std::ceil(best[d] * A.dcd[d] / A.dx);
+    c->tile_wg = (int)std::min<double>(TILE_WG, std::max(256.0, 64.0 * std::ceil(most / 64.0)));
+    long long tiles = 0;
+    for (DP& Q : c->segs) {
+        long long n = 1;
+        for (int d = 0; d < 3; ++d) {
+            Q.tdim[d] = best[d];
+            Q.ntile[d] = (Q.ncd[d] + best[d] - 1) / best[d];
+            n *= Q.ntile[d];
+        }
+        for (int d = 0; d < 3; ++d) Q.inv_tdim[d] = 1.0 / Q.tdim[d];
+        Q.inv_ntij = 1.0 / ((double)Q.ntile[0] * Q.ntile[1]);
+        Q.inv_nti = 1.0 / Q.ntile[0];
+        Q.inv_ry = 1.0 / (Q.tdim[1] + 2);
+        Q.toff = (int)tiles;
+        Q.tcap = Q.f32 ? c->tile_cap : 0;
+        tiles += (n + 255) / 256 * 256;
+    }
+    c->ntiles = (int)(A.f32 ? tiles : 0);
+    // a workgroup per tile where every tile is full, and as many again for partly filled ones
+    const double full = 2.0 * A.cap / home + 64.0;
+    c->tile_grid = (int)(std::min((double)tiles, full) / 8.0 + 1.0) * 8;
+}
 
 // Places nseg solves in one context: slots and keys of segment s follow
 // those of segment s-1 (slots and keys in whole 256-blocks).  One solve keeps
@@ -679,6 +768,7 @@ int layout_segments(sph_ctx* c, int nseg, const sph_params* p, const sph_faces* 
             return fail(2, "batch too large for one context");
     }
     for (auto& P : c->segs) P.cap = (int)slots;
+    choose_tile(c);
     c->P = c->segs[0];
     c->nkeys = (int)keys;
     c->nb_stride_max = nmaxpartj;
@@ -815,27 +905,41 @@ int upload_tables(sph_ctx* c, const sph_faces* const* f) {
     return 0;
 }
 
-// Segment maps of a segmented context: per-segment constants, segment of
-// every 256-slot block and 256-key block.
+// The constants to the device, after every change of them on the host: a
+// one-solve context's are c->P.  Waits for the kernels that read the old ones.
+int upload_constants(sph_ctx* c) {
+    if (c->nseg == 1) c->segs[0] = c->P;
+    HIPC(hipStreamSynchronize(c->stream));
+    HIPC(hipMemcpy(c->d_P, c->segs.data(), sizeof(DP) * c->nseg, hipMemcpyHostToDevice));
+    return 0;
+}
+
+// Segment maps of a segmented context: segment of
+// every 256-slot, 256-key and 256-tile block.
 int upload_segment_maps(sph_ctx* c) {
+    if (hipMalloc(&c->d_P, sizeof(DP) * c->nseg) != hipSuccess) return fail(102, "device allocation failed");
+    c->S = Seg{(DPC*)c->d_P, nullptr, nullptr, nullptr, c->nseg};
+    if (int rc = upload_constants(c)) return rc;
     if (c->nseg == 1) return 0;
-    std::vector<int> pblk(c->P.cap / 256), kblk(c->nkeys / 256);
+    std::vector<int> pblk(c->P.cap / 256), kblk(c->nkeys / 256), tblk(std::max(1, c->ntiles / 256));
     for (int s = 0; s < c->nseg; ++s) {
         const DP& P = c->segs[s];
         const int sb = (s + 1 < c->nseg ? c->segs[s + 1].base : c->P.cap);
         for (int b = P.base / 256; b < sb / 256; ++b) pblk[b] = s;
         const int ke = (s + 1 < c->nseg ? c->segs[s + 1].koff : c->nkeys);
         for (int b = P.koff / 256; b < ke / 256; ++b) kblk[b] = s;
+        const int te = (s + 1 < c->nseg ? c->segs[s + 1].toff : c->ntiles);
+        for (int b = P.toff / 256; c->ntiles && b < te / 256; ++b) tblk[b] = s;
     }
-    bool ok = hipMalloc(&c->d_P, sizeof(DP) * c->nseg) == hipSuccess &&
-              hipMemcpy(c->d_P, c->segs.data(), sizeof(DP) * c->nseg, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMalloc(&c->d_pblk, sizeof(int) * pblk.size()) == hipSuccess &&
+    bool ok = hipMalloc(&c->d_pblk, sizeof(int) * pblk.size()) == hipSuccess &&
               hipMemcpy(c->d_pblk, pblk.data(), sizeof(int) * pblk.size(), hipMemcpyHostToDevice) == hipSuccess &&
               hipMalloc(&c->d_kblk, sizeof(int) * kblk.size()) == hipSuccess &&
               hipMemcpy(c->d_kblk, kblk.data(), sizeof(int) * kblk.size(), hipMemcpyHostToDevice) == hipSuccess &&
+              hipMalloc(&c->d_tblk, sizeof(int) * tblk.size()) == hipSuccess &&
+              hipMemcpy(c->d_tblk, tblk.data(), sizeof(int) * tblk.size(), hipMemcpyHostToDevice) == hipSuccess &&
               hipMalloc(&c->d_adj, sizeof(int) * c->nseg) == hipSuccess;
     if (!ok) return fail(102, "device allocation/copy of the segment maps failed");
-    c->S = Seg{c->d_P, c->d_pblk, c->d_kblk, c->nseg};
+    c->S = Seg{(DPC*)c->d_P, c->d_pblk, c->d_kblk, c->d_tblk, c->nseg};
     return 0;
 }
 
@@ -1024,7 +1128,12 @@ int sph_ctx_create2d(const sph_params* p, const sph_sides2d* sd, sph_ctx** out) 
             return fail(102, "device allocation/copy of boundary sides failed");
         }
     }
-    return 0;
+    rc = upload_constants(c);
+    if (rc) {
+        sph_ctx_destroy(c);
+        *out = nullptr;
+    }
+    return rc;
 }
 
 int sph_ctx_destroy(sph_ctx* c) {
@@ -1116,7 +1225,7 @@ int sph_dbsph_walls(sph_ctx* c, const sph_dbsph_walls_t* w) {
     P.fs_allowed = w->fs_allowed ? 1 : 0;
     P.neg_wall_p = w->negative_wall_p_allowed ? 1 : 0;
     P.muscl_bnd = w->muscl_boundary ? 1 : 0;
-    return 0;
+    return upload_constants(c);
 }
 
 int sph_dbsph_kinematics(sph_ctx* c, int32_t nrec, const double* records, const double* centre) {
@@ -1138,7 +1247,7 @@ int sph_dbsph_kinematics(sph_ctx* c, int32_t nrec, const double* records, const 
     }
     c->P.nkin = nrec;
     for (int d = 0; d < 3; ++d) c->P.kin_c[d] = nrec > 0 ? centre[d] : 0.0;
-    return 0;
+    return upload_constants(c);
 }
 
 int sph_dbsph_state(sph_ctx* c, double* gamma, double* sigma, double* rhosph, double* dshep, int32_t* fs,
@@ -1210,14 +1319,12 @@ int sph_segment_upload(sph_ctx* c, int32_t seg, int32_t n, const double* coord, 
         DP& Q = c->nseg > 1 ? c->segs[seg] : c->P;
         Q.umass = umass;
         Q.f_mass = f_mass;
-        if (c->nseg > 1) {
-            if (seg == 0) {
-                c->P.umass = umass;
-                c->P.f_mass = f_mass;
-            }
-            HIPC(hipMemcpy(c->d_P + seg, &Q, sizeof(DP), hipMemcpyHostToDevice));
+        if (c->nseg > 1 && seg == 0) {
+            c->P.umass = umass;
+            c->P.f_mass = f_mass;
         }
-        // captured graphs hold the constants they were captured with
+        if (int rc = upload_constants(c)) return rc;
+        // captured graphs hold the momentum kernel chosen for the old masses
         for (auto& g : c->graphs) hipGraphExecDestroy(g.second);
         c->graphs.clear();
     }
@@ -1247,9 +1354,6 @@ int sph_segment_upload(sph_ctx* c, int32_t seg, int32_t n, const double* coord, 
     // the sort leaves (rho,p) in the buffer the continuity pass reads; the
     // state at rest keeps it in the buffer the momentum pass reads
     HIPC(hipMemcpyAsync(c->rp[0], c->rp[1], sizeof(double2) * c->P.cap, hipMemcpyDeviceToDevice, c->stream));
-    if (c->P.f32)
-        HIPC(hipMemcpyAsync(c->rpf[0], c->rpf[1], sizeof(float2) * c->P.cap, hipMemcpyDeviceToDevice,
-                            c->stream));
     HIPC(hipStreamSynchronize(c->stream));
     collect_timing(c);
     c->n_upload = n;
@@ -1445,7 +1549,7 @@ int sph_free_surface(sph_ctx* c, double* pelolib, double* zlft) {
         return fail(121, "the free surface is taken at a time-step boundary");
     const int nl = c->mon_nlines;
     if (nl == 0) return 0;
-    k_free_surface<<<nl, FS_WG, 0, c->stream>>>(c->P, c->xm[0], c->start, c->mon_pts, c->mon_icont, nl,
+    k_free_surface<<<nl, FS_WG, 0, c->stream>>>(c->S.P, c->xm[0], c->start, c->mon_pts, c->mon_icont, nl,
                                                 c->mon_out);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
@@ -1485,15 +1589,58 @@ int sph_get_neighbour_lists(sph_ctx* c, int32_t* count, int32_t* ids, int32_t st
     const size_t ngroups = (size_t)(kmax + NB_G - 1) / NB_G;
     std::vector<uint32_t> nb(ngroups * N * NB_G);
     if (kmax) HIPC(hipMemcpy(nb.data(), c->nbr, sizeof(uint32_t) * nb.size(), hipMemcpyDeviceToHost));
+    const uint16_t* nb16 = reinterpret_cast<const uint16_t*>(nb.data());
+    const DP& P = c->P;
+    std::vector<int> start(c->nkeys + 1, 0), cell(n);
+    if (P.tcap > 0 && n) {
+        HIPC(hipMemcpy(start.data(), c->start, sizeof(int) * c->nkeys, hipMemcpyDeviceToHost));
+        HIPC(hipMemcpy(cell.data(), c->cell, sizeof(int) * n, hipMemcpyDeviceToHost));
+    }
+    // rows of the current tile (tile_row of the device): first slot and sorted index
+    std::vector<int> rl, rg;
+    long long tile = -1;
+    bool fits = false;
+    auto rows_of = [&](int s) {
+        const int q = cell[s] - 1, nij = P.ncd[0] * P.ncd[1];
+        const int t[3] = {q % P.ncd[0] / P.tdim[0], q % nij / P.ncd[0] / P.tdim[1], q / nij / P.tdim[2]};
+        const long long id = ((long long)t[2] * P.ntile[1] + t[1]) * P.ntile[0] + t[0];
+        if (id == tile) return;
+        tile = id;
+        rl.assign(1, 0);
+        rg.clear();
+        const int i0 = t[0] * P.tdim[0] + 1, i1 = std::min(i0 + P.tdim[0] - 1, P.ncd[0]);
+        for (int k = t[2] * P.tdim[2]; k <= (t[2] + 1) * P.tdim[2] + 1; ++k)
+            for (int j = t[1] * P.tdim[1]; j <= (t[1] + 1) * P.tdim[1] + 1; ++j) {
+                int g0 = 0, g1 = 0;
+                if (j >= 1 && j <= P.ncd[1] && k >= 1 && k <= P.ncd[2]) {
+                    const int rb = ((k - 1) * P.ncd[1] + (j - 1)) * P.ncd[0] - 1;
+                    g0 = start[rb + std::max(i0 - 1, 1)];
+                    g1 = start[rb + std::min(i1 + 1, P.ncd[0]) + 1];
+                }
+                rg.push_back(g0);
+                rl.push_back(rl.back() + g1 - g0);
+            }
+        fits = rl.back() <= P.tcap;
+    };
     std::vector<int> order(n);
     std::iota(order.begin(), order.end(), 0);
     std::sort(order.begin(), order.end(), [&](int a, int b) { return hv[a].w < hv[b].w; });
     for (int r = 0; r < n; ++r) {
         const int s = order[r];
         count[r] = nn[s];
-        if (ids)
-            for (int k = 0; k < nn[s]; ++k)
-                ids[(size_t)r * stride + k] = (int32_t)hv[nb[nb_index(N, s, k)] & NB_MASK].w;
+        if (!ids) continue;
+        if (P.tcap > 0) rows_of(s);
+        for (int k = 0; k < nn[s]; ++k) {
+            int j;
+            if (fits) {
+                const int slot = nb16[nb16_index(N, s, k)] >> 4;
+                const int row = (int)(std::upper_bound(rl.begin(), rl.end(), slot) - rl.begin()) - 1;
+                j = rg[row] + slot - rl[row];
+            } else {
+                j = (int)(nb[nb_index(N, s, k)] & NB_MASK);
+            }
+            ids[(size_t)r * stride + k] = (int32_t)hv[j].w;
+        }
     }
     return 0;
 }

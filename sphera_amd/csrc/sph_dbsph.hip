@@ -49,13 +49,14 @@ struct DWall {
 // cell's run of the list, then that cell's wall elements.
 template <int MODE>
 __global__ __launch_bounds__(256) void k_dbsph_lists(
-    DP P, DWall W, const double4* __restrict__ xm, const double4* __restrict__ vel,
+    DPC* Pp, DWall W, const double4* __restrict__ xm, const double4* __restrict__ vel,
     const double2* __restrict__ rp, const int* __restrict__ cell, const uint32_t* __restrict__ nbr,
     const int* __restrict__ nnb,
     const double* __restrict__ gam_in, const double* __restrict__ dsh_in, double* __restrict__ gam_out,
     double* __restrict__ dsh_out, double* __restrict__ sig_out, double* __restrict__ rsph_out,
     int* __restrict__ fs_out, int* __restrict__ nfw, int* __restrict__ fwl, int* __restrict__ wwet,
     double* __restrict__ dden, double2* __restrict__ rp_out, const double* scal, int* iscal) {
+    DPC& P = *Pp;
     // DB_G lanes per particle: they take consecutive candidates of a cell
     // (fluid-list entries, then wall elements) side by side, and every lane
     // of the group adds the candidates' terms in candidate order, read from
@@ -216,11 +217,12 @@ __global__ __launch_bounds__(256) void k_dbsph_lists(
 // without the VSL model (slip_ID = 0), and add zeros.  acc = (tpres + tdiss
 // + tvisc) / Gamma + g; Euler's vel += dt acc (kodvel = 0) is fused.
 __global__ __launch_bounds__(256) void k_momentum_dbsph(
-    DP P, DWall W, const double4* __restrict__ xm, const double4* __restrict__ vel,
+    DPC* Pp, DWall W, const double4* __restrict__ xm, const double4* __restrict__ vel,
     const double2* __restrict__ rp, const uint32_t* __restrict__ nbr, const int* __restrict__ nnb,
     const int* __restrict__ nfw, const int* __restrict__ fwl, const double* __restrict__ gam,
     const double* __restrict__ wdens, const double* __restrict__ wpres, int* __restrict__ lam_out,
     double4* __restrict__ acc_out, double4* __restrict__ vel_out, const double* scal, const int* iscal) {
+    DPC& P = *Pp;
     // DB_G lanes per particle take consecutive list entries (then wall
     // elements) side by side; every lane of the group adds the entries'
     // terms in list order, read from their lanes with shuffles
@@ -349,7 +351,7 @@ __global__ __launch_bounds__(256) void k_momentum_dbsph(
 // Gradients_to_MUSCL.f90:47-91 for the particles with wall neighbours:
 // drho = sum r (rho_j - rho_i) PartKernel(1) m_j/rho_j and dvel(r, :) the
 // same of var(r); drho[3 i + d], dvel[9 i + 3 r + d]
-__global__ __launch_bounds__(256) void k_dbsph_muscl(DP P, DWall W, const double4* __restrict__ xm,
+__global__ __launch_bounds__(256) void k_dbsph_muscl(DPC* Pp, DWall W, const double4* __restrict__ xm,
                                                      const double4* __restrict__ vel,
                                                      const double2* __restrict__ rp,
                                                      const uint32_t* __restrict__ nbr,
@@ -358,6 +360,7 @@ __global__ __launch_bounds__(256) void k_dbsph_muscl(DP P, DWall W, const double
                                                      const double* __restrict__ wdens,
                                                      double* __restrict__ drho, double* __restrict__ dvel,
                                                      const int* iscal) {
+    DPC& P = *Pp;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= iscal[IS_N] || nfw[i] <= 0) return;
     const double4 xi = xm[i];
@@ -417,9 +420,10 @@ __global__ __launch_bounds__(256) void k_dbsph_muscl(DP P, DWall W, const double
 // element omega x (x - centre) + v; then every element moves by dt vel.
 // The elements keep their cells: OrdGrid1.f90:108 bins them on the first
 // step only.
-__global__ __launch_bounds__(256) void k_dbsph_kinematics(DP P, const double* __restrict__ kin,
+__global__ __launch_bounds__(256) void k_dbsph_kinematics(DPC* Pp, const double* __restrict__ kin,
                                                           const int* __restrict__ wids, double4* w0,
                                                           double4* w2, double4* wpos, const double* scal) {
+    DPC& P = *Pp;
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= P.nw) return;
     const int id = wids[s];
@@ -469,7 +473,7 @@ __global__ __launch_bounds__(256) void k_dbsph_kinematics(DP P, const double* __
 // the contributions; each contribution goes to its rank by pg index in LDS,
 // and one lane sums them in that order.
 constexpr int DB_WPB = 4;  // wall elements (wavefronts) per 256-thread block
-__global__ __launch_bounds__(256) void k_dbsph_walls(DP P, DWall W, const double4* __restrict__ xm,
+__global__ __launch_bounds__(256) void k_dbsph_walls(DPC* Pp, DWall W, const double4* __restrict__ xm,
                                                      const double4* __restrict__ vel,
                                                      const double2* __restrict__ rp,
                                                      const int* __restrict__ start,
@@ -477,6 +481,7 @@ __global__ __launch_bounds__(256) void k_dbsph_walls(DP P, DWall W, const double
                                                      const double* __restrict__ dvel,
                                                      double* __restrict__ wdens, double* __restrict__ wpres,
                                                      int* iscal) {
+    DPC& P = *Pp;
     __shared__ int s_m[DB_WPB];
     __shared__ int s_pre[DB_WPB][28];  // candidates of the cells before cell t
     __shared__ int s_c0[DB_WPB][27];   // first sorted slot of cell t

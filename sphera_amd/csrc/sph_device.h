@@ -12,13 +12,16 @@ constexpr uint32_t NB_MASK = (1u << NB_SHIFT) - 1u;
 // neighbour-list layout: entry k of particle p at ((k/NB_G)*N + p)*NB_G + k%NB_G,
 // i.e. groups of NB_G consecutive entries per particle, the groups of one
 // rank k/NB_G contiguous over p (32-byte vector stores and loads per lane)
-#ifndef SPH_NB_GROUP
-#define SPH_NB_GROUP 8
-#endif
-constexpr int NB_G = SPH_NB_GROUP;
+constexpr int NB_G = 8;
 __host__ __device__ inline size_t nb_index(size_t N, int p, int k) {
     const unsigned u = (unsigned)k;
     return ((size_t)(u / NB_G) * N + (size_t)p) * NB_G + (size_t)(u % NB_G);
+}
+// 16-bit entries, in the same 32 bytes per particle and group rank (so that
+// lists of both widths share one buffer): 16 consecutive entries
+__host__ __device__ inline size_t nb16_index(size_t N, int p, int k) {
+    const unsigned u = (unsigned)k;
+    return ((size_t)(u / 16) * N + (size_t)p) * 16 + (size_t)(u % 16);
 }
 // list capacity per particle: NMAXPARTJ rounded up to whole groups
 __host__ __device__ inline int nb_stride(int nmaxpartj) { return (nmaxpartj + NB_G - 1) / NB_G * NB_G; }
@@ -33,7 +36,9 @@ enum {
 // most particles one sort may remove from the grid (renumbering list)
 constexpr int RM_CAP = 4096;
 
-// per-context constants, passed by value to every kernel
+// per-segment constants; the kernels read them from device memory through the
+// constant address space (scalar loads), so a kernel's arguments stay short and
+// one-solve and segmented forms read them alike
 struct DP {
     int cap, nmaxpartj, nmax, semi, f32, nf;
     int ncd[3];
@@ -42,15 +47,15 @@ struct DP {
     double ke_coef, kacl_coef, ktdelta, GI;
     double grav[3], prif, den0, eps, celerita, alfamon, kin_visc;
     double cfl, vsc_coeff, pesodt, tetap, tetav;
-    // FP32-mixed copies
-    float f_h, f_unosuh, f_unosusquareh, f_eta, f_eta2, f_ke_coef, f_kacl_coef, f_coefke;
-    float f_dcd[3], f_alfamon, f_celerita, f_kin_visc;
+    // unit of the integer positions: 2^-28 of the largest cell side
+    double lsb, inv_lsb;
+    // FP32-mixed pair sums: h, eta and eta2 in units of lsb (f_q = lsb / h)
+    float f_q, f_etal, f_eta2l, f_dcd[3], f_kin_visc;
     // the density slot of the FP32 velocity records holds rho - den0; the
     // linear EoS p = eps/den0 (rho - den0) + prif gives the pressure from it
     float f_den0, f_eosk, f_prif;
     // every particle of the solve has the mass f_mass (one medium, one dx:
-    // SetParticleParameters.f90:56-57): the pressure smoothing then reads one
-    // (x, y, z, rho - den0) record per neighbour
+    // SetParticleParameters.f90:56-57)
     int umass;
     float f_mass;
     // density_thresholds == 1: Leapfrog_continuity.f90:61-68 clamps the
@@ -68,26 +73,41 @@ struct DP {
     int seg;   // segment index
     int base;  // first sorted slot of the segment (a multiple of 256)
     int scap;  // slots reserved for the segment
+    int toff;  // first tile id (a multiple of 256)
     int koff;  // first cell key: keys koff .. koff+nmax-1 are the cells, koff+nmax the
                // particles out of the grid (a multiple of 256)
     int foff;  // first frontier face of the segment in the context's face array
     int eoff;  // first convex edge of the segment in the context's edge array
     int ne;    // its convex edges (NumBEdges)
     int nopen; // its open faces (NumOpenFaces)
+    // tiles (boxes of tdim cells, ntile of them along each axis) and the slots
+    // a tile may have for its lists to be LDS slots (0: never)
+    int tdim[3], ntile[3], tcap;
+    // reciprocals for div_inv: ncd[0] ncd[1], ncd[0]; tdim; ntile[0] ntile[1], ntile[0]; tdim[1] + 2
+    double inv_nij, inv_ni, inv_tdim[3], inv_ntij, inv_nti, inv_ry;
     // DB-SPH walls (Domain%tipo = "bsph"): nw wall elements; the DBSPH
     // section's Gamma_limiter_flag, FS_allowed and negative_wall_p_allowed
     int dbsph, nw, gamma_lim, fs_allowed, neg_wall_p, muscl_bnd, nkin;
     double kin_c[3];  // rotation centre of the wall kinematics
 };
 
-// Segment maps of a segmented context, passed by value to the kernels that
-// take a segmented form.  Slots and keys are partitioned in whole 256-blocks,
+using DPC = const __attribute__((address_space(4))) DP;
+
+// The constants of a context's segments and, for a segmented context, the
+// segment maps.  Slots, keys and tiles are partitioned in whole 256-blocks,
 // so a workgroup of a particle or key kernel lies in one segment.
 struct Seg {
-    const DP* P;        // per-segment constants
+    DPC* P;             // per-segment constants
     const int* pblk;    // segment of each 256-slot block
     const int* kblk;    // segment of each 256-key block
+    const int* tblk;    // segment of each 256-tile block
     int nseg;
+};
+
+// the tiles that hold particles: *n ids
+struct Tiles {
+    const int* list;
+    const int* n;
 };
 
 // one convex frontier edge (BoundaryConvexEdge, FindBoundaryConvexEdges3D.f90):

@@ -7,12 +7,17 @@
 //   rp   double2 (rho, p)                 x3 buffers (sort -> continuity -> smoothing)
 //   lam  int32 laminar flag               x2 buffers
 //   acc  double4, dden, vpres             outputs of the passes
-//   FP32-mixed mirrors: xmf float4 (cell-relative x,y,z, mass), velf float4,
-//   rpf float2, written by the same kernels that write the FP64 fields.
-//   Neighbour list: entry k of particle i at nb_index(N, i, k) (groups of 8
-//   entries per particle, a group rank contiguous over i), the sorted index of
+//   xq int4 (x, y, z in units of P.lsb modulo 2^32, mass): separations of
+//   the search and of the FP32-mixed pair sums
+//   FP32-mixed: vf float4 (vx, vy, vz, rho - den0) x2 buffers, dr float rho - den0
+//   Neighbour list, in groups of 8 entries per particle, a group rank
+//   contiguous over the particles; count in nnb[i].  Tiles (below) that fit
+//   the pair passes' LDS: 16-bit entries, the neighbour's slot of the
+//   particle's tile times 16 (nb16_index), filled up to whole eights with the
+//   particle itself.
+//   Elsewhere: entry k of particle i at nb_index(N, i, k), the sorted index of
 //   the k-th neighbour in bits 0..26 and its stencil cell code
-//   (dx+1)+3(dy+1)+9(dz+1) in bits 27..31; count in nnb[i].
+//   (dx+1)+3(dy+1)+9(dz+1) in bits 27..31.
 //
 // FP64 kernels are compiled with -ffp-contract=off and evaluate every
 // expression in the order of the cited reference line, so sums over a list in
@@ -26,29 +31,15 @@
 
 namespace sph {
 
-// FP32 particle records of the passes that read velocities are interleaved:
-// slot i of a record buffer holds the cell-relative position (x, y, z, mass)
-// at float4 2i and (vx, vy, vz, rho) at 2i+1, so a neighbour's position and
-// velocity come from one 32-byte run.  F4View is the strided view of one of
-// the two halves.  The neighbour search and the pressure smoothing read the
-// positions alone from the compact array xmf.
-template <class T>
-struct F4View {
-    T* p;
-    __host__ __device__ __forceinline__ T& operator[](size_t i) const { return p[2 * i]; }
-};
-using F4In = F4View<const float4>;
-using F4Out = F4View<float4>;
-
 // ----------------------------------------------------------------------------
 // grid helpers: CellNumber.f90:53-59, ParticleCellNumber.f90:52-62,
 // CellIndices.f90:51-63 (1-based cell ids, 0 = outside)
 // ----------------------------------------------------------------------------
-__device__ __forceinline__ int d_cell_number(const DP& P, int i, int j, int k) {
+__device__ __forceinline__ int d_cell_number(DPC& P, int i, int j, int k) {
     if (i < 1 || i > P.ncd[0] || j < 1 || j > P.ncd[1] || k < 1 || k > P.ncd[2]) return 0;
     return ((k - 1) * P.ncd[1] + (j - 1)) * P.ncd[0] + i;
 }
-__device__ __forceinline__ int d_particle_cell(const DP& P, double x, double y, double z) {
+__device__ __forceinline__ int d_particle_cell(DPC& P, double x, double y, double z) {
     const double xp = x - P.extr_lo[0];
     const double yp = y - P.extr_lo[1];
     const double zp = z - P.extr_lo[2];
@@ -57,11 +48,14 @@ __device__ __forceinline__ int d_particle_cell(const DP& P, double x, double y, 
     const int j = P.dim == 2 ? 1 : (int)ceil(yp / P.dcd[1]);  // :59-61 (2D: j = 1)
     return d_cell_number(P, i, j, k);
 }
-__device__ __forceinline__ void d_cell_indices(const DP& P, int nc, int& i, int& j, int& k) {
+// x / d for 0 <= x < 2^30 from inv = 1.0 / d: (x + 1/2) / d is at least 1/(2 d)
+// away from an integer, far above the product's rounding
+__device__ __forceinline__ int div_inv(int x, double inv) { return (int)(((double)x + 0.5) * inv); }
+__device__ __forceinline__ void d_cell_indices(DPC& P, int nc, int& i, int& j, int& k) {
     const int nij = P.ncd[0] * P.ncd[1];
-    k = (nc - 1) / nij + 1;
+    k = div_inv(nc - 1, P.inv_nij) + 1;
     const int ncij = nc - nij * (k - 1);
-    j = (ncij - 1) / P.ncd[0] + 1;
+    j = div_inv(ncij - 1, P.inv_ni) + 1;
     i = ncij - P.ncd[0] * (j - 1);
 }
 
@@ -85,7 +79,7 @@ __device__ __forceinline__ int xcd_block(int nblocks) {
 // ----------------------------------------------------------------------------
 struct K64 { double K1, K2, K3, W; };
 
-__device__ __forceinline__ void kvals64(const DP& P, double rij, bool need12, bool need3,
+__device__ __forceinline__ void kvals64(DPC& P, double rij, bool need12, bool need3,
                                         bool needW, K64& K) {
     const double rij2 = rij;
     const double r = sqrt(rij);
@@ -114,55 +108,6 @@ __device__ __forceinline__ void kvals64(const DP& P, double rij, bool need12, bo
     }
 }
 
-struct K32 { float K1, K2, K3, W; };
-
-// FP32 form: same piecewise cubic spline, single-precision hardware sqrt/rcp
-__device__ __forceinline__ void kvals32(const DP& P, float rij, bool need12, bool need3,
-                                        bool needW, K32& K) {
-    const float r = __builtin_amdgcn_sqrtf(rij);
-    const float q = r * P.f_unosuh;
-    const float q2 = rij * P.f_unosusquareh;
-    // every listed pair has r <= 2h, where both branches of the spline and its
-    // derivatives vanish at q = 2, so no cut-off test is needed
-    K.K1 = K.K2 = K.K3 = K.W = 0.0f;
-    const bool outer = q >= 1.0f;
-    const float denom = __builtin_amdgcn_rcpf(r + P.f_eta);
-    if (need12) {
-        float gm = -2.0f * q + 1.5f * q2;
-        if (outer) gm = -gm + q2 - 2.0f;
-        K.K1 = gm * P.f_ke_coef * denom;
-        K.K2 = K.K1 * __builtin_amdgcn_rcpf(rij + P.f_eta2);
-    }
-    if (need3) K.K3 = (-12.0f - 3.0f * q2 + 12.0f * q) * P.f_kacl_coef * denom;
-    if (needW) {
-        const float t = 2.0f - q;
-        const float wu = outer ? t * t * t * 0.166666666667f : 0.666666667f + q2 * (q * 0.5f - 1.0f);
-        K.W = wu * P.f_coefke;
-    }
-}
-
-// The 27 stencil-cell offsets (dx,dy,dz) * dcd in FP32, indexed by the
-// stencil code of a list entry; each workgroup keeps a copy in LDS.
-__shared__ float4 g_soff[27];
-
-__device__ __forceinline__ void stencil_offsets(const DP& P) {
-    if (threadIdx.x < 27) {
-        const int c = threadIdx.x;
-        g_soff[c] = make_float4((float)(c % 3 - 1) * P.f_dcd[0], (float)((c / 3) % 3 - 1) * P.f_dcd[1],
-                                (float)(c / 9 - 1) * P.f_dcd[2], 0.0f);
-    }
-    __syncthreads();
-}
-
-// cell-relative FP32 separation x_i - x_j from the stencil code of j
-__device__ __forceinline__ void rag32(float4 xi, float4 xj, uint32_t code, float& r0, float& r1,
-                                      float& r2) {
-    const float4 o = g_soff[code >> NB_SHIFT];
-    r0 = (xi.x - xj.x) - o.x;
-    r1 = (xi.y - xj.y) - o.y;
-    r2 = (xi.z - xj.z) - o.z;
-}
-
 // ----------------------------------------------------------------------------
 // SA-SPH geometry: LocalNormalCoordinates.f90:55-87 + IsPointInternal.f90
 // ----------------------------------------------------------------------------
@@ -189,6 +134,58 @@ __device__ __forceinline__ bool d_point_internal(const DFace& F, double px0, dou
 }
 
 // ----------------------------------------------------------------------------
+// Tiles: the grid is cut into boxes of P.tdim cells.  The particles of a tile
+// (home) and those of the cells around it (halo) are, row by row (fixed j, k;
+// consecutive cells of a row are consecutive in memory), the tile's slots: a
+// particle's neighbours all have a slot of its tile.  Where the slots fit the
+// LDS of the pair passes (P.tcap), the neighbour lists hold 16-bit slot
+// offsets; elsewhere 32-bit sorted indices with the stencil code.
+// ----------------------------------------------------------------------------
+constexpr int TILE_CAP_L = 2496, TILE_CAP_M = 1632, TILE_CAP_S = 1216;  // 2, 3 and 4 workgroups a CU of 32 bytes a slot
+constexpr int TILE_WG = 512;   // most threads of a pair pass
+constexpr int TILE_U = 5;      // slots a thread stages at a time
+constexpr int TILE_G2 = 40000;  // particles below which two lanes take a particle
+constexpr int TILE_MIN = 300, TILE_MIN2 = 200, TILE_MIN_L = 500;  // tiles of water a solve is cut into (choose_tile)
+struct TileS {
+    int g[64];      // row r: sorted index of its first particle
+    int l[65];      // its first slot; l[rows] the number of slots
+    int h0[64];     // home part: sorted index of its first particle
+    int hp[65];     // and home particles before the row; hp[rows] their number
+};
+
+// rows of a tile with its halo, at most 64 (choose_tile)
+__device__ __forceinline__ int tile_rows(DPC& P) { return (P.tdim[1] + 2) * (P.tdim[2] + 2); }
+
+// row `lane` of the tile (ti, tj, tk): its slot range and home range
+__device__ __forceinline__ void tile_row(DPC& P, const int* __restrict__ start, int ti, int tj, int tk,
+                                         int lane, int& g0, int& g1, int& h0, int& h1) {
+    g0 = g1 = h0 = h1 = 0;
+    const int ry = P.tdim[1] + 2;
+    if (lane >= ry * (P.tdim[2] + 2)) return;
+    const int rk = div_inv(lane, P.inv_ry), rj = lane - rk * ry;
+    const int ni = P.ncd[0], nj = P.ncd[1], nk = P.ncd[2];
+    const int i0 = ti * P.tdim[0] + 1, i1 = min(i0 + P.tdim[0] - 1, ni);
+    const int j = tj * P.tdim[1] + rj, k = tk * P.tdim[2] + rk;
+    if (j < 1 || j > nj || k < 1 || k > nk) return;
+    const int rb = P.koff + ((k - 1) * nj + (j - 1)) * ni - 1;
+    g0 = start[rb + max(i0 - 1, 1)];
+    g1 = start[rb + min(i1 + 1, ni) + 1];
+    if (rj >= 1 && rj <= P.tdim[1] && rk >= 1 && rk <= P.tdim[2]) {
+        h0 = start[rb + i0];
+        h1 = start[rb + i1 + 1];
+    }
+}
+
+// the tile of a context's list entry: coordinates in its segment's tile grid
+__device__ __forceinline__ void tile_coords(DPC& P, int id, int& ti, int& tj, int& tk) {
+    const int t = id - P.toff;
+    tk = div_inv(t, P.inv_ntij);
+    const int r = t - tk * P.ntile[0] * P.ntile[1];
+    tj = div_inv(r, P.inv_nti);
+    ti = r - tj * P.ntile[0];
+}
+
+// ----------------------------------------------------------------------------
 // sort: OrdGrid1.f90:58-105 as a device counting sort.  The particles arrive
 // almost in cell order (they moved less than a cell since the last sort), so
 // a workgroup's 256 particles fall in a narrow window of cells: it counts
@@ -202,21 +199,22 @@ constexpr int HIST_W = 512;
 // Segmented contexts (SG): the workgroup's segment comes from the slot-block
 // map; slots, keys, ids and the removal list are the segment's.
 template <bool SG>
-__global__ __launch_bounds__(256) void k_cell_count(DP P0, Seg S, const double4* __restrict__ xm,
+__global__ __launch_bounds__(256) void k_cell_count(Seg S, const double4* __restrict__ xm,
                                                     const double4* __restrict__ vel,
                                                     int* __restrict__ key, int* __restrict__ slot,
                                                     int* __restrict__ cnt, int* __restrict__ idslot,
                                                     int* __restrict__ rmids, int* iscal,
-                                                    int* __restrict__ gone) {
+                                                    int* __restrict__ gone, int* ntile) {
     __shared__ int base[HIST_W];
     __shared__ int wcnt[4][HIST_W];  // particles of each window cell per wave
     __shared__ int cmin;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(blockIdx.x * blockDim.x) >> 8]) : 0;
-    const DP& P = SG ? S.P[sg] : P0;
+    DPC& P = S.P[sg];
     iscal += sg * IS_COUNT;
     rmids += sg * RM_CAP;
     const int n = iscal[IS_N];
+    if (i == 0) *ntile = 0;  // k_scatter counts them
     for (int b = threadIdx.x; b < HIST_W; b += blockDim.x)
         for (int w = 0; w < 4; ++w) wcnt[w][b] = 0;
     if (threadIdx.x == 0) cmin = 0x7fffffff;
@@ -316,11 +314,11 @@ __global__ __launch_bounds__(256) void k_scan_local(const int* __restrict__ in, 
 // lane; removals are rare (particles leaving a closed tank).
 // Segmented contexts: one lane per segment.
 template <bool SG>
-__global__ void k_renumber(DP P0, Seg S, int* __restrict__ rmids, const int* __restrict__ idslot,
+__global__ void k_renumber(Seg S, int* __restrict__ rmids, const int* __restrict__ idslot,
                            double4* __restrict__ vel, int* iscal) {
     const int sg = SG ? (int)(blockIdx.x * blockDim.x + threadIdx.x) : 0;
     if (SG ? sg >= S.nseg : threadIdx.x != 0) return;
-    const int pbase = SG ? S.P[sg].base : P0.base;
+    const int pbase = S.P[sg].base;
     iscal += sg * IS_COUNT;
     rmids += sg * RM_CAP;
     const int m = iscal[IS_NRM];
@@ -399,13 +397,44 @@ __global__ void k_seg_add(Seg S, int* __restrict__ start, const int* __restrict_
     if (k < m) start[k] += adj[S.kblk[k >> 8]];
 }
 
+// Workgroups past the first nsb list the tiles that hold particles (a tile per
+// lane, ids in ascending order within a workgroup) instead.
 template <bool SG>
-__global__ void k_scatter(DP P0, Seg S, const int* __restrict__ key, const int* __restrict__ slot,
-                          const int* __restrict__ start, const double4* __restrict__ vel,
-                          int* __restrict__ perm, int* __restrict__ pid, const int* iscal) {
+__global__ __launch_bounds__(256) void k_scatter(Seg S, const int* __restrict__ key,
+                                                 const int* __restrict__ slot, const int* __restrict__ start,
+                                                 const double4* __restrict__ vel, int* __restrict__ perm,
+                                                 int* __restrict__ pid, const int* iscal, int nsb,
+                                                 int* __restrict__ tlist, int* ntile) {
+    if ((int)blockIdx.x >= nsb) {
+        __shared__ int wn[4], first;
+        const int b = blockIdx.x - nsb, id = b * 256 + threadIdx.x;
+        DPC& P = S.P[SG ? __builtin_amdgcn_readfirstlane(S.tblk[b]) : 0];
+        int n = 0;
+        if (id - P.toff < P.ntile[0] * P.ntile[1] * P.ntile[2]) {
+            int ti, tj, tk;
+            tile_coords(P, id, ti, tj, tk);
+            const int i0 = ti * P.tdim[0], i1 = min(i0 + P.tdim[0], P.ncd[0]);
+            const int j1 = min((tj + 1) * P.tdim[1], P.ncd[1]), k1 = min((tk + 1) * P.tdim[2], P.ncd[2]);
+            for (int k = tk * P.tdim[2]; k < k1; ++k)
+                for (int j = tj * P.tdim[1]; j < j1; ++j) {
+                    const int rb = P.koff + (k * P.ncd[1] + j) * P.ncd[0];
+                    n += start[rb + i1] - start[rb + i0];
+                }
+        }
+        const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+        const unsigned long long m = __ballot(n > 0);
+        if (lane == 0) wn[wid] = __popcll(m);
+        __syncthreads();
+        if (threadIdx.x == 0) first = atomicAdd(ntile, wn[0] + wn[1] + wn[2] + wn[3]);
+        __syncthreads();
+        int at = first + __popcll(m & ((1ull << lane) - 1ull));
+        for (int w = 0; w < wid; ++w) at += wn[w];
+        if (n > 0) tlist[at] = id;
+        return;
+    }
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(blockIdx.x * blockDim.x) >> 8]) : 0;
-    const int pbase = SG ? S.P[sg].base : P0.base;
+    const int pbase = S.P[sg].base;
     if (i - pbase >= iscal[sg * IS_COUNT + IS_N]) return;
     const int d = start[key[i]] + slot[i];
     perm[d] = i;
@@ -418,13 +447,13 @@ __global__ void k_scatter(DP P0, Seg S, const int* __restrict__ key, const int* 
 constexpr int CSORT_CAP = 6144;
 
 template <bool SG>
-__global__ __launch_bounds__(256) void k_cell_sort(DP P0, Seg S, const int* __restrict__ start,
+__global__ __launch_bounds__(256) void k_cell_sort(Seg S, const int* __restrict__ start,
                                                    int* __restrict__ perm, int* __restrict__ pid) {
     __shared__ int sid[CSORT_CAP];
     __shared__ int sperm[CSORT_CAP];
     const int c0 = blockIdx.x * 256;
     const int sg = SG ? __builtin_amdgcn_readfirstlane(S.kblk[blockIdx.x]) : 0;
-    const DP& P = SG ? S.P[sg] : P0;
+    DPC& P = S.P[sg];
     const int c1 = min(c0 + 256, P.koff + P.nmax);
     if (c0 >= c1) return;  // a block of the out-of-grid key or of the padding
     const int g0 = start[c0], g1 = start[c1];
@@ -468,25 +497,32 @@ __global__ __launch_bounds__(256) void k_cell_sort(DP P0, Seg S, const int* __re
     }
 }
 
-// permutes the state into the new order and writes the FP32 cell-relative
-// positions (used by the neighbour test in both precisions)
+// A coordinate relative to the grid's corner in units of lsb, modulo 2^32:
+// the difference of two particles' values, as a signed integer, is their
+// separation wherever that is below 2^31 lsb (eight cells).
+__device__ __forceinline__ int lsb_units(double x, double inv) {
+    const double t = rint(x * inv);
+    return (int)(uint32_t)(t - floor(t * 0x1p-32) * 0x1p32);
+}
+
+// permutes the state into the new order and writes the integer positions (the
+// neighbour test's in both precisions)
 template <bool SG>
-__global__ void k_gather(DP P0, Seg S, const int* __restrict__ perm, const int* __restrict__ key,
+__global__ void k_gather(Seg S, const int* __restrict__ perm, const int* __restrict__ key,
                          const double4* __restrict__ xm_s, const double4* __restrict__ vel_s,
                          const double2* __restrict__ rp_s, const int* __restrict__ lam_s,
                          const double4* __restrict__ acc_s, double4* __restrict__ xm_d,
                          double4* __restrict__ vel_d, double2* __restrict__ rp_d,
                          int* __restrict__ lam_d, double4* __restrict__ acc_d,
-                         int* __restrict__ cell_d, float4* __restrict__ xmf, F4Out xmf0, F4Out xmf1,
-                         F4Out velf,
-                         float2* __restrict__ rpf, const int* __restrict__ start, int* iscal,
+                         int* __restrict__ cell_d, int4* __restrict__ xq, float4* __restrict__ vf,
+                         const int* __restrict__ start, int* iscal,
                          const double* __restrict__ dd_s, double* __restrict__ dd_d,
                          const double* __restrict__ vp_s, double* __restrict__ vp_d,
                          const double* __restrict__ g_s, double* __restrict__ g_d,
                          const double* __restrict__ h_s, double* __restrict__ h_d) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(blockIdx.x * blockDim.x) >> 8]) : 0;
-    const DP& P = SG ? S.P[sg] : P0;
+    DPC& P = S.P[sg];
     iscal += sg * IS_COUNT;
     const int nin = start[P.koff + P.nmax] - P.base;  // particles still inside the grid
     if (p == P.base) {
@@ -513,189 +549,91 @@ __global__ void k_gather(DP P0, Seg S, const int* __restrict__ perm, const int* 
     }
     const int c = key[s] - P.koff + 1;
     cell_d[p] = c;
-    int ci, cj, ck;
-    d_cell_indices(P, c, ci, cj, ck);
-    const double ox = P.extr_lo[0] + P.dcd[0] * (double)(ci - 1);
-    const double oy = P.extr_lo[1] + P.dcd[1] * (double)(cj - 1);
-    const double oz = P.extr_lo[2] + P.dcd[2] * (double)(ck - 1);
-    const float4 xr = make_float4((float)(x.x - ox), (float)(x.y - oy), (float)(x.z - oz), (float)x.w);
-    xmf[p] = xr;
-    if (P.f32) {  // the position half of both FP32 record buffers
-        xmf0[p] = xr;
-        xmf1[p] = xr;
-        velf[p] = make_float4((float)v.x, (float)v.y, (float)v.z, (float)(r.x - P.den0));
-        rpf[p] = make_float2((float)r.x, (float)r.y);
-    }
+    xq[p] = make_int4(lsb_units(x.x - P.extr_lo[0], P.inv_lsb), lsb_units(x.y - P.extr_lo[1], P.inv_lsb),
+                      lsb_units(x.z - P.extr_lo[2], P.inv_lsb), __float_as_int((float)x.w));
+    if (P.f32) vf[p] = make_float4((float)v.x, (float)v.y, (float)v.z, (float)(r.x - P.den0));
 }
 
 // ----------------------------------------------------------------------------
 // neighbour lists: CalcVarLength.f90:133-242 — stencil y -> x -> z, ascending
 // particle id in a cell, r^2 <= (2h)^2 in FP64, self included, truncation past
-// NMAXPARTJ.  Candidates are tested on FP32 cell-relative positions;
-// a candidate whose FP32 r^2 lies within a relative 4e-5 of (2h)^2 is decided
-// by the reference's FP64 expression on the FP64 positions, so the lists are
-// exactly the reference's.  (Each relative coordinate is rounded once from
-// |x - corner| <= dcd, so the FP32 separation is within ~5e-7 dcd per axis and
-// the FP32 r^2 within ~1.5e-6 relative of (2h)^2 near the cut-off.)
+// NMAXPARTJ.  Candidates are tested in FP32 on separations of the integer
+// positions; a candidate whose FP32 r^2 lies within a relative 4e-5 of (2h)^2
+// is decided by the reference's FP64 expression on the FP64 positions, so the
+// lists are exactly the reference's.
 // ----------------------------------------------------------------------------
-// List writer of one lane (cells too dense for the wavefront form below): the
-// entries are collected in a shift register of four and stored as one 16-byte
-// vector per full run; flush() stores the last, partial run (its unused tail
-// slots are past the count and never read).  A run is stored only while it
-// lies inside the particle's list capacity (nb_stride(NMAXPARTJ)); the count
-// keeps running, so the first NMAXPARTJ entries are the stored ones, as in
-// the reference.
-static_assert(NB_G == 8, "the list writer stores runs inside 8-entry groups");
-struct NbOut {
-    static constexpr int B = 4;
-    uint32_t* wp;  // first slot of the current run
-    int cnt;
-    int lim;       // list capacity: runs ending past it are not stored
-    size_t jump;   // from the last run of a group to the first slot of the particle's next group
-    uint32_t b[B]; // b[B-1] is the newest entry
-    __device__ __forceinline__ NbOut(uint32_t* nbr, size_t N, int p, int stride)
-        : wp(nbr + nb_index(N, p, 0)), cnt(0), lim(stride), jump(N * NB_G - (NB_G - B)) {
-#pragma unroll
-        for (int u = 0; u < B; ++u) b[u] = 0u;
-    }
-    __device__ __forceinline__ void store_run() {
-        uint4* q = reinterpret_cast<uint4*>(wp);
-        q[0] = make_uint4(b[0], b[1], b[2], b[3]);
-    }
-    __device__ __forceinline__ void push(uint32_t e, int) {
-#pragma unroll
-        for (int u = 0; u + 1 < B; ++u) b[u] = b[u + 1];
-        b[B - 1] = e;
-        ++cnt;
-        if ((cnt & (B - 1)) == 0) {
-            if (cnt <= lim) store_run();
-            wp += ((cnt & (NB_G - 1)) == 0) ? jump : (size_t)B;
-        }
-    }
-    // the r = cnt % B entries since the last run, moved to the run's first slots
-    __device__ __forceinline__ void flush() {
-        const int r = cnt & (B - 1);
-        if (r == 0 || cnt > lim) return;
-        uint32_t o[B];
-#pragma unroll
-        for (int u = 0; u < B; ++u) {
-            uint32_t v = 0u;
-#pragma unroll
-            for (int s = 1; s < B; ++s)  // slot u holds b[B - r + u] when u < r
-                if (r == s && u < s) v = b[B - s + u];
-            o[u] = v;
-        }
-#pragma unroll
-        for (int u = 0; u < B; ++u) b[u] = o[u];
-        store_run();
-    }
-};
-
-// The neighbour test of one candidate and the list append: FP32 on
-// cell-relative positions, and the reference's FP64 expression on the FP64
-// positions inside the guard band.  xo: FP32 position of particle p relative
-// to the candidate's cell corner (its own cell-relative position minus the
-// stencil offset), xj: the candidate's cell-relative position, m: its sorted
-// index.  The FP32 r^2 (fused multiply-adds) is within ~3e-7 relative of the
-// exact one, far inside the 4e-5 band.  Every accepted candidate is counted;
-// the first NMAXPARTJ are stored (the reference keeps the first NMAXPARTJ of
-// its list, CalcVarLength.f90:200-207), so the loops have no early exit.
-__device__ __forceinline__ void nb_test(const DP& P, const double4* __restrict__ xm, double4 xi64,
-                                        float4 xo, float4 xj, int m, uint32_t ctag, float lo, float hi,
-                                        NbOut& w, int mj) {
-    const float r0 = xo.x - xj.x, r1 = xo.y - xj.y, r2 = xo.z - xj.z;
-    const float r2f = __builtin_fmaf(r0, r0, __builtin_fmaf(r1, r1, r2 * r2));
-    if (r2f <= hi) {
-        bool acc = r2f < lo;
-        if (!acc) {  // guard band: the reference's FP64 test
-            const double4 xj64 = xm[m];
-            const double d0 = xi64.x - xj64.x;
-            const double d1 = xi64.y - xj64.y;
-            const double d2 = xi64.z - xj64.z;
-            const double rij = d0 * d0 + d1 * d1 + d2 * d2;
-            acc = !(rij > P.square_doubleh);
-        }
-        if (acc) w.push((uint32_t)m | ctag, mj);
-    }
-}
-
-// Candidates [b,e) of one stencil cell, four loads ahead: load(x) gives the
-// FP32 position of slot x.
-template <class Load>
-__device__ __forceinline__ void nb_cell(const DP& P, const double4* __restrict__ xm, double4 xi64,
-                                        float4 xi, float4 o, uint32_t ctag, int b, int e,
-                                        Load&& load, float lo, float hi, NbOut& w, int mj) {
-    const float4 xo = make_float4(xi.x - o.x, xi.y - o.y, xi.z - o.z, 0.0f);
-    int x = b;
-    for (; x + 4 <= e; x += 4) {
-        const float4 q0 = load(x), q1 = load(x + 1), q2 = load(x + 2), q3 = load(x + 3);
-        nb_test(P, xm, xi64, xo, q0, x, ctag, lo, hi, w, mj);
-        nb_test(P, xm, xi64, xo, q1, x + 1, ctag, lo, hi, w, mj);
-        nb_test(P, xm, xi64, xo, q2, x + 2, ctag, lo, hi, w, mj);
-        nb_test(P, xm, xi64, xo, q3, x + 3, ctag, lo, hi, w, mj);
-    }
-    for (; x < e; ++x) nb_test(P, xm, xi64, xo, load(x), x, ctag, lo, hi, w, mj);
-}
-
-// List of particle p from global memory (candidates gathered through L1/L2).
-__device__ int nb_particle_global(const DP& P, int p, const double4* __restrict__ xm,
-                                  const float4* __restrict__ xmf, const int* __restrict__ cell,
+// One lane per particle, candidates from global memory (cells too dense for
+// the wavefront form below).  aux: per stencil cell in list order what turns
+// a sorted index into its list entry.  Every accepted candidate is counted;
+// the first NMAXPARTJ are stored, as in the reference.
+__device__ int nb_particle_global(DPC& P, int p, const double4* __restrict__ xm,
+                                  const int4* __restrict__ xq, const int* __restrict__ cell,
                                   const int* __restrict__ start, uint32_t* __restrict__ nbr,
-                                  float lo, float hi, bool& ov) {
+                                  const int* aux, bool fits, float lo, float hi, bool& ov) {
     const int ni = P.ncd[0], nj = P.ncd[1], nk = P.ncd[2];
     const int mj = P.nmaxpartj;
     const size_t N = P.cap;
+    uint16_t* nbr16 = reinterpret_cast<uint16_t*>(nbr);
     int ic, jc, kc;
     d_cell_indices(P, cell[p], ic, jc, kc);
-    const float4 xi = xmf[p];
+    const int4 xi = xq[p];
     const double4 xi64 = xm[p];
-    NbOut w(nbr, N, p, nb_stride(mj));
-    auto load = [&](int x) { return xmf[x]; };
-    for (int dy = -1; dy <= 1; ++dy) {
-        const int jj = jc + dy;
-        if (jj < 1 || jj > nj) continue;
-        for (int dx = -1; dx <= 1; ++dx) {
-            const int ii = ic + dx;
-            if (ii < 1 || ii > ni) continue;
-            for (int dz = -1; dz <= 1; ++dz) {
-                const int kk = kc + dz;
-                if (kk < 1 || kk > nk) continue;
-                const int cn = ((kk - 1) * nj + (jj - 1)) * ni + ii;
-                const int code = (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1);
-                nb_cell(P, xm, xi64, xi, g_soff[code], (uint32_t)code << NB_SHIFT, start[P.koff + cn - 1],
-                        start[P.koff + cn], load, lo, hi, w, mj);
+    int k = 0;
+    for (int t = 0; t < 27; ++t) {
+        const int jj = jc + t / 9 - 1, ii = ic + (t / 3) % 3 - 1, kk = kc + t % 3 - 1;
+        if (ii < 1 || ii > ni || jj < 1 || jj > nj || kk < 1 || kk > nk) continue;
+        const int key = P.koff + ((kk - 1) * nj + (jj - 1)) * ni + ii - 1;
+        for (int m = start[key]; m < start[key + 1]; ++m) {
+            const int4 xj = xq[m];
+            const float r0 = (float)(xi.x - xj.x), r1 = (float)(xi.y - xj.y), r2 = (float)(xi.z - xj.z);
+            const float rr = __builtin_fmaf(r0, r0, __builtin_fmaf(r1, r1, r2 * r2));
+            if (rr > hi) continue;
+            if (!(rr < lo)) {  // guard band: the reference's FP64 test
+                const double4 xj64 = xm[m];
+                const double d0 = xi64.x - xj64.x;
+                const double d1 = xi64.y - xj64.y;
+                const double d2 = xi64.z - xj64.z;
+                if (d0 * d0 + d1 * d1 + d2 * d2 > P.square_doubleh) continue;
             }
+            if (k < mj) {
+                if (fits) nbr16[nb16_index(N, p, k)] = (uint16_t)((m + aux[t]) << 4);
+                else nbr[nb_index(N, p, k)] = (uint32_t)m | (uint32_t)aux[t];
+            }
+            ++k;
         }
     }
-    w.flush();
-    ov = w.cnt > mj;
-    return min(w.cnt, mj);
+    ov = k > mj;
+    k = min(k, mj);
+    if (fits)
+        for (int q = k; q & 7; ++q) nbr16[nb16_index(N, p, q)] = (uint16_t)((p + aux[13]) << 4);
+    return k;
 }
 
 // One wavefront per cell.  All particles of a cell share the candidates of its
 // 27 stencil cells (475 at 17.6 particles per cell), in the same order: the
 // lanes hold them in registers (candidate 64 q + lane in chunk q), relative
-// to the cell's corner, and the particles of the cell are taken one after the
-// other.  With c = |xj|^2 kept per candidate, the test
+// to the cell's first particle, and the particles of the cell are taken one
+// after the other.  With c = |xj|^2 kept per candidate, the test
 // c - 2 xi.xj <= (2h)^2 - |xi|^2 is three fused multiply-adds and a compare
 // for 64 candidates; the hits of a chunk are a lane mask, so a hit's place in
 // the list is the count of mask bits below it, and the list is built in LDS
-// and stored in 16-byte pieces.  VALU issue bounds it: 8 instructions per 64
+// and stored in 16-byte pieces.  VALU issue bounds it: 9 instructions per 64
 // candidates, against 19 per candidate and lane (with the append in the
 // divergent branch of every test) for one lane per particle.
-// 576,000 particles: 219 -> 171 us; a batch of eight solves, 536,000: 334 -> 159;
-// 1,440 particles (one lane's 475 serial tests were the time): 71 -> 17 us.
+// 576,000 particles: 219 -> 163 us; a batch of eight solves, 536,000: 334 ->
+// 152; 1,440 particles (one lane's 475 serial tests were the time): 71 -> 18 us.
 //
-// The FP32 test: a candidate's coordinates are within 2 dcd of the corner, so
-// with the rounding of the sums r^2 is within 3.5e-6 dcd^2; the guard band
-// 4e-5 (2h)^2 (wider for cells larger than 2h) goes to the FP64 test.
+// The FP32 test: a candidate's coordinates are within 2 dcd of the first
+// particle, so with the rounding of the sums r^2 is within 3.5e-6 dcd^2; the
+// guard band 4e-5 (2h)^2 (wider for cells larger than 2h) goes to the FP64 test.
 // A wavefront takes the cells whose first particle lies in its NBC_SLOTS
 // sorted slots: about one cell, so small solves spread over the chip.
 // Cells with more candidates than the registers hold (denser than 1.35 times
 // water) take one lane per particle from global memory.
 constexpr int NBC_CH = 10;             // chunks of 64 candidates in registers
 constexpr int NBC_MAX = 64 * NBC_CH;
-constexpr int NBC_SLOTS = 16;          // sorted slots per wavefront
+constexpr int NBC_SLOTS = 16, NBC_SLOTS_L = 64;  // sorted slots per wavefront: small, large solves
+constexpr int NBC_LARGE = 150000;      // particles from which the chip is full with 64 slots per wavefront
 constexpr int NBC_PAIRS = 64;          // pair counters, one 128-byte line each
 constexpr int NBC_PSTRIDE = 16;
 
@@ -705,16 +643,20 @@ __device__ __forceinline__ float readlane_f(float v, int l) {
 
 // The cell's particles hb .. hb+hc-1 against its `total` candidates, NCH chunks
 // of 64 (64 (NCH-1) < total <= 64 NCH).  A lane without a hit writes to the
-// slot past the list, so a chunk's append has no branch.  Returns the sum of
-// the list lengths without the particles themselves; over counts truncated lists.
-template <int NCH>
-__device__ __forceinline__ int nb_cell_lists(const DP& P, const double4* __restrict__ xm,
-                                             const float4* __restrict__ xmf, const uint32_t* cand,
-                                             uint32_t* list, int total, int hb, int hc, float lo, float hi,
+// slot past the list, so a chunk's append has no branch.  FIT: 16-bit entries
+// (the tile fits LDS).  Returns the sum of the list lengths without the
+// particles themselves; over counts truncated lists.
+template <int NCH, bool FIT>
+__device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__ xm,
+                                             const int4* __restrict__ xq, const uint32_t* cand, const int* aux,
+                                             uint32_t* list32, int total, int hb, int hc, float lo, float hi,
                                              uint32_t* __restrict__ nbr, int* __restrict__ nnb, int& over) {
+    using E = typename std::conditional<FIT, uint16_t, uint32_t>::type;
+    E* list = reinterpret_cast<E*>(list32);
     const int lane = threadIdx.x & 63;
-    const int mj = P.nmaxpartj, stride = nb_stride(mj);
+    const int mj = P.nmaxpartj;
     const size_t N = P.cap;
+    const int4 x0 = xq[hb];
     float cx[NCH], cy[NCH], cz[NCH], cq[NCH];
     uint32_t ce[NCH];
 #pragma unroll
@@ -724,24 +666,27 @@ __device__ __forceinline__ int nb_cell_lists(const DP& P, const double4* __restr
     }
 #pragma unroll
     for (int q = 0; q < NCH; ++q) {
-        const float4 x = xmf[ce[q] & NB_MASK];
-        const float4 o = g_soff[ce[q] >> NB_SHIFT];
-        cx[q] = x.x + o.x;
-        cy[q] = x.y + o.y;
-        cz[q] = x.z + o.z;
+        const int4 x = xq[ce[q] & NB_MASK];
+        const int a = aux[ce[q] >> NB_SHIFT];
+        ce[q] = FIT ? (uint32_t)((int)(ce[q] & NB_MASK) + a) << 4 : (ce[q] & NB_MASK) | (uint32_t)a;
+        cx[q] = (float)(x.x - x0.x);
+        cy[q] = (float)(x.y - x0.y);
+        cz[q] = (float)(x.z - x0.z);
         const float r2 = __builtin_fmaf(cx[q], cx[q], __builtin_fmaf(cy[q], cy[q], cz[q] * cz[q]));
         cq[q] = 64 * q + lane < total ? r2 : 3.0e38f;
     }
+    const int self = FIT ? aux[13] : 0;
     int pairs = 0;
     for (int h0 = 0; h0 < hc; h0 += 64) {
         // the lane's own particle of the cell, as it enters the test
         float mx = 0.f, my = 0.f, mz = 0.f, tl = 0.f, th = 0.f;
         if (h0 + lane < hc) {
-            const float4 x = xmf[hb + h0 + lane];
-            const float r2 = __builtin_fmaf(x.x, x.x, __builtin_fmaf(x.y, x.y, x.z * x.z));
-            mx = -2.0f * x.x;
-            my = -2.0f * x.y;
-            mz = -2.0f * x.z;
+            const int4 x = xq[hb + h0 + lane];
+            const float fx = (float)(x.x - x0.x), fy = (float)(x.y - x0.y), fz = (float)(x.z - x0.z);
+            const float r2 = __builtin_fmaf(fx, fx, __builtin_fmaf(fy, fy, fz * fz));
+            mx = -2.0f * fx;
+            my = -2.0f * fy;
+            mz = -2.0f * fz;
             tl = lo - r2;
             th = hi - r2;
         }
@@ -760,7 +705,7 @@ __device__ __forceinline__ int nb_cell_lists(const DP& P, const double4* __restr
                 const unsigned long long m = __ballot(in);
                 const int at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, k));
-                list[in ? at : NBC_MAX] = ce[q];
+                list[in ? at : NBC_MAX + 8] = (E)ce[q];
                 k += __popcll(m);
                 return m;
             };
@@ -777,7 +722,7 @@ __device__ __forceinline__ int nb_cell_lists(const DP& P, const double4* __restr
                     const float r2 = r2of(q);
                     bool in = r2 < al;
                     if (!in && r2 <= ah) {
-                        const double4 xj = xm[ce[q] & NB_MASK];
+                        const double4 xj = xm[cand[64 * q + lane] & NB_MASK];
                         const double d0 = xi.x - xj.x;
                         const double d1 = xi.y - xj.y;
                         const double d2 = xi.z - xj.z;
@@ -786,11 +731,18 @@ __device__ __forceinline__ int nb_cell_lists(const DP& P, const double4* __restr
                     append(q, in);
                 }
             }
-            __builtin_amdgcn_wave_barrier();
-            for (int e = 4 * lane, ke = min(k, stride); e < ke; e += 256)
-                *reinterpret_cast<uint4*>(nbr + nb_index(N, p, e)) = *reinterpret_cast<const uint4*>(list + e);
-            __builtin_amdgcn_wave_barrier();
             const int kn = min(k, mj);
+            if (FIT && lane < 8) list[kn + lane] = (E)((uint32_t)(p + self) << 4);  // fills the last group
+            __builtin_amdgcn_wave_barrier();
+            if constexpr (FIT) {
+                for (int e = 8 * lane; e < kn; e += 512)
+                    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(nbr) + nb16_index(N, p, e)) =
+                        *reinterpret_cast<const uint4*>(list + e);
+            } else {
+                for (int e = 4 * lane; e < kn; e += 256)
+                    *reinterpret_cast<uint4*>(nbr + nb_index(N, p, e)) = *reinterpret_cast<const uint4*>(list + e);
+            }
+            __builtin_amdgcn_wave_barrier();
             mine = lane == u ? kn : mine;
             pairs += kn - 1;
             over += k > mj;
@@ -801,83 +753,114 @@ __device__ __forceinline__ int nb_cell_lists(const DP& P, const double4* __restr
 }
 
 template <bool SG>
-__global__ __launch_bounds__(256, 4) void k_neighbours(DP P0, Seg S, const double4* __restrict__ xm,
-                                                    const float4* __restrict__ xmf,
+__global__ __launch_bounds__(256, 4) void k_neighbours(Seg S, const double4* __restrict__ xm,
+                                                    const int4* __restrict__ xq,
                                                     const int* __restrict__ cell,
                                                     const int* __restrict__ start,
                                                     uint32_t* __restrict__ nbr, int* __restrict__ nnb,
-                                                    int* iscal, unsigned long long* pairs) {
-    __shared__ uint32_t s_cand[4][NBC_MAX];                // a wave's candidates: sorted index | stencil code
-    __shared__ __align__(16) uint32_t s_list[4][NBC_MAX + 4];  // the list of its current particle
+                                                    int* iscal, unsigned long long* pairs, int slots) {
+    __shared__ uint32_t s_cand[4][NBC_MAX];  // a wave's candidates: sorted index | stencil cell in list order
+    __shared__ __align__(16) uint32_t s_list[4][NBC_MAX + 12];  // the list of its current particle
+    __shared__ int s_aux[4][28];  // per stencil cell: sorted index to slot, or the stencil code's bits
     __shared__ int s_pairs[4];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int vb = xcd_block(gridDim.x);
-    const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * 4 * NBC_SLOTS) >> 8]) : 0;
-    const DP& P = SG ? S.P[sg] : P0;
+    const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * 4 * slots) >> 8]) : 0;
+    DPC& P = S.P[sg];
     iscal += sg * IS_COUNT;
     const int n = iscal[IS_N];
-    if (vb * 4 * NBC_SLOTS - P.base >= n) return;
-    stencil_offsets(P);
+    if (vb * 4 * slots - P.base >= n) return;
     const int ni = P.ncd[0], nj = P.ncd[1], nk = P.ncd[2];
-    const float sq = (float)P.square_doubleh;
+    const float sq = (float)(P.square_doubleh * P.inv_lsb * P.inv_lsb);
     const float dm = fmaxf(P.f_dcd[0], fmaxf(P.f_dcd[1], P.f_dcd[2]));
-    const float band = 4.0e-5f * fmaxf(1.0f, dm * dm / sq);
+    const float band = 4.0e-5f * fmaxf(1.0f, dm * dm / (float)P.square_doubleh);
     const float lo = sq * (1.0f - band), hi = sq * (1.0f + band);
-    const int s0 = (vb * 4 + wid) * NBC_SLOTS;
+    const int s0 = (vb * 4 + wid) * slots;
     uint32_t* cand = s_cand[wid];
     uint32_t* list = s_list[wid];
     int mypairs = 0, over = 0;
     int cl = 0;
     bool first = false;  // the lane's slot starts a cell
-    if (lane < NBC_SLOTS && s0 + lane - P.base < n) {
+    if (lane < slots && s0 + lane - P.base < n) {
         cl = cell[s0 + lane];
         first = s0 + lane == P.base || cell[s0 + lane - 1] != cl;
     }
+    int tile = -1, delta = 0;
+    bool fits = false;
     unsigned long long todo = __ballot(first);
     while (todo) {
         const int l = __ffsll((long long)todo) - 1;
         todo &= todo - 1ull;
         int ic, jc, kc;
         d_cell_indices(P, __builtin_amdgcn_readlane(cl, l), ic, jc, kc);
+        // lane r: row r of the cell's tile, its slots' offset from the sorted indices
+        const int ti = div_inv(ic - 1, P.inv_tdim[0]), tj = div_inv(jc - 1, P.inv_tdim[1]),
+                  tk = div_inv(kc - 1, P.inv_tdim[2]);
+        const int id = __builtin_amdgcn_readfirstlane((tk * P.ntile[1] + tj) * P.ntile[0] + ti);
+        if (id != tile) {
+            tile = id;
+            int g0, g1, h0, h1;
+            tile_row(P, start, ti, tj, tk, lane, g0, g1, h0, h1);
+            const int rincl = wave_incl_scan(g1 - g0);
+            fits = __builtin_amdgcn_readlane(rincl, 63) <= P.tcap;
+            delta = rincl - (g1 - g0) - g0;
+        }
         // lane t: the t-th stencil cell in the order dy, dx, dz
-        int b = 0, cnt = 0;
-        uint32_t tag = 0u;
+        int b = 0, cnt = 0, row = 0;
+        const int dy = lane / 9 - 1, dx = (lane / 3) % 3 - 1, dz = lane % 3 - 1;
         if (lane < 27) {
-            const int dy = lane / 9 - 1, dx = (lane / 3) % 3 - 1, dz = lane % 3 - 1;
             const int ii = ic + dx, jj = jc + dy, kk = kc + dz;
             if (ii >= 1 && ii <= ni && jj >= 1 && jj <= nj && kk >= 1 && kk <= nk) {
                 const int key = P.koff + ((kk - 1) * nj + (jj - 1)) * ni + ii - 1;
                 b = start[key];
                 cnt = start[key + 1] - b;
-                tag = (uint32_t)((dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)) << NB_SHIFT;
+                row = (kk - tk * P.tdim[2]) * (P.tdim[1] + 2) + (jj - tj * P.tdim[1]);
             }
         }
+        const int dt = __shfl(delta, row, 64);
+        if (lane < 27) s_aux[wid][lane] = fits ? dt : (int)((uint32_t)((dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)) << NB_SHIFT);
         const int incl = wave_incl_scan(cnt);
         const int total = __builtin_amdgcn_readlane(incl, 63);
         const int hb = __builtin_amdgcn_readlane(b, 13), hc = __builtin_amdgcn_readlane(cnt, 13);
+        __builtin_amdgcn_wave_barrier();
         if (total > NBC_MAX) {
             for (int q = lane; q < hc; q += 64) {
                 bool ov;
-                const int k = nb_particle_global(P, hb + q, xm, xmf, cell, start, nbr, lo, hi, ov);
+                const int k = nb_particle_global(P, hb + q, xm, xq, cell, start, nbr, s_aux[wid], fits, lo, hi, ov);
                 nnb[hb + q] = k;
                 if (ov) atomicAdd(&iscal[IS_NB_OVERFLOW], 1);
                 atomicAdd(&pairs[(vb % NBC_PAIRS) * NBC_PSTRIDE], (unsigned long long)(k - 1));
             }
             continue;
         }
-        for (int u = 0, pre = incl - cnt; u < cnt; ++u) cand[pre + u] = (uint32_t)(b + u) | tag;
+        for (int u = 0, pre = incl - cnt; u < cnt; ++u) cand[pre + u] = (uint32_t)(b + u) | ((uint32_t)lane << NB_SHIFT);
         __builtin_amdgcn_wave_barrier();
-        switch ((total + 63) >> 6) {
-            case 1: mypairs += nb_cell_lists<1>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-            case 2: mypairs += nb_cell_lists<2>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-            case 3: mypairs += nb_cell_lists<3>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-            case 4: mypairs += nb_cell_lists<4>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-            case 5: mypairs += nb_cell_lists<5>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-            case 6: mypairs += nb_cell_lists<6>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-            case 7: mypairs += nb_cell_lists<7>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-            case 8: mypairs += nb_cell_lists<8>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-            case 9: mypairs += nb_cell_lists<9>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-            case 10: mypairs += nb_cell_lists<10>(P, xm, xmf, cand, list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+        if (fits) {
+            switch ((total + 63) >> 6) {
+                case 1: mypairs += nb_cell_lists<1, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 2: mypairs += nb_cell_lists<2, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 3: mypairs += nb_cell_lists<3, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 4: mypairs += nb_cell_lists<4, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 5: mypairs += nb_cell_lists<5, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 6: mypairs += nb_cell_lists<6, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 7: mypairs += nb_cell_lists<7, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 8: mypairs += nb_cell_lists<8, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 9: mypairs += nb_cell_lists<9, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 10: mypairs += nb_cell_lists<10, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+            }
+        } else {
+            switch ((total + 63) >> 6) {
+                case 1: mypairs += nb_cell_lists<1, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 2: mypairs += nb_cell_lists<2, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 3: mypairs += nb_cell_lists<3, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 4: mypairs += nb_cell_lists<4, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 5: mypairs += nb_cell_lists<5, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 6: mypairs += nb_cell_lists<6, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 7: mypairs += nb_cell_lists<7, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 8: mypairs += nb_cell_lists<8, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 9: mypairs += nb_cell_lists<9, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 10: mypairs += nb_cell_lists<10, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+            }
         }
     }
     // pair-interaction counter: sum_i (nPartIntorno(i) - 1), self excluded
@@ -894,7 +877,7 @@ __global__ __launch_bounds__(256, 4) void k_neighbours(DP P0, Seg S, const doubl
 // ----------------------------------------------------------------------------
 // SA-SPH volume integrals (FP64)
 // ----------------------------------------------------------------------------
-__device__ void d_volume_integrals(const DP& P, const DFace& F, const double* __restrict__ kt,
+__device__ void d_volume_integrals(DPC& P, const DFace& F, const double* __restrict__ kt,
                                    const double* __restrict__ bit, const double locx[3],
                                    double bi[8], double ig[9]) {
     double IntWdV = 0.0, IntdWrm1dV = 0.0, IntGWZrm1dV = 0.0;
@@ -986,7 +969,7 @@ __device__ void d_volume_integrals(const DP& P, const DFace& F, const double* __
 // 256-direction quadrature keeps every lane busy.
 // ----------------------------------------------------------------------------
 template <bool SG>
-__global__ __launch_bounds__(256) void k_boundary_find(DP P0, Seg S, const DFace* __restrict__ faces,
+__global__ __launch_bounds__(256) void k_boundary_find(Seg S, const DFace* __restrict__ faces,
                                                        const int* __restrict__ ncount,
                                                        const int* __restrict__ nstart,
                                                        const int* __restrict__ nvec,
@@ -995,7 +978,7 @@ __global__ __launch_bounds__(256) void k_boundary_find(DP P0, Seg S, const DFace
                                                        int* __restrict__ work, int* nwork, int* iscal) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(blockIdx.x * blockDim.x) >> 8]) : 0;
-    const DP& P = SG ? S.P[sg] : P0;
+    DPC& P = S.P[sg];
     iscal += sg * IS_COUNT;
     if (i - P.base >= iscal[IS_N]) return;
     const double4 x = xm[i];
@@ -1060,7 +1043,7 @@ __global__ __launch_bounds__(256) void k_boundary_find(DP P0, Seg S, const DFace
 // each lane reads its segment's constants and tables (kernel and direction
 // tables of every segment, consecutive) from global memory.
 template <bool SG>
-__global__ __launch_bounds__(256) void k_boundary_int(DP P0, Seg S, const DFace* __restrict__ faces,
+__global__ __launch_bounds__(256) void k_boundary_int(Seg S, const DFace* __restrict__ faces,
                                                       const double* __restrict__ kt_g,
                                                       const double* __restrict__ bit_g,
                                                       BTab* __restrict__ bt,
@@ -1078,7 +1061,7 @@ __global__ __launch_bounds__(256) void k_boundary_int(DP P0, Seg S, const DFace*
         const int e = work[w];
         const int i = e & (int)NB_MASK, q = (int)((uint32_t)e >> NB_SHIFT);
         const int sg = SG ? S.pblk[i >> 8] : 0;
-        const DP& P = SG ? S.P[sg] : P0;
+        DPC& P = S.P[sg];
         const double* kt = SG ? kt_g + (size_t)sg * (41 * 5) : kt_s;
         const double* bit = SG ? bit_g + (size_t)sg * (256 * 7) : bit_s;
         BTab& rec = bt[(size_t)q * P.cap + i];
@@ -1156,12 +1139,13 @@ __device__ __forceinline__ void d_interp2d(const double* __restrict__ tab, int n
     }
 }
 
-__global__ __launch_bounds__(256) void k_boundary_2d(DP P, const DFace* __restrict__ sides,
+__global__ __launch_bounds__(256) void k_boundary_2d(DPC* Pp, const DFace* __restrict__ sides,
                                                      const double* __restrict__ tab,
                                                      const double4* __restrict__ xm,
                                                      const int* __restrict__ cell,
                                                      int* __restrict__ bn, BTab* __restrict__ bt,
                                                      int* iscal) {
+    DPC& P = *Pp;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= P.cap) return;
     if (i >= iscal[IS_N]) {
@@ -1460,7 +1444,7 @@ __device__ void bt_pair_f32_dirs(const BtF32& T, const DFace& F, double L0, doub
 // Segmented contexts: the lanes of a pair read their segment's table (one
 // per segment, consecutive) from global memory.
 template <bool SG>
-__global__ __launch_bounds__(256) void k_boundary_int_f32(DP P0, Seg S, const DFace* __restrict__ faces,
+__global__ __launch_bounds__(256) void k_boundary_int_f32(Seg S, const DFace* __restrict__ faces,
                                                           const BtF32* __restrict__ tab,
                                                           BTab* __restrict__ bt,
                                                           const int* __restrict__ work,
@@ -1483,7 +1467,7 @@ __global__ __launch_bounds__(256) void k_boundary_int_f32(DP P0, Seg S, const DF
         const int e = work[w];
         const int i = e & (int)NB_MASK, q = (int)((uint32_t)e >> NB_SHIFT);
         const int sg = SG ? S.pblk[i >> 8] : 0;
-        const DP& P = SG ? S.P[sg] : P0;
+        DPC& P = S.P[sg];
         const BtF32& T = SG ? tab[sg] : T_s;
         BTab& rec = bt[(size_t)q * P.cap + i];
         const double L0 = rec.loc[0], L1 = rec.loc[1];
@@ -1653,7 +1637,7 @@ __global__ void k_global_final(const double* __restrict__ part, int nblocks, dou
 // ----------------------------------------------------------------------------
 constexpr int FS_WG = 256;
 
-__device__ __forceinline__ int d_point_cell(const DP& P, double x, double y, double z) {
+__device__ __forceinline__ int d_point_cell(DPC& P, double x, double y, double z) {
     const double q[3] = {x, y, z};
     int ijk[3];
 #pragma unroll
@@ -1665,11 +1649,12 @@ __device__ __forceinline__ int d_point_cell(const DP& P, double x, double y, dou
     return d_cell_number(P, ijk[0], ijk[1], ijk[2]);
 }
 
-__global__ __launch_bounds__(FS_WG) void k_free_surface(DP P, const double4* __restrict__ xm,
+__global__ __launch_bounds__(FS_WG) void k_free_surface(DPC* Pp, const double4* __restrict__ xm,
                                                        const int* __restrict__ start,
                                                        const double* __restrict__ pts,
                                                        const int* __restrict__ icont, int nlines,
                                                        double* __restrict__ out) {
+    DPC& P = *Pp;
     __shared__ double val[FS_WG][3];
     __shared__ int st[FS_WG];  // 0 outside the grid, 1 empty cell, 2 filled cell
     const int line = blockIdx.x;
@@ -1741,7 +1726,7 @@ __global__ __launch_bounds__(FS_WG) void k_free_surface(DP P, const double4* __r
 // dt: time_step_duration.f90:74-116.  Positive doubles order like their bit
 // patterns, so the minimum over particles is an exact atomicMin on uint64.
 // ----------------------------------------------------------------------------
-__device__ __forceinline__ double d_dt_cfl(const DP& P, double vx, double vy, double vz) {
+__device__ __forceinline__ double d_dt_cfl(DPC& P, double vx, double vy, double vz) {
     const double U = sqrt(vx * vx + vy * vy + vz * vz);
     return P.cfl * 2.0 * P.h / (P.celerita + U);
 }
@@ -1763,11 +1748,11 @@ __device__ __forceinline__ void block_min_to(unsigned long long v, unsigned long
 }
 
 template <bool SG>
-__global__ __launch_bounds__(256) void k_dtmin(DP P0, Seg S, const double4* __restrict__ vel,
+__global__ __launch_bounds__(256) void k_dtmin(Seg S, const double4* __restrict__ vel,
                                                unsigned long long* dtmin, const int* iscal) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(blockIdx.x * blockDim.x) >> 8]) : 0;
-    const DP& P = SG ? S.P[sg] : P0;
+    DPC& P = S.P[sg];
     dtmin += sg;
     unsigned long long v = 0x7FF0000000000000ull;
     if (i - P.base < iscal[sg * IS_COUNT + IS_N]) {
@@ -1780,10 +1765,10 @@ __global__ __launch_bounds__(256) void k_dtmin(DP P0, Seg S, const double4* __re
 // step prologue (time_step_loop.f90:180-186): dt_previous_step, dt, time
 // Segmented contexts: one lane per segment.
 template <bool SG>
-__global__ void k_dt_begin(DP P0, Seg S, double* scal, unsigned long long* dtmin, int* iscal, int advance) {
+__global__ void k_dt_begin(Seg S, double* scal, unsigned long long* dtmin, int* iscal, int advance) {
     const int sg = SG ? (int)(blockIdx.x * blockDim.x + threadIdx.x) : 0;
     if (SG ? sg >= S.nseg : (threadIdx.x != 0 || blockIdx.x != 0)) return;
-    const DP& P = SG ? S.P[sg] : P0;
+    DPC& P = S.P[sg];
     scal += sg * SC_COUNT;
     iscal += sg * IS_COUNT;
     dtmin += sg;
@@ -1817,31 +1802,78 @@ __global__ void k_dt_begin(DP P0, Seg S, double* scal, unsigned long long* dtmin
     *dtmin = 0x7FF0000000000000ull;
 }
 
-// ----------------------------------------------------------------------------
-// The four pair passes.  A persistent workgroup takes a cell block, stages the
-// block's 9 neighbour rows into LDS (coalesced, contiguous in sorted order)
-// and gives each home particle one lane that walks its neighbour list in the
-// reference's order, reading neighbour records from LDS.  Blocks whose rows
-// exceed the LDS tile read their neighbours from global memory instead.
-// FP64: the reference's expressions, operation for operation.  FP32-mixed:
-// FP32 pair math on cell-relative separations, FP32 sums per particle, FP64
-// wall terms, FP64 integration.
-// ----------------------------------------------------------------------------
-template <bool F32>
-struct Rec;
-template <>
-struct Rec<false> {
-    using X = double4;
-    using V = double4;
-    using RP = double2;
-};
-template <>
-struct Rec<true> {
-    using X = float4;
-    using V = float4;
-    using RP = float2;
-};
+// the row a with pre[a] <= x < pre[a + 1] of the prefix sums pre[0..rows]
+__device__ __forceinline__ int tile_find(const int* pre, int rows, int x) {
+    int a = 0;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1)
+        if (a + s < rows && pre[a + s] <= x) a += s;
+    return a;
+}
 
+// Runs the tiles that hold particles: stage(P, segment, sorted index, slot)
+// for every slot of a tile that fits, then part(P, segment, sorted index,
+// fits) with G lanes for every home particle, then done(P, segment).  A workgroup takes
+// the tiles of its XCD's contiguous share, so tiles that share halo rows
+// share an L2.
+template <bool SG, int G, class Stage, class Part, class Done>
+__device__ __forceinline__ void for_tiles(const Seg& S, const Tiles& T,
+                                          const int* __restrict__ start, Stage&& stage, Part&& part,
+                                          Done&& done) {
+    __shared__ TileS ts;
+    const int nt = *T.n;
+    const int per = gridDim.x >> 3, xcd = blockIdx.x & 7;  // gridDim.x is a multiple of 8
+    const int t1 = (int)((long long)nt * (xcd + 1) / 8);
+    const int lane = threadIdx.x & 63;
+    for (int t = (int)((long long)nt * xcd / 8) + (blockIdx.x >> 3); t < t1; t += per) {
+        const int id = __builtin_amdgcn_readfirstlane(T.list[t]);
+        const int sg = SG ? __builtin_amdgcn_readfirstlane(S.tblk[id >> 8]) : 0;
+        DPC& P = S.P[sg];
+        const int rows = tile_rows(P);
+        if (threadIdx.x < 64) {
+            int ti, tj, tk, g0, g1, h0, h1;
+            tile_coords(P, id, ti, tj, tk);
+            tile_row(P, start, ti, tj, tk, lane, g0, g1, h0, h1);
+            const int a = wave_incl_scan(g1 - g0), b = wave_incl_scan(h1 - h0);
+            ts.g[lane] = g0;
+            ts.h0[lane] = h0;
+            ts.l[lane + 1] = a;
+            ts.hp[lane + 1] = b;
+            if (lane == 0) ts.l[0] = ts.hp[0] = 0;
+        }
+        __syncthreads();
+        const int total = ts.l[rows], nhome = ts.hp[rows];
+        const bool fits = total <= P.tcap;
+        if (fits) {
+            // TILE_U slots per thread at a time, so that their loads are in
+            // flight together (a slot past the end repeats the last one)
+            const int bs = blockDim.x;
+            for (int e0 = threadIdx.x; e0 < total; e0 += TILE_U * bs) {
+                int e[TILE_U], g[TILE_U];
+#pragma unroll
+                for (int u = 0; u < TILE_U; ++u) {
+                    e[u] = min(e0 + u * bs, total - 1);
+                    const int r = tile_find(ts.l, rows, e[u]);
+                    g[u] = ts.g[r] + e[u] - ts.l[r];
+                }
+#pragma unroll
+                for (int u = 0; u < TILE_U; ++u) stage(P, sg, g[u], e[u]);
+            }
+        }
+        __syncthreads();
+        for (int q = threadIdx.x / G; q < nhome; q += blockDim.x / G) {
+            const int a = tile_find(ts.hp, rows, q);
+            part(P, sg, ts.h0[a] + q - ts.hp[a], fits);
+        }
+        done(P, sg);
+        __syncthreads();  // the slots and rows are reused
+    }
+}
+
+// 16 bytes at byte offset o of an LDS array
+__device__ __forceinline__ float4 lds16(const float4* a, uint32_t o) {
+    return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a) + o);
+}
 
 constexpr uint32_t NB_NONE = 0xFFFFFFFFu;
 
@@ -1855,7 +1887,7 @@ __device__ __forceinline__ void walk_list(const uint32_t* __restrict__ nbr, size
     static_assert(CH % 4 == 0, "list walks read whole 16-byte quarters of a group");
     for (int k0 = 0; k0 < nn; k0 += CH) {
         uint32_t ev[CH];
-        if constexpr (NB_G >= 4) {
+        {
 #pragma unroll
             for (int q = 0; q < CH / 4; ++q) {
                 const uint4 v = *reinterpret_cast<const uint4*>(nbr + nb_index(N, i, k0 + 4 * q));
@@ -1864,9 +1896,6 @@ __device__ __forceinline__ void walk_list(const uint32_t* __restrict__ nbr, size
                 ev[4 * q + 2] = v.z;
                 ev[4 * q + 3] = v.w;
             }
-        } else {
-#pragma unroll
-            for (int u = 0; u < CH; ++u) ev[u] = nbr[nb_index(N, i, k0 + u)];
         }
 #pragma unroll
         for (int u = 0; u < CH; ++u)
@@ -2017,7 +2046,7 @@ __device__ bool open_side_crossed(const DFace& S, const double xo[3], const doub
 
 // SA-SPH terms of the momentum equation (AddBoundaryContributions_to_ME3D.f90:
 // 118-336), FP64; tp/td/tv start at zero
-__device__ __forceinline__ void sa_momentum(const DP& P, const DFace* __restrict__ faces,
+__device__ __forceinline__ void sa_momentum(DPC& P, const DFace* __restrict__ faces,
                                             const BTab* __restrict__ bt, int i, int ncbf,
                                             const double v_i[3], double2 rpi, int lam_prev,
                                             double tp[3], double td[3], double tv[3], int* iscal) {
@@ -2091,7 +2120,7 @@ __device__ __forceinline__ void sa_momentum(const DP& P, const DFace* __restrict
 
 // AddBoundaryContributions_to_ME2D.f90:121-405 for fixe/tapi sides (2D form);
 // tp/td/tv start at zero, as the reference's tpres/tdiss/tvisc do
-__device__ __forceinline__ void sa_momentum_2d(const DP& P, const DFace* __restrict__ sides,
+__device__ __forceinline__ void sa_momentum_2d(DPC& P, const DFace* __restrict__ sides,
                                                const BTab* __restrict__ bt, int i, int ncbf,
                                                const double v_i[3], double2 rpi, int lam_prev,
                                                double tp[3], double td[3], double tv[3]) {
@@ -2163,7 +2192,7 @@ __device__ __forceinline__ void sa_momentum_2d(const DP& P, const DFace* __restr
 }
 
 // AddElasticBoundaryReaction_2D.f90:66-99 over the selected sides
-__device__ __forceinline__ void elastic_2d(const DP& P, const DFace* __restrict__ sides,
+__device__ __forceinline__ void elastic_2d(DPC& P, const DFace* __restrict__ sides,
                                            const BTab* __restrict__ bt, int i, int ncbf,
                                            const double v_i[3], double br[3]) {
     const double h = P.h;
@@ -2186,713 +2215,989 @@ __device__ __forceinline__ void elastic_2d(const DP& P, const DFace* __restrict_
 }
 
 // ----------------------------------------------------------------------------
-// momentum: RHS_momentum_equation.f90:72-179, inter_EqMoto.f90:108-283,
-// viscomon.f90:54-71, viscomorris.f90:60-71, AddElasticBoundaryReaction_3D.f90:
-// 67-98; fused Leapfrog_momentum.f90:66-86
+// Per-particle parts of the four passes outside the pair sums, FP64 in both
+// forms.
 // ----------------------------------------------------------------------------
-template <bool F32, int CH, bool SG>
-__global__ __launch_bounds__(256) void k_momentum(
-    DP P0, Seg S, const DFace* __restrict__ faces, const DEdge* __restrict__ edges,
+// elastic wall reaction (AddElasticBoundaryReaction_3D.f90:67-152, _2D) of a
+// particle with ncbf > 0 close frontiers
+__device__ __forceinline__ void elastic_walls(DPC& P, const DFace* __restrict__ faces,
+                                              const DEdge* __restrict__ edges, const BTab* __restrict__ bt,
+                                              const double4* __restrict__ xm, int i, int ncbf, double4 vi,
+                                              double br[3]) {
+    const double v_i[3] = {vi.x, vi.y, vi.z};
+    if (P.dim == 2) {
+        elastic_2d(P, faces, bt, i, ncbf, v_i, br);
+        return;
+    }
+    const double h = P.h;
+    const double zimin = 0.25 * P.dx;
+    const double celer02 = P.eps / P.den0;
+    // AddElasticBoundaryReaction_3D.f90:72-104 (faces); rea: the
+    // slots whose face reacted (ReaFace), for the edges below
+    static_assert(SPH_MB <= 32, "one ReaFace bit per boundary-table slot");
+    unsigned rea = 0u;
+    for (int q = 0; q < ncbf; ++q) {
+        const BTab& B = bt[(size_t)q * P.cap + i];
+        const DFace& F = faces[B.face];
+        if (F.btype != 0 && F.btype != 1) continue;
+        const double zi = B.loc[2];
+        if (zi < zimin && d_point_internal(F, B.loc[0], B.loc[1])) {
+            double vin = 0.0;
+            for (int sd = 0; sd < 3; ++sd) vin = vin + v_i[sd] * F.T[6 + sd];
+            if (vin < 0.0) {
+                const double nr = -1.0 * celer02 * log((h + zi - zimin) / h) / h;
+                for (int d = 0; d < 3; ++d) br[d] = br[d] + nr * F.T[6 + d];
+            }
+            rea |= 1u << q;
+        }
+    }
+    // AddElasticBoundaryReaction_3D.f90:106-152 (convex edges, in
+    // order; the reference returns at the first edge whose two
+    // faces are not both among the particle's non-reacting faces)
+    for (int ne = 0; ne < P.ne; ++ne) {
+        const DEdge& E = edges[P.eoff + ne];
+        int nclose = 0;
+        for (int q = 0; q < ncbf; ++q) {
+            const int f = bt[(size_t)q * P.cap + i].face;
+            const bool rq = (rea >> q) & 1u;
+            if (f == E.face[0] && !rq) ++nclose;
+            else if (f == E.face[1] && !rq) ++nclose;
+        }
+        if (nclose != 2) break;
+        const double4 xi = xm[i];
+        const double x[3] = {xi.x, xi.y, xi.z};
+        double scaprod = 0.0;
+        for (int sd = 0; sd < 3; ++sd) scaprod = scaprod + (x[sd] - E.gx[sd]) * E.comp[sd];
+        const double tau = scaprod / (E.len * E.len);
+        if (tau >= 0.0 && tau <= 1.0) {
+            double QP[3], d2 = 0.0;
+            for (int sd = 0; sd < 3; ++sd) QP[sd] = x[sd] - (E.gx[sd] + E.comp[sd] * tau);
+            for (int sd = 0; sd < 3; ++sd) d2 = d2 + QP[sd] * QP[sd];
+            const double zi = sqrt(d2);
+            if (zi < zimin) {
+                double cd[3], vin = 0.0;
+                for (int sd = 0; sd < 3; ++sd) cd[sd] = QP[sd] / zi;
+                for (int sd = 0; sd < 3; ++sd) vin = vin + v_i[sd] * cd[sd];
+                if (vin < 0.0) {
+                    const double nr = -1.0 * celer02 * log(zi / zimin) / zimin;
+                    for (int d = 0; d < 3; ++d) br[d] = br[d] + nr * cd[d];
+                }
+            }
+        }
+    }
+}
+
+// The wall terms of the FP32-mixed momentum pass as calls: inlined, their FP64
+// values raise the kernel above the 128 registers that two workgroups a CU
+// allow, and it spills (576,000 particles: 151 us
+// against 116).  Few particles take them.
+struct Walls6 {
+    double tp[3], tdv[3];  // pressure terms; Monaghan's and the shear terms
+};
+struct Walls3 {
+    double r[3];
+};
+__device__ __attribute__((noinline)) Walls6 wall_terms(DPC* P, const DFace* __restrict__ faces,
+                                                       const BTab* __restrict__ bt, int i, int ncbf, double vx,
+                                                       double vy, double vz, double rho, double p, int lam,
+                                                       int* iscal) {
+    double tp[3] = {0.0, 0.0, 0.0}, td[3] = {0.0, 0.0, 0.0}, tv[3] = {0.0, 0.0, 0.0};
+    const double v_i[3] = {vx, vy, vz};
+    if (P->dim == 2)
+        sa_momentum_2d(*P, faces, bt, i, ncbf, v_i, make_double2(rho, p), lam, tp, td, tv);
+    else
+        sa_momentum(*P, faces, bt, i, ncbf, v_i, make_double2(rho, p), lam, tp, td, tv, iscal);
+    return Walls6{{tp[0], tp[1], tp[2]}, {td[0] + tv[0], td[1] + tv[1], td[2] + tv[2]}};
+}
+__device__ __attribute__((noinline)) Walls3 wall_elastic(DPC* P, const DFace* __restrict__ faces,
+                                                         const DEdge* __restrict__ edges,
+                                                         const BTab* __restrict__ bt,
+                                                         const double4* __restrict__ xm, int i, int ncbf,
+                                                         double vx, double vy, double vz) {
+    double br[3] = {0.0, 0.0, 0.0};
+    elastic_walls(*P, faces, edges, bt, xm, i, ncbf, make_double4(vx, vy, vz, 0.0), br);
+    return Walls3{{br[0], br[1], br[2]}};
+}
+
+// laminar flag, acceleration and Leapfrog_momentum.f90:66-86 (RK1:
+// Euler.f90:85-93); br: the elastic wall reaction, for ncbf > 0.  Returns the
+// new velocity.
+__device__ __forceinline__ double4 momentum_end(DPC& P, int i, int ncbf, double4 vi, double dtvel,
+                                                const double tp[3], const double td[3], const double tv[3],
+                                                const double rvs[3], const double br[3],
+                                                int* __restrict__ lam_out, double4* __restrict__ acc_out,
+                                                double4* __restrict__ vel_out) {
+    int lam = 0;
+    if (P.kin_visc > 0.0) {
+        const double apg = sqrt(tp[0] * tp[0] + tp[1] * tp[1] + tp[2] * tp[2]) + P.GI;
+        const double amo = sqrt(rvs[0] * rvs[0] + rvs[1] * rvs[1] + rvs[2] * rvs[2]);
+        double w = 0.0;
+        if (apg != 0.0) w = amo / apg * 100.0;
+        lam = (w > 5.0 || apg == 0.0) ? 1 : 0;
+    }
+    lam_out[i] = lam;
+    double a[3];
+    for (int d = 0; d < 3; ++d) a[d] = tp[d] + td[d] + tv[d] + P.grav[d];
+    if (ncbf > 0)
+        for (int d = 0; d < 3; ++d) a[d] = a[d] + br[d];
+    acc_out[i] = make_double4(a[0], a[1], a[2], 0.0);
+    // vel = vel + dtvel*acc (kodvel == 0)
+    const double4 vn =
+        make_double4(vi.x + dtvel * a[0], vi.y + dtvel * a[1], vi.z + dtvel * a[2], vi.w);
+    vel_out[i] = vn;
+    return vn;
+}
+
+// wall terms of the velocity smoothing (velocity_smoothing_SA_SPH_3D.f90:64-122, _2D)
+__device__ __forceinline__ void vsmooth_walls(DPC& P, const DFace* __restrict__ faces,
+                                              const BTab* __restrict__ bt, int i, int ncbf, double4 vi,
+                                              double v[3]) {
+    // velocity_smoothing_SA_SPH_2D.f90:64-118 (fixe/tapi sides)
+    for (int q = 0; q < ncbf && P.dim == 2; ++q) {
+        const BTab& B = bt[(size_t)q * P.cap + i];
+        const DFace& S = faces[B.face];
+        if (S.btype != 0 && S.btype != 1) continue;
+        const double s0 = S.T[0], s1 = S.T[2], n0 = S.T[6], n1 = S.T[8];
+        const double DVG0 = 2.0 * (S.tvel[0] - vi.x), DVG1 = 2.0 * (S.tvel[2] - vi.z);
+        const double DVL0 = s0 * DVG0 + s1 * DVG1;
+        const double DVL1 = n0 * DVG0 + n1 * DVG1;
+        const double IntWdV = B.bi[2];
+        double slip = S.mode == 1 ? S.slip : 0.0;
+        if (S.mode == 2) {
+            // velocity_smoothing_SA_SPH_2D.f90:93-106
+            const double u0 = (S.tvel[0] - vi.x) - (0.5 * DVL1 * S.T[6]);
+            const double u1 = (S.tvel[1] - vi.y) - (0.5 * DVL1 * S.T[7]);
+            const double u2 = (S.tvel[2] - vi.z) - (0.5 * DVL1 * S.T[8]);
+            double nut;
+            wall_function(sqrt(u0 * u0 + u1 * u1 + u2 * u2), S.slip * 10.0, B.loc[1], P.dx,
+                          slip, nut);
+        }
+        const double BCL0 = DVL0 * IntWdV * slip;
+        const double BCL1 = DVL1 * IntWdV;
+        v[0] = v[0] + (s0 * BCL0 + n0 * BCL1);
+        v[2] = v[2] + (s1 * BCL0 + n1 * BCL1);
+    }
+    for (int q = 0; q < ncbf && P.dim == 3; ++q) {
+        const BTab& B = bt[(size_t)q * P.cap + i];
+        const DFace& F = faces[B.face];
+        if (F.btype == 3 || F.btype == 4 || F.btype == 5) {
+            v[0] = v[1] = v[2] = 0.0;
+            break;
+        }
+        if (F.btype != 0 && F.btype != 1) continue;
+        const double DVG[3] = {2.0 * (F.tvel[0] - vi.x), 2.0 * (F.tvel[1] - vi.y),
+                               2.0 * (F.tvel[2] - vi.z)};
+        double DVL[3];
+        for (int ii = 0; ii < 3; ++ii) {
+            double a = 0.0;
+            for (int jj = 0; jj < 3; ++jj) a = a + F.T[3 * ii + jj] * DVG[jj];
+            DVL[ii] = a;
+        }
+        const double IntWdV = B.bi[1];
+        double slip = F.mode == 1 ? F.slip : 0.0;
+        if (F.mode == 2) {
+            // velocity_smoothing_SA_SPH_3D.f90:89-110
+            double ut[3], nut;
+            for (int d = 0; d < 3; ++d) ut[d] = 0.5 * (DVG[d] - DVL[2] * F.T[6 + d]);
+            wall_function(sqrt(ut[0] * ut[0] + ut[1] * ut[1] + ut[2] * ut[2]), F.slip * 10.0,
+                          B.loc[2], P.dx, slip, nut);
+        }
+        const double BCL[3] = {DVL[0] * IntWdV * slip, DVL[1] * IntWdV * slip,
+                               DVL[2] * IntWdV};
+        for (int ii = 0; ii < 3; ++ii) {
+            double a = 0.0;
+            for (int jj = 0; jj < 3; ++jj) a = a + F.T[3 * jj + ii] * BCL[jj];
+            v[ii] = v[ii] + a;
+        }
+    }
+}
+
+// CancelOutgoneParticles_3D / _2D: the step from xo to xn crosses an open frontier
+__device__ __forceinline__ int open_crossed(DPC& P, const DFace* __restrict__ faces, const double xo[3],
+                                            const double xn[3]) {
+    int g = 0;
+    for (int f = P.foff; f < P.foff + P.nf; ++f)
+        if (faces[f].btype == 2 &&
+            (P.dim == 2 ? open_side_crossed(faces[f], xo, xn) : open_face_crossed(faces[f], xo, xn)))
+            g = 1;
+    return g;
+}
+
+// The same two as calls, for the FP32-mixed pass (see wall_terms)
+__device__ __attribute__((noinline)) int open_crossed_call(DPC* P, const DFace* __restrict__ faces, double x0,
+                                                           double y0, double z0, double x1, double y1, double z1) {
+    const double xo[3] = {x0, y0, z0}, xn[3] = {x1, y1, z1};
+    return open_crossed(*P, faces, xo, xn);
+}
+__device__ __attribute__((noinline)) Walls3 wall_smooth(DPC* P, const DFace* __restrict__ faces,
+                                                        const BTab* __restrict__ bt, int i, int ncbf, double vx,
+                                                        double vy, double vz, double sx, double sy, double sz) {
+    double v[3] = {sx, sy, sz};
+    vsmooth_walls(*P, faces, bt, i, ncbf, make_double4(vx, vy, vz, 0.0), v);
+    return Walls3{{v[0], v[1], v[2]}};
+}
+
+// velocity_smoothing_2.f90:59-103, Leapfrog_trajectories.f90:48-76, the open
+// faces, RK1's density update and the particle part of the next
+// time_step_duration; returns the bits of the particle's time step limit
+template <bool CALL>
+__device__ __forceinline__ unsigned long long vsmooth_end(
+    DPC& P, const DFace* __restrict__ faces, int i, double4 xi, double4 vi, const double v[3],
+    bool smooth, double tv1, double dt, bool eos, const double* __restrict__ dden_in,
+    const double2* __restrict__ rp, double4* __restrict__ vel_out, double4* __restrict__ xm_out,
+    double2* __restrict__ rp_out, float* __restrict__ dr_out, int* __restrict__ gone) {
+    double4 vn = vi;
+    if (smooth) vn = make_double4(vi.x + tv1 * v[0], vi.y + tv1 * v[1], vi.z + tv1 * v[2], vi.w);
+    vel_out[i] = vn;
+
+    const double xn[3] = {xi.x + dt * vn.x, xi.y + dt * vn.y, xi.z + dt * vn.z};
+    xm_out[i] = make_double4(xn[0], xn[1], xn[2], xi.w);
+    // the next time_step_duration runs over the particles the coming
+    // OrdGrid1 keeps: not those out of the grid, nor those that left
+    // through an open face
+    bool stays = d_particle_cell(P, xn[0], xn[1], xn[2]) > 0;
+    if (P.nopen > 0) {  // open frontiers, on the step just made
+        const double xo[3] = {xi.x, xi.y, xi.z};
+        const int g = CALL ? open_crossed_call(&P, faces, xo[0], xo[1], xo[2], xn[0], xn[1], xn[2])
+                           : open_crossed(P, faces, xo, xn);
+        gone[i] = g;
+        stays = stays && !g;
+    }
+    if (P.rk1 && !P.dbsph) {
+        // explicit RK1: Euler.f90:231-241 (dens = dens + dt dden) and
+        // EoS_fluid_loop.f90:59-70 (time_integration.f90:52-65); the
+        // pressure smoothing that follows reads these with the
+        // stage's kernel values, hence the old positions
+        const double2 rpi = rp[i];
+        const double rho1 = rpi.x + dt * dden_in[i];
+        const double p1 = eos ? P.eps / P.den0 * (rho1 - P.den0) + P.prif : rpi.y;
+        rp_out[i] = make_double2(rho1, p1);
+        if (P.f32) dr_out[i] = (float)(rho1 - P.den0);
+    }
+    if (!stays) return 0x7FF0000000000000ull;
+    return (unsigned long long)__double_as_longlong(d_dt_cfl(P, vn.x, vn.y, vn.z));
+}
+
+// wall part of the continuity equation: AddBoundaryContribution_to_CE3D.f90:82-169, _CE2D
+__device__ __forceinline__ double continuity_walls(DPC& P, const DFace* __restrict__ faces,
+                                                   const BTab* __restrict__ bt, int i, int ncbf, double4 vi,
+                                                   double rhoi, int* iscal) {
+    double dd = 0.0;
+    if (ncbf > 0 && P.dim == 2) {
+        // SASPH_continuity.f90:126-169 with AddBoundaryContribution_to_CE2D
+        // .f90:74-150 (fixe/tapi sides): grad_u_SA(1) and grad_w_SA(3)
+        double gu0 = 0.0, gw2 = 0.0;
+        for (int q = 0; q < ncbf; ++q) {
+            const BTab& B = bt[(size_t)q * P.cap + i];
+            const DFace& S = faces[B.face];
+            if (S.btype != 0 && S.btype != 1) continue;
+            const double IntWdS = B.bi[0];
+            double dv0, dv1;
+            if (S.btype == 0) {
+                dv0 = 2.0 * (-vi.x);
+                dv1 = 2.0 * (-vi.z);
+            } else {
+                dv0 = 2.0 * (S.vel[0] - vi.x);
+                dv1 = 2.0 * (S.vel[2] - vi.z);
+            }
+            gu0 = gu0 - dv0 * S.T[6] * IntWdS;
+            gw2 = gw2 - dv1 * S.T[8] * IntWdS;
+        }
+        dd = dd - rhoi * (gu0 + 0.0 + gw2);
+    } else if (ncbf > 0) {
+        double gu = 0.0, gv = 0.0, gw = 0.0;
+        const double v_i[3] = {vi.x, vi.y, vi.z};
+        for (int q = 0; q < ncbf; ++q) {
+            const BTab& B = bt[(size_t)q * P.cap + i];
+            const DFace& F = faces[B.face];
+            if (F.btype == 0 || F.btype == 1) {
+                if (B.loc[2] > 0.0) {
+                    double a2[3];
+                    for (int d = 0; d < 3; ++d) a2[d] = 2.0 * (F.vel[d] - v_i[d]);
+                    const double dp = a2[0] * F.T[6] + a2[1] * F.T[7] + a2[2] * F.T[8];
+                    double av[3];
+                    for (int r = 0; r < 3; ++r) {
+                        double a = 0.0;
+                        for (int k = 0; k < 3; ++k) a = a + F.T[3 * k + r] * B.bi[3 + k];
+                        av[r] = a;
+                    }
+                    gu = gu - dp * F.T[6] * av[0];
+                    gv = gv - dp * F.T[7] * av[1];
+                    gw = gw - dp * F.T[8] * av[2];
+                }
+            } else if (F.btype >= 3) {
+                atomicAdd(&iscal[IS_UNSUPPORTED], 1);
+                break;
+            }
+        }
+        dd = dd - rhoi * (gu + gv + gw);
+    }
+    return dd;
+}
+
+// Leapfrog_continuity.f90:51-68 (with the density_thresholds clamp) and
+// EoS_fluid_loop.f90:59-70.  RK1: the density is integrated after the
+// velocities and positions (Euler.f90:231-241, in vsmooth_end).
+__device__ __forceinline__ void continuity_end(DPC& P, int i, double2 rpi, double dden, double dt, bool eos,
+                                               double* __restrict__ dden_out, double2* __restrict__ rp_out,
+                                               float* __restrict__ dr_out) {
+    dden_out[i] = dden;
+    if (P.rk1) return;
+    double rho1 = rpi.x + dt * dden;
+    if (P.dthr) {  // Leapfrog_continuity.f90:61-68
+        if (rho1 < 0.9 * P.den0) rho1 = 0.9 * P.den0;
+        if (rho1 > 1.1 * P.den0) rho1 = 1.1 * P.den0;
+    }
+    const double p1 = eos ? P.eps / P.den0 * (rho1 - P.den0) + P.prif : rpi.y;
+    rp_out[i] = make_double2(rho1, p1);
+    if (P.f32) dr_out[i] = (float)(rho1 - P.den0);
+}
+
+// the wall part of PressureSmoothing_3D.f90 / _2D.f90 and the update of p and rho;
+// returns the new rho
+__device__ __forceinline__ double psmooth_end(DPC& P, const DFace* __restrict__ faces,
+                                              const int* __restrict__ bn, const BTab* __restrict__ bt, int i,
+                                              int nsp, double2 rpi, double tp1, double somp, double app,
+                                              double* __restrict__ vpres_out, double2* __restrict__ rp_out) {
+    const double p0i = P.prif, pi = rpi.y;
+    double diffp = 0.0;
+    if (nsp > 0) {
+    const int ncbf = P.semi ? bn[i] : 0;
+    if (P.dim == 2) {
+        // PressureSmoothing_2D.f90:124-214, SmoothVersion "b", fixe/tapi
+        // sides; vpres is the smoothed pressure itself
+        double VFT = 0.0;
+        for (int q = 0; q < ncbf; ++q) {
+            const BTab& B = bt[(size_t)q * P.cap + i];
+            const DFace& S = faces[B.face];
+            if (S.btype != 0 && S.btype != 1) continue;
+            const double mf0 = S.T[0] * P.grav[0] + S.T[2] * P.grav[2];
+            const double mf1 = S.T[6] * P.grav[0] + S.T[8] * P.grav[2];
+            VFT = VFT + B.bi[1];
+            somp = somp + P.den0 * (mf0 * B.bi[3] + mf1 * B.bi[4]);
+        }
+        app = app + VFT + 0.0 + 0.0 + 0.0;
+        const double pz = (pi - pi) * 0.0;
+        diffp = pi + tp1 * (somp + pz + pz + (p0i - pi) * (1.0 - app));
+    } else {
+        for (int q = 0; q < ncbf; ++q) {
+            const BTab& B = bt[(size_t)q * P.cap + i];
+            if (B.loc[2] > 0.0) app = app + B.bi[1];
+        }
+        if (P.dbsph) diffp = somp / app;  // PressureSmoothing_3D.f90:110-112
+        else if (app < 0.95) diffp = somp + (p0i - pi) * (1.0 - app);
+        else diffp = somp / app;
+    }
+    } else if (P.dim == 2) {
+        diffp = rpi.y;  // no list (never: self is listed): pressure unchanged
+    }
+    vpres_out[i] = diffp;
+    double p2 = rpi.y, rho2 = rpi.x;
+    if (P.dim == 2) {  // PressureSmoothing_2D.f90:217-231: p = vpres, rho = EoS^-1(p)
+        if (P.tetap > 0.0) {
+            p2 = diffp;
+            rho2 = P.den0 * (1.0 + (p2 - P.prif) / P.eps);
+        }
+    } else if (P.tetap > 0.0) {
+        p2 = rpi.y + tp1 * diffp;
+        rho2 = P.den0 * (1.0 + (p2 - P.prif) / P.eps);
+    }
+    rp_out[i] = make_double2(rho2, p2);
+    return rho2;
+}
+
+// ----------------------------------------------------------------------------
+// The four passes in FP64: one lane per particle, records gathered through
+// L1/L2, the reference's expressions operation for operation.
+// ----------------------------------------------------------------------------
+// momentum: RHS_momentum_equation.f90:72-179, inter_EqMoto.f90:108-283,
+// viscomon.f90:54-71, viscomorris.f90:60-71
+template <bool SG>
+__global__ __launch_bounds__(256) void k_momentum64(
+    Seg S, const DFace* __restrict__ faces, const DEdge* __restrict__ edges,
     const int* __restrict__ bn, const BTab* __restrict__ bt, const double4* __restrict__ xm,
-    const double4* __restrict__ vel, const double2* __restrict__ rp, F4In xmf,
-    F4In velf, const float2* __restrict__ rpf, const int* __restrict__ lam_in,
+    const double4* __restrict__ vel, const double2* __restrict__ rp, const int* __restrict__ lam_in,
     int* __restrict__ lam_out, const uint32_t* __restrict__ nbr, const int* __restrict__ nnb,
-    double4* __restrict__ acc_out, double4* __restrict__ vel_out, F4Out velf_out,
-    const double* scal, int* iscal) {
+    double4* __restrict__ acc_out, double4* __restrict__ vel_out, const double* scal, int* iscal) {
     const int vb = xcd_block(gridDim.x);
     const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * (int)blockDim.x) >> 8]) : 0;
-    const DP& P = SG ? S.P[sg] : P0;
+    DPC& P = S.P[sg];
     scal += sg * SC_COUNT;
     iscal += sg * IS_COUNT;
-    stencil_offsets(P);
     const double h = P.h;
     // Leapfrog_momentum.f90:66-86 integrates with dtvel; the explicit RK1
     // branch (Euler.f90:85-93) with dt
     const double dtvel = P.rk1 ? scal[SC_DT] : scal[SC_DTVEL];
     const size_t N = P.cap;
-    {
-        const int i = vb * blockDim.x + threadIdx.x;
-        if (i - P.base < iscal[IS_N]) {
-            const double4 vi = vel[i];  // var == vel here
-            const double2 rpi = rp[i];
-            double tp[3] = {0.0, 0.0, 0.0}, td[3] = {0.0, 0.0, 0.0}, tv[3] = {0.0, 0.0, 0.0};
-            const int ncbf = P.semi ? bn[i] : 0;
-            const double v_i[3] = {vi.x, vi.y, vi.z};
-            if (ncbf > 0) {
-                if (P.dim == 2)
-                    sa_momentum_2d(P, faces, bt, i, ncbf, v_i, rpi, lam_in[i], tp, td, tv);
-                else
-                    sa_momentum(P, faces, bt, i, ncbf, v_i, rpi, lam_in[i], tp, td, tv, iscal);
-            }
-            const int nn = nnb[i];
-            double rvs[3];
-            if constexpr (!F32) {
-                const double4 xi = xm[i];
-                const double rhoi = rpi.x, pi = rpi.y;
-                double tpa[3] = {0, 0, 0}, ale[3] = {0, 0, 0};
-                rvs[0] = rvs[1] = rvs[2] = 0.0;
-                const double celt = P.celerita + P.celerita;
-                const double nui = P.kin_visc, nuj = P.kin_visc;
-                const bool morris = nui > 1.0e-12 && nuj > 1.0e-12;
-                using RM = NRec<double4, double4, double2>;
-                auto fetch = [&](uint32_t e) {
-                    const int j = (int)(e & NB_MASK);
-                    return RM{xm[j], vel[j], rp[j]};
-                };
-                walk_list<4, RM>(nbr, N, i, nn, fetch, [&](uint32_t e, const RM& q) {
-                    if ((int)(e & NB_MASK) == i) return;
-                    const double4 xj = q.x;
-                    const double4 vj = q.v;
-                    const double2 rpj = q.r;
-                    const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
-                    const double rij = R0 * R0 + R1 * R1 + R2 * R2;
-                    K64 K;
-                    kvals64(P, rij, true, true, false, K);
-                    const double rhoj = rpj.x, pj = rpj.y, amassj = xj.w;
-                    const double dv0 = vj.x - vi.x, dv1 = vj.y - vi.y, dv2 = vj.z - vi.z;
-                    double alpha = (pj - pi) / (rhoi * rhoj);
-                    tpa[0] = tpa[0] + -amassj * alpha * R0 * K.K3;
-                    tpa[1] = tpa[1] + -amassj * alpha * R1 * K.K3;
-                    tpa[2] = tpa[2] + -amassj * alpha * R2 * K.K3;
-                    alpha = (pi * (rhoj / rhoi + 1.0) + pj * (rhoi / rhoj - 1.0)) / (rhoi * rhoj);
-                    ale[0] = ale[0] - amassj * alpha * R0 * K.K3;
-                    ale[1] = ale[1] - amassj * alpha * R1 * K.K3;
-                    ale[2] = ale[2] - amassj * alpha * R2 * K.K3;
-                    const double vrij = -dv0 * R0 - dv1 * R1 - dv2 * R2;
-                    const double TermMon = P.alfamon * celt * h / (rhoi + rhoj);
-                    td[0] = td[0] + (amassj * TermMon * vrij * R0 * K.K2 + 0.0);
-                    td[1] = td[1] + (amassj * TermMon * vrij * R1 * K.K2 + 0.0);
-                    td[2] = td[2] + (amassj * TermMon * vrij * R2 * K.K2 + 0.0);
-                    if (morris) {
-                        const double rtil = nui * rhoi + nuj * rhoj + 1.0e-3;
-                        const double atil = 4.0 * (nui * nuj);
-                        const double fac = amassj * atil / rtil;
-                        const double rr = R0 * R0 + R1 * R1 + R2 * R2;
-                        const double w0 = fac * (-dv0 * K.K2 * rr);
-                        const double w1 = fac * (-dv1 * K.K2 * rr);
-                        const double w2 = fac * (-dv2 * K.K2 * rr);
-                        tv[0] = tv[0] + w0; tv[1] = tv[1] + w1; tv[2] = tv[2] + w2;
-                        rvs[0] = rvs[0] + w0; rvs[1] = rvs[1] + w1; rvs[2] = rvs[2] + w2;
-                    }
-                });
-                for (int d = 0; d < 3; ++d) tp[d] = tp[d] + tpa[d] + ale[d];
-            } else {
-                                // symmetric form -m_j (p_i/rho_i^2 + p_j/rho_j^2) r K3 of the
-                // reference's difference term plus its ALE1 complement
-                const float4 xf = xmf[i];
-                const float4 vf = velf[i];
-                const float2 rpfi = rpf[i];
-                const float rhoi = rpfi.x, pi = rpfi.y;
-                const float pri = pi * __builtin_amdgcn_rcpf(rhoi * rhoi);
-                float s_p0 = 0.f, s_p1 = 0.f, s_p2 = 0.f, s_d0 = 0.f, s_d1 = 0.f, s_d2 = 0.f;
-                float s_v0 = 0.f, s_v1 = 0.f, s_v2 = 0.f;
-                const float mon = P.f_alfamon * (P.f_celerita + P.f_celerita) * P.f_h;
-                const float nu = P.f_kin_visc;
-                const float atil = 4.0f * (nu * nu);
-                const bool morris = P.kin_visc > 1.0e-12;
-                // neighbour records: (x, m) and (v, rho - den0); the pressure
-                // follows from the linear EoS, so one 32-byte run per neighbour
-                using RM = NRec2<float4, float4>;
-                auto fetch = [&](uint32_t e) {
-                    const int j = (int)(e & NB_MASK);
-                    return RM{xmf[j], velf[j]};
-                };
-                walk_list<CH, RM>(nbr, N, i, nn, fetch, [&](uint32_t e, const RM& q) {
-                    if ((int)(e & NB_MASK) == i) return;
-                    const float4 xj = q.x;
-                    const float4 vj = q.r;
-                    float R0, R1, R2;
-                    rag32(xf, xj, e, R0, R1, R2);
-                    const float rij = R0 * R0 + R1 * R1 + R2 * R2;
-                    K32 K;
-                    kvals32(P, rij, true, true, false, K);
-                    const float rhoj = P.f_den0 + vj.w, pj = __builtin_fmaf(P.f_eosk, vj.w, P.f_prif);
-                    const float mj = xj.w;
-                    const float dv0 = vj.x - vf.x, dv1 = vj.y - vf.y, dv2 = vj.z - vf.z;
-                    const float cp = -mj * (pri + pj * __builtin_amdgcn_rcpf(rhoj * rhoj)) * K.K3;
-                    s_p0 += cp * R0; s_p1 += cp * R1; s_p2 += cp * R2;
-                    const float vrij = -(dv0 * R0 + dv1 * R1 + dv2 * R2);
-                    const float cd = mj * mon * __builtin_amdgcn_rcpf(rhoi + rhoj) * vrij * K.K2;
-                    s_d0 += cd * R0; s_d1 += cd * R1; s_d2 += cd * R2;
-                    if (morris) {
-                        const float fac = mj * atil * __builtin_amdgcn_rcpf(nu * rhoi + nu * rhoj + 1.0e-3f);
-                        const float cv = -fac * K.K2 * rij;
-                        s_v0 += cv * dv0; s_v1 += cv * dv1; s_v2 += cv * dv2;
-                    }
-                });
-                tp[0] = tp[0] + (double)s_p0; tp[1] = tp[1] + (double)s_p1; tp[2] = tp[2] + (double)s_p2;
-                td[0] = td[0] + (double)s_d0; td[1] = td[1] + (double)s_d1; td[2] = td[2] + (double)s_d2;
-                tv[0] = tv[0] + (double)s_v0; tv[1] = tv[1] + (double)s_v1; tv[2] = tv[2] + (double)s_v2;
-                rvs[0] = s_v0; rvs[1] = s_v1; rvs[2] = s_v2;
-            }
-            int lam = 0;
-            if (P.kin_visc > 0.0) {
-                const double apg = sqrt(tp[0] * tp[0] + tp[1] * tp[1] + tp[2] * tp[2]) + P.GI;
-                const double amo = sqrt(rvs[0] * rvs[0] + rvs[1] * rvs[1] + rvs[2] * rvs[2]);
-                double w = 0.0;
-                if (apg != 0.0) w = amo / apg * 100.0;
-                lam = (w > 5.0 || apg == 0.0) ? 1 : 0;
-            }
-            lam_out[i] = lam;
-            double a[3];
-            if (ncbf > 0 && P.dim == 2) {
-                double br[3] = {0.0, 0.0, 0.0};
-                elastic_2d(P, faces, bt, i, ncbf, v_i, br);
-                for (int d = 0; d < 3; ++d) a[d] = tp[d] + td[d] + tv[d] + P.grav[d] + br[d];
-            } else if (ncbf > 0) {
-                double br[3] = {0.0, 0.0, 0.0};
-                const double zimin = 0.25 * P.dx;
-                const double celer02 = P.eps / P.den0;
-                // AddElasticBoundaryReaction_3D.f90:72-104 (faces); rea: the
-                // slots whose face reacted (ReaFace), for the edges below
-                static_assert(SPH_MB <= 32, "one ReaFace bit per boundary-table slot");
-                unsigned rea = 0u;
-                for (int q = 0; q < ncbf; ++q) {
-                    const BTab& B = bt[(size_t)q * P.cap + i];
-                    const DFace& F = faces[B.face];
-                    if (F.btype != 0 && F.btype != 1) continue;
-                    const double zi = B.loc[2];
-                    if (zi < zimin && d_point_internal(F, B.loc[0], B.loc[1])) {
-                        double vin = 0.0;
-                        for (int sd = 0; sd < 3; ++sd) vin = vin + v_i[sd] * F.T[6 + sd];
-                        if (vin < 0.0) {
-                            const double nr = -1.0 * celer02 * log((h + zi - zimin) / h) / h;
-                            for (int d = 0; d < 3; ++d) br[d] = br[d] + nr * F.T[6 + d];
-                        }
-                        rea |= 1u << q;
-                    }
-                }
-                // AddElasticBoundaryReaction_3D.f90:106-152 (convex edges, in
-                // order; the reference returns at the first edge whose two
-                // faces are not both among the particle's non-reacting faces)
-                for (int ne = 0; ne < P.ne; ++ne) {
-                    const DEdge& E = edges[P.eoff + ne];
-                    int nclose = 0;
-                    for (int q = 0; q < ncbf; ++q) {
-                        const int f = bt[(size_t)q * P.cap + i].face;
-                        const bool rq = (rea >> q) & 1u;
-                        if (f == E.face[0] && !rq) ++nclose;
-                        else if (f == E.face[1] && !rq) ++nclose;
-                    }
-                    if (nclose != 2) break;
-                    const double4 xi = xm[i];
-                    const double x[3] = {xi.x, xi.y, xi.z};
-                    double scaprod = 0.0;
-                    for (int sd = 0; sd < 3; ++sd) scaprod = scaprod + (x[sd] - E.gx[sd]) * E.comp[sd];
-                    const double tau = scaprod / (E.len * E.len);
-                    if (tau >= 0.0 && tau <= 1.0) {
-                        double QP[3], d2 = 0.0;
-                        for (int sd = 0; sd < 3; ++sd) QP[sd] = x[sd] - (E.gx[sd] + E.comp[sd] * tau);
-                        for (int sd = 0; sd < 3; ++sd) d2 = d2 + QP[sd] * QP[sd];
-                        const double zi = sqrt(d2);
-                        if (zi < zimin) {
-                            double cd[3], vin = 0.0;
-                            for (int sd = 0; sd < 3; ++sd) cd[sd] = QP[sd] / zi;
-                            for (int sd = 0; sd < 3; ++sd) vin = vin + v_i[sd] * cd[sd];
-                            if (vin < 0.0) {
-                                const double nr = -1.0 * celer02 * log(zi / zimin) / zimin;
-                                for (int d = 0; d < 3; ++d) br[d] = br[d] + nr * cd[d];
-                            }
-                        }
-                    }
-                }
-                for (int d = 0; d < 3; ++d) a[d] = tp[d] + td[d] + tv[d] + P.grav[d] + br[d];
-            } else {
-                for (int d = 0; d < 3; ++d) a[d] = tp[d] + td[d] + tv[d] + P.grav[d];
-            }
-            acc_out[i] = make_double4(a[0], a[1], a[2], 0.0);
-            // Leapfrog_momentum (RK1: Euler): vel = vel + dtvel*acc (kodvel == 0)
-            const double4 vn =
-                make_double4(vi.x + dtvel * a[0], vi.y + dtvel * a[1], vi.z + dtvel * a[2], vi.w);
-            vel_out[i] = vn;
-            if (F32) velf_out[i] = make_float4((float)vn.x, (float)vn.y, (float)vn.z, (float)(rpi.x - P.den0));
+    const int i = vb * blockDim.x + threadIdx.x;
+    if (i - P.base < iscal[IS_N]) {
+        const double4 vi = vel[i];  // var == vel here
+        const double2 rpi = rp[i];
+        double tp[3] = {0.0, 0.0, 0.0}, td[3] = {0.0, 0.0, 0.0}, tv[3] = {0.0, 0.0, 0.0};
+        const int ncbf = P.semi ? bn[i] : 0;
+        const double v_i[3] = {vi.x, vi.y, vi.z};
+        if (ncbf > 0) {
+            if (P.dim == 2)
+                sa_momentum_2d(P, faces, bt, i, ncbf, v_i, rpi, lam_in[i], tp, td, tv);
+            else
+                sa_momentum(P, faces, bt, i, ncbf, v_i, rpi, lam_in[i], tp, td, tv, iscal);
         }
-        __syncthreads();
+        const int nn = nnb[i];
+        double rvs[3];
+        const double4 xi = xm[i];
+        const double rhoi = rpi.x, pi = rpi.y;
+        double tpa[3] = {0, 0, 0}, ale[3] = {0, 0, 0};
+        rvs[0] = rvs[1] = rvs[2] = 0.0;
+        const double celt = P.celerita + P.celerita;
+        const double nui = P.kin_visc, nuj = P.kin_visc;
+        const bool morris = nui > 1.0e-12 && nuj > 1.0e-12;
+        using RM = NRec<double4, double4, double2>;
+        auto fetch = [&](uint32_t e) {
+            const int j = (int)(e & NB_MASK);
+            return RM{xm[j], vel[j], rp[j]};
+        };
+        walk_list<4, RM>(nbr, N, i, nn, fetch, [&](uint32_t e, const RM& q) {
+            if ((int)(e & NB_MASK) == i) return;
+            const double4 xj = q.x;
+            const double4 vj = q.v;
+            const double2 rpj = q.r;
+            const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
+            const double rij = R0 * R0 + R1 * R1 + R2 * R2;
+            K64 K;
+            kvals64(P, rij, true, true, false, K);
+            const double rhoj = rpj.x, pj = rpj.y, amassj = xj.w;
+            const double dv0 = vj.x - vi.x, dv1 = vj.y - vi.y, dv2 = vj.z - vi.z;
+            double alpha = (pj - pi) / (rhoi * rhoj);
+            tpa[0] = tpa[0] + -amassj * alpha * R0 * K.K3;
+            tpa[1] = tpa[1] + -amassj * alpha * R1 * K.K3;
+            tpa[2] = tpa[2] + -amassj * alpha * R2 * K.K3;
+            alpha = (pi * (rhoj / rhoi + 1.0) + pj * (rhoi / rhoj - 1.0)) / (rhoi * rhoj);
+            ale[0] = ale[0] - amassj * alpha * R0 * K.K3;
+            ale[1] = ale[1] - amassj * alpha * R1 * K.K3;
+            ale[2] = ale[2] - amassj * alpha * R2 * K.K3;
+            const double vrij = -dv0 * R0 - dv1 * R1 - dv2 * R2;
+            const double TermMon = P.alfamon * celt * h / (rhoi + rhoj);
+            td[0] = td[0] + (amassj * TermMon * vrij * R0 * K.K2 + 0.0);
+            td[1] = td[1] + (amassj * TermMon * vrij * R1 * K.K2 + 0.0);
+            td[2] = td[2] + (amassj * TermMon * vrij * R2 * K.K2 + 0.0);
+            if (morris) {
+                const double rtil = nui * rhoi + nuj * rhoj + 1.0e-3;
+                const double atil = 4.0 * (nui * nuj);
+                const double fac = amassj * atil / rtil;
+                const double rr = R0 * R0 + R1 * R1 + R2 * R2;
+                const double w0 = fac * (-dv0 * K.K2 * rr);
+                const double w1 = fac * (-dv1 * K.K2 * rr);
+                const double w2 = fac * (-dv2 * K.K2 * rr);
+                tv[0] = tv[0] + w0; tv[1] = tv[1] + w1; tv[2] = tv[2] + w2;
+                rvs[0] = rvs[0] + w0; rvs[1] = rvs[1] + w1; rvs[2] = rvs[2] + w2;
+            }
+        });
+        for (int d = 0; d < 3; ++d) tp[d] = tp[d] + tpa[d] + ale[d];
+        double br[3] = {0.0, 0.0, 0.0};
+        if (ncbf > 0) elastic_walls(P, faces, edges, bt, xm, i, ncbf, vi, br);
+        momentum_end(P, i, ncbf, vi, dtvel, tp, td, tv, rvs, br, lam_out, acc_out, vel_out);
     }
 }
 
-// ----------------------------------------------------------------------------
-// velocity smoothing: velocity_smoothing.f90:74-133, velocity_smoothing_SA_SPH
-// _3D.f90:64-122 (FP64), velocity_smoothing_2.f90:59-103; fused
-// Leapfrog_trajectories.f90:48-76 and the particle part of the next
-// time_step_duration.  Neighbour density travels in velf.w (FP32).  Explicit
-// RK1: the same smoothing, update and positions (Euler.f90:94-139), then the
-// density update and EoS of Euler.f90:231-241 and time_integration.f90:52-65.
-// ----------------------------------------------------------------------------
-template <bool F32, int CH, bool SG>
-__global__ __launch_bounds__(256) void k_vsmooth(
-    DP P0, Seg S, const DFace* __restrict__ faces,
+// velocity smoothing: velocity_smoothing.f90:74-133
+template <bool SG>
+__global__ __launch_bounds__(256) void k_vsmooth64(
+    Seg S, const DFace* __restrict__ faces,
     const int* __restrict__ bn, const BTab* __restrict__ bt, const double4* __restrict__ xm,
-    const double4* __restrict__ vel1, const double2* __restrict__ rp, F4In xmf,
-    F4In velf1, const uint32_t* __restrict__ nbr, const int* __restrict__ nnb,
-    double4* __restrict__ vel_out, double4* __restrict__ xm_out,
+    const double4* __restrict__ vel1, const double2* __restrict__ rp, const uint32_t* __restrict__ nbr,
+    const int* __restrict__ nnb, double4* __restrict__ vel_out, double4* __restrict__ xm_out,
     const double* scal, unsigned long long* dtmin, int* iscal, const double* __restrict__ dden_in,
-    double2* __restrict__ rp_out, float2* __restrict__ rpf_out, float4* __restrict__ xrf_out,
-    int* __restrict__ gone) {
-    using X = typename Rec<F32>::X;
-    using V = typename Rec<F32>::V;
-    using RT = typename std::conditional<F32, float, double>::type;
+    double2* __restrict__ rp_out, int* __restrict__ gone) {
     const int vb = xcd_block(gridDim.x);
     const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * (int)blockDim.x) >> 8]) : 0;
-    const DP& P = SG ? S.P[sg] : P0;
+    DPC& P = S.P[sg];
     scal += sg * SC_COUNT;
     iscal += sg * IS_COUNT;
     const bool eos = iscal[IS_ONGOING] > 0;
     dtmin += sg;
-    stencil_offsets(P);
     const size_t N = P.cap;
     const bool smooth = P.tetav > 1.0e-9;
-    const double tv1 = scal[SC_TV1];
-    const double dt = scal[SC_DT];
     unsigned long long dtbits = 0x7FF0000000000000ull;
-    {
-        const int i = vb * blockDim.x + threadIdx.x;
-        if (i - P.base < iscal[IS_N]) {
-            const double4 xi = xm[i];
-            const double4 vi = vel1[i];
-            double v[3] = {0.0, 0.0, 0.0};
-            if (smooth) {
-                const int nn = nnb[i];
-                if constexpr (!F32) {
-                    using RV = NRec<double4, double4, double>;
-                    auto fetch = [&](uint32_t e) {
-                        const int j = (int)(e & NB_MASK);
-                            return RV{xm[j], vel1[j], rp[j].x};
-                    };
-                    walk_list<4, RV>(nbr, N, i, nn, fetch, [&](uint32_t e, const RV& q) {
-                        const double4 xj = q.x;
-                        const double4 vj = q.v;
-                        const double rhoj = q.r;
-                        const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
-                        const double rij = R0 * R0 + R1 * R1 + R2 * R2;
-                        K64 K;
-                        kvals64(P, rij, false, false, true, K);
-                        const double pes = xj.w * K.W / rhoj;
-                        v[0] = v[0] + (vj.x - vi.x) * pes;
-                        v[1] = v[1] + (vj.y - vi.y) * pes;
-                        v[2] = v[2] + (vj.z - vi.z) * pes;
-                                        });
-                } else {
-                                        const float4 xf = xmf[i];
-                    const float4 vf = velf1[i];
-                    float s0 = 0.f, s1 = 0.f, s2 = 0.f;
-                    using RV = NRec2<float4, float4>;
-                    auto fetch = [&](uint32_t e) {
-                        const int j = (int)(e & NB_MASK);
-                            return RV{xmf[j], velf1[j]};
-                    };
-                    walk_list<CH, RV>(nbr, N, i, nn, fetch, [&](uint32_t e, const RV& q) {
-                        const float4 xj = q.x;
-                        const float4 vj = q.r;
-                        float R0, R1, R2;
-                        rag32(xf, xj, e, R0, R1, R2);
-                        K32 K;
-                        kvals32(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true, K);
-                        const float pes = xj.w * K.W * __builtin_amdgcn_rcpf(P.f_den0 + vj.w);
-                        s0 += (vj.x - vf.x) * pes;
-                        s1 += (vj.y - vf.y) * pes;
-                        s2 += (vj.z - vf.z) * pes;
-                                        });
-                    v[0] = s0; v[1] = s1; v[2] = s2;
-                }
-                const int ncbf = P.semi ? bn[i] : 0;
-                // velocity_smoothing_SA_SPH_2D.f90:64-118 (fixe/tapi sides)
-                for (int q = 0; q < ncbf && P.dim == 2; ++q) {
-                    const BTab& B = bt[(size_t)q * P.cap + i];
-                    const DFace& S = faces[B.face];
-                    if (S.btype != 0 && S.btype != 1) continue;
-                    const double s0 = S.T[0], s1 = S.T[2], n0 = S.T[6], n1 = S.T[8];
-                    const double DVG0 = 2.0 * (S.tvel[0] - vi.x), DVG1 = 2.0 * (S.tvel[2] - vi.z);
-                    const double DVL0 = s0 * DVG0 + s1 * DVG1;
-                    const double DVL1 = n0 * DVG0 + n1 * DVG1;
-                    const double IntWdV = B.bi[2];
-                    double slip = S.mode == 1 ? S.slip : 0.0;
-                    if (S.mode == 2) {
-                        // velocity_smoothing_SA_SPH_2D.f90:93-106
-                        const double u0 = (S.tvel[0] - vi.x) - (0.5 * DVL1 * S.T[6]);
-                        const double u1 = (S.tvel[1] - vi.y) - (0.5 * DVL1 * S.T[7]);
-                        const double u2 = (S.tvel[2] - vi.z) - (0.5 * DVL1 * S.T[8]);
-                        double nut;
-                        wall_function(sqrt(u0 * u0 + u1 * u1 + u2 * u2), S.slip * 10.0, B.loc[1], P.dx,
-                                      slip, nut);
-                    }
-                    const double BCL0 = DVL0 * IntWdV * slip;
-                    const double BCL1 = DVL1 * IntWdV;
-                    v[0] = v[0] + (s0 * BCL0 + n0 * BCL1);
-                    v[2] = v[2] + (s1 * BCL0 + n1 * BCL1);
-                }
-                for (int q = 0; q < ncbf && P.dim == 3; ++q) {
-                    const BTab& B = bt[(size_t)q * P.cap + i];
-                    const DFace& F = faces[B.face];
-                    if (F.btype == 3 || F.btype == 4 || F.btype == 5) {
-                        v[0] = v[1] = v[2] = 0.0;
-                        break;
-                    }
-                    if (F.btype != 0 && F.btype != 1) continue;
-                    const double DVG[3] = {2.0 * (F.tvel[0] - vi.x), 2.0 * (F.tvel[1] - vi.y),
-                                           2.0 * (F.tvel[2] - vi.z)};
-                    double DVL[3];
-                    for (int ii = 0; ii < 3; ++ii) {
-                        double a = 0.0;
-                        for (int jj = 0; jj < 3; ++jj) a = a + F.T[3 * ii + jj] * DVG[jj];
-                        DVL[ii] = a;
-                    }
-                    const double IntWdV = B.bi[1];
-                    double slip = F.mode == 1 ? F.slip : 0.0;
-                    if (F.mode == 2) {
-                        // velocity_smoothing_SA_SPH_3D.f90:89-110
-                        double ut[3], nut;
-                        for (int d = 0; d < 3; ++d) ut[d] = 0.5 * (DVG[d] - DVL[2] * F.T[6 + d]);
-                        wall_function(sqrt(ut[0] * ut[0] + ut[1] * ut[1] + ut[2] * ut[2]), F.slip * 10.0,
-                                      B.loc[2], P.dx, slip, nut);
-                    }
-                    const double BCL[3] = {DVL[0] * IntWdV * slip, DVL[1] * IntWdV * slip,
-                                           DVL[2] * IntWdV};
-                    for (int ii = 0; ii < 3; ++ii) {
-                        double a = 0.0;
-                        for (int jj = 0; jj < 3; ++jj) a = a + F.T[3 * jj + ii] * BCL[jj];
-                        v[ii] = v[ii] + a;
-                    }
-                }
-            }
-            double4 vn = vi;
-            if (smooth) vn = make_double4(vi.x + tv1 * v[0], vi.y + tv1 * v[1], vi.z + tv1 * v[2], vi.w);
-            vel_out[i] = vn;
-
-            const double xn[3] = {xi.x + dt * vn.x, xi.y + dt * vn.y, xi.z + dt * vn.z};
-            xm_out[i] = make_double4(xn[0], xn[1], xn[2], xi.w);
-            // the next time_step_duration runs over the particles the coming
-            // OrdGrid1 keeps: not those out of the grid, nor those that left
-            // through an open face
-            bool stays = d_particle_cell(P, xn[0], xn[1], xn[2]) > 0;
-            if (P.nopen > 0) {  // CancelOutgoneParticles_3D / _2D on the step just made
-                const double xo[3] = {xi.x, xi.y, xi.z};
-                int g = 0;
-                for (int f = P.foff; f < P.foff + P.nf; ++f)
-                    if (faces[f].btype == 2 &&
-                        (P.dim == 2 ? open_side_crossed(faces[f], xo, xn) : open_face_crossed(faces[f], xo, xn)))
-                        g = 1;
-                gone[i] = g;
-                stays = stays && !g;
-            }
-            if (P.rk1 && !P.dbsph) {
-                // explicit RK1: Euler.f90:231-241 (dens = dens + dt dden) and
-                // EoS_fluid_loop.f90:59-70 (time_integration.f90:52-65); the
-                // pressure smoothing that follows reads these with the
-                // stage's kernel values, hence the old cell-relative position
-                const double2 rpi = rp[i];
-                const double rho1 = rpi.x + dt * dden_in[i];
-                const double p1 = eos ? P.eps / P.den0 * (rho1 - P.den0) + P.prif : rpi.y;
-                rp_out[i] = make_double2(rho1, p1);
-                if (F32) {
-                    rpf_out[i] = make_float2((float)rho1, (float)p1);
-                    const float4 xo = xmf[i];
-                    xrf_out[i] = make_float4(xo.x, xo.y, xo.z, (float)(rho1 - P.den0));
-                }
-            }
-            if (stays) {
-                const unsigned long long b =
-                    (unsigned long long)__double_as_longlong(d_dt_cfl(P, vn.x, vn.y, vn.z));
-                dtbits = b < dtbits ? b : dtbits;
-            }
+    const int i = vb * blockDim.x + threadIdx.x;
+    if (i - P.base < iscal[IS_N]) {
+        const double4 xi = xm[i];
+        const double4 vi = vel1[i];
+        double v[3] = {0.0, 0.0, 0.0};
+        if (smooth) {
+            const int nn = nnb[i];
+            using RV = NRec<double4, double4, double>;
+            auto fetch = [&](uint32_t e) {
+                const int j = (int)(e & NB_MASK);
+                    return RV{xm[j], vel1[j], rp[j].x};
+            };
+            walk_list<4, RV>(nbr, N, i, nn, fetch, [&](uint32_t e, const RV& q) {
+                const double4 xj = q.x;
+                const double4 vj = q.v;
+                const double rhoj = q.r;
+                const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
+                const double rij = R0 * R0 + R1 * R1 + R2 * R2;
+                K64 K;
+                kvals64(P, rij, false, false, true, K);
+                const double pes = xj.w * K.W / rhoj;
+                v[0] = v[0] + (vj.x - vi.x) * pes;
+                v[1] = v[1] + (vj.y - vi.y) * pes;
+                v[2] = v[2] + (vj.z - vi.z) * pes;
+                                });
+            vsmooth_walls(P, faces, bt, i, P.semi ? bn[i] : 0, vi, v);
         }
-        __syncthreads();
+        dtbits = vsmooth_end<false>(P, faces, i, xi, vi, v, smooth, scal[SC_TV1], scal[SC_DT], eos, dden_in, rp,
+                             vel_out, xm_out, rp_out, nullptr, gone);
     }
     block_min_to(dtbits, dtmin);
 }
 
-// ----------------------------------------------------------------------------
-// continuity: SASPH_continuity.f90:89-169 with AddBoundaryContribution_to_CE3D
-// .f90:82-169 (FP64), Continuity_Equation.f90:97-235; fused
-// Leapfrog_continuity.f90:51-68 (with the density_thresholds clamp) and EoS_fluid_loop.f90:59-70
-// ----------------------------------------------------------------------------
-template <bool F32, int CH, bool SG>
-__global__ __launch_bounds__(256) void k_continuity(
-    DP P0, Seg S, const DFace* __restrict__ faces,
+// continuity: SASPH_continuity.f90:89-169, Continuity_Equation.f90:97-235
+template <bool SG>
+__global__ __launch_bounds__(256) void k_continuity64(
+    Seg S, const DFace* __restrict__ faces,
     const int* __restrict__ bn, const BTab* __restrict__ bt, const double4* __restrict__ xm,
-    const double4* __restrict__ vel, const double2* __restrict__ rp, F4In xmf,
-    F4In velf, const uint32_t* __restrict__ nbr, const int* __restrict__ nnb,
-    double* __restrict__ dden_out, double2* __restrict__ rp_out, float2* __restrict__ rpf_out,
-    float4* __restrict__ xrf_out,
+    const double4* __restrict__ vel, const double2* __restrict__ rp, const uint32_t* __restrict__ nbr,
+    const int* __restrict__ nnb, double* __restrict__ dden_out, double2* __restrict__ rp_out,
     const double* scal, int* iscal) {
-    using X = typename Rec<F32>::X;
-    using V = typename Rec<F32>::V;
-    using RT = typename std::conditional<F32, float, double>::type;
     const int vb = xcd_block(gridDim.x);
     const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * (int)blockDim.x) >> 8]) : 0;
-    const DP& P = SG ? S.P[sg] : P0;
+    DPC& P = S.P[sg];
     scal += sg * SC_COUNT;
     iscal += sg * IS_COUNT;
-    stencil_offsets(P);
     const size_t N = P.cap;
-    const double dt = scal[SC_DT];
-    const bool eos = iscal[IS_ONGOING] > 0;
-    {
-        const int i = vb * blockDim.x + threadIdx.x;
-        if (i - P.base < iscal[IS_N]) {
-            const double4 vi = vel[i];
-            const double2 rpi = rp[i];
-            const double rhoi = rpi.x;
-            double dd = 0.0;
-            const int ncbf = P.semi ? bn[i] : 0;
-            if (ncbf > 0 && P.dim == 2) {
-                // SASPH_continuity.f90:126-169 with AddBoundaryContribution_to_CE2D
-                // .f90:74-150 (fixe/tapi sides): grad_u_SA(1) and grad_w_SA(3)
-                double gu0 = 0.0, gw2 = 0.0;
-                for (int q = 0; q < ncbf; ++q) {
-                    const BTab& B = bt[(size_t)q * P.cap + i];
-                    const DFace& S = faces[B.face];
-                    if (S.btype != 0 && S.btype != 1) continue;
-                    const double IntWdS = B.bi[0];
-                    double dv0, dv1;
-                    if (S.btype == 0) {
-                        dv0 = 2.0 * (-vi.x);
-                        dv1 = 2.0 * (-vi.z);
-                    } else {
-                        dv0 = 2.0 * (S.vel[0] - vi.x);
-                        dv1 = 2.0 * (S.vel[2] - vi.z);
-                    }
-                    gu0 = gu0 - dv0 * S.T[6] * IntWdS;
-                    gw2 = gw2 - dv1 * S.T[8] * IntWdS;
-                }
-                dd = dd - rhoi * (gu0 + 0.0 + gw2);
-            } else if (ncbf > 0) {
-                double gu = 0.0, gv = 0.0, gw = 0.0;
-                const double v_i[3] = {vi.x, vi.y, vi.z};
-                for (int q = 0; q < ncbf; ++q) {
-                    const BTab& B = bt[(size_t)q * P.cap + i];
-                    const DFace& F = faces[B.face];
-                    if (F.btype == 0 || F.btype == 1) {
-                        if (B.loc[2] > 0.0) {
-                            double a2[3];
-                            for (int d = 0; d < 3; ++d) a2[d] = 2.0 * (F.vel[d] - v_i[d]);
-                            const double dp = a2[0] * F.T[6] + a2[1] * F.T[7] + a2[2] * F.T[8];
-                            double av[3];
-                            for (int r = 0; r < 3; ++r) {
-                                double a = 0.0;
-                                for (int k = 0; k < 3; ++k) a = a + F.T[3 * k + r] * B.bi[3 + k];
-                                av[r] = a;
-                            }
-                            gu = gu - dp * F.T[6] * av[0];
-                            gv = gv - dp * F.T[7] * av[1];
-                            gw = gw - dp * F.T[8] * av[2];
-                        }
-                    } else if (F.btype >= 3) {
-                        atomicAdd(&iscal[IS_UNSUPPORTED], 1);
-                        break;
-                    }
-                }
-                dd = dd - rhoi * (gu + gv + gw);
-            }
-            const int nn = nnb[i];
-            double inner;
-            if constexpr (!F32) {
-                const double4 xi = xm[i];
-                double a1 = 0.0, a2 = 0.0, a3 = 0.0;
-                using RC = NRec<double4, double4, double>;
-                auto fetch = [&](uint32_t e) {
-                    const int j = (int)(e & NB_MASK);
-                    return RC{xm[j], vel[j], rp[j].x};
-                };
-                walk_list<4, RC>(nbr, N, i, nn, fetch, [&](uint32_t e, const RC& q) {
-                    const double4 xj = q.x;
-                    const double4 vj = q.v;
-                    const double rhoj = q.r;
-                    const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
-                    const double rij = R0 * R0 + R1 * R1 + R2 * R2;
-                    K64 K;
-                    kvals64(P, rij, true, false, false, K);
-                    const double amassj = xj.w;
-                    a1 = a1 + rhoi * (amassj / rhoj) * K.K1 * (vj.x - vi.x) * R0;
-                    a2 = a2 + rhoi * (amassj / rhoj) * K.K1 * (vj.y - vi.y) * R1;
-                    a3 = a3 + rhoi * (amassj / rhoj) * K.K1 * (vj.z - vi.z) * R2;
+    const int i = vb * blockDim.x + threadIdx.x;
+    if (i - P.base < iscal[IS_N]) {
+        const double4 vi = vel[i];
+        const double2 rpi = rp[i];
+        const double rhoi = rpi.x;
+        const double dd = continuity_walls(P, faces, bt, i, P.semi ? bn[i] : 0, vi, rhoi, iscal);
+        const int nn = nnb[i];
+        const double4 xi = xm[i];
+        double a1 = 0.0, a2 = 0.0, a3 = 0.0;
+        using RC = NRec<double4, double4, double>;
+        auto fetch = [&](uint32_t e) {
+            const int j = (int)(e & NB_MASK);
+            return RC{xm[j], vel[j], rp[j].x};
+        };
+        walk_list<4, RC>(nbr, N, i, nn, fetch, [&](uint32_t e, const RC& q) {
+            const double4 xj = q.x;
+            const double4 vj = q.v;
+            const double rhoj = q.r;
+            const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
+            const double rij = R0 * R0 + R1 * R1 + R2 * R2;
+            K64 K;
+            kvals64(P, rij, true, false, false, K);
+            const double amassj = xj.w;
+            a1 = a1 + rhoi * (amassj / rhoj) * K.K1 * (vj.x - vi.x) * R0;
+            a2 = a2 + rhoi * (amassj / rhoj) * K.K1 * (vj.y - vi.y) * R1;
+            a3 = a3 + rhoi * (amassj / rhoj) * K.K1 * (vj.z - vi.z) * R2;
+                        });
+        const double inner = a1 + a2 + a3;
+        continuity_end(P, i, rpi, dd - inner, scal[SC_DT], iscal[IS_ONGOING] > 0, dden_out, rp_out, nullptr);
+    }
+}
+
+// pressure smoothing: PressureSmoothing_3D.f90:80-161 (both loops)
+template <bool SG>
+__global__ __launch_bounds__(256) void k_psmooth64(
+    Seg S, const DFace* __restrict__ faces, const int* __restrict__ bn, const BTab* __restrict__ bt,
+    const double4* __restrict__ xm, const double2* __restrict__ rp, const uint32_t* __restrict__ nbr,
+    const int* __restrict__ nnb, double* __restrict__ vpres_out, double2* __restrict__ rp_out,
+    const double* scal, const int* iscal) {
+    const int vb = xcd_block(gridDim.x);
+    const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * (int)blockDim.x) >> 8]) : 0;
+    DPC& P = S.P[sg];
+    scal += sg * SC_COUNT;
+    iscal += sg * IS_COUNT;
+    const size_t N = P.cap;
+    const int i = vb * blockDim.x + threadIdx.x;
+    if (i - P.base < iscal[IS_N]) {
+        const double2 rpi = rp[i];
+        const int nsp = nnb[i];
+        const double pi = rpi.y;
+        double somp = 0.0, app = 0.0;
+        if (nsp > 0) {
+            const double4 xi = xm[i];
+            somp = 0.0;
+            app = 0.0;
+            using RP2 = NRec2<double4, double2>;
+            auto fetch = [&](uint32_t e) {
+                const int j = (int)(e & NB_MASK);
+                    return RP2{xm[j], rp[j]};
+            };
+            walk_list<4, RP2>(nbr, N, i, nsp, fetch, [&](uint32_t e, const RP2& q) {
+                const double4 xj = q.x;
+                const double2 rpj = q.r;
+                const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
+                K64 K;
+                kvals64(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true, K);
+                const double pes = xj.w * K.W / rpj.x;
+                app = app + pes;
+                somp = somp + (rpj.y - pi) * pes;
                                 });
-                inner = a1 + a2 + a3;
-            } else {
-                                const float4 xf = xmf[i];
-                const float4 vf = velf[i];
-                float s = 0.f;
-                using RC = NRec2<float4, float4>;
-                auto fetch = [&](uint32_t e) {
-                    const int j = (int)(e & NB_MASK);
-                    return RC{xmf[j], velf[j]};
-                };
-                walk_list<CH, RC>(nbr, N, i, nn, fetch, [&](uint32_t e, const RC& q) {
-                    const float4 xj = q.x;
-                    const float4 vj = q.r;
-                    float R0, R1, R2;
-                    rag32(xf, xj, e, R0, R1, R2);
-                    K32 K;
-                    kvals32(P, R0 * R0 + R1 * R1 + R2 * R2, true, false, false, K);
-                    s += xj.w * __builtin_amdgcn_rcpf(P.f_den0 + vj.w) * K.K1 *
-                         ((vj.x - vf.x) * R0 + (vj.y - vf.y) * R1 + (vj.z - vf.z) * R2);
-                                });
-                inner = rhoi * (double)s;
-            }
-            const double dden = dd - inner;
-            dden_out[i] = dden;
-            // RK1: the density is integrated after the velocities and positions
-            // (Euler.f90:231-241, in k_vsmooth)
-            if (!P.rk1) {
-                double rho1 = rhoi + dt * dden;
-                if (P.dthr) {  // Leapfrog_continuity.f90:61-68
-                    if (rho1 < 0.9 * P.den0) rho1 = 0.9 * P.den0;
-                    if (rho1 > 1.1 * P.den0) rho1 = 1.1 * P.den0;
-                }
-                const double p1 = eos ? P.eps / P.den0 * (rho1 - P.den0) + P.prif : rpi.y;
-                rp_out[i] = make_double2(rho1, p1);
-                if (F32) {
-                    rpf_out[i] = make_float2((float)rho1, (float)p1);
-                    // (cell-relative position, rho - den0) for the pressure smoothing
-                    const float4 xo = xmf[i];
-                    xrf_out[i] = make_float4(xo.x, xo.y, xo.z, (float)(rho1 - P.den0));
-                }
-            }
         }
-        __syncthreads();
+        psmooth_end(P, faces, bn, bt, i, nsp, rpi, scal[SC_TP1], somp, app, vpres_out, rp_out);
     }
 }
 
 // ----------------------------------------------------------------------------
-// pressure smoothing: PressureSmoothing_3D.f90:80-161 (both loops)
+// The four passes in FP32-mixed form, one workgroup per tile (see Tiles): the
+// records of the tile's particles and of the cells around it are staged in
+// LDS once, with the parts of a pair's term that belong to the neighbour
+// alone (m_j / rho_j, p_j / rho_j^2) computed there, and a lane walks its
+// particle's list of LDS slots.  The passes were bound by their gathers: 64
+// lanes reading 64 different lines take about 75 cycles of the CU's L1 per
+// 16-byte load, 78 neighbours and one or two loads each; a 16-byte LDS gather
+// takes about a quarter of it, and the pair sums' own instructions bound now.
+// The tile is as large as two workgroups a CU allow (80 KB of LDS each: one
+// stages while the other computes), smaller for small solves (choose_tile).
+// Pair math on xq's integer positions: a separation is exact to 2^-28 of a
+// cell, in units of P.lsb, whose powers are taken out of the sums.
+// Tiles with more candidates than the LDS holds gather from global memory
+// with the same expressions, so a sum does not depend on the tile.
+// 576,000 particles: momentum 186 -> 120 us, velocity smoothing 202 -> 87,
+// continuity 185 -> 79, pressure smoothing 101 -> 55; 25,000 particles: 33 ->
+// 28, 24 -> 17, 23 -> 16, 19 -> 13.
 // ----------------------------------------------------------------------------
-template <bool F32, int CH, bool SG>
-__global__ __launch_bounds__(256) void k_psmooth(
-    DP P0, Seg S, const DFace* __restrict__ faces, const int* __restrict__ bn, const BTab* __restrict__ bt,
-    const double4* __restrict__ xm, const double2* __restrict__ rp, const float4* __restrict__ xmf,
-    const float2* __restrict__ rpf, const float4* __restrict__ xrf, const uint32_t* __restrict__ nbr,
-    const int* __restrict__ nnb,
-    double* __restrict__ vpres_out, double2* __restrict__ rp_out, float2* __restrict__ rpf_out,
-    float* __restrict__ velw_out,
-    const double* scal, const int* iscal) {
-    using X = typename Rec<F32>::X;
-    using RPT = typename Rec<F32>::RP;
-    const int vb = xcd_block(gridDim.x);
-    const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * (int)blockDim.x) >> 8]) : 0;
-    const DP& P = SG ? S.P[sg] : P0;
-    scal += sg * SC_COUNT;
-    iscal += sg * IS_COUNT;
-    stencil_offsets(P);
-    const size_t N = P.cap;
-    const double tp1 = scal[SC_TP1];
-    {
-        const int i = vb * blockDim.x + threadIdx.x;
-        if (i - P.base < iscal[IS_N]) {
-            const double2 rpi = rp[i];
-            const int nsp = nnb[i];
-            double diffp = 0.0;
-            if (nsp > 0) {
-                const double p0i = P.prif, pi = rpi.y;
-                double somp, app;
-                if constexpr (!F32) {
-                    const double4 xi = xm[i];
-                    somp = 0.0;
-                    app = 0.0;
-                    using RP2 = NRec2<double4, double2>;
-                    auto fetch = [&](uint32_t e) {
-                        const int j = (int)(e & NB_MASK);
-                            return RP2{xm[j], rp[j]};
-                    };
-                    walk_list<4, RP2>(nbr, N, i, nsp, fetch, [&](uint32_t e, const RP2& q) {
-                        const double4 xj = q.x;
-                        const double2 rpj = q.r;
-                        const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
-                        K64 K;
-                        kvals64(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true, K);
-                        const double pes = xj.w * K.W / rpj.x;
-                        app = app + pes;
-                        somp = somp + (rpj.y - pi) * pes;
-                                        });
-                } else {
-                    const float4 xf = xmf[i];
-                    const float pif = rpf[i].y;
-                    float s_a = 0.f, s_p = 0.f;
-                    if (P.umass) {
-                        // one (x, y, z, rho - den0) record per neighbour: m_j is
-                        // the solve's mass, p_j - p_i the linear EoS of the
-                        // density difference
-                        const float wi = xrf[i].w;
-                        auto fetch = [&](uint32_t e) { return xrf[(int)(e & NB_MASK)]; };
-                        walk_list<CH, float4>(nbr, N, i, nsp, fetch, [&](uint32_t e, const float4& xj) {
-                            float R0, R1, R2;
-                            rag32(xf, xj, e, R0, R1, R2);
-                            K32 K;
-                            kvals32(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true, K);
-                            const float pes = P.f_mass * K.W * __builtin_amdgcn_rcpf(P.f_den0 + xj.w);
-                            s_a += pes;
-                            s_p += P.f_eosk * (xj.w - wi) * pes;
-                        });
-                    } else {
-                        using RP2 = NRec2<float4, float2>;
-                        auto fetch = [&](uint32_t e) {
-                            const int j = (int)(e & NB_MASK);
-                            return RP2{xmf[j], rpf[j]};
-                        };
-                        walk_list<CH, RP2>(nbr, N, i, nsp, fetch, [&](uint32_t e, const RP2& q) {
-                            const float4 xj = q.x;
-                            const float2 rpj = q.r;
-                            float R0, R1, R2;
-                            rag32(xf, xj, e, R0, R1, R2);
-                            K32 K;
-                            kvals32(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true, K);
-                            const float pes = xj.w * K.W * __builtin_amdgcn_rcpf(rpj.x);
-                            s_a += pes;
-                            s_p += (rpj.y - pif) * pes;
-                        });
-                    }
-                    somp = s_p;
-                    app = s_a;
-                }
-                const int ncbf = P.semi ? bn[i] : 0;
-                if (P.dim == 2) {
-                    // PressureSmoothing_2D.f90:124-214, SmoothVersion "b", fixe/tapi
-                    // sides; vpres is the smoothed pressure itself
-                    double VFT = 0.0;
-                    for (int q = 0; q < ncbf; ++q) {
-                        const BTab& B = bt[(size_t)q * P.cap + i];
-                        const DFace& S = faces[B.face];
-                        if (S.btype != 0 && S.btype != 1) continue;
-                        const double mf0 = S.T[0] * P.grav[0] + S.T[2] * P.grav[2];
-                        const double mf1 = S.T[6] * P.grav[0] + S.T[8] * P.grav[2];
-                        VFT = VFT + B.bi[1];
-                        somp = somp + P.den0 * (mf0 * B.bi[3] + mf1 * B.bi[4]);
-                    }
-                    app = app + VFT + 0.0 + 0.0 + 0.0;
-                    const double pz = (pi - pi) * 0.0;
-                    diffp = pi + tp1 * (somp + pz + pz + (p0i - pi) * (1.0 - app));
-                } else {
-                    for (int q = 0; q < ncbf; ++q) {
-                        const BTab& B = bt[(size_t)q * P.cap + i];
-                        if (B.loc[2] > 0.0) app = app + B.bi[1];
-                    }
-                    if (P.dbsph) diffp = somp / app;  // PressureSmoothing_3D.f90:110-112
-                    else if (app < 0.95) diffp = somp + (p0i - pi) * (1.0 - app);
-                    else diffp = somp / app;
-                }
-            } else if (P.dim == 2) {
-                diffp = rpi.y;  // no list (never: self is listed): pressure unchanged
+// q = r/h from a squared separation in lsb^2
+struct PairR {
+    float R0, R1, R2, rij, r;
+};
+__device__ __forceinline__ PairR pair_r(int4 a, float4 b) {
+    PairR d;
+    d.R0 = (float)(a.x - __float_as_int(b.x));
+    d.R1 = (float)(a.y - __float_as_int(b.y));
+    d.R2 = (float)(a.z - __float_as_int(b.z));
+    d.rij = __builtin_fmaf(d.R0, d.R0, __builtin_fmaf(d.R1, d.R1, d.R2 * d.R2));
+    d.r = __builtin_amdgcn_sqrtf(d.rij);
+    return d;
+}
+// the spline over coefke, and its derivative times h over coefke
+// (CalcVarLength.f90:243-265); every listed pair has r <= 2h, where both
+// branches vanish, so no cut-off test is needed
+__device__ __forceinline__ float spline_w(float q) {
+    const float b = 2.0f - q, q2 = q * q;
+    const float in = __builtin_fmaf(q2, __builtin_fmaf(q, 0.5f, -1.0f), 0.666666667f);
+    const float out = b * b * b * 0.166666666667f;
+    return q >= 1.0f ? out : in;
+}
+__device__ __forceinline__ float spline_g(float q, float b2) {
+    return q >= 1.0f ? -0.5f * b2 : q * __builtin_fmaf(1.5f, q, -2.0f);
+}
+
+__device__ __forceinline__ float4 bits4(int4 x, float w) {
+    return make_float4(__int_as_float(x.x), __int_as_float(x.y), __int_as_float(x.z), w);
+}
+
+// The NS pair sums of particle i over its list, by G lanes (1 or 2, lane g of
+// them).  The entries go by eights to two partial sums in turn, which are
+// added at the end, so a sum is the same for both G: few particles take two
+// lanes each (a lane's serial walk over 80 neighbours is then the time: 1,440
+// particles, continuity 18 -> 14 us), many take one.  (Four partial sums: 12
+// us there, but one lane holding 36 of them spilled: 116 -> 206 us for the
+// momentum pass at 576,000.)
+// fits: 16-bit entries (LDS slot times 16), 16 of them per 32 bytes, filled up
+// with the particle itself to whole eights; lds(sums, byte offset of the
+// neighbour's 16-byte record, place in the list).  Else glob(sums, sorted
+// index).  The next entries are loaded while some are used.
+template <int G, int NS, class Lds, class Glob>
+__device__ __forceinline__ void pair_sums(const uint32_t* __restrict__ nbr, size_t N, int i, int nn, int g,
+                                          bool fits, float (&sum)[NS], Lds&& lds, Glob&& glob) {
+#pragma unroll
+    for (int c = 0; c < NS; ++c) sum[c] = 0.0f;
+#pragma unroll 1
+    for (int m = g; m < 2; m += G) {  // the partial sums of the lane, one walk each
+        float a[NS];
+#pragma unroll
+        for (int c = 0; c < NS; ++c) a[c] = 0.0f;
+        if (fits) {
+            const uint4* L = reinterpret_cast<const uint4*>(nbr) + 2 * (size_t)i + m;
+            uint4 next = *L;
+            for (int k = 8 * m; k < nn; k += 16) {
+                const uint4 cur = next;
+                L += 2 * N;
+                if (k + 16 < nn) next = *L;
+                const uint32_t w[4] = {cur.x, cur.y, cur.z, cur.w};
+#pragma unroll
+                for (int u = 0; u < 8; ++u) lds(a, (u & 1) ? w[u >> 1] >> 16 : w[u >> 1] & 0xFFFFu, k + u);
             }
-            vpres_out[i] = diffp;
-            double p2 = rpi.y, rho2 = rpi.x;
-            if (P.dim == 2) {  // PressureSmoothing_2D.f90:217-231: p = vpres, rho = EoS^-1(p)
-                if (P.tetap > 0.0) {
-                    p2 = diffp;
-                    rho2 = P.den0 * (1.0 + (p2 - P.prif) / P.eps);
-                }
-            } else if (P.tetap > 0.0) {
-                p2 = rpi.y + tp1 * diffp;
-                rho2 = P.den0 * (1.0 + (p2 - P.prif) / P.eps);
-            }
-            rp_out[i] = make_double2(rho2, p2);
-            if (F32) {
-                rpf_out[i] = make_float2((float)rho2, (float)p2);
-                // the density slot of the velocity record the next momentum
-                // pass reads (element 8 i: 32-byte records, w of the second half)
-                velw_out[8 * (size_t)i] = (float)(rho2 - P.den0);
-            }
+        } else {
+            for (int k0 = 8 * m; k0 < nn; k0 += 16)
+                for (int k = k0; k < min(nn, k0 + 8); ++k) glob(a, (int)(nbr[nb_index(N, i, k)] & NB_MASK));
         }
-        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < NS; ++c) sum[c] += a[c];
     }
+    if constexpr (G == 2)
+#pragma unroll
+        for (int c = 0; c < NS; ++c) sum[c] += __shfl_xor(sum[c], 1, 64);
+}
+
+#define TILE_ARGS Seg S, Tiles T, const int* __restrict__ start
+
+// momentum; UM: every particle of the context has its solve's mass
+template <int CAP, bool SG, int G, bool UM>
+__global__ __launch_bounds__(TILE_WG, 4) void k_momentum(
+    TILE_ARGS, const DFace* __restrict__ faces, const DEdge* __restrict__ edges,
+    const int* __restrict__ bn, const BTab* __restrict__ bt, const double4* __restrict__ xm,
+    const double4* __restrict__ vel, const double2* __restrict__ rp, const int4* __restrict__ xq,
+    const float4* __restrict__ vf, const int* __restrict__ lam_in, int* __restrict__ lam_out,
+    const uint32_t* __restrict__ nbr, const int* __restrict__ nnb, double4* __restrict__ acc_out,
+    double4* __restrict__ vel_out, float4* __restrict__ vf_out, const double* scal0, int* iscal0) {
+    __shared__ float4 sA[CAP], sB[CAP];
+    // UM: (position, p_j / rho_j^2), (velocity, rho - den0); else (position, rho - den0), (velocity, mass)
+    auto rec_a = [](DPC& P, int4 x, float4 v) {
+        if constexpr (!UM) return bits4(x, v.w);
+        const float rhoj = P.f_den0 + v.w, pj = __builtin_fmaf(P.f_eosk, v.w, P.f_prif);
+        return bits4(x, pj * __builtin_amdgcn_rcpf(rhoj * rhoj));
+    };
+    auto rec_b = [](int4 x, float4 v) {
+        return make_float4(v.x, v.y, v.z, UM ? v.w : __int_as_float(x.w));
+    };
+    for_tiles<SG, G>(S, T, start,
+        [&](DPC& P, int, int j, int slot) {
+            const int4 x = xq[j];
+            const float4 v = vf[j];
+            sA[slot] = rec_a(P, x, v);
+            sB[slot] = rec_b(x, v);
+        },
+        [&](DPC& P, int sg, int i, bool fits) {
+            const double* scal = scal0 + sg * SC_COUNT;
+            const int4 xi = xq[i];
+            const float4 vf_i = vf[i];
+            const double2 rpi = rp[i];
+            const float rhoi = (float)rpi.x;
+            const float pri = (float)rpi.y * __builtin_amdgcn_rcpf(rhoi * rhoi);
+            const float nu = P.f_kin_visc;
+            // symmetric form -m_j (p_i/rho_i^2 + p_j/rho_j^2) r K3 of the
+            // reference's difference term plus its ALE1 complement, with
+            // K3 = -3 (2-q)^2 kacl / (r + eta); Monaghan's and Morris's terms
+            // with K2 = g ke / ((r + eta)(r^2 + eta2)).  The particle itself
+            // adds zeros.
+            auto pair = [&](float* s, float4 A, float4 B) {
+                const PairR d = pair_r(xi, A);
+                const float q = d.r * P.f_q, b = 2.0f - q, b2 = b * b;
+                const float e2 = d.rij + P.f_eta2l;
+                const float D2 = __builtin_amdgcn_rcpf((d.r + P.f_etal) * e2);
+                float k2 = spline_g(q, b2) * D2, k3 = b2 * (e2 * D2);
+                float prj = A.w, drj = B.w;
+                if constexpr (!UM) {
+                    drj = A.w;
+                    const float rhoj = P.f_den0 + drj, pj = __builtin_fmaf(P.f_eosk, drj, P.f_prif);
+                    prj = pj * __builtin_amdgcn_rcpf(rhoj * rhoj);
+                    k2 *= B.w;
+                    k3 *= B.w;
+                }
+                const float cp = (pri + prj) * k3;
+                s[0] = __builtin_fmaf(cp, d.R0, s[0]);
+                s[1] = __builtin_fmaf(cp, d.R1, s[1]);
+                s[2] = __builtin_fmaf(cp, d.R2, s[2]);
+                const float v0 = B.x - vf_i.x, v1 = B.y - vf_i.y, v2 = B.z - vf_i.z;
+                const float vr = __builtin_fmaf(v0, d.R0, __builtin_fmaf(v1, d.R1, v2 * d.R2));
+                // 1 / (rho_i + rho_j) and 1 / (nu (rho_i + rho_j) + 1e-3) from one reciprocal
+                const float t = rhoi + (P.f_den0 + drj), nt = __builtin_fmaf(nu, t, 1.0e-3f);
+                const float Dm = __builtin_amdgcn_rcpf(t * nt);
+                const float cd = Dm * nt * vr * k2;
+                s[3] = __builtin_fmaf(cd, d.R0, s[3]);
+                s[4] = __builtin_fmaf(cd, d.R1, s[4]);
+                s[5] = __builtin_fmaf(cd, d.R2, s[5]);
+                const float cv = Dm * t * (k2 * d.rij);
+                s[6] = __builtin_fmaf(cv, v0, s[6]);
+                s[7] = __builtin_fmaf(cv, v1, s[7]);
+                s[8] = __builtin_fmaf(cv, v2, s[8]);
+            };
+            float s[9];
+            pair_sums<G>(nbr, (size_t)P.cap, i, nnb[i], threadIdx.x % G, fits, s,
+                         [&](float* a, uint32_t o, int) { pair(a, lds16(sA, o), lds16(sB, o)); },
+                         [&](float* a, int j) {
+                             const int4 x = xq[j];
+                             const float4 v = vf[j];
+                             pair(a, rec_a(P, x, v), rec_b(x, v));
+                         });
+            if (threadIdx.x % G) return;
+            const double m = UM ? (double)P.f_mass : 1.0, ke = P.ke_coef * P.inv_lsb;
+            const double sp = 3.0 * P.kacl_coef * m;
+            const double sd = -(P.alfamon * (P.celerita + P.celerita) * P.h * m * ke);
+            const double sv = P.kin_visc > 1.0e-12 ? -(4.0 * (P.kin_visc * P.kin_visc) * m * ke) : 0.0;
+            // wall terms (AddBoundaryContributions_to_ME3D.f90), then the sums
+            const double4 vi = vel[i];  // var == vel here
+            const int ncbf = P.semi ? bn[i] : 0;
+            Walls6 W = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+            Walls3 E = {{0.0, 0.0, 0.0}};
+            if (ncbf > 0) {
+                W = wall_terms(&P, faces, bt, i, ncbf, vi.x, vi.y, vi.z, rpi.x, rpi.y, lam_in[i], iscal0 + sg * IS_COUNT);
+                E = wall_elastic(&P, faces, edges, bt, xm, i, ncbf, vi.x, vi.y, vi.z);
+            }
+            const double rvs[3] = {sv * (double)s[6], sv * (double)s[7], sv * (double)s[8]};
+            const double tp[3] = {W.tp[0] + sp * (double)s[0], W.tp[1] + sp * (double)s[1], W.tp[2] + sp * (double)s[2]};
+            const double td[3] = {W.tdv[0] + sd * (double)s[3], W.tdv[1] + sd * (double)s[4], W.tdv[2] + sd * (double)s[5]};
+            const double dtvel = P.rk1 ? scal[SC_DT] : scal[SC_DTVEL];
+            const double4 vn = momentum_end(P, i, ncbf, vi, dtvel, tp, td, rvs, rvs, E.r, lam_out, acc_out, vel_out);
+            vf_out[i] = make_float4((float)vn.x, (float)vn.y, (float)vn.z, (float)(rpi.x - P.den0));
+        },
+        [](DPC&, int) {});
+}
+
+// velocity smoothing
+template <int CAP, bool SG, int G>
+__global__ __launch_bounds__(TILE_WG, 4) void k_vsmooth(
+    TILE_ARGS, const DFace* __restrict__ faces, const int* __restrict__ bn, const BTab* __restrict__ bt,
+    const double4* __restrict__ xm, const double4* __restrict__ vel1, const double2* __restrict__ rp,
+    const int4* __restrict__ xq, const float4* __restrict__ vf, const uint32_t* __restrict__ nbr,
+    const int* __restrict__ nnb, double4* __restrict__ vel_out, double4* __restrict__ xm_out,
+    const double* scal0, unsigned long long* dtmin, const int* iscal0, const double* __restrict__ dden_in,
+    double2* __restrict__ rp_out, float* __restrict__ dr_out, int* __restrict__ gone) {
+    __shared__ float4 sA[CAP], sB[CAP];  // (position, m_j / rho_j), velocity
+    auto rec_a = [](DPC& P, int4 x, float4 v) {
+        return bits4(x, __int_as_float(x.w) * __builtin_amdgcn_rcpf(P.f_den0 + v.w));
+    };
+    unsigned long long dtbits = 0x7FF0000000000000ull;
+    for_tiles<SG, G>(S, T, start,
+        [&](DPC& P, int, int j, int slot) {
+            if (!(P.tetav > 1.0e-9)) return;
+            const float4 v = vf[j];
+            sA[slot] = rec_a(P, xq[j], v);
+            sB[slot] = v;
+        },
+        [&](DPC& P, int sg, int i, bool fits) {
+            const double* scal = scal0 + sg * SC_COUNT;
+            const bool smooth = P.tetav > 1.0e-9;
+            double v[3] = {0.0, 0.0, 0.0};
+            if (smooth) {
+                const int4 xi = xq[i];
+                const float4 vi = vf[i];
+                auto pair = [&](float* s, float4 A, float4 B) {
+                    const PairR d = pair_r(xi, A);
+                    const float pes = A.w * spline_w(d.r * P.f_q);
+                    s[0] = __builtin_fmaf(B.x - vi.x, pes, s[0]);
+                    s[1] = __builtin_fmaf(B.y - vi.y, pes, s[1]);
+                    s[2] = __builtin_fmaf(B.z - vi.z, pes, s[2]);
+                };
+                float s[3];
+                pair_sums<G>(nbr, (size_t)P.cap, i, nnb[i], threadIdx.x % G, fits, s,
+                             [&](float* a, uint32_t o, int) { pair(a, lds16(sA, o), lds16(sB, o)); },
+                             [&](float* a, int j) {
+                                 const float4 vj = vf[j];
+                                 pair(a, rec_a(P, xq[j], vj), vj);
+                             });
+                v[0] = P.coefke * (double)s[0];
+                v[1] = P.coefke * (double)s[1];
+                v[2] = P.coefke * (double)s[2];
+            }
+            if (threadIdx.x % G) return;
+            const double4 vi = vel1[i];
+            const int ncbf = smooth && P.semi ? bn[i] : 0;
+            if (ncbf > 0) {
+                const Walls3 W = wall_smooth(&P, faces, bt, i, ncbf, vi.x, vi.y, vi.z, v[0], v[1], v[2]);
+                for (int d = 0; d < 3; ++d) v[d] = W.r[d];
+            }
+            const unsigned long long b =
+                vsmooth_end<true>(P, faces, i, xm[i], vi, v, smooth, scal[SC_TV1], scal[SC_DT],
+                            iscal0[sg * IS_COUNT + IS_ONGOING] > 0, dden_in, rp, vel_out, xm_out, rp_out,
+                            dr_out, gone);
+            dtbits = b < dtbits ? b : dtbits;
+        },
+        [&](DPC&, int sg) {
+            for (int o = 32; o > 0; o >>= 1) {
+                const unsigned long long t = __shfl_xor(dtbits, o, 64);
+                dtbits = t < dtbits ? t : dtbits;
+            }
+            // the minimum only falls: a value read before is an upper bound of it
+            if ((threadIdx.x & 63) == 0 && dtbits < *(volatile unsigned long long*)(dtmin + sg))
+                atomicMin(dtmin + sg, dtbits);
+            dtbits = 0x7FF0000000000000ull;
+        });
+}
+
+// continuity
+template <int CAP, bool SG, int G>
+__global__ __launch_bounds__(TILE_WG, 4) void k_continuity(
+    TILE_ARGS, const DFace* __restrict__ faces, const int* __restrict__ bn, const BTab* __restrict__ bt,
+    const double4* __restrict__ vel, const double2* __restrict__ rp, const int4* __restrict__ xq,
+    const float4* __restrict__ vf, const uint32_t* __restrict__ nbr, const int* __restrict__ nnb,
+    double* __restrict__ dden_out, double2* __restrict__ rp_out, float* __restrict__ dr_out,
+    const double* scal0, int* iscal0) {
+    __shared__ float4 sA[CAP], sB[CAP];  // (position, m_j / rho_j), velocity
+    auto rec_a = [](DPC& P, int4 x, float4 v) {
+        return bits4(x, __int_as_float(x.w) * __builtin_amdgcn_rcpf(P.f_den0 + v.w));
+    };
+    for_tiles<SG, G>(S, T, start,
+        [&](DPC& P, int, int j, int slot) {
+            const float4 v = vf[j];
+            sA[slot] = rec_a(P, xq[j], v);
+            sB[slot] = v;
+        },
+        [&](DPC& P, int sg, int i, bool fits) {
+            const int4 xi = xq[i];
+            const float4 vi = vf[i];
+            auto pair = [&](float* s, float4 A, float4 B) {
+                const PairR d = pair_r(xi, A);
+                const float q = d.r * P.f_q, b = 2.0f - q;
+                const float k = A.w * spline_g(q, b * b) * __builtin_amdgcn_rcpf(d.r + P.f_etal);
+                const float dv = __builtin_fmaf(B.x - vi.x, d.R0, __builtin_fmaf(B.y - vi.y, d.R1, (B.z - vi.z) * d.R2));
+                s[0] = __builtin_fmaf(k, dv, s[0]);
+            };
+            float s[1];
+            pair_sums<G>(nbr, (size_t)P.cap, i, nnb[i], threadIdx.x % G, fits, s,
+                         [&](float* a, uint32_t o, int) { pair(a, lds16(sA, o), lds16(sB, o)); },
+                         [&](float* a, int j) {
+                             const float4 vj = vf[j];
+                             pair(a, rec_a(P, xq[j], vj), vj);
+                         });
+            if (threadIdx.x % G) return;
+            const double2 rpi = rp[i];
+            int* iscal = iscal0 + sg * IS_COUNT;
+            const double dd = continuity_walls(P, faces, bt, i, P.semi ? bn[i] : 0, vel[i], rpi.x, iscal);
+            const double inner = rpi.x * (P.ke_coef * (double)s[0]);
+            continuity_end(P, i, rpi, dd - inner, scal0[sg * SC_COUNT + SC_DT], iscal[IS_ONGOING] > 0, dden_out,
+                           rp_out, dr_out);
+        },
+        [](DPC&, int) {});
+}
+
+// pressure smoothing; p_j - p_i is the linear EoS of the density difference
+template <int CAP, bool SG, int G>
+__global__ __launch_bounds__(TILE_WG, 4) void k_psmooth(
+    TILE_ARGS, const DFace* __restrict__ faces, const int* __restrict__ bn, const BTab* __restrict__ bt,
+    const double2* __restrict__ rp, const int4* __restrict__ xq, const float* __restrict__ dr,
+    const uint32_t* __restrict__ nbr, const int* __restrict__ nnb, double* __restrict__ vpres_out,
+    double2* __restrict__ rp_out, float4* __restrict__ vf_out, const double* scal0) {
+    __shared__ float4 sA[CAP];  // (position, m_j / rho_j)
+    __shared__ float sD[CAP];   // rho_j - den0
+    auto rec_a = [](DPC& P, int4 x, float d) {
+        return bits4(x, __int_as_float(x.w) * __builtin_amdgcn_rcpf(P.f_den0 + d));
+    };
+    for_tiles<SG, G>(S, T, start,
+        [&](DPC& P, int, int j, int slot) {
+            const float d = dr[j];
+            sA[slot] = rec_a(P, xq[j], d);
+            sD[slot] = d;
+        },
+        [&](DPC& P, int sg, int i, bool fits) {
+            const int4 xi = xq[i];
+            const float di = dr[i];
+            const int nn = nnb[i];
+            auto pair = [&](float* s, float4 A, float dj, bool in) {
+                const PairR d = pair_r(xi, A);
+                const float pes = in ? A.w * spline_w(d.r * P.f_q) : 0.0f;
+                s[0] += pes;
+                s[1] = __builtin_fmaf(dj - di, pes, s[1]);
+            };
+            float s[2];
+            pair_sums<G>(nbr, (size_t)P.cap, i, nn, threadIdx.x % G, fits, s,
+                         [&](float* a, uint32_t o, int k) {
+                             const float dj = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(sD) + (o >> 2));
+                             pair(a, lds16(sA, o), dj, k < nn);
+                         },
+                         [&](float* a, int j) { pair(a, rec_a(P, xq[j], dr[j]), dr[j], true); });
+            if (threadIdx.x % G) return;
+            const double rho2 = psmooth_end(P, faces, bn, bt, i, nn, rp[i], scal0[sg * SC_COUNT + SC_TP1],
+                                            P.eps / P.den0 * P.coefke * (double)s[1], P.coefke * (double)s[0],
+                                            vpres_out, rp_out);
+            // the density slot of the velocity record the next momentum pass reads
+            reinterpret_cast<float*>(vf_out + i)[3] = (float)(rho2 - P.den0);
+        },
+        [](DPC&, int) {});
 }
 
 }  // namespace sph
