@@ -1386,6 +1386,34 @@ int sph_segment_download(sph_ctx* c, int32_t seg, double* coord, double* vel, do
     int n;
     HIPC(hipMemcpy(&n, c->iscal + (size_t)seg * IS_COUNT + IS_N, sizeof(int), hipMemcpyDeviceToHost));
     const size_t b = c->nseg > 1 ? c->segs[seg].base : 0;
+    // Rows in pg order by the device, in buffers that hold nothing at a step
+    // boundary: xm[1], vel[1] and acc[1] (written by the next step before they
+    // are read) take the vectors, vel[2] the four scalars
+    if (n) {
+        double* o[4] = {reinterpret_cast<double*>(c->xm[1] + b), reinterpret_cast<double*>(c->vel[1] + b),
+                        reinterpret_cast<double*>(c->acc[1] + b), reinterpret_cast<double*>(c->vel[2] + b)};
+        k_fill_int<<<1, 64, 0, c->stream>>>(c->nwork, 0, 1);  // the boundary table clears its counter itself
+        k_pack_state<<<nblk(n), 256, 0, c->stream>>>(c->xm[0] + b, c->vel[0] + b, c->acc[0] + b,
+                                                     c->rp[cur_rp(c)] + b, (c->P.rk1 ? c->dden2 : c->dden) + b,
+                                                     (c->P.rk1 ? c->vpres2 : c->vpres) + b, n, o[0], o[1], o[2],
+                                                     o[3], c->nwork);
+        HIPC(hipGetLastError());
+        int bad = 0;
+        HIPC(hipMemcpyAsync(&bad, c->nwork, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        const size_t m = (size_t)n;
+        const struct { double* to; const double* from; size_t len; } part[7] = {
+            {coord, o[0], 3 * m}, {vel, o[1], 3 * m}, {acc, o[2], 3 * m}, {dens, o[3], m},
+            {pres, o[3] + m, m}, {dden, o[3] + 2 * m, m}, {vpres, o[3] + 3 * m, m}};
+        HIPC(hipStreamSynchronize(c->stream));
+        if (!bad) {
+            for (const auto& q : part)
+                if (q.to) HIPC(hipMemcpy(q.to, q.from, sizeof(double) * q.len, hipMemcpyDeviceToHost));
+            for (int r = 0; ids && r < n; ++r) ids[r] = r;
+            return 0;
+        }
+    }
+    // ids with gaps (a sort that removed more particles than it can renumber,
+    // status 102): rows by ascending id
     std::vector<double4> hx(n), hv(n), ha(n);
     std::vector<double2> hr(n);
     std::vector<double> hd(n), hp(n);
