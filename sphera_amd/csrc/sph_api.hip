@@ -53,7 +53,7 @@ struct sph_ctx {
     std::vector<DP> segs;
     Seg S{};
     DP* d_P = nullptr;
-    int *d_pblk = nullptr, *d_kblk = nullptr, *d_tblk = nullptr, *d_adj = nullptr;
+    int *d_pblk = nullptr, *d_kblk = nullptr, *d_tblk = nullptr;
     int nkeys = 1;             // cell keys (cells + out-of-grid bucket per segment)
     int nb_stride_max = 1;     // largest NMAXPARTJ of the segments (list capacity)
     std::vector<int> staged;   // segments uploaded since the last commit
@@ -82,6 +82,7 @@ struct sph_ctx {
     int* gone = nullptr;  // 1: the last trajectory step left through an open face
     int *cell = nullptr, *key = nullptr, *slot = nullptr, *cnt = nullptr, *start = nullptr,
         *perm = nullptr, *pid = nullptr, *bsum = nullptr;
+    int nrep = 1;  // copies of the scan blocks' sums
     int *tlist = nullptr, *ntile = nullptr;  // the tiles that hold particles, their number
     int ntiles = 0;                          // tile ids of all segments (whole 256-blocks)
     int tile_cap = 0, tile_grid = 8, tile_wg = 64, tile_g = 1;  // slots of the pair passes' LDS form, their launch shape
@@ -191,24 +192,12 @@ int collect_timing(sph_ctx* c) {
 }
 
 // ---- device steps --------------------------------------------------------
-void scan_ints(sph_ctx* c, const int* in, int* out, int* bs, int m, int* total) {
-    const int nb = (m + 1023) / 1024;
-    k_scan_local<<<nb, 256, 0, c->stream>>>(in, out, bs, m);
-    k_scan_sums<<<1, 1024, 0, c->stream>>>(bs, nb, total);
-    k_scan_add<<<nblk(m), 256, 0, c->stream>>>(out, bs, m);
-}
-
 // Launches kernel K in its one-solve (<false>) or segmented (<true>) form.
 #define SEGL(K, G, B, ...)                                                                 \
     do {                                                                                   \
         if (c->nseg > 1) K<true><<<(G), (B), 0, c->stream>>>(c->S, __VA_ARGS__);      \
         else K<false><<<(G), (B), 0, c->stream>>>(c->S, __VA_ARGS__);                 \
     } while (0)
-
-__global__ void k_fill_strided(int* p, int stride, int v, int m) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < m) p[(size_t)i * stride] = v;
-}
 
 // Buffer of the current (rho, p) at a step boundary: the pressure smoothing
 // writes rp[0]; the leapfrog step's sort comes before it, the RK1 step's sort
@@ -219,35 +208,28 @@ inline int cur_rp(const sph_ctx* c) { return c->P.dbsph ? 0 : (c->P.rk1 ? 1 : 0)
 int run_sort(sph_ctx* c) {
     const int m = c->nkeys;
     const int cap = c->P.cap;
-    const int ns = c->nseg;
+    const int nsb = nblk(m, SCAN_B);
     {
         KTime t(c, "sort_count");
-        k_fill_int<<<nblk(m), 256, 0, c->stream>>>(c->cnt, 0, m);
-        k_fill_strided<<<nblk(ns, 64), 64, 0, c->stream>>>(c->iscal + IS_NRM, IS_COUNT, 0, ns);
         SEGL(k_cell_count, nblk(cap), 256, c->xm[1], c->vel[2], c->key, c->slot, c->cnt, c->idslot, c->rmids,
-             c->iscal, c->gone, c->ntile);
-        SEGL(k_renumber, nblk(ns, 64), 64, c->rmids, c->idslot, c->vel[2], c->iscal);
+             c->iscal, c->gone, c->ntile, c->bsum, c->nrep, nsb);
     }
     {
         KTime t(c, "sort_scan");
-        scan_ints(c, c->cnt, c->start, c->bsum, m, nullptr);
-        if (ns > 1) {  // each segment's slots start at its base
-            k_seg_adj<<<nblk(ns, 64), 64, 0, c->stream>>>(c->S, c->start, c->d_adj);
-            k_seg_add<<<nblk(m), 256, 0, c->stream>>>(c->S, c->start, c->d_adj, m);
-        }
+        SEGL(k_cell_scan, nblk(m, SCAN_B) + 1, 256, c->cnt, c->start, c->bsum, c->nrep, nsb, m, c->rmids, c->idslot, c->vel[2],
+             c->iscal);
     }
     {
         KTime t(c, "sort_scatter");
         SEGL(k_scatter, nblk(cap) + c->ntiles / 256, 256, c->key, c->slot, c->start, c->vel[2], c->perm, c->pid,
              c->iscal, nblk(cap), c->tlist, c->ntile);
-        SEGL(k_cell_sort, ns > 1 ? m / 256 : (c->P.nmax + 255) / 256, 256, c->start, c->perm, c->pid);
     }
     {
         KTime t(c, "sort_gather");
-        SEGL(k_gather, nblk(cap), 256, c->perm, c->key, c->xm[1], c->vel[2], c->rp[0], c->lam[0], c->acc[1],
+        SEGL(k_gather, nblk(cap), 256, c->perm, c->pid, c->key, c->xm[1], c->vel[2], c->rp[0], c->lam[0], c->acc[1],
              c->xm[0], c->vel[0], c->rp[1], c->lam[1], c->acc[0], c->cell, c->xq, c->vf[0], c->start, c->iscal, c->P.rk1 ? c->dden : nullptr, c->dden2,
              c->P.rk1 ? c->vpres : nullptr, c->vpres2, c->P.dbsph ? c->gam[0] : nullptr, c->gam[1],
-             c->dsh[0], c->dsh[1]);
+             c->dsh[0], c->dsh[1], c->cnt, m, c->bsum, c->nrep * nsb, c->nwork);
     }
     return 0;
 }
@@ -260,7 +242,8 @@ int run_neighbours(sph_ctx* c) {
     return 0;
 }
 
-int run_btab(sph_ctx* c) {
+// again: the table of this sort may have been built before
+int run_btab(sph_ctx* c, bool again = false) {
     if (!c->P.semi || c->P.nf == 0) {
         k_fill_int<<<nblk(c->P.cap), 256, 0, c->stream>>>(c->bn, 0, c->P.cap);
         return 0;
@@ -273,7 +256,7 @@ int run_btab(sph_ctx* c) {
     }
     {
         KTime t(c, "boundary_find");
-        k_fill_int<<<1, 64, 0, c->stream>>>(c->nwork, 0, 1);
+        if (again) k_fill_int<<<1, 64, 0, c->stream>>>(c->nwork, 0, 1);  // else the sort has cleared it
         SEGL(k_boundary_find, nblk(c->P.cap), 256, c->d_faces, c->d_gcount, c->d_gstart, c->d_gvec,
              c->xm[0], c->bn, c->bt, c->work, c->nwork, c->iscal);
     }
@@ -477,7 +460,7 @@ sph_ctx::~sph_ctx() {
         if (p) hipFree(p);
     };
     F(d_faces); F(d_edges); F(d_gcount); F(d_gstart); F(d_gvec); F(d_kt); F(d_bit); F(d_btf);
-    F(d_P); F(d_pblk); F(d_kblk); F(d_tblk); F(d_adj);
+    F(d_P); F(d_pblk); F(d_kblk); F(d_tblk);
     for (auto p : xm) F(p);
     for (auto p : vel) F(p);
     for (auto p : acc) F(p);
@@ -526,7 +509,8 @@ int sph_ctx::alloc() {
     HIPC(da(&nwork, 1));
     HIPC(da(&cnt, m));
     HIPC(da(&start, m + 1));
-    HIPC(da(&bsum, (m + 1023) / 1024 + 1));
+    nrep = nblk((int)m, SCAN_B) <= 256 ? 16 : nblk((int)m, SCAN_B) <= 1024 ? 4 : 1;
+    HIPC(da(&bsum, (size_t)nrep * nblk((int)m, SCAN_B)));
     HIPC(da(&idslot, N));
     HIPC(da(&rmids, RM_CAP * ns));
     HIPC(da(&nbr, N * (size_t)nb_stride(nb_stride_max)));
@@ -550,6 +534,10 @@ int sph_ctx::alloc() {
         HIPC(hipMemset(vpres2, 0, sizeof(double) * N));
     }
     HIPC(hipMemset(ntile, 0, sizeof(int)));
+    // every sort leaves its counters cleared for the next
+    HIPC(hipMemset(cnt, 0, sizeof(int) * m));
+    HIPC(hipMemset(bsum, 0, sizeof(int) * (size_t)nrep * nblk((int)m, SCAN_B)));
+    HIPC(hipMemset(nwork, 0, sizeof(int)));
     HIPC(hipMemset(nnb, 0, sizeof(int) * N));
     HIPC(hipMemset(gone, 0, sizeof(int) * N));
     HIPC(hipMemset(bn, 0, sizeof(int) * N));
@@ -936,8 +924,7 @@ int upload_segment_maps(sph_ctx* c) {
               hipMalloc(&c->d_kblk, sizeof(int) * kblk.size()) == hipSuccess &&
               hipMemcpy(c->d_kblk, kblk.data(), sizeof(int) * kblk.size(), hipMemcpyHostToDevice) == hipSuccess &&
               hipMalloc(&c->d_tblk, sizeof(int) * tblk.size()) == hipSuccess &&
-              hipMemcpy(c->d_tblk, tblk.data(), sizeof(int) * tblk.size(), hipMemcpyHostToDevice) == hipSuccess &&
-              hipMalloc(&c->d_adj, sizeof(int) * c->nseg) == hipSuccess;
+              hipMemcpy(c->d_tblk, tblk.data(), sizeof(int) * tblk.size(), hipMemcpyHostToDevice) == hipSuccess;
     if (!ok) return fail(102, "device allocation/copy of the segment maps failed");
     c->S = Seg{(DPC*)c->d_P, c->d_pblk, c->d_kblk, c->d_tblk, c->nseg};
     return 0;
@@ -1392,7 +1379,7 @@ int sph_segment_download(sph_ctx* c, int32_t seg, double* coord, double* vel, do
     if (n) {
         double* o[4] = {reinterpret_cast<double*>(c->xm[1] + b), reinterpret_cast<double*>(c->vel[1] + b),
                         reinterpret_cast<double*>(c->acc[1] + b), reinterpret_cast<double*>(c->vel[2] + b)};
-        k_fill_int<<<1, 64, 0, c->stream>>>(c->nwork, 0, 1);  // the boundary table clears its counter itself
+        k_fill_int<<<1, 64, 0, c->stream>>>(c->nwork, 0, 1);  // the next sort clears the boundary table's counter
         k_pack_state<<<nblk(n), 256, 0, c->stream>>>(c->xm[0] + b, c->vel[0] + b, c->acc[0] + b,
                                                      c->rp[cur_rp(c)] + b, (c->P.rk1 ? c->dden2 : c->dden) + b,
                                                      (c->P.rk1 ? c->vpres2 : c->vpres) + b, n, o[0], o[1], o[2],
@@ -1760,7 +1747,7 @@ int sph_boundary_tab(sph_ctx* c) {
     if (c->P.rk1) return expect(c, c->phase, "sph_boundary_tab");
     if (c->phase != PH_NB && c->phase != PH_SORTED)
         return fail(120, "sph_boundary_tab called out of the time_step_loop order");
-    run_btab(c);
+    run_btab(c, true);
     c->phase = c->phase == PH_SORTED ? PH_SORTED : PH_BT;
     return 0;
 }
@@ -1793,7 +1780,7 @@ int sph_preloop(sph_ctx* c) {
     if (!c) return fail(1, "null argument");
     if (c->phase != PH_SORTED) return fail(120, "sph_preloop needs a freshly uploaded state");
     run_neighbours(c);
-    run_btab(c);
+    run_btab(c, true);
     if (c->P.dbsph) {
         // time_step_loop.f90:82-135 for bsph: CalcVarLength with Gamma from
         // sigma, then again after OrdGrid1 (nothing has moved since the

@@ -195,6 +195,7 @@ __device__ __forceinline__ void tile_coords(DPC& P, int id, int& ti, int& tj, in
 // their previous (ascending-id) order and k_cell_sort finds its runs sorted.
 // ----------------------------------------------------------------------------
 constexpr int HIST_W = 512;
+constexpr int SCAN_B = 4096;  // keys per scan block (HIST_W < SCAN_B)
 
 // Segmented contexts (SG): the workgroup's segment comes from the slot-block
 // map; slots, keys, ids and the removal list are the segment's.
@@ -204,8 +205,9 @@ __global__ __launch_bounds__(256) void k_cell_count(Seg S, const double4* __rest
                                                     int* __restrict__ key, int* __restrict__ slot,
                                                     int* __restrict__ cnt, int* __restrict__ idslot,
                                                     int* __restrict__ rmids, int* iscal,
-                                                    int* __restrict__ gone, int* ntile) {
+                                                    int* __restrict__ gone, int* ntile, int* __restrict__ bsum, int nrep, int nsb) {
     __shared__ int base[HIST_W];
+    __shared__ int part[2];  // particles in the two scan blocks that the window can touch
     __shared__ int wcnt[4][HIST_W];  // particles of each window cell per wave
     __shared__ int cmin;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -215,9 +217,11 @@ __global__ __launch_bounds__(256) void k_cell_count(Seg S, const double4* __rest
     rmids += sg * RM_CAP;
     const int n = iscal[IS_N];
     if (i == 0) *ntile = 0;  // k_scatter counts them
+    bsum += (blockIdx.x % nrep) * nsb;
     for (int b = threadIdx.x; b < HIST_W; b += blockDim.x)
         for (int w = 0; w < 4; ++w) wcnt[w][b] = 0;
     if (threadIdx.x == 0) cmin = 0x7fffffff;
+    if (threadIdx.x < 2) part[threadIdx.x] = 0;
     __syncthreads();
     int k = -1;
     if (i - P.base < n) {
@@ -244,8 +248,12 @@ __global__ __launch_bounds__(256) void k_cell_count(Seg S, const double4* __rest
     int loc = -1, rank = 0;
     if (k >= 0) {
         const int d = k - c0;
-        if (k < P.koff + P.nmax && d < HIST_W) loc = d;
-        else slot[i] = atomicAdd(&cnt[k], 1);
+        if (k < P.koff + P.nmax && d < HIST_W) {
+            loc = d;
+        } else {
+            slot[i] = atomicAdd(&cnt[k], 1);
+            atomicAdd(&bsum[k / SCAN_B], 1);
+        }
     }
     // rank within the wave among the lanes of the same window cell, one
     // ballot per distinct cell of the wave
@@ -265,10 +273,14 @@ __global__ __launch_bounds__(256) void k_cell_count(Seg S, const double4* __rest
         for (int w = 0; w < wid; ++w) rank += wcnt[w][loc];
     for (int b = threadIdx.x; b < HIST_W; b += blockDim.x) {
         const int tot = wcnt[0][b] + wcnt[1][b] + wcnt[2][b] + wcnt[3][b];
-        if (tot > 0) base[b] = atomicAdd(&cnt[c0 + b], tot);
+        if (tot > 0) {
+            base[b] = atomicAdd(&cnt[c0 + b], tot);
+            atomicAdd(&part[(c0 + b) / SCAN_B - c0 / SCAN_B], tot);
+        }
     }
     __syncthreads();
     if (loc >= 0) slot[i] = base[loc] + rank;
+    if (threadIdx.x < 2 && part[threadIdx.x]) atomicAdd(&bsum[c0 / SCAN_B + threadIdx.x], part[threadIdx.x]);
 }
 
 // wave64 inclusive scan
@@ -282,30 +294,6 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
     return v;
 }
 
-// block-level exclusive scan of 4*256 elements; writes per-block totals
-__global__ __launch_bounds__(256) void k_scan_local(const int* __restrict__ in, int* __restrict__ out,
-                                                    int* __restrict__ bsum, int m) {
-    __shared__ int wsum[4];
-    const int base = blockIdx.x * 1024 + threadIdx.x * 4;
-    int v[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] = (base + q < m) ? in[base + q] : 0;
-    const int tsum = v[0] + v[1] + v[2] + v[3];
-    const int incl = wave_incl_scan(tsum);
-    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 63) wsum[wid] = incl;
-    __syncthreads();
-    int woff = 0;
-    for (int w = 0; w < wid; ++w) woff += wsum[w];
-    int run = woff + incl - tsum;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        if (base + q < m) out[base + q] = run;
-        run += v[q];
-    }
-    if (threadIdx.x == 255) bsum[blockIdx.x] = woff + incl;
-}
-
 // Ids after the removals of this sort, as OrdGrid1.f90:62-83 leaves pg: the
 // first loop walks npi upwards; a particle out of the grid is overwritten by
 // pg(nag), nag decreases and the same npi is tested again.  So, for the removed
@@ -313,11 +301,8 @@ __global__ __launch_bounds__(256) void k_scan_local(const int* __restrict__ in, 
 // it is itself removed (then it is dropped and the next last is tried).  One
 // lane; removals are rare (particles leaving a closed tank).
 // Segmented contexts: one lane per segment.
-template <bool SG>
-__global__ void k_renumber(Seg S, int* __restrict__ rmids, const int* __restrict__ idslot,
-                           double4* __restrict__ vel, int* iscal) {
-    const int sg = SG ? (int)(blockIdx.x * blockDim.x + threadIdx.x) : 0;
-    if (SG ? sg >= S.nseg : threadIdx.x != 0) return;
+__device__ void renumber(const Seg& S, int sg, int* __restrict__ rmids, const int* __restrict__ idslot,
+                         double4* __restrict__ vel, int* iscal) {
     const int pbase = S.P[sg].base;
     iscal += sg * IS_COUNT;
     rmids += sg * RM_CAP;
@@ -356,45 +341,57 @@ __global__ void k_renumber(Seg S, int* __restrict__ rmids, const int* __restrict
     }
 }
 
-// exclusive scan of the block totals by one workgroup
-__global__ __launch_bounds__(1024) void k_scan_sums(int* __restrict__ bsum, int nb, int* total) {
-    __shared__ int wsum[16];
-    __shared__ int carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int base = 0; base < nb; base += 1024) {
-        const int idx = base + threadIdx.x;
-        const int v = idx < nb ? bsum[idx] : 0;
-        const int incl = wave_incl_scan(v);
-        const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        if (lane == 63) wsum[wid] = incl;
-        __syncthreads();
-        int woff = 0;
-        for (int w = 0; w < wid; ++w) woff += wsum[w];
-        const int c0 = carry;
-        if (idx < nb) bsum[idx] = c0 + woff + incl - v;
-        __syncthreads();
-        if (threadIdx.x == 1023) carry = c0 + woff + incl;
-        __syncthreads();
+// Cell starts: exclusive scan of the counts, a block of SCAN_B keys per
+// workgroup.  k_cell_count has summed the counts by block (in nrep copies:
+// its workgroups run through the keys together, and on one copy their atomics
+// queued, 45 against 18 us at 576,000 particles), so a workgroup adds up the
+// blocks before its own and scans its keys: one launch for what took
+// three (local scan, scan of the totals, their addition; a launch costs 4.5 us
+// in a step whatever it does, and the sort had ten: now four).  Segmented contexts: a
+// segment's slots begin at its base, and the particles before its keys are
+// the earlier segments' particles.  The last workgroup renumbers the ids
+// after removals.
+template <bool SG>
+__global__ __launch_bounds__(256) void k_cell_scan(Seg S, const int* __restrict__ cnt, int* __restrict__ start,
+                                                   const int* __restrict__ bsum, int nrep, int nsb, int m, int* __restrict__ rmids,
+                                                   const int* __restrict__ idslot, double4* __restrict__ vel,
+                                                   int* iscal) {
+    if (blockIdx.x == gridDim.x - 1) {
+        for (int sg = threadIdx.x; sg < (SG ? S.nseg : 1); sg += blockDim.x) renumber(S, sg, rmids, idslot, vel, iscal);
+        return;
     }
-    if (threadIdx.x == 0 && total) *total = carry;
-}
-
-__global__ void k_scan_add(int* __restrict__ out, const int* __restrict__ bsum, int m) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < m) out[i] += bsum[i >> 10];
-}
-
-// Segmented contexts: the scan over the whole key space gives every key its
-// start counted from slot 0; a segment's slots begin at its base instead.
-// adj[s] = base_s - start[koff_s], added to every key of segment s.
-__global__ void k_seg_adj(Seg S, const int* __restrict__ start, int* __restrict__ adj) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < S.nseg) adj[s] = S.P[s].base - start[S.P[s].koff];
-}
-__global__ void k_seg_add(Seg S, int* __restrict__ start, const int* __restrict__ adj, int m) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < m) start[k] += adj[S.kblk[k >> 8]];
+    __shared__ int wsum[4], wtot[4];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    int before = 0;
+    // nrep is a power of two up to 16: copy t % nrep, blocks t / nrep + 256 / nrep * ...
+    for (int b = threadIdx.x / nrep; b < (int)blockIdx.x; b += 256 / nrep)
+        before += bsum[(threadIdx.x & (nrep - 1)) * nsb + b];
+    constexpr int U = SCAN_B / 256;
+    const int k0 = blockIdx.x * SCAN_B + threadIdx.x * U;
+    int v[U], tsum = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        v[u] = k0 + u < m ? cnt[k0 + u] : 0;
+        tsum += v[u];
+    }
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+    const int incl = wave_incl_scan(tsum);
+    if (lane == 63) wsum[wid] = incl;
+    if (lane == 0) wtot[wid] = before;
+    __syncthreads();
+    int run = wtot[0] + wtot[1] + wtot[2] + wtot[3] + incl - tsum;
+    for (int w = 0; w < wid; ++w) run += wsum[w];
+    if (SG && k0 < m) {  // a thread's keys lie in one 256-block, hence in one segment
+        const int sg = S.kblk[k0 >> 8];
+        int earlier = 0;
+        for (int q = 0; q < sg; ++q) earlier += iscal[q * IS_COUNT + IS_N];
+        run += S.P[sg].base - earlier;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (k0 + u < m) start[k0 + u] = run;
+        run += v[u];
+    }
 }
 
 // Workgroups past the first nsb list the tiles that hold particles (a tile per
@@ -441,62 +438,6 @@ __global__ __launch_bounds__(256) void k_scatter(Seg S, const int* __restrict__ 
     pid[d] = (int)vel[i].w;
 }
 
-// ascending particle id inside every cell: the order OrdGrid1's 4th loop
-// produces (NPartOrd), hence the reference's neighbour-list order.  A
-// workgroup sorts the segments of 256 consecutive cells in LDS.
-constexpr int CSORT_CAP = 6144;
-
-template <bool SG>
-__global__ __launch_bounds__(256) void k_cell_sort(Seg S, const int* __restrict__ start,
-                                                   int* __restrict__ perm, int* __restrict__ pid) {
-    __shared__ int sid[CSORT_CAP];
-    __shared__ int sperm[CSORT_CAP];
-    const int c0 = blockIdx.x * 256;
-    const int sg = SG ? __builtin_amdgcn_readfirstlane(S.kblk[blockIdx.x]) : 0;
-    DPC& P = S.P[sg];
-    const int c1 = min(c0 + 256, P.koff + P.nmax);
-    if (c0 >= c1) return;  // a block of the out-of-grid key or of the padding
-    const int g0 = start[c0], g1 = start[c1];
-    const int len = g1 - g0;
-    const int c = c0 + threadIdx.x;
-    if (len <= CSORT_CAP) {
-        for (int t = threadIdx.x; t < len; t += blockDim.x) {
-            sid[t] = pid[g0 + t];
-            sperm[t] = perm[g0 + t];
-        }
-        __syncthreads();
-        if (c < c1) {
-            const int b = start[c] - g0, e = start[c + 1] - g0;
-            for (int a = b + 1; a < e; ++a) {
-                const int kv = sid[a], pv = sperm[a];
-                int q = a - 1;
-                while (q >= b && sid[q] > kv) {
-                    sid[q + 1] = sid[q];
-                    sperm[q + 1] = sperm[q];
-                    --q;
-                }
-                sid[q + 1] = kv;
-                sperm[q + 1] = pv;
-            }
-        }
-        __syncthreads();
-        for (int t = threadIdx.x; t < len; t += blockDim.x) perm[g0 + t] = sperm[t];
-    } else if (c < c1) {  // dense window: sort in place in global memory
-        const int b = start[c], e = start[c + 1];
-        for (int a = b + 1; a < e; ++a) {
-            const int kv = pid[a], pv = perm[a];
-            int q = a - 1;
-            while (q >= b && pid[q] > kv) {
-                pid[q + 1] = pid[q];
-                perm[q + 1] = perm[q];
-                --q;
-            }
-            pid[q + 1] = kv;
-            perm[q + 1] = pv;
-        }
-    }
-}
-
 // A coordinate relative to the grid's corner in units of lsb, modulo 2^32:
 // the difference of two particles' values, as a signed integer, is their
 // separation wherever that is below 2^31 lsb (eight cells).
@@ -505,10 +446,18 @@ __device__ __forceinline__ int lsb_units(double x, double inv) {
     return (int)(uint32_t)(t - floor(t * 0x1p-32) * 0x1p32);
 }
 
-// permutes the state into the new order and writes the integer positions (the
-// neighbour test's in both precisions)
+// Permutes the state into the new order and writes the integer positions (the
+// neighbour test's in both precisions).  Inside a cell the order is by
+// ascending particle id, which OrdGrid1's 4th loop produces (NPartOrd), hence
+// the reference's neighbour-list order: a particle's place is the number of
+// smaller ids among the cell's (18) particles, whose ids are a few cache lines
+// for a wavefront.  (A kernel that sorted each cell's run by insertion before
+// this one took 33 us at 576,000 particles and 17 at 1,440.)
+// Also clears the counters that the next sort counts in: m keys, their
+// scan blocks, the removed ids, the boundary table's work counter.
 template <bool SG>
-__global__ void k_gather(Seg S, const int* __restrict__ perm, const int* __restrict__ key,
+__global__ void k_gather(Seg S, const int* __restrict__ perm, const int* __restrict__ pid,
+                         const int* __restrict__ key,
                          const double4* __restrict__ xm_s, const double4* __restrict__ vel_s,
                          const double2* __restrict__ rp_s, const int* __restrict__ lam_s,
                          const double4* __restrict__ acc_s, double4* __restrict__ xm_d,
@@ -519,18 +468,26 @@ __global__ void k_gather(Seg S, const int* __restrict__ perm, const int* __restr
                          const double* __restrict__ dd_s, double* __restrict__ dd_d,
                          const double* __restrict__ vp_s, double* __restrict__ vp_d,
                          const double* __restrict__ g_s, double* __restrict__ g_d,
-                         const double* __restrict__ h_s, double* __restrict__ h_d) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+                         const double* __restrict__ h_s, double* __restrict__ h_d,
+                         int* __restrict__ cnt, int m, int* __restrict__ bsum, int nbsum, int* nwork) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
     const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(blockIdx.x * blockDim.x) >> 8]) : 0;
     DPC& P = S.P[sg];
     iscal += sg * IS_COUNT;
+    for (int k = q; k < m; k += gridDim.x * blockDim.x) cnt[k] = 0;
+    for (int k = q; k < nbsum; k += gridDim.x * blockDim.x) bsum[k] = 0;
+    if (q == 0) *nwork = 0;
     const int nin = start[P.koff + P.nmax] - P.base;  // particles still inside the grid
-    if (p == P.base) {
+    if (q == P.base) {
         iscal[IS_NPREV] = iscal[IS_N];
         iscal[IS_N] = nin;
+        iscal[IS_NRM] = 0;
     }
-    if (p - P.base >= nin) return;
-    const int s = perm[p];
+    if (q - P.base >= nin) return;
+    const int s = perm[q], id = pid[q];
+    const int b = start[key[s]], e = start[key[s] + 1];
+    int p = b;
+    for (int t = b; t < e; ++t) p += pid[t] < id;
     const double4 x = xm_s[s];
     const double4 v = vel_s[s];
     const double2 r = rp_s[s];
