@@ -275,15 +275,8 @@ int run_dt(sph_ctx* c, int advance, bool reduce) {
     return 0;
 }
 
-// The pair passes in FP64: one lane per particle, one-solve or segmented form.
-#define PAIR64(K, ...)                                                                            \
-    do {                                                                                          \
-        if (c->nseg > 1) K<true><<<c->grid, c->wg, 0, c->stream>>>(c->S, __VA_ARGS__);      \
-        else K<false><<<c->grid, c->wg, 0, c->stream>>>(c->S, __VA_ARGS__);                 \
-    } while (0)
-
-// The pair passes in FP32-mixed form: launch(CAP, SG, G) of the context's tile
-// form (more than one lane per particle only with the smallest tiles).
+// The pair passes: launch(CAP, SG, G) of the context's tile form (more than one
+// lane per particle only with the smallest tiles; TILE_CAP_0: no LDS form).
 template <int V>
 using IntC = std::integral_constant<int, V>;
 template <class Launch>
@@ -297,14 +290,32 @@ void tile_dispatch(sph_ctx* c, Launch&& launch) {
     if (c->nseg > 1) form(std::true_type{});
     else form(std::false_type{});
 }
+// The FP64 passes; TILE_CAP_0 has no LDS form (lists with stencil codes).
+template <class Launch>
+void tile_dispatch64(sph_ctx* c, Launch&& launch) {
+    auto lanes = [&](auto cap, auto sg) {
+        if (c->tile_g == 1) launch(cap, sg, IntC<1>{});
+        else if (c->tile_g == 2) launch(cap, sg, IntC<2>{});
+        else launch(cap, sg, IntC<4>{});
+    };
+    auto form = [&](auto sg) {
+        if (c->tile_cap == TILE_CAP_L) lanes(IntC<TILE_CAP_L>{}, sg);
+        else if (c->tile_cap == TILE_CAP_S) lanes(IntC<TILE_CAP_S>{}, sg);
+        else lanes(IntC<TILE_CAP_0>{}, sg);
+    };
+    if (c->nseg > 1) form(std::true_type{});
+    else form(std::false_type{});
+}
 #define TILE_RUN(...) \
     <<<c->tile_grid, c->tile_wg, 0, c->stream>>>(c->S, Tiles{c->tlist, c->ntile}, c->start, __VA_ARGS__)
 
 int run_momentum(sph_ctx* c) {
     KTime t(c, "momentum");
     if (!c->P.f32) {
-        PAIR64(k_momentum64, c->d_faces, c->d_edges, c->bn, c->bt, c->xm[0], c->vel[0], c->rp[cur_rp(c)], c->lam[1],
-               c->lam[0], c->nbr, c->nnb, c->acc[1], c->vel[1], c->scal, c->iscal);
+        tile_dispatch64(c, [&](auto cap, auto sg, auto g) {
+            k_momentum64<cap.value, sg.value, g.value> TILE_RUN(c->d_faces, c->d_edges, c->bn, c->bt, c->xm[0], c->vel[0],
+                c->rp[cur_rp(c)], c->lam[1], c->lam[0], c->nbr, c->nnb, c->acc[1], c->vel[1], c->scal, c->iscal);
+        });
         return 0;
     }
     bool um = c->nseg == 1 ? c->P.umass != 0 : true;
@@ -322,8 +333,11 @@ int run_momentum(sph_ctx* c) {
 int run_vsmooth(sph_ctx* c) {
     KTime t(c, "velocity_smoothing");
     if (!c->P.f32)
-        PAIR64(k_vsmooth64, c->d_faces, c->bn, c->bt, c->xm[0], c->vel[1], c->rp[cur_rp(c)], c->nbr, c->nnb, c->vel[2],
-               c->xm[1], c->scal, c->dtmin, c->iscal, c->dden, c->rp[2], c->gone);
+        tile_dispatch64(c, [&](auto cap, auto sg, auto g) {
+            k_vsmooth64<cap.value, sg.value, g.value> TILE_RUN(c->d_faces, c->bn, c->bt, c->xm[0], c->vel[1],
+                c->rp[cur_rp(c)], c->nbr, c->nnb, c->vel[2], c->xm[1], c->scal, c->dtmin, c->iscal, c->dden, c->rp[2],
+                c->gone);
+        });
     else
         tile_dispatch(c, [&](auto cap, auto sg, auto g) {
             k_vsmooth<cap.value, sg.value, g.value> TILE_RUN(c->d_faces, c->bn, c->bt, c->xm[0], c->vel[1], c->rp[cur_rp(c)], c->xq, c->vf[1],
@@ -335,8 +349,10 @@ int run_vsmooth(sph_ctx* c) {
 int run_continuity(sph_ctx* c) {
     KTime t(c, "continuity");
     if (!c->P.f32)
-        PAIR64(k_continuity64, c->d_faces, c->bn, c->bt, c->xm[0], c->vel[0], c->P.dbsph ? c->rp[0] : c->rp[1], c->nbr,
-               c->nnb, c->dden, c->rp[2], c->scal, c->iscal);
+        tile_dispatch64(c, [&](auto cap, auto sg, auto g) {
+            k_continuity64<cap.value, sg.value, g.value> TILE_RUN(c->d_faces, c->bn, c->bt, c->xm[0], c->vel[0],
+                c->P.dbsph ? c->rp[0] : c->rp[1], c->nbr, c->nnb, c->dden, c->rp[2], c->scal, c->iscal);
+        });
     else
         tile_dispatch(c, [&](auto cap, auto sg, auto g) {
             k_continuity<cap.value, sg.value, g.value> TILE_RUN(c->d_faces, c->bn, c->bt, c->vel[0], c->rp[1], c->xq, c->vf[0], c->nbr, c->nnb,
@@ -345,11 +361,17 @@ int run_continuity(sph_ctx* c) {
     return 0;
 }
 
+void run_psmooth64(sph_ctx* c, double* vpres) {
+    tile_dispatch64(c, [&](auto cap, auto sg, auto g) {
+        k_psmooth64<cap.value, sg.value, g.value> TILE_RUN(c->d_faces, c->bn, c->bt, c->xm[0], c->rp[2], c->nbr, c->nnb,
+            vpres, c->rp[0], c->scal);
+    });
+}
+
 int run_psmooth(sph_ctx* c) {
     KTime t(c, "pressure_smoothing");
     if (!c->P.f32)
-        PAIR64(k_psmooth64, c->d_faces, c->bn, c->bt, c->xm[0], c->rp[2], c->nbr, c->nnb, c->vpres, c->rp[0], c->scal,
-               c->iscal);
+        run_psmooth64(c, c->vpres);
     else
         tile_dispatch(c, [&](auto cap, auto sg, auto g) {
             k_psmooth<cap.value, sg.value, g.value> TILE_RUN(c->d_faces, c->bn, c->bt, c->rp[2], c->xq, c->dr, c->nbr, c->nnb, c->vpres,
@@ -396,8 +418,7 @@ int run_momentum_dbsph(sph_ctx* c) {
 // PressureSmoothing_3D.f90 for bsph on the new lists: rp[2] -> rp[0]
 int run_psmooth_dbsph(sph_ctx* c) {
     KTime t(c, "pressure_smoothing");
-    PAIR64(k_psmooth64, c->d_faces, c->bn, c->bt, c->xm[0], c->rp[2], c->nbr, c->nnb, c->vpres2, c->rp[0], c->scal,
-           c->iscal);
+    run_psmooth64(c, c->vpres2);
     return 0;
 }
 
@@ -632,6 +653,8 @@ int fill_dp(const sph_params* p, const sph_faces* f, DP& P, bool dry = false) {
     P.eta = p->eta;
     P.eta2 = p->eta2;
     P.squareh = p->h * p->h;
+    P.inv_h = 1.0 / P.h;
+    P.inv_squareh = 1.0 / P.squareh;
     P.doubleh = 2.0 * p->h;
     P.square_doubleh = P.doubleh * P.doubleh;
     P.ke_coef = p->coefke / p->h;
@@ -664,7 +687,7 @@ int fill_dp(const sph_params* p, const sph_faces* f, DP& P, bool dry = false) {
 
 inline int round256(long long v) { return (int)((v + 255) / 256 * 256); }
 
-// The tile of the FP32-mixed pair passes, one for all segments: the largest
+// The tile of the pair passes, one for all segments: the largest
 // box of cells of the ladder that cuts the solve's water into TILE_MIN tiles
 // (2D: TILE_MIN2) - fewer leave CUs idle, smaller ones read more halo - and whose
 // cells with their halo, an eighth denser than water, fit the largest LDS
@@ -673,6 +696,15 @@ inline int round256(long long v) { return (int)((v + 255) / 256 * 256); }
 // 4x3x2 740; 250,000 409, 439; 185,000 (390 tiles) 3x3x3 446, 3x3x2 377,
 // 3x2x1 411; 103,000 3x3x2 294, 3x2x2 334, 3x3x3 396; 72,000 3x2x2 229, 3x3x2
 // 245, 3x1x1 292; 2D 61,000 7x6 182, 6x5 185, 4x4 189.
+// FP64, one workgroup a CU: TILE_MIN64 (2D TILE_MIN64_2) tiles, enough for a
+// round of half the CUs, and lanes a particle (1, 2, 4) up to a workgroup.
+// 576,000 particles 3x3x3 1465, 3x3x2 1827, 3x2x2 1906; 72,000 (152 tiles)
+// 3x3x3 379, 3x2x2 436, 3x3x2 468; 50,000 3x3x2 327, 3x3x3 353, 3x2x2 396;
+// 30,000 3x2x2 284, 3x3x2 317, 3x2x1 328; 20,000 3x2x1 270, 3x2x2 276; 5,000
+// 2x1x1 236, 1x1x1 252, 3x1x1 258; 2D 61,000 7x6 167, 8x8 172, 6x5 183; 20,000
+// 4x4 130, 6x5 142, 3x3 143; 5,000 3x3 115, 2x2 119, 4x4 122.  Lanes: 72,000
+// one 379, two 410; 50,000 (3x3x2) two 327, one 355; 20,000 (3x2x2) two 276,
+// four 306; 2D 20,000 four 130, two 139; 5,000 four 119, two 123.
 void choose_tile(sph_ctx* c) {
     const int L3[][3] = {{3, 3, 3}, {3, 3, 2}, {3, 2, 2}, {3, 2, 1}, {3, 1, 1}, {2, 1, 1}, {1, 1, 1}};
     const int L2[][3] = {{8, 1, 8}, {7, 1, 6}, {6, 1, 5}, {4, 1, 4}, {3, 1, 3}, {2, 1, 2}, {1, 1, 1}};
@@ -690,10 +722,15 @@ void choose_tile(sph_ctx* c) {
         best = flat ? L2[k] : L3[k];
         home = ppc * best[0] * best[1] * best[2];
         need = 1.125 * ppc * (best[0] + 2) * (flat ? 1 : best[1] + 2) * (best[2] + 2);
-        if (need <= TILE_CAP_L && A.cap >= (k == 0 ? TILE_MIN_L : flat ? TILE_MIN2 : TILE_MIN) * home) break;
+        const int least = !A.f32 ? (flat ? TILE_MIN64_2 : TILE_MIN64) : k == 0 ? TILE_MIN_L : flat ? TILE_MIN2 : TILE_MIN;
+        if (need <= TILE_CAP_L && A.cap >= least * home) break;
     }
     c->tile_cap = need <= TILE_CAP_S ? TILE_CAP_S : need <= TILE_CAP_M ? TILE_CAP_M : TILE_CAP_L;
     c->tile_g = c->tile_cap != TILE_CAP_S ? 1 : A.cap < TILE_G2 ? 2 : 1;
+    if (!A.f32) {
+        c->tile_cap = need <= TILE_CAP_S ? TILE_CAP_S : TILE_CAP_L;
+        c->tile_g = 4 * home <= TILE_WG ? 4 : 2 * home <= 1.25 * TILE_WG ? 2 : 1;
+    }
     // threads for the most particles a tile of lattice water holds
     double most = c->tile_g;
     for (int d = 0; d < 3; d += flat ? 2 : 1) most *= std::ceil(best[d] * A.dcd[d] / A.dx);
@@ -711,10 +748,10 @@ void choose_tile(sph_ctx* c) {
         Q.inv_nti = 1.0 / Q.ntile[0];
         Q.inv_ry = 1.0 / (Q.tdim[1] + 2);
         Q.toff = (int)tiles;
-        Q.tcap = Q.f32 ? c->tile_cap : 0;
+        Q.tcap = Q.f32 ? c->tile_cap : 0;  // FP64: set by the upload
         tiles += (n + 255) / 256 * 256;
     }
-    c->ntiles = (int)(A.f32 ? tiles : 0);
+    c->ntiles = (int)tiles;
     // a workgroup per tile where every tile is full, and as many again for partly filled ones
     const double full = 2.0 * A.cap / home + 64.0;
     c->tile_grid = (int)(std::min((double)tiles, full) / 8.0 + 1.0) * 8;
@@ -909,7 +946,7 @@ int upload_segment_maps(sph_ctx* c) {
     c->S = Seg{(DPC*)c->d_P, nullptr, nullptr, nullptr, c->nseg};
     if (int rc = upload_constants(c)) return rc;
     if (c->nseg == 1) return 0;
-    std::vector<int> pblk(c->P.cap / 256), kblk(c->nkeys / 256), tblk(std::max(1, c->ntiles / 256));
+    std::vector<int> pblk(c->P.cap / 256), kblk(c->nkeys / 256), tblk(c->ntiles / 256);
     for (int s = 0; s < c->nseg; ++s) {
         const DP& P = c->segs[s];
         const int sb = (s + 1 < c->nseg ? c->segs[s + 1].base : c->P.cap);
@@ -917,7 +954,7 @@ int upload_segment_maps(sph_ctx* c) {
         const int ke = (s + 1 < c->nseg ? c->segs[s + 1].koff : c->nkeys);
         for (int b = P.koff / 256; b < ke / 256; ++b) kblk[b] = s;
         const int te = (s + 1 < c->nseg ? c->segs[s + 1].toff : c->ntiles);
-        for (int b = P.toff / 256; c->ntiles && b < te / 256; ++b) tblk[b] = s;
+        for (int b = P.toff / 256; b < te / 256; ++b) tblk[b] = s;
     }
     bool ok = hipMalloc(&c->d_pblk, sizeof(int) * pblk.size()) == hipSuccess &&
               hipMemcpy(c->d_pblk, pblk.data(), sizeof(int) * pblk.size(), hipMemcpyHostToDevice) == hipSuccess &&
@@ -1212,6 +1249,8 @@ int sph_dbsph_walls(sph_ctx* c, const sph_dbsph_walls_t* w) {
     P.fs_allowed = w->fs_allowed ? 1 : 0;
     P.neg_wall_p = w->negative_wall_p_allowed ? 1 : 0;
     P.muscl_bnd = w->muscl_boundary ? 1 : 0;
+    P.tcap = 0;  // the DB-SPH kernels read the lists' stencil codes
+    c->tile_cap = TILE_CAP_0;
     return upload_constants(c);
 }
 
@@ -1306,9 +1345,11 @@ int sph_segment_upload(sph_ctx* c, int32_t seg, int32_t n, const double* coord, 
         DP& Q = c->nseg > 1 ? c->segs[seg] : c->P;
         Q.umass = umass;
         Q.f_mass = f_mass;
+        if (!Q.f32) Q.tcap = umass && !Q.dbsph ? c->tile_cap : 0;  // the FP64 slots hold no mass
         if (c->nseg > 1 && seg == 0) {
             c->P.umass = umass;
             c->P.f_mass = f_mass;
+            c->P.tcap = Q.tcap;
         }
         if (int rc = upload_constants(c)) return rc;
         // captured graphs hold the momentum kernel chosen for the old masses

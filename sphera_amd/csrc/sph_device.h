@@ -48,6 +48,7 @@ struct DP {
     double grav[3], prif, den0, eps, celerita, alfamon, kin_visc;
     double cfl, vsc_coeff, pesodt, tetap, tetav;
     // unit of the integer positions: 2^-28 of the largest cell side
+    double inv_h, inv_squareh;  // reciprocals of h and squareh
     double lsb, inv_lsb;
     // FP32-mixed pair sums: h, eta and eta2 in units of lsb (f_q = lsb / h)
     float f_q, f_etal, f_eta2l, f_dcd[3], f_kin_visc;

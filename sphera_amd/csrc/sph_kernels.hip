@@ -108,6 +108,79 @@ __device__ __forceinline__ void kvals64(DPC& P, double rij, bool need12, bool ne
     }
 }
 
+// The pair loops form the terms of two list entries side by side: an FP64
+// operation's result is ready after several issue slots, and two wavefronts a
+// SIMD (what the registers and the LDS leave) do not fill them.
+using d2 = double __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ d2 fma2(d2 a, d2 b, d2 c) { return __builtin_elementwise_fma(a, b, c); }
+
+// FP64 quotients and roots of the pair loops, correctly rounded as `/` and
+// sqrt() are, without the scaling steps those take for operands near the ends
+// of the exponent range: Newton's iteration for the reciprocal and Markstein's
+// final correction, q + (a - d q) y with y = 1/d (P. Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990).  A
+// divisor that several quotients share is inverted once.
+__device__ __forceinline__ d2 newton64(d2 d, d2 y) { return fma2(fma2(-d, y, d2(1.0)), y, y); }
+__device__ __forceinline__ d2 inv64(d2 d) {
+    return newton64(d, newton64(d, d2{__builtin_amdgcn_rcp(d.x), __builtin_amdgcn_rcp(d.y)}));
+}
+__device__ __forceinline__ d2 quot64(d2 a, d2 d, d2 y) {
+    const d2 q = a * y;
+    return fma2(fma2(-d, q, a), y, q);
+}
+// with zeros, infinities and NaN as `/` gives them
+__device__ __forceinline__ d2 div64(d2 a, d2 d, d2 y) {
+    const d2 q = quot64(a, d, y);
+    return d2{__builtin_amdgcn_div_fixup(q.x, d.x, a.x), __builtin_amdgcn_div_fixup(q.y, d.y, a.y)};
+}
+__device__ __forceinline__ d2 sqrt64(d2 x) {
+    const d2 y = {__builtin_amdgcn_rsq(x.x), __builtin_amdgcn_rsq(x.y)};
+    d2 g = x * y, h = 0.5 * y;
+    const d2 e = fma2(-h, g, d2(0.5));
+    g = fma2(g, e, g);
+    h = fma2(h, e, h);
+    g = fma2(fma2(-g, g, x), h, g);
+    g = fma2(fma2(-g, g, x), h, g);
+    auto ends = [](double a, double r) { return a > 0.0 && a < __builtin_inf() ? r : a; };
+    return d2{ends(x.x, g.x), ends(x.y, g.y)};
+}
+
+// kvals64 of two pairs without branches (a wavefront's lanes differ), its
+// quotients by the reciprocals of the constants
+struct K64x2 { d2 K1, K2, K3, W; };
+__device__ __forceinline__ K64x2 kvals64x2(DPC& P, d2 rij2, bool need12, bool need3, bool needW) {
+    const d2 r = sqrt64(rij2);
+    const d2 q = quot64(r, d2(P.h), d2(P.inv_h));
+    const d2 q2 = quot64(rij2, d2(P.squareh), d2(P.inv_squareh));
+    auto near = [&](double k) { return d2{q.x >= 2.0 ? 0.0 : k, q.y >= 2.0 ? 0.0 : k}; };
+    auto part = [&](d2 outer, d2 inner) { return d2{q.x >= 1.0 ? outer.x : inner.x, q.y >= 1.0 ? outer.y : inner.y}; };
+    K64x2 K;
+    K.K1 = K.K2 = K.K3 = K.W = d2(0.0);
+    d2 denom = d2(0.0);
+    if (need12 || need3) {
+        const d2 d = r + P.eta;
+        denom = quot64(d2(1.0), d, inv64(d));
+    }
+    if (need12) {
+        d2 gm = -2.0 * q + 1.5 * q2;
+        gm = part(-gm + q2 - 2.0, gm);
+        gm = gm * near(P.ke_coef);
+        K.K1 = gm * denom;
+        const d2 d = rij2 + P.eta2;
+        K.K2 = quot64(K.K1, d, inv64(d));
+    }
+    if (need3) {
+        d2 gw = -12.0 - 3.0 * q2 + 12.0 * q;
+        gw = gw * near(P.kacl_coef);
+        K.K3 = gw * denom;
+    }
+    if (needW) {
+        const d2 a = 0.666666667 + q2 * (q * 0.5 - 1.0), b = (2.0 - q) * (2.0 - q) * (2.0 - q) * 0.166666666667;
+        K.W = part(b, a) * near(P.coefke);
+    }
+    return K;
+}
+
 // ----------------------------------------------------------------------------
 // SA-SPH geometry: LocalNormalCoordinates.f90:55-87 + IsPointInternal.f90
 // ----------------------------------------------------------------------------
@@ -141,11 +214,14 @@ __device__ __forceinline__ bool d_point_internal(const DFace& F, double px0, dou
 // LDS of the pair passes (P.tcap), the neighbour lists hold 16-bit slot
 // offsets; elsewhere 32-bit sorted indices with the stencil code.
 // ----------------------------------------------------------------------------
-constexpr int TILE_CAP_L = 2496, TILE_CAP_M = 1632, TILE_CAP_S = 1216;  // 2, 3 and 4 workgroups a CU of 32 bytes a slot
+// slots: 2, 3 and 4 workgroups a CU of 32 bytes a slot, 1, 1 and 2 of 64
+constexpr int TILE_CAP_L = 2496, TILE_CAP_M = 1632, TILE_CAP_S = 1216, TILE_CAP_0 = 16;
 constexpr int TILE_WG = 512;   // most threads of a pair pass
-constexpr int TILE_U = 5;      // slots a thread stages at a time
+constexpr int TILE_U = 5;      // slots a thread stages at a time (FP64: 3)
 constexpr int TILE_G2 = 40000;  // particles below which two lanes take a particle
-constexpr int TILE_MIN = 300, TILE_MIN2 = 200, TILE_MIN_L = 500;  // tiles of water a solve is cut into (choose_tile)
+// tiles of water a solve is cut into (choose_tile); FP64
+constexpr int TILE_MIN = 300, TILE_MIN2 = 200, TILE_MIN_L = 500;
+constexpr int TILE_MIN64 = 130, TILE_MIN64_2 = 150;
 struct TileS {
     int g[64];      // row r: sorted index of its first particle
     int l[65];      // its first slot; l[rows] the number of slots
@@ -1741,6 +1817,17 @@ __device__ __forceinline__ void block_min_to(unsigned long long v, unsigned long
     }
 }
 
+// The wave's minimum of v into *dst, and v reset.  The minimum only falls: a
+// value read before the atomic is an upper bound of it.
+__device__ __forceinline__ void wave_min_to(unsigned long long& v, unsigned long long* dst) {
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long t = __shfl_xor(v, o, 64);
+        v = t < v ? t : v;
+    }
+    if ((threadIdx.x & 63) == 0 && v < *(volatile unsigned long long*)dst) atomicMin(dst, v);
+    v = 0x7FF0000000000000ull;
+}
+
 template <bool SG>
 __global__ __launch_bounds__(256) void k_dtmin(Seg S, const double4* __restrict__ vel,
                                                unsigned long long* dtmin, const int* iscal) {
@@ -1807,10 +1894,10 @@ __device__ __forceinline__ int tile_find(const int* pre, int rows, int x) {
 
 // Runs the tiles that hold particles: stage(P, segment, sorted index, slot)
 // for every slot of a tile that fits, then part(P, segment, sorted index,
-// fits) with G lanes for every home particle, then done(P, segment).  A workgroup takes
-// the tiles of its XCD's contiguous share, so tiles that share halo rows
-// share an L2.
-template <bool SG, int G, class Stage, class Part, class Done>
+// slot, fits) with G lanes for every home particle, then done(P, segment).  A
+// workgroup takes the tiles of its XCD's contiguous share, so tiles that share
+// halo rows share an L2.
+template <bool SG, int G, int U, class Stage, class Part, class Done>
 __device__ __forceinline__ void for_tiles(const Seg& S, const Tiles& T,
                                           const int* __restrict__ start, Stage&& stage, Part&& part,
                                           Done&& done) {
@@ -1839,25 +1926,26 @@ __device__ __forceinline__ void for_tiles(const Seg& S, const Tiles& T,
         const int total = ts.l[rows], nhome = ts.hp[rows];
         const bool fits = total <= P.tcap;
         if (fits) {
-            // TILE_U slots per thread at a time, so that their loads are in
-            // flight together (a slot past the end repeats the last one)
+            // U slots per thread at a time, so that their loads are in flight
+            // together (a slot past the end repeats the last one)
             const int bs = blockDim.x;
-            for (int e0 = threadIdx.x; e0 < total; e0 += TILE_U * bs) {
-                int e[TILE_U], g[TILE_U];
+            for (int e0 = threadIdx.x; e0 < total; e0 += U * bs) {
+                int e[U], g[U];
 #pragma unroll
-                for (int u = 0; u < TILE_U; ++u) {
+                for (int u = 0; u < U; ++u) {
                     e[u] = min(e0 + u * bs, total - 1);
                     const int r = tile_find(ts.l, rows, e[u]);
                     g[u] = ts.g[r] + e[u] - ts.l[r];
                 }
 #pragma unroll
-                for (int u = 0; u < TILE_U; ++u) stage(P, sg, g[u], e[u]);
+                for (int u = 0; u < U; ++u) stage(P, sg, g[u], e[u]);
             }
         }
         __syncthreads();
         for (int q = threadIdx.x / G; q < nhome; q += blockDim.x / G) {
             const int a = tile_find(ts.hp, rows, q);
-            part(P, sg, ts.h0[a] + q - ts.hp[a], fits);
+            const int i = ts.h0[a] + q - ts.hp[a];
+            part(P, sg, i, i - ts.g[a] + ts.l[a], fits);
         }
         done(P, sg);
         __syncthreads();  // the slots and rows are reused
@@ -2601,237 +2689,359 @@ __device__ __forceinline__ double psmooth_end(DPC& P, const DFace* __restrict__ 
 }
 
 // ----------------------------------------------------------------------------
-// The four passes in FP64: one lane per particle, records gathered through
-// L1/L2, the reference's expressions operation for operation.
+// The four passes in FP64, one workgroup per tile: as the FP32-mixed ones
+// below, with FP64 records (48 to 64 bytes a slot, so the largest tiles leave
+// one workgroup of eight wavefronts a CU).  The expressions are the
+// reference's, operation for operation, and every sum is formed in list order.
+// They were bound by their gathers, five 16-byte loads a neighbour from records
+// of three cell planes, more than an XCD's L2 (0.9-1.9 GB a launch from HBM);
+// now by FP64 issue (measured: an operation every 4.9-5.7 cycles of a SIMD, a
+// reciprocal or root 16.5), so the quotients share reciprocals and nothing
+// branches on a pair.  576,000 particles: momentum 499 -> 448 us, velocity
+// smoothing 595 -> 203, continuity 527 -> 206, pressure smoothing 315 -> 170;
+// 72,000: 102 -> 74, 58 -> 33, 58 -> 33, 46 -> 28.  Twice the wavefronts (two
+// lanes a particle, 1024 threads) measured the same, reading a neighbour's
+// records ahead of the previous one's arithmetic 1% slower.
+// Tiles that do not fit, solves of several masses, and lists that carry stencil
+// codes (DB-SPH walls) gather from global memory with the same expressions.
 // ----------------------------------------------------------------------------
+#define TILE_ARGS Seg S, Tiles T, const int* __restrict__ start
+
+// lane u's value for lane 0 of each group of G (the other lanes: any)
+template <int G>
+__device__ __forceinline__ double group_lane(double v, int u) {
+    if (u == 0) return v;
+    auto pick = [&](int w) {
+        if constexpr (G == 2) return __builtin_amdgcn_mov_dpp(w, 0xF5, 0xF, 0xF, true);  // quad_perm (1,1,3,3)
+        return u == 1 ? __builtin_amdgcn_mov_dpp(w, 0x55, 0xF, 0xF, true)
+             : u == 2 ? __builtin_amdgcn_mov_dpp(w, 0xAA, 0xF, 0xF, true)
+                      : __builtin_amdgcn_mov_dpp(w, 0xFF, 0xF, 0xF, true);
+    };
+    return __hiloint2double(pick(__double2hiint(v)), pick(__double2loint(v)));
+}
+
+// Adds particle i's NS pair terms to sum in list order, by G lanes (1, 2 or 4,
+// lane g of them): each lane forms the terms of two entries, the lanes' entries
+// consecutive, and lane 0 adds them all in order.  lds(byte offset of a
+// neighbour's 16-byte records) and glob(its sorted index) read a neighbour,
+// term(terms, one, other, one counts, other counts).  Past the list's end they
+// are given the particle itself (`self`, i), whose differences vanish: a term
+// that is a multiple of one is then a zero and leaves the sum as it is.
+template <int G, int NS, class Lds, class Glob, class Term>
+__device__ __forceinline__ void pair_sums64(const uint32_t* __restrict__ nbr, size_t N, int i, int nn, int g,
+                                            bool fits, uint32_t self, double (&sum)[NS], Lds&& lds, Glob&& glob,
+                                            Term&& term) {
+    auto add = [&](const d2 (&t)[NS]) {
+#pragma unroll
+        for (int u = 0; u < G; ++u)
+#pragma unroll
+            for (int c = 0; c < NS; ++c) sum[c] = sum[c] + group_lane<G>(t[c].x, u);
+#pragma unroll
+        for (int u = 0; u < G; ++u)
+#pragma unroll
+            for (int c = 0; c < NS; ++c) sum[c] = sum[c] + group_lane<G>(t[c].y, u);
+    };
+    if (fits) {
+        const uint4* L = reinterpret_cast<const uint4*>(nbr) + 2 * (size_t)i;
+        uint4 next = *L;
+        for (int k0 = 0; k0 < nn; k0 += 8) {
+            const uint4 cur = next;
+            L += (k0 & 8) ? 2 * N - 1 : (size_t)1;
+            if (k0 + 8 < nn) next = *L;
+            const uint32_t w[4] = {cur.x, cur.y, cur.z, cur.w};
+            auto slot = [&](int u) {  // this lane's of the G entries from u on
+                uint32_t o = w[u >> 1];
+                if constexpr (G == 4) {
+                    const uint32_t o2 = w[(u >> 1) + 1];
+                    o = g & 2 ? o2 : o;
+                }
+                o = (G == 1 ? u & 1 : g & 1) ? o >> 16 : o & 0xFFFFu;
+                return k0 + u + g < nn ? o : self;
+            };
+#pragma unroll
+            for (int u = 0; u < 8; u += 2 * G) {
+                __builtin_amdgcn_sched_barrier(0);
+                d2 t[NS];
+                term(t, lds(slot(u)), lds(slot(u + G)), k0 + u + g < nn, k0 + u + G + g < nn);
+                add(t);
+            }
+        }
+    } else {
+        for (int k0 = 0; k0 < nn; k0 += 2 * G) {
+            const int ka = k0 + g, kb = k0 + G + g;
+            const int ja = ka < nn ? (int)(nbr[nb_index(N, i, ka)] & NB_MASK) : i;
+            const int jb = kb < nn ? (int)(nbr[nb_index(N, i, kb)] & NB_MASK) : i;
+            d2 t[NS];
+            term(t, glob(ja), glob(jb), ka < nn, kb < nn);
+            add(t);
+        }
+    }
+}
+
+// 16 bytes at byte offset o of an LDS array, 8 bytes of the slot at offset o
+__device__ __forceinline__ double2 lds16(const double2* a, uint32_t o) {
+    return *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(a) + o);
+}
+__device__ __forceinline__ double lds8(const double* a, uint32_t o) {
+    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(a) + (o >> 1));
+}
+
+struct Nb { double x, y, z, u, v, w, rho, p, inv, m; };  // a neighbour, as far as a pass needs it
+
 // momentum: RHS_momentum_equation.f90:72-179, inter_EqMoto.f90:108-283,
 // viscomon.f90:54-71, viscomorris.f90:60-71
-template <bool SG>
-__global__ __launch_bounds__(256) void k_momentum64(
-    Seg S, const DFace* __restrict__ faces, const DEdge* __restrict__ edges,
+template <int CAP, bool SG, int G>
+__global__ __launch_bounds__(TILE_WG, 2) void k_momentum64(
+    TILE_ARGS, const DFace* __restrict__ faces, const DEdge* __restrict__ edges,
     const int* __restrict__ bn, const BTab* __restrict__ bt, const double4* __restrict__ xm,
     const double4* __restrict__ vel, const double2* __restrict__ rp, const int* __restrict__ lam_in,
     int* __restrict__ lam_out, const uint32_t* __restrict__ nbr, const int* __restrict__ nnb,
-    double4* __restrict__ acc_out, double4* __restrict__ vel_out, const double* scal, int* iscal) {
-    const int vb = xcd_block(gridDim.x);
-    const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * (int)blockDim.x) >> 8]) : 0;
-    DPC& P = S.P[sg];
-    scal += sg * SC_COUNT;
-    iscal += sg * IS_COUNT;
-    const double h = P.h;
-    // Leapfrog_momentum.f90:66-86 integrates with dtvel; the explicit RK1
-    // branch (Euler.f90:85-93) with dt
-    const double dtvel = P.rk1 ? scal[SC_DT] : scal[SC_DTVEL];
-    const size_t N = P.cap;
-    const int i = vb * blockDim.x + threadIdx.x;
-    if (i - P.base < iscal[IS_N]) {
-        const double4 vi = vel[i];  // var == vel here
-        const double2 rpi = rp[i];
-        double tp[3] = {0.0, 0.0, 0.0}, td[3] = {0.0, 0.0, 0.0}, tv[3] = {0.0, 0.0, 0.0};
-        const int ncbf = P.semi ? bn[i] : 0;
-        const double v_i[3] = {vi.x, vi.y, vi.z};
-        if (ncbf > 0) {
-            if (P.dim == 2)
-                sa_momentum_2d(P, faces, bt, i, ncbf, v_i, rpi, lam_in[i], tp, td, tv);
-            else
-                sa_momentum(P, faces, bt, i, ncbf, v_i, rpi, lam_in[i], tp, td, tv, iscal);
-        }
-        const int nn = nnb[i];
-        double rvs[3];
-        const double4 xi = xm[i];
-        const double rhoi = rpi.x, pi = rpi.y;
-        double tpa[3] = {0, 0, 0}, ale[3] = {0, 0, 0};
-        rvs[0] = rvs[1] = rvs[2] = 0.0;
-        const double celt = P.celerita + P.celerita;
-        const double nui = P.kin_visc, nuj = P.kin_visc;
-        const bool morris = nui > 1.0e-12 && nuj > 1.0e-12;
-        using RM = NRec<double4, double4, double2>;
-        auto fetch = [&](uint32_t e) {
-            const int j = (int)(e & NB_MASK);
-            return RM{xm[j], vel[j], rp[j]};
-        };
-        walk_list<4, RM>(nbr, N, i, nn, fetch, [&](uint32_t e, const RM& q) {
-            if ((int)(e & NB_MASK) == i) return;
-            const double4 xj = q.x;
-            const double4 vj = q.v;
-            const double2 rpj = q.r;
-            const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
-            const double rij = R0 * R0 + R1 * R1 + R2 * R2;
-            K64 K;
-            kvals64(P, rij, true, true, false, K);
-            const double rhoj = rpj.x, pj = rpj.y, amassj = xj.w;
-            const double dv0 = vj.x - vi.x, dv1 = vj.y - vi.y, dv2 = vj.z - vi.z;
-            double alpha = (pj - pi) / (rhoi * rhoj);
-            tpa[0] = tpa[0] + -amassj * alpha * R0 * K.K3;
-            tpa[1] = tpa[1] + -amassj * alpha * R1 * K.K3;
-            tpa[2] = tpa[2] + -amassj * alpha * R2 * K.K3;
-            alpha = (pi * (rhoj / rhoi + 1.0) + pj * (rhoi / rhoj - 1.0)) / (rhoi * rhoj);
-            ale[0] = ale[0] - amassj * alpha * R0 * K.K3;
-            ale[1] = ale[1] - amassj * alpha * R1 * K.K3;
-            ale[2] = ale[2] - amassj * alpha * R2 * K.K3;
-            const double vrij = -dv0 * R0 - dv1 * R1 - dv2 * R2;
-            const double TermMon = P.alfamon * celt * h / (rhoi + rhoj);
-            td[0] = td[0] + (amassj * TermMon * vrij * R0 * K.K2 + 0.0);
-            td[1] = td[1] + (amassj * TermMon * vrij * R1 * K.K2 + 0.0);
-            td[2] = td[2] + (amassj * TermMon * vrij * R2 * K.K2 + 0.0);
-            if (morris) {
-                const double rtil = nui * rhoi + nuj * rhoj + 1.0e-3;
-                const double atil = 4.0 * (nui * nuj);
-                const double fac = amassj * atil / rtil;
-                const double rr = R0 * R0 + R1 * R1 + R2 * R2;
-                const double w0 = fac * (-dv0 * K.K2 * rr);
-                const double w1 = fac * (-dv1 * K.K2 * rr);
-                const double w2 = fac * (-dv2 * K.K2 * rr);
-                tv[0] = tv[0] + w0; tv[1] = tv[1] + w1; tv[2] = tv[2] + w2;
-                rvs[0] = rvs[0] + w0; rvs[1] = rvs[1] + w1; rvs[2] = rvs[2] + w2;
+    double4* __restrict__ acc_out, double4* __restrict__ vel_out, const double* scal0, int* iscal0) {
+    __shared__ double2 sA[CAP], sB[CAP], sC[CAP], sD[CAP];  // (x, y), (z, vx), (vy, vz), (rho, p)
+    const int g = threadIdx.x % G;
+    for_tiles<SG, G, 3>(S, T, start,
+        [&](DPC&, int, int j, int slot) {
+            const double4 x = xm[j], v = vel[j];
+            sA[slot] = make_double2(x.x, x.y);
+            sB[slot] = make_double2(x.z, v.x);
+            sC[slot] = make_double2(v.y, v.z);
+            sD[slot] = rp[j];
+        },
+        [&](DPC& P, int sg, int i, int slot, bool fits) {
+            const double* scal = scal0 + sg * SC_COUNT;
+            const double h = P.h;
+            const double4 vi = vel[i];  // var == vel here
+            const double2 rpi = rp[i];
+            double tp[3] = {0.0, 0.0, 0.0};
+            // sums: td, tv (from the wall terms on), rvs, tpa, ale
+            double s[15];
+            for (int c = 0; c < 15; ++c) s[c] = 0.0;
+            const int ncbf = P.semi ? bn[i] : 0;
+            const double v_i[3] = {vi.x, vi.y, vi.z};
+            if (ncbf > 0) {
+                double td[3] = {0.0, 0.0, 0.0}, tv[3] = {0.0, 0.0, 0.0};
+                if (P.dim == 2)
+                    sa_momentum_2d(P, faces, bt, i, ncbf, v_i, rpi, lam_in[i], tp, td, tv);
+                else
+                    sa_momentum(P, faces, bt, i, ncbf, v_i, rpi, lam_in[i], tp, td, tv, iscal0 + sg * IS_COUNT);
+                for (int c = 0; c < 3; ++c) {
+                    s[c] = td[c];
+                    s[3 + c] = tv[c];
+                }
             }
-        });
-        for (int d = 0; d < 3; ++d) tp[d] = tp[d] + tpa[d] + ale[d];
-        double br[3] = {0.0, 0.0, 0.0};
-        if (ncbf > 0) elastic_walls(P, faces, edges, bt, xm, i, ncbf, vi, br);
-        momentum_end(P, i, ncbf, vi, dtvel, tp, td, tv, rvs, br, lam_out, acc_out, vel_out);
-    }
+            const double4 xi = xm[i];
+            const double rhoi = rpi.x, pi = rpi.y;
+            const double celt = P.celerita + P.celerita;
+            const double nui = P.kin_visc, nuj = P.kin_visc;
+            const bool morris = nui > 1.0e-12 && nuj > 1.0e-12;
+            const d2 invi = inv64(d2(rhoi));
+            pair_sums64<G, 15>(nbr, (size_t)P.cap, i, nnb[i], g, fits, (uint32_t)slot << 4, s,
+                [&](uint32_t o) {
+                    const double2 a = lds16(sA, o), b = lds16(sB, o), c = lds16(sC, o), d = lds16(sD, o);
+                    return Nb{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y, 0.0, xi.w};
+                },
+                [&](int j) {
+                    const double4 x = xm[j], v = vel[j];
+                    const double2 q = rp[j];
+                    return Nb{x.x, x.y, x.z, v.x, v.y, v.z, q.x, q.y, 0.0, x.w};
+                },
+                [&](d2 (&t)[15], const Nb& a, const Nb& b, bool, bool) {
+                    const d2 R0 = xi.x - d2{a.x, b.x}, R1 = xi.y - d2{a.y, b.y}, R2 = xi.z - d2{a.z, b.z};
+                    const d2 rij = R0 * R0 + R1 * R1 + R2 * R2;
+                    const K64x2 K = kvals64x2(P, rij, true, true, false);
+                    const d2 dv0 = d2{a.u, b.u} - vi.x, dv1 = d2{a.v, b.v} - vi.y, dv2 = d2{a.w, b.w} - vi.z;
+                    const d2 rhoj = {a.rho, b.rho}, pj = {a.p, b.p}, amassj = {a.m, b.m};
+                    const d2 rr = rhoi * rhoj;
+                    const d2 inv = inv64(rr), invj = newton64(rhoj, inv * rhoi);
+                    d2 alpha = div64(pj - pi, rr, inv);
+                    t[9] = -amassj * alpha * R0 * K.K3;
+                    t[10] = -amassj * alpha * R1 * K.K3;
+                    t[11] = -amassj * alpha * R2 * K.K3;
+                    alpha = div64(pi * (div64(rhoj, d2(rhoi), invi) + 1.0) + pj * (div64(d2(rhoi), rhoj, invj) - 1.0), rr,
+                                  inv);
+                    t[12] = -(amassj * alpha * R0 * K.K3);
+                    t[13] = -(amassj * alpha * R1 * K.K3);
+                    t[14] = -(amassj * alpha * R2 * K.K3);
+                    const d2 vrij = -dv0 * R0 - dv1 * R1 - dv2 * R2;
+                    const d2 rsum = rhoi + rhoj;
+                    const d2 TermMon = div64(d2(P.alfamon * celt * h), rsum, inv64(rsum));
+                    t[0] = amassj * TermMon * vrij * R0 * K.K2;
+                    t[1] = amassj * TermMon * vrij * R1 * K.K2;
+                    t[2] = amassj * TermMon * vrij * R2 * K.K2;
+                    // no branch: the compiler would keep the entries' values across it
+                    const d2 rtil = nui * rhoi + nuj * rhoj + 1.0e-3;
+                    const double atil = 4.0 * (nui * nuj);
+                    const d2 visc = div64(amassj * atil, rtil, inv64(rtil));
+                    const d2 fac = {morris ? visc.x : 0.0, morris ? visc.y : 0.0};
+                    t[3] = t[6] = fac * (-dv0 * K.K2 * rij);
+                    t[4] = t[7] = fac * (-dv1 * K.K2 * rij);
+                    t[5] = t[8] = fac * (-dv2 * K.K2 * rij);
+                });
+            if (g) return;
+            for (int d = 0; d < 3; ++d) tp[d] = tp[d] + s[9 + d] + s[12 + d];
+            double br[3] = {0.0, 0.0, 0.0};
+            if (ncbf > 0) elastic_walls(P, faces, edges, bt, xm, i, ncbf, vi, br);
+            // Leapfrog_momentum.f90:66-86 integrates with dtvel; the explicit RK1
+            // branch (Euler.f90:85-93) with dt
+            momentum_end(P, i, ncbf, vi, P.rk1 ? scal[SC_DT] : scal[SC_DTVEL], tp, s, s + 3, s + 6, br, lam_out,
+                         acc_out, vel_out);
+        },
+        [](DPC&, int) {});
 }
 
 // velocity smoothing: velocity_smoothing.f90:74-133
-template <bool SG>
-__global__ __launch_bounds__(256) void k_vsmooth64(
-    Seg S, const DFace* __restrict__ faces,
-    const int* __restrict__ bn, const BTab* __restrict__ bt, const double4* __restrict__ xm,
-    const double4* __restrict__ vel1, const double2* __restrict__ rp, const uint32_t* __restrict__ nbr,
-    const int* __restrict__ nnb, double4* __restrict__ vel_out, double4* __restrict__ xm_out,
-    const double* scal, unsigned long long* dtmin, int* iscal, const double* __restrict__ dden_in,
-    double2* __restrict__ rp_out, int* __restrict__ gone) {
-    const int vb = xcd_block(gridDim.x);
-    const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * (int)blockDim.x) >> 8]) : 0;
-    DPC& P = S.P[sg];
-    scal += sg * SC_COUNT;
-    iscal += sg * IS_COUNT;
-    const bool eos = iscal[IS_ONGOING] > 0;
-    dtmin += sg;
-    const size_t N = P.cap;
-    const bool smooth = P.tetav > 1.0e-9;
+template <int CAP, bool SG, int G>
+__global__ __launch_bounds__(TILE_WG, 2) void k_vsmooth64(
+    TILE_ARGS, const DFace* __restrict__ faces, const int* __restrict__ bn, const BTab* __restrict__ bt,
+    const double4* __restrict__ xm, const double4* __restrict__ vel1, const double2* __restrict__ rp,
+    const uint32_t* __restrict__ nbr, const int* __restrict__ nnb, double4* __restrict__ vel_out,
+    double4* __restrict__ xm_out, const double* scal0, unsigned long long* dtmin, const int* iscal0,
+    const double* __restrict__ dden_in, double2* __restrict__ rp_out, int* __restrict__ gone) {
+    __shared__ double2 sA[CAP], sB[CAP], sC[CAP], sD[CAP];  // (x, y), (z, vx), (vy, vz), (rho, 1 / rho)
+    const int g = threadIdx.x % G;
     unsigned long long dtbits = 0x7FF0000000000000ull;
-    const int i = vb * blockDim.x + threadIdx.x;
-    if (i - P.base < iscal[IS_N]) {
-        const double4 xi = xm[i];
-        const double4 vi = vel1[i];
-        double v[3] = {0.0, 0.0, 0.0};
-        if (smooth) {
-            const int nn = nnb[i];
-            using RV = NRec<double4, double4, double>;
-            auto fetch = [&](uint32_t e) {
-                const int j = (int)(e & NB_MASK);
-                    return RV{xm[j], vel1[j], rp[j].x};
-            };
-            walk_list<4, RV>(nbr, N, i, nn, fetch, [&](uint32_t e, const RV& q) {
-                const double4 xj = q.x;
-                const double4 vj = q.v;
-                const double rhoj = q.r;
-                const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
-                const double rij = R0 * R0 + R1 * R1 + R2 * R2;
-                K64 K;
-                kvals64(P, rij, false, false, true, K);
-                const double pes = xj.w * K.W / rhoj;
-                v[0] = v[0] + (vj.x - vi.x) * pes;
-                v[1] = v[1] + (vj.y - vi.y) * pes;
-                v[2] = v[2] + (vj.z - vi.z) * pes;
-                                });
-            vsmooth_walls(P, faces, bt, i, P.semi ? bn[i] : 0, vi, v);
-        }
-        dtbits = vsmooth_end<false>(P, faces, i, xi, vi, v, smooth, scal[SC_TV1], scal[SC_DT], eos, dden_in, rp,
-                             vel_out, xm_out, rp_out, nullptr, gone);
-    }
-    block_min_to(dtbits, dtmin);
+    for_tiles<SG, G, 3>(S, T, start,
+        [&](DPC& P, int, int j, int slot) {
+            if (!(P.tetav > 1.0e-9)) return;
+            const double4 x = xm[j], v = vel1[j];
+            sA[slot] = make_double2(x.x, x.y);
+            sB[slot] = make_double2(x.z, v.x);
+            sC[slot] = make_double2(v.y, v.z);
+            const double rho = rp[j].x;
+            sD[slot] = make_double2(rho, 1.0 / rho);
+        },
+        [&](DPC& P, int sg, int i, int slot, bool fits) {
+            const double* scal = scal0 + sg * SC_COUNT;
+            const bool smooth = P.tetav > 1.0e-9;
+            const double4 xi = xm[i];
+            const double4 vi = vel1[i];
+            double v[3] = {0.0, 0.0, 0.0};
+            if (smooth) {
+                pair_sums64<G, 3>(nbr, (size_t)P.cap, i, nnb[i], g, fits, (uint32_t)slot << 4, v,
+                    [&](uint32_t o) {
+                        const double2 a = lds16(sA, o), b = lds16(sB, o), c = lds16(sC, o), d = lds16(sD, o);
+                        return Nb{a.x, a.y, b.x, b.y, c.x, c.y, d.x, 0.0, d.y, xi.w};
+                    },
+                    [&](int j) {
+                        const double4 x = xm[j], u = vel1[j];
+                        const double rho = rp[j].x;
+                        return Nb{x.x, x.y, x.z, u.x, u.y, u.z, rho, 0.0, 1.0 / rho, x.w};
+                    },
+                    [&](d2 (&t)[3], const Nb& a, const Nb& b, bool, bool) {
+                        const d2 R0 = xi.x - d2{a.x, b.x}, R1 = xi.y - d2{a.y, b.y}, R2 = xi.z - d2{a.z, b.z};
+                        const K64x2 K = kvals64x2(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true);
+                        const d2 pes = div64(d2{a.m, b.m} * K.W, d2{a.rho, b.rho}, d2{a.inv, b.inv});
+                        t[0] = (d2{a.u, b.u} - vi.x) * pes;
+                        t[1] = (d2{a.v, b.v} - vi.y) * pes;
+                        t[2] = (d2{a.w, b.w} - vi.z) * pes;
+                    });
+            }
+            if (g) return;
+            if (smooth) vsmooth_walls(P, faces, bt, i, P.semi ? bn[i] : 0, vi, v);
+            const unsigned long long b =
+                vsmooth_end<false>(P, faces, i, xi, vi, v, smooth, scal[SC_TV1], scal[SC_DT],
+                                   iscal0[sg * IS_COUNT + IS_ONGOING] > 0, dden_in, rp, vel_out, xm_out, rp_out,
+                                   nullptr, gone);
+            dtbits = b < dtbits ? b : dtbits;
+        },
+        [&](DPC&, int sg) { wave_min_to(dtbits, dtmin + sg); });
 }
 
 // continuity: SASPH_continuity.f90:89-169, Continuity_Equation.f90:97-235
-template <bool SG>
-__global__ __launch_bounds__(256) void k_continuity64(
-    Seg S, const DFace* __restrict__ faces,
-    const int* __restrict__ bn, const BTab* __restrict__ bt, const double4* __restrict__ xm,
-    const double4* __restrict__ vel, const double2* __restrict__ rp, const uint32_t* __restrict__ nbr,
-    const int* __restrict__ nnb, double* __restrict__ dden_out, double2* __restrict__ rp_out,
-    const double* scal, int* iscal) {
-    const int vb = xcd_block(gridDim.x);
-    const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * (int)blockDim.x) >> 8]) : 0;
-    DPC& P = S.P[sg];
-    scal += sg * SC_COUNT;
-    iscal += sg * IS_COUNT;
-    const size_t N = P.cap;
-    const int i = vb * blockDim.x + threadIdx.x;
-    if (i - P.base < iscal[IS_N]) {
-        const double4 vi = vel[i];
-        const double2 rpi = rp[i];
-        const double rhoi = rpi.x;
-        const double dd = continuity_walls(P, faces, bt, i, P.semi ? bn[i] : 0, vi, rhoi, iscal);
-        const int nn = nnb[i];
-        const double4 xi = xm[i];
-        double a1 = 0.0, a2 = 0.0, a3 = 0.0;
-        using RC = NRec<double4, double4, double>;
-        auto fetch = [&](uint32_t e) {
-            const int j = (int)(e & NB_MASK);
-            return RC{xm[j], vel[j], rp[j].x};
-        };
-        walk_list<4, RC>(nbr, N, i, nn, fetch, [&](uint32_t e, const RC& q) {
-            const double4 xj = q.x;
-            const double4 vj = q.v;
-            const double rhoj = q.r;
-            const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
-            const double rij = R0 * R0 + R1 * R1 + R2 * R2;
-            K64 K;
-            kvals64(P, rij, true, false, false, K);
-            const double amassj = xj.w;
-            a1 = a1 + rhoi * (amassj / rhoj) * K.K1 * (vj.x - vi.x) * R0;
-            a2 = a2 + rhoi * (amassj / rhoj) * K.K1 * (vj.y - vi.y) * R1;
-            a3 = a3 + rhoi * (amassj / rhoj) * K.K1 * (vj.z - vi.z) * R2;
-                        });
-        const double inner = a1 + a2 + a3;
-        continuity_end(P, i, rpi, dd - inner, scal[SC_DT], iscal[IS_ONGOING] > 0, dden_out, rp_out, nullptr);
-    }
+template <int CAP, bool SG, int G>
+__global__ __launch_bounds__(TILE_WG, 2) void k_continuity64(
+    TILE_ARGS, const DFace* __restrict__ faces, const int* __restrict__ bn, const BTab* __restrict__ bt,
+    const double4* __restrict__ xm, const double4* __restrict__ vel, const double2* __restrict__ rp,
+    const uint32_t* __restrict__ nbr, const int* __restrict__ nnb, double* __restrict__ dden_out,
+    double2* __restrict__ rp_out, const double* scal0, int* iscal0) {
+    __shared__ double2 sA[CAP], sB[CAP], sC[CAP];  // (x, y), (z, vx), (vy, vz)
+    __shared__ double sD[CAP];                     // m / rho
+    const int g = threadIdx.x % G;
+    for_tiles<SG, G, 3>(S, T, start,
+        [&](DPC&, int, int j, int slot) {
+            const double4 x = xm[j], v = vel[j];
+            sA[slot] = make_double2(x.x, x.y);
+            sB[slot] = make_double2(x.z, v.x);
+            sC[slot] = make_double2(v.y, v.z);
+            sD[slot] = x.w / rp[j].x;
+        },
+        [&](DPC& P, int sg, int i, int slot, bool fits) {
+            const double4 xi = xm[i];
+            const double4 vi = vel[i];
+            const double2 rpi = rp[i];
+            const double rhoi = rpi.x;
+            double s[3] = {0.0, 0.0, 0.0};
+            pair_sums64<G, 3>(nbr, (size_t)P.cap, i, nnb[i], g, fits, (uint32_t)slot << 4, s,
+                [&](uint32_t o) {
+                    const double2 a = lds16(sA, o), b = lds16(sB, o), c = lds16(sC, o);
+                    return Nb{a.x, a.y, b.x, b.y, c.x, c.y, 0.0, 0.0, 0.0, lds8(sD, o)};
+                },
+                [&](int j) {
+                    const double4 x = xm[j], v = vel[j];
+                    return Nb{x.x, x.y, x.z, v.x, v.y, v.z, 0.0, 0.0, 0.0, x.w / rp[j].x};
+                },
+                [&](d2 (&t)[3], const Nb& a, const Nb& b, bool, bool) {  // m: the neighbour's volume
+                    const d2 R0 = xi.x - d2{a.x, b.x}, R1 = xi.y - d2{a.y, b.y}, R2 = xi.z - d2{a.z, b.z};
+                    const K64x2 K = kvals64x2(P, R0 * R0 + R1 * R1 + R2 * R2, true, false, false);
+                    const d2 f = rhoi * d2{a.m, b.m} * K.K1;
+                    t[0] = f * (d2{a.u, b.u} - vi.x) * R0;
+                    t[1] = f * (d2{a.v, b.v} - vi.y) * R1;
+                    t[2] = f * (d2{a.w, b.w} - vi.z) * R2;
+                });
+            if (g) return;
+            int* iscal = iscal0 + sg * IS_COUNT;
+            const double dd = continuity_walls(P, faces, bt, i, P.semi ? bn[i] : 0, vi, rhoi, iscal);
+            const double inner = s[0] + s[1] + s[2];
+            continuity_end(P, i, rpi, dd - inner, scal0[sg * SC_COUNT + SC_DT], iscal[IS_ONGOING] > 0, dden_out,
+                           rp_out, nullptr);
+        },
+        [](DPC&, int) {});
 }
 
 // pressure smoothing: PressureSmoothing_3D.f90:80-161 (both loops)
-template <bool SG>
-__global__ __launch_bounds__(256) void k_psmooth64(
-    Seg S, const DFace* __restrict__ faces, const int* __restrict__ bn, const BTab* __restrict__ bt,
+template <int CAP, bool SG, int G>
+__global__ __launch_bounds__(TILE_WG, 2) void k_psmooth64(
+    TILE_ARGS, const DFace* __restrict__ faces, const int* __restrict__ bn, const BTab* __restrict__ bt,
     const double4* __restrict__ xm, const double2* __restrict__ rp, const uint32_t* __restrict__ nbr,
     const int* __restrict__ nnb, double* __restrict__ vpres_out, double2* __restrict__ rp_out,
-    const double* scal, const int* iscal) {
-    const int vb = xcd_block(gridDim.x);
-    const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * (int)blockDim.x) >> 8]) : 0;
-    DPC& P = S.P[sg];
-    scal += sg * SC_COUNT;
-    iscal += sg * IS_COUNT;
-    const size_t N = P.cap;
-    const int i = vb * blockDim.x + threadIdx.x;
-    if (i - P.base < iscal[IS_N]) {
-        const double2 rpi = rp[i];
-        const int nsp = nnb[i];
-        const double pi = rpi.y;
-        double somp = 0.0, app = 0.0;
-        if (nsp > 0) {
+    const double* scal0) {
+    __shared__ double2 sA[CAP], sB[CAP], sC[CAP];  // (x, y), (z, p), (rho, 1 / rho)
+    const int g = threadIdx.x % G;
+    for_tiles<SG, G, 3>(S, T, start,
+        [&](DPC&, int, int j, int slot) {
+            const double4 x = xm[j];
+            const double2 q = rp[j];
+            sA[slot] = make_double2(x.x, x.y);
+            sB[slot] = make_double2(x.z, q.y);
+            sC[slot] = make_double2(q.x, 1.0 / q.x);
+        },
+        [&](DPC& P, int sg, int i, int slot, bool fits) {
             const double4 xi = xm[i];
-            somp = 0.0;
-            app = 0.0;
-            using RP2 = NRec2<double4, double2>;
-            auto fetch = [&](uint32_t e) {
-                const int j = (int)(e & NB_MASK);
-                    return RP2{xm[j], rp[j]};
-            };
-            walk_list<4, RP2>(nbr, N, i, nsp, fetch, [&](uint32_t e, const RP2& q) {
-                const double4 xj = q.x;
-                const double2 rpj = q.r;
-                const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
-                K64 K;
-                kvals64(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true, K);
-                const double pes = xj.w * K.W / rpj.x;
-                app = app + pes;
-                somp = somp + (rpj.y - pi) * pes;
-                                });
-        }
-        psmooth_end(P, faces, bn, bt, i, nsp, rpi, scal[SC_TP1], somp, app, vpres_out, rp_out);
-    }
+            const double2 rpi = rp[i];
+            const int nsp = nnb[i];
+            const double pi = rpi.y;
+            double s[2] = {0.0, 0.0};
+            pair_sums64<G, 2>(nbr, (size_t)P.cap, i, nsp, g, fits, (uint32_t)slot << 4, s,
+                [&](uint32_t o) {
+                    const double2 a = lds16(sA, o), b = lds16(sB, o), c = lds16(sC, o);
+                    return Nb{a.x, a.y, b.x, 0.0, 0.0, 0.0, c.x, b.y, c.y, xi.w};
+                },
+                [&](int j) {
+                    const double4 x = xm[j];
+                    const double2 q = rp[j];
+                    return Nb{x.x, x.y, x.z, 0.0, 0.0, 0.0, q.x, q.y, 1.0 / q.x, x.w};
+                },
+                [&](d2 (&t)[2], const Nb& a, const Nb& b, bool ona, bool onb) {
+                    const d2 R0 = xi.x - d2{a.x, b.x}, R1 = xi.y - d2{a.y, b.y}, R2 = xi.z - d2{a.z, b.z};
+                    const K64x2 K = kvals64x2(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true);
+                    const d2 pes = div64(d2{a.m, b.m} * K.W, d2{a.rho, b.rho}, d2{a.inv, b.inv});
+                    t[0] = d2{ona ? pes.x : 0.0, onb ? pes.y : 0.0};
+                    t[1] = (d2{a.p, b.p} - pi) * pes;
+                });
+            if (g) return;
+            psmooth_end(P, faces, bn, bt, i, nsp, rpi, scal0[sg * SC_COUNT + SC_TP1], s[1], s[0], vpres_out, rp_out);
+        },
+        [](DPC&, int) {});
 }
 
 // ----------------------------------------------------------------------------
@@ -2927,8 +3137,6 @@ __device__ __forceinline__ void pair_sums(const uint32_t* __restrict__ nbr, size
         for (int c = 0; c < NS; ++c) sum[c] += __shfl_xor(sum[c], 1, 64);
 }
 
-#define TILE_ARGS Seg S, Tiles T, const int* __restrict__ start
-
 // momentum; UM: every particle of the context has its solve's mass
 template <int CAP, bool SG, int G, bool UM>
 __global__ __launch_bounds__(TILE_WG, 4) void k_momentum(
@@ -2948,14 +3156,14 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_momentum(
     auto rec_b = [](int4 x, float4 v) {
         return make_float4(v.x, v.y, v.z, UM ? v.w : __int_as_float(x.w));
     };
-    for_tiles<SG, G>(S, T, start,
+    for_tiles<SG, G, TILE_U>(S, T, start,
         [&](DPC& P, int, int j, int slot) {
             const int4 x = xq[j];
             const float4 v = vf[j];
             sA[slot] = rec_a(P, x, v);
             sB[slot] = rec_b(x, v);
         },
-        [&](DPC& P, int sg, int i, bool fits) {
+        [&](DPC& P, int sg, int i, int, bool fits) {
             const double* scal = scal0 + sg * SC_COUNT;
             const int4 xi = xq[i];
             const float4 vf_i = vf[i];
@@ -3046,14 +3254,14 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_vsmooth(
         return bits4(x, __int_as_float(x.w) * __builtin_amdgcn_rcpf(P.f_den0 + v.w));
     };
     unsigned long long dtbits = 0x7FF0000000000000ull;
-    for_tiles<SG, G>(S, T, start,
+    for_tiles<SG, G, TILE_U>(S, T, start,
         [&](DPC& P, int, int j, int slot) {
             if (!(P.tetav > 1.0e-9)) return;
             const float4 v = vf[j];
             sA[slot] = rec_a(P, xq[j], v);
             sB[slot] = v;
         },
-        [&](DPC& P, int sg, int i, bool fits) {
+        [&](DPC& P, int sg, int i, int, bool fits) {
             const double* scal = scal0 + sg * SC_COUNT;
             const bool smooth = P.tetav > 1.0e-9;
             double v[3] = {0.0, 0.0, 0.0};
@@ -3091,16 +3299,7 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_vsmooth(
                             dr_out, gone);
             dtbits = b < dtbits ? b : dtbits;
         },
-        [&](DPC&, int sg) {
-            for (int o = 32; o > 0; o >>= 1) {
-                const unsigned long long t = __shfl_xor(dtbits, o, 64);
-                dtbits = t < dtbits ? t : dtbits;
-            }
-            // the minimum only falls: a value read before is an upper bound of it
-            if ((threadIdx.x & 63) == 0 && dtbits < *(volatile unsigned long long*)(dtmin + sg))
-                atomicMin(dtmin + sg, dtbits);
-            dtbits = 0x7FF0000000000000ull;
-        });
+        [&](DPC&, int sg) { wave_min_to(dtbits, dtmin + sg); });
 }
 
 // continuity
@@ -3115,13 +3314,13 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_continuity(
     auto rec_a = [](DPC& P, int4 x, float4 v) {
         return bits4(x, __int_as_float(x.w) * __builtin_amdgcn_rcpf(P.f_den0 + v.w));
     };
-    for_tiles<SG, G>(S, T, start,
+    for_tiles<SG, G, TILE_U>(S, T, start,
         [&](DPC& P, int, int j, int slot) {
             const float4 v = vf[j];
             sA[slot] = rec_a(P, xq[j], v);
             sB[slot] = v;
         },
-        [&](DPC& P, int sg, int i, bool fits) {
+        [&](DPC& P, int sg, int i, int, bool fits) {
             const int4 xi = xq[i];
             const float4 vi = vf[i];
             auto pair = [&](float* s, float4 A, float4 B) {
@@ -3161,13 +3360,13 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_psmooth(
     auto rec_a = [](DPC& P, int4 x, float d) {
         return bits4(x, __int_as_float(x.w) * __builtin_amdgcn_rcpf(P.f_den0 + d));
     };
-    for_tiles<SG, G>(S, T, start,
+    for_tiles<SG, G, TILE_U>(S, T, start,
         [&](DPC& P, int, int j, int slot) {
             const float d = dr[j];
             sA[slot] = rec_a(P, xq[j], d);
             sD[slot] = d;
         },
-        [&](DPC& P, int sg, int i, bool fits) {
+        [&](DPC& P, int sg, int i, int, bool fits) {
             const int4 xi = xq[i];
             const float di = dr[i];
             const int nn = nnb[i];
