@@ -290,9 +290,15 @@ void tile_dispatch(sph_ctx* c, Launch&& launch) {
     if (c->nseg > 1) form(std::true_type{});
     else form(std::false_type{});
 }
-// The FP64 passes; TILE_CAP_0 has no LDS form (lists with stencil codes).
+// The FP64 passes.  TILE_CAP_0 (lists with stencil codes): no LDS form, lanes
+// by particles.
 template <class Launch>
 void tile_dispatch64(sph_ctx* c, Launch&& launch) {
+    if (c->tile_cap == TILE_CAP_0) {
+        if (c->tile_g == 4) launch(IntC<TILE_CAP_0>{}, std::false_type{}, IntC<4>{});
+        else launch(IntC<TILE_CAP_0>{}, std::false_type{}, IntC<8>{});
+        return;
+    }
     auto lanes = [&](auto cap, auto sg) {
         if (c->tile_g == 1) launch(cap, sg, IntC<1>{});
         else if (c->tile_g == 2) launch(cap, sg, IntC<2>{});
@@ -300,8 +306,7 @@ void tile_dispatch64(sph_ctx* c, Launch&& launch) {
     };
     auto form = [&](auto sg) {
         if (c->tile_cap == TILE_CAP_L) lanes(IntC<TILE_CAP_L>{}, sg);
-        else if (c->tile_cap == TILE_CAP_S) lanes(IntC<TILE_CAP_S>{}, sg);
-        else lanes(IntC<TILE_CAP_0>{}, sg);
+        else lanes(IntC<TILE_CAP_S>{}, sg);
     };
     if (c->nseg > 1) form(std::true_type{});
     else form(std::false_type{});
@@ -388,30 +393,42 @@ DWall dwall(const sph_ctx* c) { return DWall{c->d_w0, c->d_w1, c->d_w2, c->d_wst
 int run_dbsph_lists(sph_ctx* c, int mode) {
     KTime t(c, "dbsph_lists");
     const int cap = c->P.cap;
+    // a block of 256 threads, or of one wavefront where its LDS would not fit
+    const size_t each = (size_t)(db_words(c->P.nmaxpartj, cap) + DB_INTS) * 4;
+    const int wg = each * (256 / DB_G) <= 65536 ? 256 : 64;
+    const size_t lds = each * (wg / DB_G);
     if (mode == 0)
-        k_dbsph_lists<0><<<nblk(DB_G * cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->cell,
+        k_dbsph_lists<0><<<nblk(DB_G * cap, wg), wg, lds, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->cell,
                                                            c->nbr, c->nnb, c->gam[0], c->dsh[0], c->gam[0], c->dsh[0],
                                                            c->sig, c->rsph, c->fsf, c->nfw, c->fwl, c->d_wwet,
                                                            c->dden2, c->rp[2], c->scal, c->iscal);
     else if (mode == 1)
-        k_dbsph_lists<1><<<nblk(DB_G * cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->cell,
+        k_dbsph_lists<1><<<nblk(DB_G * cap, wg), wg, lds, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->cell,
                                                            c->nbr, c->nnb, c->gam[0], c->dsh[0], c->gam[0], c->dsh[0],
                                                            c->sig, c->rsph, c->fsf, c->nfw, c->fwl, c->d_wwet,
                                                            c->dden2, c->rp[2], c->scal, c->iscal);
     else
-        k_dbsph_lists<2><<<nblk(DB_G * cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[1], c->cell,
+        k_dbsph_lists<2><<<nblk(DB_G * cap, wg), wg, lds, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[1], c->cell,
                                                            c->nbr, c->nnb, c->gam[1], c->dsh[1], c->gam[0], c->dsh[0],
                                                            c->sig, c->rsph, c->fsf, c->nfw, c->fwl, c->d_wwet,
                                                            c->dden2, c->rp[2], c->scal, c->iscal);
     return 0;
 }
 
+template <class Launch>
+void dbsph_lanes(sph_ctx* c, Launch&& launch) {
+    if (c->tile_g == 4) launch(IntC<4>{});
+    else launch(IntC<8>{});
+}
+
 int run_momentum_dbsph(sph_ctx* c) {
     KTime t(c, "momentum");
-    k_momentum_dbsph<<<nblk(DB_G * c->P.cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->nbr,
+    dbsph_lanes(c, [&](auto g) {
+    k_momentum_dbsph<g.value><<<nblk(g.value * c->P.cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->nbr,
                                                             c->nnb, c->nfw, c->fwl, c->gam[0], c->d_wdens,
                                                             c->d_wpres, c->lam[0], c->acc[1], c->vel[1], c->scal,
                                                             c->iscal);
+    });
     return 0;
 }
 
@@ -433,9 +450,11 @@ int run_dbsph_kinematics(sph_ctx* c) {
 // Gradients_to_MUSCL and BC_wall_elements on the step's final state
 int run_dbsph_walls(sph_ctx* c) {
     KTime t(c, "dbsph_walls");
-    k_dbsph_muscl<<<nblk(c->P.cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->nbr,
+    dbsph_lanes(c, [&](auto g) {
+    k_dbsph_muscl<g.value><<<nblk(g.value * c->P.cap), 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->nbr,
                                                          c->nnb, c->nfw, c->fwl, c->sig, c->d_wdens, c->drho,
                                                          c->dvelg, c->iscal);
+    });
     k_dbsph_walls<<<(c->P.nw + DB_WPB - 1) / DB_WPB, 256, 0, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->start,
                                                         c->drho, c->dvelg, c->d_wdens, c->d_wpres, c->iscal);
     return 0;
@@ -1251,6 +1270,9 @@ int sph_dbsph_walls(sph_ctx* c, const sph_dbsph_walls_t* w) {
     P.muscl_bnd = w->muscl_boundary ? 1 : 0;
     P.tcap = 0;  // the DB-SPH kernels read the lists' stencil codes
     c->tile_cap = TILE_CAP_0;
+    c->tile_g = P.cap < TILE_G8 ? 8 : 4;
+    c->tile_wg = 256;
+    c->tile_grid = nblk((long long)P.cap * c->tile_g);
     return upload_constants(c);
 }
 

@@ -25,7 +25,21 @@ namespace sph {
 
 constexpr int SPH_MW = 128;   // fluid-wall list capacity per particle
 constexpr int SPH_WF = 128;   // fluid neighbours a wall element gathers
-constexpr int DB_G = 4;       // lanes per particle in k_dbsph_lists
+constexpr int DB_G = 8;       // lanes per particle in k_dbsph_lists
+
+// k_dbsph_lists's LDS of a particle: a bit for every place of the merged
+// sequence, and DB_INTS words
+constexpr int DB_INTS = 3 * 28 + SPH_MW;
+__host__ __device__ __forceinline__ int db_words(int nmaxpartj, int cap) {
+    return ((nmaxpartj < cap ? nmaxpartj : cap) + SPH_MW + 2 * DB_G) / 32 + 1;
+}
+
+// LDS written by one lane of a wavefront is read by another
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // wall-element tables: w0 = (x, y, z, weight), w1 = (normal, volume),
 // w2 = (velocity, mass)
@@ -43,10 +57,14 @@ struct DWall {
 // or 1 without wall neighbours); 1: its second call (Gamma kept, FS set);
 // 2: inside Euler after OrdGrid1 (Gamma += dShep dt before the sums, then
 // dden / Gamma and the density and pressure of the particle)
-// The fluid sums walk the particle's neighbour list, whose entries carry the
-// stencil code (dx+1) + 3(dy+1) + 9(dz+1) of their cell and come in the
-// reference's cell order (y, x, z nest; ascending pg index in a cell): each
-// cell's run of the list, then that cell's wall elements.
+// The sums take the cells in the reference's order (y, x, z nest): the fluid
+// neighbours of a cell (their list entries carry the stencil code (dx+1) +
+// 3(dy+1) + 9(dz+1) and come in this order, ascending pg index in a cell), then
+// its wall elements.  Bound by latency: walking the 27 cells one after the
+// other, each with its dependent loads, took 139 us at 2,000 particles and 191
+// at 70,000.  So DB_G lanes of a particle first find the wall elements of all
+// cells side by side and mark their places in the merged sequence, then run
+// through that sequence two places a lane at a time: 42 and 114 us.
 template <int MODE>
 __global__ __launch_bounds__(256) void k_dbsph_lists(
     DPC* Pp, DWall W, const double4* __restrict__ xm, const double4* __restrict__ vel,
@@ -57,12 +75,15 @@ __global__ __launch_bounds__(256) void k_dbsph_lists(
     int* __restrict__ fs_out, int* __restrict__ nfw, int* __restrict__ fwl, int* __restrict__ wwet,
     double* __restrict__ dden, double2* __restrict__ rp_out, const double* scal, int* iscal) {
     DPC& P = *Pp;
-    // DB_G lanes per particle: they take consecutive candidates of a cell
-    // (fluid-list entries, then wall elements) side by side, and every lane
-    // of the group adds the candidates' terms in candidate order, read from
-    // their lanes with shuffles, so the sums keep the serial order
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = t / DB_G, g = t % DB_G;
+    extern __shared__ uint32_t db_lds[];
+    const int np = blockDim.x / DB_G, words = db_words(P.nmaxpartj, P.cap);
+    const int q = threadIdx.x / DB_G, g = threadIdx.x % DB_G;
+    uint32_t* bm = db_lds + q * (words + DB_INTS);  // merged positions that are wall elements
+    int* wa = reinterpret_cast<int*>(bm + words);   // first wall element of cell t
+    int* pre = wa + 28;                             // wall elements of the cells before cell t
+    int* cnt = pre + 28;                            // fluid entries of the cells up to cell t
+    int* ids = cnt + 28;                            // the particle's wall elements
+    const int i = xcd_block(gridDim.x) * np + q;
     const int gb = (threadIdx.x & 63) & ~(DB_G - 1);  // the group's first lane
     const uint64_t gmask = (1ull << DB_G) - 1ull;
     if (i >= iscal[IS_N]) return;  // whole groups leave together
@@ -75,107 +96,132 @@ __global__ __launch_bounds__(256) void k_dbsph_lists(
     } else if (MODE == 1) {
         gamma = gam_in[i];
     }
-    double sigma = 0.0, rsph = 0.0, dshep = 0.0;
     int nf = 0;
     const int cap = SPH_MW < P.nmaxpartj ? SPH_MW : P.nmaxpartj;
     int ci, cj, ck;
     d_cell_indices(P, cell[i], ci, cj, ck);
     const size_t N = P.cap;
     const int nn = nnb[i];
-    int kl = 0;
-    for (int dy = -1; dy <= 1; ++dy)
-        for (int dx = -1; dx <= 1; ++dx)
-            for (int dz = -1; dz <= 1; ++dz) {
-                // the cell's fluid neighbours, then its wall elements
-                const uint32_t code = (uint32_t)((dx + 1) + 3 * (dy + 1) + 9 * (dz + 1));
-                for (;;) {
-                    const int k = kl + g;
-                    uint32_t e = NB_NONE;
-                    if (k < nn) e = nbr[nb_index(N, i, k)];
-                    const bool val = e != NB_NONE && (e >> NB_SHIFT) == code;
-                    double cs = 0.0, cr = 0.0;
-                    if (val) {
-                        const double4 xj = xm[e & NB_MASK];
-                        const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
-                        K64 K;
-                        kvals64(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true, K);
-                        cs = xj.w * K.W / rp[e & NB_MASK].x;
-                        cr = xj.w * K.W;
-                    }
-                    // the run of this code's entries is a prefix of the group
-                    const int cnt = __popcll((__ballot(val) >> gb) & gmask);
-#pragma unroll
-                    for (int u = 0; u < DB_G; ++u) {
-                        const double su = __shfl(cs, u, DB_G);
-                        const double ru = __shfl(cr, u, DB_G);
-                        if (u < cnt) {
-                            sigma = sigma + su;
-                            rsph = rsph + ru;
-                        }
-                    }
-                    kl += cnt;
-                    if (cnt < DB_G) break;
-                }
-                const int c = d_cell_number(P, ci + dx, cj + dy, ck + dz);
-                if (c == 0) continue;
-                const int wa = W.wstart[c - 1], wz = W.wstart[c];
-                for (int wb = wa; wb < wz; wb += DB_G) {
-                    const int w = wb + g;
-                    bool inr = false, add = false;
-                    int id = 0;
-                    double dv = 0.0, sv = 0.0, rv = 0.0;
-                    bool wet = false;
-                    if (w < wz) {
-                        const double4 a = W.wpos[w];
-                        const double R0 = xi.x - a.x, R1 = xi.y - a.y, R2 = xi.z - a.z;
-                        const double rij = R0 * R0 + R1 * R1 + R2 * R2;
-                        if (rij <= P.square_doubleh) {
-                            inr = true;
-                            id = (int)a.w;
-                            const double q = sqrt(rij) / P.h;
-                            const double q2 = rij / P.squareh;
-                            const int iq = (int)q;
-                            if (iq < 2) {
-                                add = true;
-                                const double aw = W.w0[id].w;
-                                const double4 b = W.w1[id];
-                                const double4 gv = W.w2[id];
-                                double wu = 0.666666667 + q2 * (q * 0.5 - 1.0);
-                                if (iq > 0) wu = (2.0 - q) * (2.0 - q) * (2.0 - q) * 0.166666666667;
-                                const double k1 = wu * P.coefke;
-                                dv = k1 * aw * (b.x * (gv.x - vi.x) + b.y * (gv.y - vi.y) + b.z * (gv.z - vi.z));
-                                wet = (q * P.h) <= (1.3 * P.dx + aw / 2.0);
-                                sv = b.w * k1;
-                                rv = gv.w * k1;
-                            }
-                        }
-                    }
-                    // in candidate order: the elements within 2h take the
-                    // next list slots while there are any left
-                    const uint64_t mk = (__ballot(inr) >> gb) & gmask;
-                    const int slot = nf + __popcll(mk & ((1ull << g) - 1ull));
-                    const bool listed = inr && slot < cap;
-                    if (inr && !listed) atomicAdd(&iscal[IS_DB_OVERFLOW], 1);
-                    if (listed) {
-                        fwl[(size_t)slot * P.cap + i] = id;
-                        if (add && wet) wwet[id] = 1;
-                    }
-                    nf = nf + __popcll(mk);
-                    if (nf > cap) nf = cap;
-                    const uint64_t ma = (__ballot(listed && add) >> gb) & gmask;
-#pragma unroll
-                    for (int u = 0; u < DB_G; ++u) {
-                        const double du = __shfl(dv, u, DB_G);
-                        const double su = __shfl(sv, u, DB_G);
-                        const double ru = __shfl(rv, u, DB_G);
-                        if ((ma >> u) & 1ull) {
-                            dshep = dshep + du;
-                            sigma = sigma + su;
-                            rsph = rsph + ru;
-                        }
-                    }
+    // the wall elements of the 27 cells, in the order of the nest
+    int mine = 0;
+    for (int t = g; t < 27; t += DB_G) {
+        const int c = d_cell_number(P, ci + (t / 3) % 3 - 1, cj + t / 9 - 1, ck + t % 3 - 1);
+        const int w0 = c ? W.wstart[c - 1] : 0, n = c ? W.wstart[c] - w0 : 0;
+        wa[t] = w0;
+        pre[t + 1] = n;
+        cnt[t] = 0;
+        mine += n;
+    }
+    if ((__ballot(mine > 0) >> gb) & gmask) {
+        for (int w = g; w < words; w += DB_G) bm[w] = 0;
+        wave_lds_sync();
+        for (int k = g; k < nn; k += DB_G) {  // code (dx+1) + 3(dy+1) + 9(dz+1) -> place in the nest
+            const int e = (int)(nbr[nb_index(N, i, k)] >> NB_SHIFT);
+            atomicAdd(&cnt[9 * (e / 3 % 3) + 3 * (e % 3) + e / 9], 1);
+        }
+        wave_lds_sync();
+        if (g == 0) {
+            int a = 0, b = 0;
+            pre[0] = 0;
+            for (int t = 0; t < 27; ++t) {
+                a += cnt[t];
+                cnt[t] = a;
+                b += pre[t + 1];
+                pre[t + 1] = b;
+            }
+        }
+        wave_lds_sync();
+        const int total = pre[27];
+        for (int w0 = 0; w0 < total; w0 += DB_G) {
+            const int w = w0 + g;
+            bool inr = false, wet = false;
+            int id = 0, t = 0;
+            if (w < total) {
+                for (int d = 16; d > 0; d >>= 1)
+                    if (t + d < 27 && pre[t + d] <= w) t += d;
+                const double4 a = W.wpos[wa[t] + w - pre[t]];
+                const double R0 = xi.x - a.x, R1 = xi.y - a.y, R2 = xi.z - a.z;
+                const double rij = R0 * R0 + R1 * R1 + R2 * R2;
+                if (rij <= P.square_doubleh) {
+                    inr = true;
+                    id = (int)a.w;
+                    const double qh = sqrt(rij) / P.h;
+                    wet = (int)qh < 2 && (qh * P.h) <= (1.3 * P.dx + W.w0[id].w / 2.0);
                 }
             }
+            // in candidate order: the elements within 2h take the next list
+            // slots while there are any left
+            const uint64_t mk = (__ballot(inr) >> gb) & gmask;
+            const int slot = nf + __popcll(mk & ((1ull << g) - 1ull));
+            if (inr && slot >= cap) atomicAdd(&iscal[IS_DB_OVERFLOW], 1);
+            if (inr && slot < cap) {
+                fwl[(size_t)slot * P.cap + i] = id;
+                if (wet) wwet[id] = 1;
+                ids[slot] = id;
+                const int pos = cnt[t] + slot;  // after the fluid entries of its cell
+                atomicOr(&bm[pos >> 5], 1u << (pos & 31));
+            }
+            nf = nf + __popcll(mk);
+            if (nf > cap) nf = cap;
+        }
+        wave_lds_sync();
+    }
+    // the merged sequence, two places a lane at a time
+    double s[3] = {0.0, 0.0, 0.0};  // sigma, rhoSPH_new, dShep
+    const int len = nn + nf;
+    auto entry = [&](int k) { return k < nn ? (int)(nbr[nb_index(N, i, k)] & NB_MASK) : i; };
+    int walls = 0;  // before the current places
+    for (int p0 = 0; p0 < len; p0 += 2 * DB_G) {
+        const uint32_t mask = nf ? (bm[p0 >> 5] >> (p0 & 31)) & ((1u << (2 * DB_G)) - 1u) : 0u;
+        d2 x, y, z, rho, c1 = d2(0.0);
+        bool on[2];
+        d2 m = d2(0.0), vn = d2(0.0), mw = d2(0.0);
+        bool wall[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int o = u * DB_G + g, p = p0 + o;
+            const int nw = walls + __popc(mask & ((1u << o) - 1u));
+            wall[u] = (mask >> o) & 1u;
+            on[u] = p < len;
+            if (!wall[u]) {
+                const int j = on[u] ? entry(p - nw) : i;
+                const double4 xj = xm[j];
+                x[u] = xj.x;
+                y[u] = xj.y;
+                z[u] = xj.z;
+                m[u] = xj.w;
+                rho[u] = rp[j].x;
+                vn[u] = 0.0;
+            } else {
+                const int id = ids[nw];
+                const double4 a = W.w0[id], b = W.w1[id], gv = W.w2[id];
+                x[u] = a.x;
+                y[u] = a.y;
+                z[u] = a.z;
+                m[u] = b.w;
+                mw[u] = gv.w;
+                rho[u] = 1.0;
+                c1[u] = a.w;
+                vn[u] = b.x * (gv.x - vi.x) + b.y * (gv.y - vi.y) + b.z * (gv.z - vi.z);
+            }
+        }
+        walls += __popc(mask);
+        const d2 R0 = xi.x - x, R1 = xi.y - y, R2 = xi.z - z;
+        const K64x2 K = kvals64x2(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true);
+        const d2 mW = m * K.W;
+        const d2 vol = div64(mW, rho, inv64(rho));
+        double t[2][3];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const double k1 = on[u] ? K.W[u] : 0.0;
+            t[u][0] = !on[u] ? 0.0 : wall[u] ? mW[u] : vol[u];
+            t[u][1] = !on[u] ? 0.0 : wall[u] ? mw[u] * k1 : mW[u];
+            t[u][2] = wall[u] ? k1 * c1[u] * vn[u] : 0.0;
+        }
+        add_lanes<DB_G>(s, t[0]);
+        add_lanes<DB_G>(s, t[1]);
+    }
+    const double sigma = s[0], rsph = s[1], dshep = s[2];
     if (g != 0) return;
     nfw[i] = nf;
     sig_out[i] = sigma;
@@ -216,6 +262,7 @@ __global__ __launch_bounds__(256) void k_dbsph_lists(
 // terms read the VSL gradients and semi-particle viscosities, which are zero
 // without the VSL model (slip_ID = 0), and add zeros.  acc = (tpres + tdiss
 // + tvisc) / Gamma + g; Euler's vel += dt acc (kodvel = 0) is fused.
+template <int G>
 __global__ __launch_bounds__(256) void k_momentum_dbsph(
     DPC* Pp, DWall W, const double4* __restrict__ xm, const double4* __restrict__ vel,
     const double2* __restrict__ rp, const uint32_t* __restrict__ nbr, const int* __restrict__ nnb,
@@ -223,13 +270,8 @@ __global__ __launch_bounds__(256) void k_momentum_dbsph(
     const double* __restrict__ wdens, const double* __restrict__ wpres, int* __restrict__ lam_out,
     double4* __restrict__ acc_out, double4* __restrict__ vel_out, const double* scal, const int* iscal) {
     DPC& P = *Pp;
-    // DB_G lanes per particle take consecutive list entries (then wall
-    // elements) side by side; every lane of the group adds the entries'
-    // terms in list order, read from their lanes with shuffles
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = t / DB_G, g = t % DB_G;
-    const int gb = (threadIdx.x & 63) & ~(DB_G - 1);
-    const uint64_t gmask = (1ull << DB_G) - 1ull;
+    // G lanes per particle; lane 0 adds their terms in list order
+    const int i = (xcd_block(gridDim.x) * 256 + (int)threadIdx.x) / G, g = threadIdx.x % G;
     if (i >= iscal[IS_N]) return;  // whole groups leave together
     const size_t N = P.cap;
     const double h = P.h;
@@ -237,70 +279,48 @@ __global__ __launch_bounds__(256) void k_momentum_dbsph(
     const double2 rpi = rp[i];
     const double4 xi = xm[i];
     const double rhoi = rpi.x, pi = rpi.y;
-    double tp[3] = {0.0, 0.0, 0.0}, td[3] = {0.0, 0.0, 0.0}, tv[3] = {0.0, 0.0, 0.0};
-    double tpa[3] = {0.0, 0.0, 0.0}, rvs[3] = {0.0, 0.0, 0.0};
+    double tp[3] = {0.0, 0.0, 0.0};
+    double s[12];  // td, tv, rvs, tpa
+    for (int c = 0; c < 12; ++c) s[c] = 0.0;
     const double celt = P.celerita + P.celerita;
     const double nui = P.kin_visc, nuj = P.kin_visc;
     const bool morris = nui > 1.0e-12 && nuj > 1.0e-12;
-    const int nn = nnb[i];
-    for (int k0 = 0; k0 < nn; k0 += DB_G) {
-        const int k = k0 + g;
-        bool val = false;
-        double cp[3] = {0.0, 0.0, 0.0}, cd[3] = {0.0, 0.0, 0.0}, cv[3] = {0.0, 0.0, 0.0};
-        if (k < nn) {
-            const int j = (int)(nbr[nb_index(N, i, k)] & NB_MASK);
-            if (j != i) {
-                val = true;
-                const double4 xj = xm[j];
-                const double4 vj = vel[j];
-                const double2 rpj = rp[j];
-                const double R0 = xi.x - xj.x, R1 = xi.y - xj.y, R2 = xi.z - xj.z;
-                const double rij = R0 * R0 + R1 * R1 + R2 * R2;
-                K64 K;
-                kvals64(P, rij, true, false, false, K);
-                const double rhoj = rpj.x, pj = rpj.y, amassj = xj.w;
-                const double dv0 = vj.x - vi.x, dv1 = vj.y - vi.y, dv2 = vj.z - vi.z;
-                const double alpha = pi / (rhoi * rhoi) + pj / (rhoj * rhoj);
-                cp[0] = -amassj * alpha * R0 * K.K1;
-                cp[1] = -amassj * alpha * R1 * K.K1;
-                cp[2] = -amassj * alpha * R2 * K.K1;
-                const double vrij = -dv0 * R0 - dv1 * R1 - dv2 * R2;
-                const double TermMon = P.alfamon * celt * h / (rhoi + rhoj);
-                cd[0] = amassj * TermMon * vrij * R0 * K.K2 + 0.0;
-                cd[1] = amassj * TermMon * vrij * R1 * K.K2 + 0.0;
-                cd[2] = amassj * TermMon * vrij * R2 * K.K2 + 0.0;
-                if (morris) {
-                    const double rtil = nui * rhoi + nuj * rhoj + 1.0e-3;
-                    const double atil = 4.0 * (nui * nuj);
-                    const double fac = amassj * atil / rtil;
-                    const double rr = R0 * R0 + R1 * R1 + R2 * R2;
-                    cv[0] = fac * (-dv0 * K.K2 * rr);
-                    cv[1] = fac * (-dv1 * K.K2 * rr);
-                    cv[2] = fac * (-dv2 * K.K2 * rr);
-                }
-            }
-        }
-        const uint64_t mv = (__ballot(val) >> gb) & gmask;
-#pragma unroll
-        for (int u = 0; u < DB_G; ++u) {
-            double p_[3], d_[3], v_[3];
-            for (int d = 0; d < 3; ++d) {
-                p_[d] = __shfl(cp[d], u, DB_G);
-                d_[d] = __shfl(cd[d], u, DB_G);
-            }
-            if (morris)
-                for (int d = 0; d < 3; ++d) v_[d] = __shfl(cv[d], u, DB_G);
-            if ((mv >> u) & 1ull) {
-                for (int d = 0; d < 3; ++d) tpa[d] = tpa[d] + p_[d];
-                for (int d = 0; d < 3; ++d) td[d] = td[d] + d_[d];
-                if (morris) {
-                    for (int d = 0; d < 3; ++d) tv[d] = tv[d] + v_[d];
-                    for (int d = 0; d < 3; ++d) rvs[d] = rvs[d] + v_[d];
-                }
-            }
-        }
-    }
-    for (int d = 0; d < 3; ++d) tp[d] = tp[d] + tpa[d] + 0.0;
+    const double ai = pi / (rhoi * rhoi);
+    pair_sums64<G, 12>(nbr, N, i, nnb[i], g, false, 0u, s, [](uint32_t) { return Nb{}; },
+        [&](int j) {
+            const double4 x = xm[j], v = vel[j];
+            const double2 q = rp[j];
+            return Nb{x.x, x.y, x.z, v.x, v.y, v.z, q.x, q.y, 0.0, x.w};
+        },
+        [&](d2 (&t)[12], const Nb& a, const Nb& b, bool, bool) {
+            const d2 R0 = xi.x - d2{a.x, b.x}, R1 = xi.y - d2{a.y, b.y}, R2 = xi.z - d2{a.z, b.z};
+            const d2 rij = R0 * R0 + R1 * R1 + R2 * R2;
+            const K64x2 K = kvals64x2(P, rij, true, false, false);
+            const d2 rhoj = {a.rho, b.rho}, pj = {a.p, b.p}, amassj = {a.m, b.m};
+            const d2 dv0 = d2{a.u, b.u} - vi.x, dv1 = d2{a.v, b.v} - vi.y, dv2 = d2{a.w, b.w} - vi.z;
+            const d2 r2 = rhoj * rhoj;
+            const d2 alpha = ai + div64(pj, r2, inv64(r2));
+            t[9] = -amassj * alpha * R0 * K.K1;
+            t[10] = -amassj * alpha * R1 * K.K1;
+            t[11] = -amassj * alpha * R2 * K.K1;
+            const d2 vrij = -dv0 * R0 - dv1 * R1 - dv2 * R2;
+            const d2 rsum = rhoi + rhoj;
+            const d2 TermMon = div64(d2(P.alfamon * celt * h), rsum, inv64(rsum));
+            t[0] = amassj * TermMon * vrij * R0 * K.K2;
+            t[1] = amassj * TermMon * vrij * R1 * K.K2;
+            t[2] = amassj * TermMon * vrij * R2 * K.K2;
+            const d2 rtil = nui * rhoi + nuj * rhoj + 1.0e-3;
+            const double atil = 4.0 * (nui * nuj);
+            const d2 visc = div64(amassj * atil, rtil, inv64(rtil));
+            const d2 fac = {morris ? visc.x : 0.0, morris ? visc.y : 0.0};
+            t[3] = t[6] = fac * (-dv0 * K.K2 * rij);
+            t[4] = t[7] = fac * (-dv1 * K.K2 * rij);
+            t[5] = t[8] = fac * (-dv2 * K.K2 * rij);
+        });
+    const double* td = s;
+    const double* tv = s + 3;
+    const double* rvs = s + 6;
+    for (int d = 0; d < 3; ++d) tp[d] = tp[d] + s[9 + d] + 0.0;
     int lam = 0;
     if (P.kin_visc > 0.0) {
         const double apg = sqrt(tp[0] * tp[0] + tp[1] * tp[1] + tp[2] * tp[2]) + P.GI;
@@ -310,7 +330,7 @@ __global__ __launch_bounds__(256) void k_momentum_dbsph(
         lam = (w > 5.0 || apg == 0.0) ? 1 : 0;
     }
     const int nf = nfw[i];
-    for (int k0 = 0; k0 < nf; k0 += DB_G) {  // inter_EqMoto.f90:286-297
+    for (int k0 = 0; k0 < nf; k0 += G) {  // inter_EqMoto.f90:286-297
         const int k = k0 + g;
         double ap[3] = {0.0, 0.0, 0.0};
         if (k < nf) {
@@ -329,17 +349,10 @@ __global__ __launch_bounds__(256) void k_momentum_dbsph(
                 ap[d] = ap[d] - wm * A * R[d] * K.K1;
             }
         }
-#pragma unroll
-        for (int u = 0; u < DB_G; ++u) {
-            double a_[3];
-            for (int d = 0; d < 3; ++d) a_[d] = __shfl(ap[d], u, DB_G);
-            if (k0 + u < nf)
-                for (int d = 0; d < 3; ++d) tp[d] = tp[d] + a_[d];
-        }
+        add_lanes<G>(tp, ap);  // past the end: zeros
     }
     if (g != 0) return;
     lam_out[i] = lam;
-    for (int d = 0; d < 3; ++d) tv[d] = tv[d] + 0.0 + 0.0;
     const double gm = gam[i];
     double a[3];
     for (int d = 0; d < 3; ++d) a[d] = (tp[d] + td[d] + tv[d]) / gm + P.grav[d];
@@ -351,6 +364,7 @@ __global__ __launch_bounds__(256) void k_momentum_dbsph(
 // Gradients_to_MUSCL.f90:47-91 for the particles with wall neighbours:
 // drho = sum r (rho_j - rho_i) PartKernel(1) m_j/rho_j and dvel(r, :) the
 // same of var(r); drho[3 i + d], dvel[9 i + 3 r + d]
+template <int G>
 __global__ __launch_bounds__(256) void k_dbsph_muscl(DPC* Pp, DWall W, const double4* __restrict__ xm,
                                                      const double4* __restrict__ vel,
                                                      const double2* __restrict__ rp,
@@ -361,56 +375,63 @@ __global__ __launch_bounds__(256) void k_dbsph_muscl(DPC* Pp, DWall W, const dou
                                                      double* __restrict__ drho, double* __restrict__ dvel,
                                                      const int* iscal) {
     DPC& P = *Pp;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (xcd_block(gridDim.x) * 256 + (int)threadIdx.x) / G, g = threadIdx.x % G;
     if (i >= iscal[IS_N] || nfw[i] <= 0) return;
     const double4 xi = xm[i];
     const double4 vi = vel[i];
     const double rhoi = rp[i].x;
-    double g[3] = {0.0, 0.0, 0.0}, V[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    using RM = NRec<double4, double4, double2>;
-    auto fetch = [&](uint32_t e) {
-        const int j = (int)(e & NB_MASK);
-        return RM{xm[j], vel[j], rp[j]};
-    };
-    walk_list<4, RM>(nbr, (size_t)P.cap, i, nnb[i], fetch, [&](uint32_t e, const RM& q) {
-        const double4 xj = q.x;
-        const double R[3] = {xi.x - xj.x, xi.y - xj.y, xi.z - xj.z};
-        K64 K;
-        kvals64(P, R[0] * R[0] + R[1] * R[1] + R[2] * R[2], true, false, false, K);
-        const double vol = xj.w / q.r.x;
-        const double dv[3] = {q.v.x - vi.x, q.v.y - vi.y, q.v.z - vi.z};
-        for (int d = 0; d < 3; ++d) g[d] = g[d] + R[d] * (q.r.x - rhoi) * K.K1 * vol;
-        for (int r = 0; r < 3; ++r)
-            for (int d = 0; d < 3; ++d) V[3 * r + d] = V[3 * r + d] + R[d] * dv[r] * K.K1 * vol;
-    });
+    double s[12];  // drho, dvel
+    for (int c = 0; c < 12; ++c) s[c] = 0.0;
+    pair_sums64<G, 12>(nbr, (size_t)P.cap, i, nnb[i], g, false, 0u, s, [](uint32_t) { return Nb{}; },
+        [&](int j) {
+            const double4 x = xm[j], v = vel[j];
+            return Nb{x.x, x.y, x.z, v.x, v.y, v.z, rp[j].x, 0.0, 0.0, x.w};
+        },
+        [&](d2 (&t)[12], const Nb& a, const Nb& b, bool, bool) {
+            const d2 R[3] = {xi.x - d2{a.x, b.x}, xi.y - d2{a.y, b.y}, xi.z - d2{a.z, b.z}};
+            const K64x2 K = kvals64x2(P, R[0] * R[0] + R[1] * R[1] + R[2] * R[2], true, false, false);
+            const d2 rhoj = {a.rho, b.rho};
+            const d2 vol = div64(d2{a.m, b.m}, rhoj, inv64(rhoj));
+            const d2 dv[3] = {d2{a.u, b.u} - vi.x, d2{a.v, b.v} - vi.y, d2{a.w, b.w} - vi.z};
+            for (int d = 0; d < 3; ++d) t[d] = R[d] * (rhoj - rhoi) * K.K1 * vol;
+            for (int r = 0; r < 3; ++r)
+                for (int d = 0; d < 3; ++d) t[3 + 3 * r + d] = R[d] * dv[r] * K.K1 * vol;
+        });
     if (P.muscl_bnd) {  // Gradients_to_MUSCL_boundary.f90:44-86 (one medium)
         const double sg = sig[i];
         const int nf = nfw[i];
         const double v[3] = {vi.x, vi.y, vi.z};
-        for (int k = 0; k < nf; ++k) {
-            const int id = fwl[(size_t)k * P.cap + i];
-            const double4 a = W.w0[id];
-            const double4 b = W.w1[id];
-            const double4 wv = W.w2[id];
-            const double wd = wdens[id];
-            const double R[3] = {xi.x - a.x, xi.y - a.y, xi.z - a.z};
-            K64 K;  // kernel_fw(1) = W, kernel_fw(2) = K1
-            kvals64(P, R[0] * R[0] + R[1] * R[1] + R[2] * R[2], true, false, true, K);
-            const double nw[3] = {b.x, b.y, b.z};
-            const double vw[3] = {wv.x, wv.y, wv.z};
-            const double dr = wd - rhoi;
-            const double Ww = a.w * K.W / sg;
-            for (int d = 0; d < 3; ++d) g[d] = g[d] + dr * nw[d] * Ww;
-            for (int r = 0; r < 3; ++r)
-                for (int d = 0; d < 3; ++d) V[3 * r + d] = V[3 * r + d] + (vw[r] - v[r]) * nw[d] * Ww;
-            const double vol = wv.w / wd / sg;
-            for (int d = 0; d < 3; ++d) g[d] = g[d] + R[d] * dr * K.K1 * vol;
-            for (int r = 0; r < 3; ++r)
-                for (int d = 0; d < 3; ++d) V[3 * r + d] = V[3 * r + d] + R[d] * (vw[r] - v[r]) * K.K1 * vol;
+        for (int k0 = 0; k0 < nf; k0 += G) {
+            const int k = k0 + g;
+            double ta[12], tb[12];  // past the end: zeros
+            for (int c = 0; c < 12; ++c) ta[c] = tb[c] = 0.0;
+            if (k < nf) {
+                const int id = fwl[(size_t)k * P.cap + i];
+                const double4 a = W.w0[id];
+                const double4 b = W.w1[id];
+                const double4 wv = W.w2[id];
+                const double wd = wdens[id];
+                const double R[3] = {xi.x - a.x, xi.y - a.y, xi.z - a.z};
+                K64 K;  // kernel_fw(1) = W, kernel_fw(2) = K1
+                kvals64(P, R[0] * R[0] + R[1] * R[1] + R[2] * R[2], true, false, true, K);
+                const double nw[3] = {b.x, b.y, b.z};
+                const double vw[3] = {wv.x, wv.y, wv.z};
+                const double dr = wd - rhoi;
+                const double Ww = a.w * K.W / sg;
+                for (int d = 0; d < 3; ++d) ta[d] = dr * nw[d] * Ww;
+                for (int r = 0; r < 3; ++r)
+                    for (int d = 0; d < 3; ++d) ta[3 + 3 * r + d] = (vw[r] - v[r]) * nw[d] * Ww;
+                const double vol = wv.w / wd / sg;
+                for (int d = 0; d < 3; ++d) tb[d] = R[d] * dr * K.K1 * vol;
+                for (int r = 0; r < 3; ++r)
+                    for (int d = 0; d < 3; ++d) tb[3 + 3 * r + d] = R[d] * (vw[r] - v[r]) * K.K1 * vol;
+            }
+            add_lanes<G>(s, ta, tb);
         }
     }
-    for (int d = 0; d < 3; ++d) drho[3 * (size_t)i + d] = g[d];
-    for (int d = 0; d < 9; ++d) dvel[9 * (size_t)i + d] = V[d];
+    if (g != 0) return;
+    for (int d = 0; d < 3; ++d) drho[3 * (size_t)i + d] = s[d];
+    for (int d = 0; d < 9; ++d) dvel[9 * (size_t)i + d] = s[3 + d];
 }
 
 // DBSPH_kinematics.f90:52-107 and Euler.f90:152-159, one thread per sorted

@@ -219,6 +219,7 @@ constexpr int TILE_CAP_L = 2496, TILE_CAP_M = 1632, TILE_CAP_S = 1216, TILE_CAP_
 constexpr int TILE_WG = 512;   // most threads of a pair pass
 constexpr int TILE_U = 5;      // slots a thread stages at a time (FP64: 3)
 constexpr int TILE_G2 = 40000;  // particles below which two lanes take a particle
+constexpr int TILE_G8 = 20000;  // DB-SPH: particles below which eight lanes take a particle, else four
 // tiles of water a solve is cut into (choose_tile); FP64
 constexpr int TILE_MIN = 300, TILE_MIN2 = 200, TILE_MIN_L = 500;
 constexpr int TILE_MIN64 = 130, TILE_MIN64_2 = 150;
@@ -1896,11 +1897,19 @@ __device__ __forceinline__ int tile_find(const int* pre, int rows, int x) {
 // for every slot of a tile that fits, then part(P, segment, sorted index,
 // slot, fits) with G lanes for every home particle, then done(P, segment).  A
 // workgroup takes the tiles of its XCD's contiguous share, so tiles that share
-// halo rows share an L2.
-template <bool SG, int G, int U, class Stage, class Part, class Done>
+// halo rows share an L2.  TILED false: G lanes for every particle of one
+// solve, 256 threads a block, nothing staged.
+template <bool SG, int G, int U, bool TILED = true, class Stage, class Part, class Done>
 __device__ __forceinline__ void for_tiles(const Seg& S, const Tiles& T,
                                           const int* __restrict__ start, Stage&& stage, Part&& part,
                                           Done&& done) {
+    if constexpr (!TILED) {
+        DPC& P = S.P[0];
+        const int i = (xcd_block(gridDim.x) * 256 + (int)threadIdx.x) / G;
+        if (i < start[P.nmax]) part(P, 0, i, 0, false);
+        done(P, 0);
+        return;
+    }
     __shared__ TileS ts;
     const int nt = *T.n;
     const int per = gridDim.x >> 3, xcd = blockIdx.x & 7;  // gridDim.x is a multiple of 8
@@ -1958,51 +1967,6 @@ __device__ __forceinline__ float4 lds16(const float4* a, uint32_t o) {
 }
 
 constexpr uint32_t NB_NONE = 0xFFFFFFFFu;
-
-// Walks particle i's neighbour list in the reference's order, CH entries at a
-// time: the CH list entries and then the CH neighbour records are all loaded
-// before any is used, so their latencies overlap; body() then consumes them
-// strictly in list order (the FP64 sums keep the reference's order).
-template <int CH, class R, class Fetch, class Body>
-__device__ __forceinline__ void walk_list(const uint32_t* __restrict__ nbr, size_t N, int i, int nn,
-                                          Fetch&& fetch, Body&& body) {
-    static_assert(CH % 4 == 0, "list walks read whole 16-byte quarters of a group");
-    for (int k0 = 0; k0 < nn; k0 += CH) {
-        uint32_t ev[CH];
-        {
-#pragma unroll
-            for (int q = 0; q < CH / 4; ++q) {
-                const uint4 v = *reinterpret_cast<const uint4*>(nbr + nb_index(N, i, k0 + 4 * q));
-                ev[4 * q + 0] = v.x;
-                ev[4 * q + 1] = v.y;
-                ev[4 * q + 2] = v.z;
-                ev[4 * q + 3] = v.w;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < CH; ++u)
-            if (k0 + u >= nn) ev[u] = NB_NONE;
-        R rq[CH];
-#pragma unroll
-        for (int u = 0; u < CH; ++u)
-            if (ev[u] != NB_NONE) rq[u] = fetch(ev[u]);
-#pragma unroll
-        for (int u = 0; u < CH; ++u)
-            if (ev[u] != NB_NONE) body(ev[u], rq[u]);
-    }
-}
-
-template <class X, class V, class RP>
-struct NRec {
-    X x;
-    V v;
-    RP r;
-};
-template <class X, class RP>
-struct NRec2 {
-    X x;
-    RP r;
-};
 
 // wall_function_for_SASPH.f90:56-80 (no land-cover map), FP64: slip
 // coefficient and mixing-length viscosity of one particle-frontier pair at
@@ -2708,20 +2672,27 @@ __device__ __forceinline__ double psmooth_end(DPC& P, const DFace* __restrict__ 
 #define TILE_ARGS Seg S, Tiles T, const int* __restrict__ start
 
 // lane u's value for lane 0 of each group of G (the other lanes: any)
-template <int G>
-__device__ __forceinline__ double group_lane(double v, int u) {
-    if (u == 0) return v;
-    auto pick = [&](int w) {
-        if constexpr (G == 2) return __builtin_amdgcn_mov_dpp(w, 0xF5, 0xF, 0xF, true);  // quad_perm (1,1,3,3)
-        return u == 1 ? __builtin_amdgcn_mov_dpp(w, 0x55, 0xF, 0xF, true)
-             : u == 2 ? __builtin_amdgcn_mov_dpp(w, 0xAA, 0xF, 0xF, true)
-                      : __builtin_amdgcn_mov_dpp(w, 0xFF, 0xF, 0xF, true);
-    };
-    return __hiloint2double(pick(__double2hiint(v)), pick(__double2loint(v)));
+template <int U>
+__device__ __forceinline__ double group_lane(double v) {
+    if constexpr (U == 0) return v;
+    else  // row_shl: lane l of a row of 16 takes lane l + U
+        return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), 0x100 + U, 0xF, 0xF, true),
+                                __builtin_amdgcn_mov_dpp(__double2loint(v), 0x100 + U, 0xF, 0xF, true));
+}
+// adds lane 0's, 1's, .. lane G-1's terms (each lane's t, then its more) to
+// lane 0's sums, in that order
+template <int G, int U = 0, int NS, class... More>
+__device__ __forceinline__ void add_lanes(double (&sum)[NS], const double (&t)[NS], const More&... more) {
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+        sum[c] = sum[c] + group_lane<U>(t[c]);
+        ((sum[c] = sum[c] + group_lane<U>(more[c])), ...);
+    }
+    if constexpr (U + 1 < G) add_lanes<G, U + 1>(sum, t, more...);
 }
 
-// Adds particle i's NS pair terms to sum in list order, by G lanes (1, 2 or 4,
-// lane g of them): each lane forms the terms of two entries, the lanes' entries
+// Adds particle i's NS pair terms to sum in list order, by G lanes (lane g of
+// them; LDS form: 1, 2 or 4): each lane forms the terms of two entries, the lanes' entries
 // consecutive, and lane 0 adds them all in order.  lds(byte offset of a
 // neighbour's 16-byte records) and glob(its sorted index) read a neighbour,
 // term(terms, one, other, one counts, other counts).  Past the list's end they
@@ -2732,14 +2703,13 @@ __device__ __forceinline__ void pair_sums64(const uint32_t* __restrict__ nbr, si
                                             bool fits, uint32_t self, double (&sum)[NS], Lds&& lds, Glob&& glob,
                                             Term&& term) {
     auto add = [&](const d2 (&t)[NS]) {
+        double v[NS];
 #pragma unroll
-        for (int u = 0; u < G; ++u)
+        for (int c = 0; c < NS; ++c) v[c] = t[c].x;
+        add_lanes<G>(sum, v);
 #pragma unroll
-            for (int c = 0; c < NS; ++c) sum[c] = sum[c] + group_lane<G>(t[c].x, u);
-#pragma unroll
-        for (int u = 0; u < G; ++u)
-#pragma unroll
-            for (int c = 0; c < NS; ++c) sum[c] = sum[c] + group_lane<G>(t[c].y, u);
+        for (int c = 0; c < NS; ++c) v[c] = t[c].y;
+        add_lanes<G>(sum, v);
     };
     if (fits) {
         const uint4* L = reinterpret_cast<const uint4*>(nbr) + 2 * (size_t)i;
@@ -2767,12 +2737,21 @@ __device__ __forceinline__ void pair_sums64(const uint32_t* __restrict__ nbr, si
             }
         }
     } else {
+        // a step's records are gathered during the step before it, and their
+        // list entries a step earlier
+        auto entry = [&](int k) { return k < nn ? (int)(nbr[nb_index(N, i, k)] & NB_MASK) : i; };
+        int ja = entry(g), jb = entry(G + g);
+        auto a = glob(ja), b = glob(jb);
+        ja = entry(2 * G + g);
+        jb = entry(3 * G + g);
         for (int k0 = 0; k0 < nn; k0 += 2 * G) {
-            const int ka = k0 + g, kb = k0 + G + g;
-            const int ja = ka < nn ? (int)(nbr[nb_index(N, i, ka)] & NB_MASK) : i;
-            const int jb = kb < nn ? (int)(nbr[nb_index(N, i, kb)] & NB_MASK) : i;
+            const auto ca = a, cb = b;
+            a = glob(ja);
+            b = glob(jb);
+            ja = entry(k0 + 4 * G + g);
+            jb = entry(k0 + 5 * G + g);
             d2 t[NS];
-            term(t, glob(ja), glob(jb), ka < nn, kb < nn);
+            term(t, ca, cb, k0 + g < nn, k0 + G + g < nn);
             add(t);
         }
     }
@@ -2799,7 +2778,7 @@ __global__ __launch_bounds__(TILE_WG, 2) void k_momentum64(
     double4* __restrict__ acc_out, double4* __restrict__ vel_out, const double* scal0, int* iscal0) {
     __shared__ double2 sA[CAP], sB[CAP], sC[CAP], sD[CAP];  // (x, y), (z, vx), (vy, vz), (rho, p)
     const int g = threadIdx.x % G;
-    for_tiles<SG, G, 3>(S, T, start,
+    for_tiles<SG, G, 3, CAP != TILE_CAP_0>(S, T, start,
         [&](DPC&, int, int j, int slot) {
             const double4 x = xm[j], v = vel[j];
             sA[slot] = make_double2(x.x, x.y);
@@ -2900,7 +2879,7 @@ __global__ __launch_bounds__(TILE_WG, 2) void k_vsmooth64(
     __shared__ double2 sA[CAP], sB[CAP], sC[CAP], sD[CAP];  // (x, y), (z, vx), (vy, vz), (rho, 1 / rho)
     const int g = threadIdx.x % G;
     unsigned long long dtbits = 0x7FF0000000000000ull;
-    for_tiles<SG, G, 3>(S, T, start,
+    for_tiles<SG, G, 3, CAP != TILE_CAP_0>(S, T, start,
         [&](DPC& P, int, int j, int slot) {
             if (!(P.tetav > 1.0e-9)) return;
             const double4 x = xm[j], v = vel1[j];
@@ -2925,12 +2904,13 @@ __global__ __launch_bounds__(TILE_WG, 2) void k_vsmooth64(
                     [&](int j) {
                         const double4 x = xm[j], u = vel1[j];
                         const double rho = rp[j].x;
-                        return Nb{x.x, x.y, x.z, u.x, u.y, u.z, rho, 0.0, 1.0 / rho, x.w};
+                        return Nb{x.x, x.y, x.z, u.x, u.y, u.z, rho, 0.0, 0.0, x.w};
                     },
                     [&](d2 (&t)[3], const Nb& a, const Nb& b, bool, bool) {
                         const d2 R0 = xi.x - d2{a.x, b.x}, R1 = xi.y - d2{a.y, b.y}, R2 = xi.z - d2{a.z, b.z};
                         const K64x2 K = kvals64x2(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true);
-                        const d2 pes = div64(d2{a.m, b.m} * K.W, d2{a.rho, b.rho}, d2{a.inv, b.inv});
+                        const d2 rhoj = {a.rho, b.rho};
+                        const d2 pes = div64(d2{a.m, b.m} * K.W, rhoj, fits ? d2{a.inv, b.inv} : inv64(rhoj));
                         t[0] = (d2{a.u, b.u} - vi.x) * pes;
                         t[1] = (d2{a.v, b.v} - vi.y) * pes;
                         t[2] = (d2{a.w, b.w} - vi.z) * pes;
@@ -2957,7 +2937,7 @@ __global__ __launch_bounds__(TILE_WG, 2) void k_continuity64(
     __shared__ double2 sA[CAP], sB[CAP], sC[CAP];  // (x, y), (z, vx), (vy, vz)
     __shared__ double sD[CAP];                     // m / rho
     const int g = threadIdx.x % G;
-    for_tiles<SG, G, 3>(S, T, start,
+    for_tiles<SG, G, 3, CAP != TILE_CAP_0>(S, T, start,
         [&](DPC&, int, int j, int slot) {
             const double4 x = xm[j], v = vel[j];
             sA[slot] = make_double2(x.x, x.y);
@@ -3007,7 +2987,7 @@ __global__ __launch_bounds__(TILE_WG, 2) void k_psmooth64(
     const double* scal0) {
     __shared__ double2 sA[CAP], sB[CAP], sC[CAP];  // (x, y), (z, p), (rho, 1 / rho)
     const int g = threadIdx.x % G;
-    for_tiles<SG, G, 3>(S, T, start,
+    for_tiles<SG, G, 3, CAP != TILE_CAP_0>(S, T, start,
         [&](DPC&, int, int j, int slot) {
             const double4 x = xm[j];
             const double2 q = rp[j];
@@ -3029,12 +3009,13 @@ __global__ __launch_bounds__(TILE_WG, 2) void k_psmooth64(
                 [&](int j) {
                     const double4 x = xm[j];
                     const double2 q = rp[j];
-                    return Nb{x.x, x.y, x.z, 0.0, 0.0, 0.0, q.x, q.y, 1.0 / q.x, x.w};
+                    return Nb{x.x, x.y, x.z, 0.0, 0.0, 0.0, q.x, q.y, 0.0, x.w};
                 },
                 [&](d2 (&t)[2], const Nb& a, const Nb& b, bool ona, bool onb) {
                     const d2 R0 = xi.x - d2{a.x, b.x}, R1 = xi.y - d2{a.y, b.y}, R2 = xi.z - d2{a.z, b.z};
                     const K64x2 K = kvals64x2(P, R0 * R0 + R1 * R1 + R2 * R2, false, false, true);
-                    const d2 pes = div64(d2{a.m, b.m} * K.W, d2{a.rho, b.rho}, d2{a.inv, b.inv});
+                    const d2 rhoj = {a.rho, b.rho};
+                    const d2 pes = div64(d2{a.m, b.m} * K.W, rhoj, fits ? d2{a.inv, b.inv} : inv64(rhoj));
                     t[0] = d2{ona ? pes.x : 0.0, onb ? pes.y : 0.0};
                     t[1] = (d2{a.p, b.p} - pi) * pes;
                 });
