@@ -264,7 +264,7 @@ int run_btab(sph_ctx* c, bool again = false) {
     if (c->P.f32)  // eight lanes per pair
         SEGL(k_boundary_int_f32, 4 * c->bt_grid, 256, c->d_faces, c->d_btf, c->bt, c->work, c->nwork);
     else
-        SEGL(k_boundary_int, c->bt_grid, 256, c->d_faces, c->d_kt, c->d_bit, c->bt, c->work, c->nwork);
+        SEGL(k_boundary_int, 2 * c->bt_grid, 256, c->d_faces, c->d_kt, c->d_bit, c->d_btf, c->bt, c->work, c->nwork);
     return 0;
 }
 

@@ -908,10 +908,37 @@ __global__ __launch_bounds__(256, 4) void k_neighbours(Seg S, const double4* __r
                   (unsigned long long)((long long)s_pairs[0] + s_pairs[1] + s_pairs[2] + s_pairs[3]));
 }
 
+// kernel-table values at rob times the weight da, FP64 (InterpolateTable.f90:58-82)
+__device__ __forceinline__ void d_kt_values(DPC& P, const double* __restrict__ kt, double rob, double da, double J[4]) {
+    const double deltaX = P.ktdelta;
+    const int nr0 = (int)((rob - kt[0]) / deltaX);
+    if (nr0 <= 0) {
+        for (int c = 0; c < 4; ++c) J[c] = kt[1 + c] * da;
+    } else if (nr0 >= 40) {
+        for (int c = 0; c < 4; ++c) J[c] = kt[40 * 5 + 1 + c] * da;
+    } else {
+        const double* r0 = &kt[nr0 * 5];
+        const double* r1 = &kt[(nr0 + 1) * 5];
+        const double csi = (rob - r0[0]) / deltaX;
+        for (int c = 0; c < 4; ++c) J[c] = (r0[1 + c] + csi * (r1[1 + c] - r0[1 + c])) * da;
+    }
+}
+
+// lane u's value for the lanes of its group of four
+__device__ __forceinline__ int quad_lane(int v, int u) {
+    return u == 0 ? __builtin_amdgcn_mov_dpp(v, 0x00, 0xF, 0xF, true)
+         : u == 1 ? __builtin_amdgcn_mov_dpp(v, 0x55, 0xF, 0xF, true)
+         : u == 2 ? __builtin_amdgcn_mov_dpp(v, 0xAA, 0xF, 0xF, true)
+                  : __builtin_amdgcn_mov_dpp(v, 0xFF, 0xF, 0xF, true);
+}
+__device__ __forceinline__ double quad_lane(double v, int u) {
+    return __hiloint2double(quad_lane(__double2hiint(v), u), quad_lane(__double2loint(v), u));
+}
+
 // ----------------------------------------------------------------------------
 // SA-SPH volume integrals (FP64)
 // ----------------------------------------------------------------------------
-__device__ void d_volume_integrals(DPC& P, const DFace& F, const double* __restrict__ kt,
+__device__ __attribute__((noinline)) void d_volume_integrals(DPC& P, const DFace& F, const double* __restrict__ kt,
                                    const double* __restrict__ bit, const double locx[3],
                                    double bi[8], double ig[9]) {
     double IntWdV = 0.0, IntdWrm1dV = 0.0, IntGWZrm1dV = 0.0;
@@ -945,26 +972,12 @@ __device__ void d_volume_integrals(DPC& P, const DFace& F, const double* __restr
         const double da = b[3];
         const double rob = dist / P.h;
         if (fabs(rob - robpre) > 1.0e-3) {
-            const double deltaX = P.ktdelta;
-            const int nr0 = (int)((rob - kt[0]) / deltaX);
-            double iv0, iv1, iv2, iv3;
-            if (nr0 <= 0) {
-                iv0 = kt[1]; iv1 = kt[2]; iv2 = kt[3]; iv3 = kt[4];
-            } else if (nr0 >= 40) {
-                iv0 = kt[40 * 5 + 1]; iv1 = kt[40 * 5 + 2]; iv2 = kt[40 * 5 + 3]; iv3 = kt[40 * 5 + 4];
-            } else {
-                const double* r0 = &kt[nr0 * 5];
-                const double* r1 = &kt[(nr0 + 1) * 5];
-                const double csi = (rob - r0[0]) / deltaX;
-                iv0 = r0[1] + csi * (r1[1] - r0[1]);
-                iv1 = r0[2] + csi * (r1[2] - r0[2]);
-                iv2 = r0[3] + csi * (r1[3] - r0[3]);
-                iv3 = r0[4] + csi * (r1[4] - r0[4]);
-            }
-            J0 = iv0 * da;
-            J1 = iv1 * da;
-            J2 = iv2 * da;
-            J3 = iv3 * da;
+            double J[4];
+            d_kt_values(P, kt, rob, da, J);
+            J0 = J[0];
+            J1 = J[1];
+            J2 = J[2];
+            J3 = J[3];
             robpre = rob;
         }
         const double R0 = b[4], R1 = b[5], R2 = b[6];
@@ -999,8 +1012,7 @@ __device__ void d_volume_integrals(DPC& P, const DFace& F, const double* __restr
 // boundary table: ComputeBoundaryDataTab_3D.f90:62-106 in two kernels.
 // k_boundary_find: FindCloseBoundaryFaces3D.f90:78-188 per particle, appends
 // every (particle, close face) pair to a compact work list; k_boundary_int:
-// ComputeBoundaryVolumeIntegrals_P0.f90:76-155 for one pair per thread, so the
-// 256-direction quadrature keeps every lane busy.
+// ComputeBoundaryVolumeIntegrals_P0.f90:76-155 over that list.
 // ----------------------------------------------------------------------------
 template <bool SG>
 __global__ __launch_bounds__(256) void k_boundary_find(Seg S, const DFace* __restrict__ faces,
@@ -1076,37 +1088,6 @@ __global__ __launch_bounds__(256) void k_boundary_find(Seg S, const DFace* __res
 // Segmented contexts: a workgroup's pairs may belong to several segments, so
 // each lane reads its segment's constants and tables (kernel and direction
 // tables of every segment, consecutive) from global memory.
-template <bool SG>
-__global__ __launch_bounds__(256) void k_boundary_int(Seg S, const DFace* __restrict__ faces,
-                                                      const double* __restrict__ kt_g,
-                                                      const double* __restrict__ bit_g,
-                                                      BTab* __restrict__ bt,
-                                                      const int* __restrict__ work,
-                                                      const int* nwork) {
-    __shared__ double kt_s[SG ? 1 : 41 * 5];
-    __shared__ double bit_s[SG ? 1 : 256 * 7];
-    if (!SG) {
-        for (int t = threadIdx.x; t < 41 * 5; t += blockDim.x) kt_s[t] = kt_g[t];
-        for (int t = threadIdx.x; t < 256 * 7; t += blockDim.x) bit_s[t] = bit_g[t];
-        __syncthreads();
-    }
-    const int nw = *nwork;
-    for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < nw; w += gridDim.x * blockDim.x) {
-        const int e = work[w];
-        const int i = e & (int)NB_MASK, q = (int)((uint32_t)e >> NB_SHIFT);
-        const int sg = SG ? S.pblk[i >> 8] : 0;
-        DPC& P = S.P[sg];
-        const double* kt = SG ? kt_g + (size_t)sg * (41 * 5) : kt_s;
-        const double* bit = SG ? bit_g + (size_t)sg * (256 * 7) : bit_s;
-        BTab& rec = bt[(size_t)q * P.cap + i];
-        const double loc[3] = {rec.loc[0], rec.loc[1], rec.loc[2]};
-        double bi[8], ig[9];
-        d_volume_integrals(P, faces[rec.face], kt, bit, loc, bi, ig);
-        for (int t = 0; t < 8; ++t) rec.bi[t] = bi[t];
-        for (int t = 0; t < 9; ++t) rec.ig[t] = ig[t];
-    }
-}
-
 // ----------------------------------------------------------------------------
 // 2D form (x-z plane): boundary table over the boundary sides.
 // FindCloseBoundarySides2D.f90:68-170, SelectCloseBoundarySides2D.f90:66-120,
@@ -1417,6 +1398,160 @@ __device__ __forceinline__ int ring_side(const DFace& F, const PIC& c, double c0
         out = out || u2 + m2 < 0.0 || u2 - m2 > 1.0;
     }
     return in ? 1 : (out ? -1 : 0);
+}
+
+// The volume integrals in FP64, bit for bit as d_volume_integrals sums them
+// over the 256 directions, by four lanes of a pair.  One lane a pair walked the
+// directions one after the other: 101 us at 72,000 particles, 134 at 576,000.
+// A ring's directions share b_z and the weight (RingC), so the plane test, ts
+// and the table values belong to the ring: each lane takes two rings, decides
+// them whole by ring_side where it can and tests direction by direction where
+// it cannot.  Then every lane adds three of the twelve sums over the kept
+// directions in order, the factors from an LDS table: 32 and 60 us.  The
+// table values are refreshed where rob moves by more than 1e-3: within a ring
+// it moves by rounding only, so a ring is refreshed by its first kept direction
+// or not at all; a pair in which a ring's move is within 1e-9 of 1e-3, and any
+// table whose rings are not of this form, goes through d_volume_integrals.
+template <bool SG>
+__global__ __launch_bounds__(256) void k_boundary_int(Seg S, const DFace* __restrict__ faces,
+                                                      const double* __restrict__ kt_g,
+                                                      const double* __restrict__ bit_g,
+                                                      const BtF32* __restrict__ tab, BTab* __restrict__ bt,
+                                                      const int* __restrict__ work, const int* nwork) {
+    constexpr int ND = BT_RINGS * BT_RDIRS, G = 4;
+    __shared__ double kt_s[SG ? 1 : 41 * 5];
+    __shared__ double2 b_s[SG ? 1 : ND];
+    __shared__ double f_s[SG ? 1 : ND * 12];  // lane l's factors of direction k: [12 k + 3 l, + 3)
+    const int nw = *nwork;
+    if ((int)blockIdx.x * (256 / G) >= nw) return;  // no pair for this workgroup
+    auto factors = [](const double* R, int l, double f[3]) {
+        f[0] = l == 0 ? 1.0 : l == 1 ? R[0] : l == 2 ? R[0] * R[0] : R[1] * R[1];
+        f[1] = l == 0 ? 1.0 : l == 1 ? R[1] : l == 2 ? R[0] * R[1] : R[1] * R[2];
+        f[2] = l == 0 ? R[2] * R[2] : l == 1 ? R[2] : l == 2 ? R[0] * R[2] : R[2] * R[2];
+    };
+    if (!SG) {
+        for (int t = threadIdx.x; t < 41 * 5; t += 256) kt_s[t] = kt_g[t];
+        for (int t = threadIdx.x; t < ND; t += 256) {
+            const double* b = &bit_g[t * 7];
+            b_s[t] = make_double2(b[0], b[1]);
+            for (int l = 0; l < G; ++l) factors(b + 4, l, &f_s[12 * t + 3 * l]);
+        }
+        __syncthreads();
+    }
+    const int l = threadIdx.x % G;
+    for (int w = (blockIdx.x * 256 + threadIdx.x) / G; w < nw; w += gridDim.x * (256 / G)) {
+        const int e = work[w];
+        const int i = e & (int)NB_MASK, q = (int)((uint32_t)e >> NB_SHIFT);
+        const int sg = SG ? S.pblk[i >> 8] : 0;
+        DPC& P = S.P[sg];
+        const BtF32& T = tab[sg];
+        const double* ktg = kt_g + (size_t)sg * (41 * 5);
+        const double* bitg = bit_g + (size_t)sg * (ND * 7);
+        const double* kt = SG ? ktg : kt_s;
+        auto dir = [&](int k) { return SG ? make_double2(bitg[k * 7], bitg[k * 7 + 1]) : b_s[k]; };
+        BTab& rec = bt[(size_t)q * P.cap + i];
+        const DFace& F = faces[rec.face];
+        const double loc[3] = {rec.loc[0], rec.loc[1], rec.loc[2]};
+        const double zpmin = 0.05 * P.h;
+        const double L0 = loc[0], L1 = loc[1], L2 = loc[2] < zpmin ? zpmin : loc[2];
+        const PIC pic = pic_of(F);
+        uint32_t mask[2] = {0u, 0u};  // the kept directions of the rings l and l + 4
+        double rob[2] = {0.0, 0.0}, J[2][4];
+        bool serial = !T.all_ok;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            J[u][0] = J[u][1] = J[u][2] = J[u][3] = 0.0;
+            const int r = l + 4 * u;
+            const double Pj2 = L2 + T.rc[r].bz;
+            if (loc[2] < 0.0 || serial || !(Pj2 <= 0.0)) continue;
+            const double ts = L2 / (L2 - Pj2);
+            auto point = [&](int k, double& X0, double& X1) {
+                const double2 b = dir(r * BT_RDIRS + k);
+                const double Pj0 = L0 + b.x, Pj1 = L1 + b.y;
+                X0 = L0 + (Pj0 - L0) * ts;
+                X1 = L1 + (Pj1 - L1) * ts;
+            };
+            double X0, X1;
+            const int side = ring_side(F, pic, L0, L1, ts * T.rc[r].rho);
+            uint32_t m = side > 0 ? ~0u : 0u;
+            if (side == 0)
+                for (int k = 0; k < BT_RDIRS; ++k) {
+                    point(k, X0, X1);
+                    if (d_point_internal(pic, X0, X1)) m |= 1u << k;
+                }
+            mask[u] = m;
+            if (m == 0u) continue;
+            point(__ffs(m) - 1, X0, X1);
+            double dist = 0.0;
+            const double d0 = X0 - L0, d1 = X1 - L1, d2 = 0.0 - L2;
+            dist = dist + d0 * d0;
+            dist = dist + d1 * d1;
+            dist = dist + d2 * d2;
+            dist = sqrt(dist);
+            rob[u] = dist / P.h;
+            d_kt_values(P, kt, rob[u], bitg[r * BT_RDIRS * 7 + 3], J[u]);
+        }
+        double s[3] = {0.0, 0.0, 0.0}, ja = 0.0, jb = 0.0, robpre = 2.1;
+#pragma unroll
+        for (int r = 0; r < BT_RINGS; ++r) {
+            const int u = r / G;
+            const uint32_t m = (uint32_t)quad_lane((int)mask[u], r % G);
+            const double rr = quad_lane(rob[u], r % G);
+            double Jr[4];
+            for (int c = 0; c < 4; ++c) Jr[c] = quad_lane(J[u][c], r % G);
+            const double move = fabs(rr - robpre);
+            if (m != 0u && fabs(move - 1.0e-3) < 1.0e-9) serial = true;
+            if (m != 0u && move > 1.0e-3) {
+                ja = l == 0 ? Jr[0] : l == 1 ? Jr[2] : Jr[3];
+                jb = l == 0 ? Jr[1] : ja;
+                robpre = rr;
+            }
+            if (!__any(m != 0u)) continue;
+            const bool part = __any(m != 0u && m != ~0u);
+            const double ma = m ? ja : 0.0, mb = m ? jb : 0.0;  // a direction left out adds a zero
+#pragma unroll 4
+            for (int k = 0; k < BT_RDIRS; ++k) {
+                const int d = r * BT_RDIRS + k;
+                double f[3];
+                if (SG) {
+                    factors(&bitg[d * 7 + 4], l, f);
+                } else {
+                    f[0] = f_s[12 * d + 3 * l];
+                    f[1] = f_s[12 * d + 3 * l + 1];
+                    f[2] = f_s[12 * d + 3 * l + 2];
+                }
+                const bool on = !part || ((m >> k) & 1u);
+                const double ka = on ? ma : 0.0, kb = on ? mb : 0.0;
+                s[0] = s[0] + f[0] * ka;
+                s[1] = s[1] + f[1] * kb;
+                s[2] = s[2] + f[2] * kb;
+            }
+        }
+        if (serial) {
+            if (l == 0) {
+                double bi[8], ig[9];
+                d_volume_integrals(P, F, ktg, bitg, loc, bi, ig);
+                for (int t = 0; t < 8; ++t) rec.bi[t] = bi[t];
+                for (int t = 0; t < 9; ++t) rec.ig[t] = ig[t];
+            }
+        } else if (l == 0) {
+            rec.bi[0] = 0.0;
+            rec.bi[1] = loc[2] >= 0.0 && L2 == zpmin ? (d_point_internal(F, L0, L1) ? 0.5 : 0.0) : s[0];
+            rec.bi[2] = s[1];
+            rec.bi[6] = s[2];
+            rec.bi[7] = 0.0;
+        } else if (l == 1) {
+            for (int t = 0; t < 3; ++t) rec.bi[3 + t] = s[t];
+        } else if (l == 2) {
+            for (int t = 0; t < 3; ++t) rec.ig[t] = s[t];
+            rec.ig[3] = s[1];
+            rec.ig[6] = s[2];
+        } else {
+            rec.ig[4] = s[0];
+            rec.ig[5] = rec.ig[7] = s[1];
+            rec.ig[8] = s[2];
+        }
+    }
 }
 
 // kernel-table values at rob times the weight da (InterpolateTable.f90:58-82)
@@ -2663,7 +2798,7 @@ __device__ __forceinline__ double psmooth_end(DPC& P, const DFace* __restrict__ 
 // reciprocal or root 16.5), so the quotients share reciprocals and nothing
 // branches on a pair.  576,000 particles: momentum 499 -> 448 us, velocity
 // smoothing 595 -> 203, continuity 527 -> 206, pressure smoothing 315 -> 170;
-// 72,000: 102 -> 74, 58 -> 33, 58 -> 33, 46 -> 28.  Twice the wavefronts (two
+// 72,000: 102 -> 80, 58 -> 38, 58 -> 37, 46 -> 31.  Twice the wavefronts (two
 // lanes a particle, 1024 threads) measured the same, reading a neighbour's
 // records ahead of the previous one's arithmetic 1% slower.
 // Tiles that do not fit, solves of several masses, and lists that carry stencil
