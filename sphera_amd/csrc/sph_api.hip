@@ -250,7 +250,7 @@ int run_btab(sph_ctx* c, bool again = false) {
     }
     if (c->P.dim == 2) {  // ComputeBoundaryDataTab_2D
         KTime t(c, "boundary_2d");
-        k_boundary_2d<<<nblk(c->P.cap), 256, 0, c->stream>>>(c->S.P, c->d_faces, c->d_bit, c->xm[0], c->cell,
+        k_boundary_2d<<<nblk(c->P.cap, BT2_WG), BT2_WG, 0, c->stream>>>(c->S.P, c->d_faces, c->d_bit, c->xm[0], c->cell,
                                                             c->bn, c->bt, c->iscal);
         return 0;
     }

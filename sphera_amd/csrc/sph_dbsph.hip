@@ -34,13 +34,6 @@ __host__ __device__ __forceinline__ int db_words(int nmaxpartj, int cap) {
     return ((nmaxpartj < cap ? nmaxpartj : cap) + SPH_MW + 2 * DB_G) / 32 + 1;
 }
 
-// LDS written by one lane of a wavefront is read by another
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // wall-element tables: w0 = (x, y, z, weight), w1 = (normal, volume),
 // w2 = (velocity, mass)
 struct DWall {

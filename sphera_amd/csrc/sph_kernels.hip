@@ -145,6 +145,33 @@ __device__ __forceinline__ d2 sqrt64(d2 x) {
     return d2{ends(x.x, g.x), ends(x.y, g.y)};
 }
 
+// lane U's value for lane 0 of each group of up to 16 lanes (the other lanes: any)
+template <int U>
+__device__ __forceinline__ double group_lane(double v) {
+    if constexpr (U == 0) return v;
+    else  // row_shl: lane l of a row of 16 takes lane l + U
+        return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), 0x100 + U, 0xF, 0xF, true),
+                                __builtin_amdgcn_mov_dpp(__double2loint(v), 0x100 + U, 0xF, 0xF, true));
+}
+// adds lane 0's, 1's, .. lane G-1's terms (each lane's t, then its more) to
+// lane 0's sums, in that order
+template <int G, int U = 0, int NS, class... More>
+__device__ __forceinline__ void add_lanes(double (&sum)[NS], const double (&t)[NS], const More&... more) {
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+        sum[c] = sum[c] + group_lane<U>(t[c]);
+        ((sum[c] = sum[c] + group_lane<U>(more[c])), ...);
+    }
+    if constexpr (U + 1 < G) add_lanes<G, U + 1>(sum, t, more...);
+}
+
+// LDS written by one lane of a wavefront is read by another
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // kvals64 of two pairs without branches (a wavefront's lanes differ), its
 // quotients by the reciprocals of the constants
 struct K64x2 { d2 K1, K2, K3, W; };
@@ -1154,27 +1181,34 @@ __device__ __forceinline__ void d_interp2d(const double* __restrict__ tab, int n
     }
 }
 
-__global__ __launch_bounds__(256) void k_boundary_2d(DPC* Pp, const DFace* __restrict__ sides,
+constexpr int BT2_WG = 512;
+struct Corner2D {  // a particle with two close sides
+    int i, side[2];
+    double x[2], y[2];
+};
+
+__global__ __launch_bounds__(BT2_WG) void k_boundary_2d(DPC* Pp, const DFace* __restrict__ sides,
                                                      const double* __restrict__ tab,
                                                      const double4* __restrict__ xm,
                                                      const int* __restrict__ cell,
                                                      int* __restrict__ bn, BTab* __restrict__ bt,
                                                      int* iscal) {
     DPC& P = *Pp;
+    __shared__ Corner2D corners[BT2_WG];
+    __shared__ int ncorner;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= P.cap) return;
-    if (i >= iscal[IS_N]) {
-        bn[i] = 0;
-        return;
-    }
+    if (threadIdx.x == 0) ncorner = 0;
+    __syncthreads();
+    const bool live = i < P.cap && i < iscal[IS_N];
     int nint = 0;
-    const double4 X = xm[i];
+    double4 X = make_double4(0.0, 0.0, 0.0, 0.0);
+    if (live) X = xm[i];
     const double px = X.x, pz = X.z;
     const double dh = P.doubleh;
     int ncbs = 0;
     int clo[4];
     double loc[8];
-    bool bad = false;
+    bool bad = !live;
     for (int isi = 0; isi < P.nf && !bad; ++isi) {
         const DFace& S = sides[isi];
         if (S.btype == 6) continue;  // peri
@@ -1216,11 +1250,8 @@ __global__ __launch_bounds__(256) void k_boundary_2d(DPC* Pp, const DFace* __res
             bad = true;
         }
     }
-    if (bad) {
-        if (ncbs >= 4) atomicAdd(&iscal[IS_BT_OVERFLOW], 1);
-        bn[i] = 0;
-        return;
-    }
+    if (bad && ncbs >= 4) atomicAdd(&iscal[IS_BT_OVERFLOW], 1);
+    if (bad) ncbs = 0;
     if (ncbs == 2) {
         const int a = clo[0], b = clo[1];
         if (sides[a].prev == b + 1)
@@ -1244,126 +1275,163 @@ __global__ __launch_bounds__(256) void k_boundary_2d(DPC* Pp, const DFace* __res
     }
     if (nint > 2) {
         atomicAdd(&iscal[IS_BT_OVERFLOW], 1);
-        bn[i] = 0;
-        return;
+        nint = 0;
     }
     const double h = P.h;
     const double yplimite = 0.05 * h;
     const double dalfarif = PIGRECO_D / 10;
     for (int icbs = 0; icbs < nint; ++icbs) {
         BTab& B = bt[(size_t)icbs * P.cap + i];
-        const double xpi = iloc[2 * icbs];
-        double ypi = iloc[2 * icbs + 1];
+        const double ypi = iloc[2 * icbs + 1];
         B.face = iside[icbs];
-        B.loc[0] = xpi;
+        B.loc[0] = iloc[2 * icbs];
         B.loc[1] = ypi;
         B.loc[2] = 0.0;
+        if (nint == 2) continue;
+        double F[5];
+        const int cols[5] = {1, 2, 3, 4, 5};
+        d_interp2d(tab, 5, cols, ypi / h, F);
+        B.bi[0] = F[0] / h;
+        B.bi[1] = F[1];
+        B.bi[2] = F[1];
+        B.bi[3] = 0.0;
+        B.bi[4] = 0.0;
+        B.bi[5] = F[2] / P.squareh;
+        B.bi[6] = F[3] / P.squareh;
+        B.bi[7] = F[4] / P.squareh;
+    }
+    if (i < P.cap) bn[i] = nint;
+    // The particles near a corner: three quadratures of about ten points a side.
+    // Bound by their latency (sin, cos, tan, atan2; one point after the other
+    // and one side after the other took 32 us at 5,000 particles), so a point is
+    // a lane's, a side 16 lanes', and the third quadrature the other half of the
+    // workgroup's; the sums are formed in order: 13 us.
+    if (nint == 2) {
+        Corner2D& C = corners[atomicAdd(&ncorner, 1)];
+        C.i = i;
+        for (int q = 0; q < 2; ++q) {
+            C.side[q] = iside[q];
+            C.x[q] = iloc[2 * q];
+            C.y[q] = iloc[2 * q + 1];
+        }
+    }
+    __syncthreads();
+    constexpr int HALF = BT2_WG / 2;
+    const int g = threadIdx.x % 16;
+    const bool third = threadIdx.x >= HALF;
+    for (int n = (threadIdx.x % HALF) / 16; n < 2 * ncorner; n += HALF / 16) {
+        const Corner2D& C = corners[n >> 1];
+        const int icbs = n & 1;
+        // point k (from 1) of a sum that steps by d from x0: the running sum itself
+        auto step = [](double x0, double d, int k) {
+            double x = x0;
+            for (int t = 0; t < k; ++t) x = x + d;
+            return x;
+        };
+        BTab& B = bt[(size_t)icbs * P.cap + C.i];
+        const double xpi = C.x[icbs], ypi = C.y[icbs];
         const double deltai = ypi / h;
         double F[5];
-        if (nint == 2) {
-            // FindBoundaryIntersection2D (ypi > 0 here)
-            const double halfchord = sqrt(P.square_doubleh - ypi * ypi);
-            const double XA = xpi - halfchord, XB = xpi + halfchord;
-            double xpmin = 0.0;
-            if (XA > xpmin) xpmin = XA;
-            double xpmax = sides[iside[icbs]].len;
-            if (XB < xpmax) xpmax = XB;
-            double interlen = xpmax - xpmin;
-            if (interlen <= 0.01 * h) interlen = 0.0;
-            // ComputeSurfaceIntegral_WdS2D
-            double IntWdS = 0.0;
-            if (interlen > 0.0) {
-                const double dsrif = h / 2.0;
-                const double ypiq = ypi * ypi;
-                int ndiv = (int)(interlen / dsrif + 0.5);
-                if (ndiv < 2) ndiv = 2;
-                const double deltas = interlen / ndiv;
-                double xpip = xpmin - 0.5 * deltas;
-                for (int ipt = 1; ipt <= ndiv; ++ipt) {
-                    xpip = xpip + deltas;
-                    const double dxpip = xpip - xpi;
+        // FindBoundaryIntersection2D (ypi > 0 here)
+        const double halfchord = sqrt(P.square_doubleh - ypi * ypi);
+        const double XA = xpi - halfchord, XB = xpi + halfchord;
+        double xpmin = 0.0;
+        if (XA > xpmin) xpmin = XA;
+        double xpmax = sides[C.side[icbs]].len;
+        if (XB < xpmax) xpmax = XB;
+        double interlen = xpmax - xpmin;
+        if (interlen <= 0.01 * h) interlen = 0.0;
+        // ComputeSurfaceIntegral_WdS2D
+        double IntWdS[1] = {0.0};
+        if (!third && interlen > 0.0) {
+            const double dsrif = h / 2.0;
+            const double ypiq = ypi * ypi;
+            int ndiv = (int)(interlen / dsrif + 0.5);
+            if (ndiv < 2) ndiv = 2;
+            const double deltas = interlen / ndiv;
+            for (int k0 = 1; k0 <= ndiv; k0 += 16) {
+                double t[1] = {0.0};
+                if (k0 + g <= ndiv) {
+                    const double dxpip = step(xpmin - 0.5 * deltas, deltas, k0 + g) - xpi;
                     const double ris = sqrt(dxpip * dxpip + ypiq);
-                    IntWdS = IntWdS + d_w2(ris, h, P.coefke) * deltas;
+                    t[0] = d_w2(ris, h, P.coefke) * deltas;
                 }
+                add_lanes<16>(IntWdS, t);
             }
-            // BoundaryVolumeIntegrals2D
-            double IntWdV = 0.0, Dp0 = 0.0, Dp1 = 0.0;
-            if (interlen > 0.0) {
-                double yb = ypi;
-                if (yb < yplimite) yb = yplimite;
-                const double alfaA = atan2(xpmin - xpi, yb), alfaB = atan2(xpmax - xpi, yb);
-                const double intalfa = alfaB - alfaA;
-                int ndiv = (int)(intalfa / dalfarif + 0.5);
-                if (ndiv < 1) ndiv = 1;
-                const double dalfa = intalfa / ndiv;
-                double alfa_k = alfaA - 0.5 * dalfa;
-                for (int k = 1; k <= ndiv; ++k) {
-                    alfa_k = alfa_k + dalfa;
+        }
+        // BoundaryVolumeIntegrals2D
+        double V[3] = {0.0, 0.0, 0.0};  // IntWdV, Dp
+        if (!third && interlen > 0.0) {
+            double yb = ypi;
+            if (yb < yplimite) yb = yplimite;
+            const double alfaA = atan2(xpmin - xpi, yb), alfaB = atan2(xpmax - xpi, yb);
+            const double intalfa = alfaB - alfaA;
+            int ndiv = (int)(intalfa / dalfarif + 0.5);
+            if (ndiv < 1) ndiv = 1;
+            const double dalfa = intalfa / ndiv;
+            for (int k0 = 1; k0 <= ndiv; k0 += 16) {
+                double t[3] = {0.0, 0.0, 0.0};
+                if (k0 + g <= ndiv) {
+                    const double alfa_k = step(alfaA - 0.5 * dalfa, dalfa, k0 + g);
                     const double sa = sin(alfa_k), ca = cos(alfa_k);
                     const double rb = yb / ca;
                     const double mult = h * d_j2wro2(rb / h) * dalfa;
-                    Dp0 = Dp0 + sa * mult;
-                    Dp1 = Dp1 - ca * mult;
-                    IntWdV = IntWdV + d_wintegr(rb, h) * dalfa;
+                    t[0] = d_wintegr(rb, h) * dalfa;
+                    t[1] = sa * mult;
+                    t[2] = -(ca * mult);
                 }
-                if (yb == yplimite) IntWdV = 0.5;
+                add_lanes<16>(V, t);
             }
-            // ComputeVolumeIntegral_WdV2D (Ncbslocal = 2)
-            double IntWdV1 = 0.0;
-            if (interlen > 0.0) {
-                if (ypi >= yplimite) {
-                    const double alfaA = atan2(xpmin - xpi, ypi), alfaB = atan2(xpmax - xpi, ypi);
-                    const double intalfa = alfaB - alfaA;
-                    int ndiv = (int)(intalfa / dalfarif + 0.5);
-                    if (ndiv < 2) ndiv = 2;
-                    const double dalfa = intalfa / ndiv;
-                    double alfa = alfaA - 0.5 * dalfa;
-                    for (int ipt = 1; ipt <= ndiv; ++ipt) {
-                        alfa = alfa + dalfa;
-                        const double ta = tan(alfa);
+            if (yb == yplimite) V[0] = 0.5;
+        }
+        // ComputeVolumeIntegral_WdV2D (Ncbslocal = 2)
+        double IntWdV1[1] = {0.0};
+        if (third && interlen > 0.0) {
+            if (ypi >= yplimite) {
+                const double alfaA = atan2(xpmin - xpi, ypi), alfaB = atan2(xpmax - xpi, ypi);
+                const double intalfa = alfaB - alfaA;
+                int ndiv = (int)(intalfa / dalfarif + 0.5);
+                if (ndiv < 2) ndiv = 2;
+                const double dalfa = intalfa / ndiv;
+                for (int k0 = 1; k0 <= ndiv; k0 += 16) {
+                    double t[1] = {0.0};
+                    if (k0 + g <= ndiv) {
+                        const double ta = tan(step(alfaA - 0.5 * dalfa, dalfa, k0 + g));
                         const double ris = ypi * sqrt(1.0 + ta * ta);
-                        IntWdV1 = IntWdV1 + d_wintegr(ris, h) * dalfa;
+                        t[0] = d_wintegr(ris, h) * dalfa;
                     }
+                    add_lanes<16>(IntWdV1, t);
+                }
+            } else {
+                const double ypj = C.y[1 - icbs];
+                if (ypj <= yplimite) {
+                    double angle = 0.0;
+                    if (sides[C.side[0]].prev == C.side[1] + 1)
+                        angle = sides[C.side[0]].angle;
+                    else if (sides[C.side[1]].prev == C.side[0] + 1)
+                        angle = sides[C.side[1]].angle;
+                    else if (g == 0)
+                        atomicAdd(&iscal[IS_UNSUPPORTED], 1);  // sides not consecutive
+                    IntWdV1[0] = 0.5 * (angle + PIGRECO_D) / (2.0 * PIGRECO_D);
                 } else {
-                    const double ypj = iloc[2 * (1 - icbs) + 1];
-                    if (ypj <= yplimite) {
-                        double angle = 0.0;
-                        if (sides[iside[0]].prev == iside[1] + 1)
-                            angle = sides[iside[0]].angle;
-                        else if (sides[iside[1]].prev == iside[0] + 1)
-                            angle = sides[iside[1]].angle;
-                        else
-                            atomicAdd(&iscal[IS_UNSUPPORTED], 1);  // sides not consecutive
-                        IntWdV1 = 0.5 * (angle + PIGRECO_D) / (2.0 * PIGRECO_D);
-                    } else {
-                        IntWdV1 = (xpmin >= xpi && xpi <= xpmax) ? 0.5 : 0.0;
-                    }
+                    IntWdV1[0] = (xpmin >= xpi && xpi <= xpmax) ? 0.5 : 0.0;
                 }
             }
+        }
+        if (g == 0 && third) {
             const int cols[3] = {3, 4, 5};
             d_interp2d(tab, 3, cols, deltai, F);
-            B.bi[0] = IntWdS;
-            B.bi[1] = IntWdV;
-            B.bi[2] = IntWdV1;
-            B.bi[3] = Dp0;
-            B.bi[4] = Dp1;
+            B.bi[2] = IntWdV1[0];
             B.bi[5] = F[0] / P.squareh;
             B.bi[6] = F[1] / P.squareh;
             B.bi[7] = F[2] / P.squareh;
-        } else {
-            const int cols[5] = {1, 2, 3, 4, 5};
-            d_interp2d(tab, 5, cols, deltai, F);
-            B.bi[0] = F[0] / h;
-            B.bi[1] = F[1];
-            B.bi[2] = F[1];
-            B.bi[3] = 0.0;
-            B.bi[4] = 0.0;
-            B.bi[5] = F[2] / P.squareh;
-            B.bi[6] = F[3] / P.squareh;
-            B.bi[7] = F[4] / P.squareh;
+        } else if (g == 0) {
+            B.bi[0] = IntWdS[0];
+            B.bi[1] = V[0];
+            B.bi[3] = V[1];
+            B.bi[4] = V[2];
         }
     }
-    bn[i] = nint;
 }
 
 // ----------------------------------------------------------------------------
@@ -2805,26 +2873,6 @@ __device__ __forceinline__ double psmooth_end(DPC& P, const DFace* __restrict__ 
 // codes (DB-SPH walls) gather from global memory with the same expressions.
 // ----------------------------------------------------------------------------
 #define TILE_ARGS Seg S, Tiles T, const int* __restrict__ start
-
-// lane u's value for lane 0 of each group of G (the other lanes: any)
-template <int U>
-__device__ __forceinline__ double group_lane(double v) {
-    if constexpr (U == 0) return v;
-    else  // row_shl: lane l of a row of 16 takes lane l + U
-        return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), 0x100 + U, 0xF, 0xF, true),
-                                __builtin_amdgcn_mov_dpp(__double2loint(v), 0x100 + U, 0xF, 0xF, true));
-}
-// adds lane 0's, 1's, .. lane G-1's terms (each lane's t, then its more) to
-// lane 0's sums, in that order
-template <int G, int U = 0, int NS, class... More>
-__device__ __forceinline__ void add_lanes(double (&sum)[NS], const double (&t)[NS], const More&... more) {
-#pragma unroll
-    for (int c = 0; c < NS; ++c) {
-        sum[c] = sum[c] + group_lane<U>(t[c]);
-        ((sum[c] = sum[c] + group_lane<U>(more[c])), ...);
-    }
-    if constexpr (U + 1 < G) add_lanes<G, U + 1>(sum, t, more...);
-}
 
 // Adds particle i's NS pair terms to sum in list order, by G lanes (lane g of
 // them; LDS form: 1, 2 or 4): each lane forms the terms of two entries, the lanes' entries
