@@ -48,9 +48,9 @@ typedef struct sph_params {
     int32_t semi;        /* 1: SA-SPH frontiers active (Domain%tipo=="semi") */
     /* launch tunables of the particle kernels (0 = default; the autotuner in
      * sphera_amd/autotune.py picks them per case) */
-    int32_t wg_size;     /* threads per workgroup of the FP64 pair passes: 64 (default), 128, 192 or 256 */
-    int32_t chunk;       /* 4 or 8 (default), accepted for callers that set it, as are the next three: */
-    int32_t chunk_v, chunk_c, chunk_p; /* the list walks have one form each */
+    int32_t wg_size;     /* 64 (default), 128, 192 or 256: accepted for callers that set it, as are the next */
+    int32_t chunk;       /* four, 4 or 8 (default): the pair passes choose their own launch shape */
+    int32_t chunk_v, chunk_c, chunk_p;
     int32_t nb_shape;    /* 0 to 4, accepted for callers that set it: the neighbour search has
                             one launch shape, and the lists never depended on it */
     int32_t options;     /* SPH_OPT_* flags of the deck (below) */
@@ -316,8 +316,8 @@ int sph_segment_download(sph_ctx* ctx, int32_t seg, double* coord, double* vel, 
 int sph_segment_scalars(sph_ctx* ctx, int32_t seg, double out[5]);
 int sph_segment_count(sph_ctx* ctx, int32_t seg, int32_t* n);
 
-/* Launch shape in use: wg_size, list entries prefetched per step of the
- * FP32 list walks, grid of the particle kernels. */
+/* wg_size and chunk as set (both without effect), and the number of wg_size
+ * groups the particles fill. */
 int sph_get_launch(sph_ctx* ctx, int32_t out[3]);
 /* Per-kernel timing of the last sph_step: name/avg-ms pairs, for the bench. */
 int sph_set_timing(sph_ctx* ctx, int32_t on);
