@@ -246,7 +246,10 @@ constexpr int TILE_CAP_L = 2496, TILE_CAP_M = 1632, TILE_CAP_S = 1216, TILE_CAP_
 constexpr int TILE_WG = 512;   // most threads of a pair pass
 constexpr int TILE_U = 5;      // slots a thread stages at a time (FP64: 3)
 constexpr int TILE_G2 = 40000;  // particles below which two lanes take a particle
-constexpr int TILE_G8 = 20000;  // DB-SPH: particles below which eight lanes take a particle, else four
+// DB-SPH: particles below which eight lanes take a particle, else four (step
+// times, us: 2,000 particles eight 265, four 292, two 357; 70,000 eight 611,
+// four 582, two 623)
+constexpr int TILE_G8 = 20000;
 // tiles of water a solve is cut into (choose_tile); FP64
 constexpr int TILE_MIN = 300, TILE_MIN2 = 200, TILE_MIN_L = 500;
 constexpr int TILE_MIN64 = 130, TILE_MIN64_2 = 150;
