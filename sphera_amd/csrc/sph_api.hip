@@ -393,9 +393,10 @@ DWall dwall(const sph_ctx* c) { return DWall{c->d_w0, c->d_w1, c->d_w2, c->d_wst
 int run_dbsph_lists(sph_ctx* c, int mode) {
     KTime t(c, "dbsph_lists");
     const int cap = c->P.cap;
-    // a block of 256 threads, or of one wavefront where its LDS would not fit
+    // a block of 256 threads, or of one wavefront or one particle's lanes where
+    // its LDS would not fit
     const size_t each = (size_t)(db_words(c->P.nmaxpartj, cap) + DB_INTS) * 4;
-    const int wg = each * (256 / DB_G) <= 65536 ? 256 : 64;
+    const int wg = each * (256 / DB_G) <= 65536 ? 256 : each * (64 / DB_G) <= 65536 ? 64 : DB_G;
     const size_t lds = each * (wg / DB_G);
     if (mode == 0)
         k_dbsph_lists<0><<<nblk(DB_G * cap, wg), wg, lds, c->stream>>>(c->S.P, dwall(c), c->xm[0], c->vel[0], c->rp[0], c->cell,

@@ -1,6 +1,6 @@
 """DB-SPH launch forms: lanes per particle by capacity (eight, four) and the
-list kernel's block size by its LDS (long neighbour lists: one wavefront a
-block) give the same bits, and the oracle's."""
+list kernel's block size by its LDS (long neighbour lists: one wavefront or one
+particle a block) give the same bits, and the oracle's."""
 import numpy as np
 import pytest
 
@@ -23,7 +23,7 @@ def small():
     return tb, coord, o.state(), o.dbsph_state()
 
 
-@pytest.mark.parametrize("capacity,nmaxpartj", [(None, None), (19999, None), (20000, None), (20000, 10000)])
+@pytest.mark.parametrize("capacity,nmaxpartj", [(None, None), (19999, None), (20000, None), (20000, 10000), (60000, 60000)])
 def test_dbsph_forms(small, capacity, nmaxpartj):
     from sphera_amd import runtime as rt
     tb, coord, so, do = small
