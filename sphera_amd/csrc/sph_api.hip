@@ -950,6 +950,13 @@ int upload_tables(sph_ctx* c, const sph_faces* const* f) {
     return 0;
 }
 
+// Captured steps hold buffer addresses and the kernels chosen by the constants:
+// dropped where either changes.
+void drop_graphs(sph_ctx* c) {
+    for (auto& g : c->graphs) hipGraphExecDestroy(g.second);
+    c->graphs.clear();
+}
+
 // The constants to the device, after every change of them on the host: a
 // one-solve context's are c->P.  Waits for the kernels that read the old ones.
 int upload_constants(sph_ctx* c) {
@@ -1270,6 +1277,7 @@ int sph_dbsph_walls(sph_ctx* c, const sph_dbsph_walls_t* w) {
     P.neg_wall_p = w->negative_wall_p_allowed ? 1 : 0;
     P.muscl_bnd = w->muscl_boundary ? 1 : 0;
     P.tcap = 0;  // the DB-SPH kernels read the lists' stencil codes
+    drop_graphs(c);
     c->tile_cap = TILE_CAP_0;
     c->tile_g = P.cap < TILE_G8 ? 8 : 4;
     c->tile_wg = 256;
@@ -1296,6 +1304,7 @@ int sph_dbsph_kinematics(sph_ctx* c, int32_t nrec, const double* records, const 
     }
     c->P.nkin = nrec;
     for (int d = 0; d < 3; ++d) c->P.kin_c[d] = nrec > 0 ? centre[d] : 0.0;
+    drop_graphs(c);  // they hold the address of the records replaced, and the kernel reads nkin from the constants
     return upload_constants(c);
 }
 
@@ -1375,9 +1384,7 @@ int sph_segment_upload(sph_ctx* c, int32_t seg, int32_t n, const double* coord, 
             c->P.tcap = Q.tcap;
         }
         if (int rc = upload_constants(c)) return rc;
-        // captured graphs hold the momentum kernel chosen for the old masses
-        for (auto& g : c->graphs) hipGraphExecDestroy(g.second);
-        c->graphs.clear();
+        drop_graphs(c);  // they hold the momentum kernel chosen for the old masses
     }
     if (c->staged.empty()) {  // first segment of a new upload: clear the whole context
         HIPC(hipMemsetAsync(c->lam[0], 0, sizeof(int) * c->P.cap, c->stream));
