@@ -165,7 +165,8 @@ __device__ __forceinline__ void add_lanes(double (&sum)[NS], const double (&t)[N
     if constexpr (U + 1 < G) add_lanes<G, U + 1>(sum, t, more...);
 }
 
-// LDS written by one lane of a wavefront is read by another
+// LDS written by one lane of a wavefront is read by another: the barrier alone
+// orders the lanes but not the compiler's LDS accesses
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -797,16 +798,19 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
             }
             const int kn = min(k, mj);
             if (FIT && lane < 8) list[kn + lane] = (E)((uint32_t)(p + self) << 4);  // fills the last group
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
+            auto run = [&](int e) {  // 16 bytes of the list, stored as entries of either width
+                uint4 v;
+                __builtin_memcpy(&v, __builtin_assume_aligned(list + e, 16), 16);
+                return v;
+            };
             if constexpr (FIT) {
                 for (int e = 8 * lane; e < kn; e += 512)
-                    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(nbr) + nb16_index(N, p, e)) =
-                        *reinterpret_cast<const uint4*>(list + e);
+                    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(nbr) + nb16_index(N, p, e)) = run(e);
             } else {
-                for (int e = 4 * lane; e < kn; e += 256)
-                    *reinterpret_cast<uint4*>(nbr + nb_index(N, p, e)) = *reinterpret_cast<const uint4*>(list + e);
+                for (int e = 4 * lane; e < kn; e += 256) *reinterpret_cast<uint4*>(nbr + nb_index(N, p, e)) = run(e);
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
             mine = lane == u ? kn : mine;
             pairs += kn - 1;
             over += k > mj;
@@ -886,7 +890,7 @@ __global__ __launch_bounds__(256, 4) void k_neighbours(Seg S, const double4* __r
         const int incl = wave_incl_scan(cnt);
         const int total = __builtin_amdgcn_readlane(incl, 63);
         const int hb = __builtin_amdgcn_readlane(b, 13), hc = __builtin_amdgcn_readlane(cnt, 13);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         if (total > NBC_MAX) {
             for (int q = lane; q < hc; q += 64) {
                 bool ov;
@@ -895,10 +899,11 @@ __global__ __launch_bounds__(256, 4) void k_neighbours(Seg S, const double4* __r
                 if (ov) atomicAdd(&iscal[IS_NB_OVERFLOW], 1);
                 atomicAdd(&pairs[(vb % NBC_PAIRS) * NBC_PSTRIDE], (unsigned long long)(k - 1));
             }
+            wave_lds_sync();  // s_aux is reused
             continue;
         }
         for (int u = 0, pre = incl - cnt; u < cnt; ++u) cand[pre + u] = (uint32_t)(b + u) | ((uint32_t)lane << NB_SHIFT);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         if (fits) {
             switch ((total + 63) >> 6) {
                 case 1: mypairs += nb_cell_lists<1, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
