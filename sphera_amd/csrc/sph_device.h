@@ -23,6 +23,11 @@ __host__ __device__ inline size_t nb16_index(size_t N, int p, int k) {
     const unsigned u = (unsigned)k;
     return ((size_t)(u / 16) * N + (size_t)p) * 16 + (size_t)(u % 16);
 }
+// a - b of two integer positions, which count modulo 2^32 (a grid longer than 16
+// cells wraps): subtracted without sign, since a signed difference overflows
+// where a pair lies across a wrap
+__host__ __device__ inline int lsb_diff(int a, int b) { return (int)((uint32_t)a - (uint32_t)b); }
+
 // list capacity per particle: NMAXPARTJ rounded up to whole groups
 __host__ __device__ inline int nb_stride(int nmaxpartj) { return (nmaxpartj + NB_G - 1) / NB_G * NB_G; }
 

@@ -547,8 +547,8 @@ __global__ __launch_bounds__(256) void k_scatter(Seg S, const int* __restrict__ 
 }
 
 // A coordinate relative to the grid's corner in units of lsb, modulo 2^32:
-// the difference of two particles' values, as a signed integer, is their
-// separation wherever that is below 2^31 lsb (eight cells).
+// lsb_diff of two particles' values is their separation wherever that is below
+// 2^31 lsb (eight cells).
 __device__ __forceinline__ int lsb_units(double x, double inv) {
     const double t = rint(x * inv);
     return (int)(uint32_t)(t - floor(t * 0x1p-32) * 0x1p32);
@@ -650,7 +650,8 @@ __device__ int nb_particle_global(DPC& P, int p, const double4* __restrict__ xm,
         const int key = P.koff + ((kk - 1) * nj + (jj - 1)) * ni + ii - 1;
         for (int m = start[key]; m < start[key + 1]; ++m) {
             const int4 xj = xq[m];
-            const float r0 = (float)(xi.x - xj.x), r1 = (float)(xi.y - xj.y), r2 = (float)(xi.z - xj.z);
+            const float r0 = (float)lsb_diff(xi.x, xj.x), r1 = (float)lsb_diff(xi.y, xj.y),
+                        r2 = (float)lsb_diff(xi.z, xj.z);
             const float rr = __builtin_fmaf(r0, r0, __builtin_fmaf(r1, r1, r2 * r2));
             if (rr > hi) continue;
             if (!(rr < lo)) {  // guard band: the reference's FP64 test
@@ -734,9 +735,9 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
         const int4 x = xq[ce[q] & NB_MASK];
         const int a = aux[ce[q] >> NB_SHIFT];
         ce[q] = FIT ? (uint32_t)((int)(ce[q] & NB_MASK) + a) << 4 : (ce[q] & NB_MASK) | (uint32_t)a;
-        cx[q] = (float)(x.x - x0.x);
-        cy[q] = (float)(x.y - x0.y);
-        cz[q] = (float)(x.z - x0.z);
+        cx[q] = (float)lsb_diff(x.x, x0.x);
+        cy[q] = (float)lsb_diff(x.y, x0.y);
+        cz[q] = (float)lsb_diff(x.z, x0.z);
         const float r2 = __builtin_fmaf(cx[q], cx[q], __builtin_fmaf(cy[q], cy[q], cz[q] * cz[q]));
         cq[q] = 64 * q + lane < total ? r2 : 3.0e38f;
     }
@@ -747,7 +748,8 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
         float mx = 0.f, my = 0.f, mz = 0.f, tl = 0.f, th = 0.f;
         if (h0 + lane < hc) {
             const int4 x = xq[hb + h0 + lane];
-            const float fx = (float)(x.x - x0.x), fy = (float)(x.y - x0.y), fz = (float)(x.z - x0.z);
+            const float fx = (float)lsb_diff(x.x, x0.x), fy = (float)lsb_diff(x.y, x0.y),
+                        fz = (float)lsb_diff(x.z, x0.z);
             const float r2 = __builtin_fmaf(fx, fx, __builtin_fmaf(fy, fy, fz * fz));
             mx = -2.0f * fx;
             my = -2.0f * fy;
@@ -3241,9 +3243,9 @@ struct PairR {
 };
 __device__ __forceinline__ PairR pair_r(int4 a, float4 b) {
     PairR d;
-    d.R0 = (float)(a.x - __float_as_int(b.x));
-    d.R1 = (float)(a.y - __float_as_int(b.y));
-    d.R2 = (float)(a.z - __float_as_int(b.z));
+    d.R0 = (float)lsb_diff(a.x, __float_as_int(b.x));
+    d.R1 = (float)lsb_diff(a.y, __float_as_int(b.y));
+    d.R2 = (float)lsb_diff(a.z, __float_as_int(b.z));
     d.rij = __builtin_fmaf(d.R0, d.R0, __builtin_fmaf(d.R1, d.R1, d.R2 * d.R2));
     d.r = __builtin_amdgcn_sqrtf(d.rij);
     return d;

@@ -1,6 +1,7 @@
 """Rules of the device sources that no run shows: the order of LDS accesses
-between the lanes of a wavefront."""
+between the lanes of a wavefront, integer positions across their wrap."""
 import re
+import subprocess
 from pathlib import Path
 
 CSRC = Path(__file__).resolve().parent.parent / "sphera_amd" / "csrc"
@@ -30,3 +31,43 @@ def test_list_runs_are_read_as_bytes():
     before the entries' stores."""
     src = _code("sph_kernels.hip")
     assert not re.search(r"reinterpret_cast<(const )?(uint4|int4)\s*\*>\(list", src)
+
+
+WRAP = r"""
+#define __host__
+#define __device__
+#include "sph_device.h"
+#include <cstdio>
+static int at(long long u) { return (int)(uint32_t)((unsigned long long)u & 0xFFFFFFFFull); }
+int main() {
+    const long long cell = 1ll << 28;
+    long long n = 0;
+    // particles of a grid of 64 cells, two cells apart at most, on both sides of every wrap
+    for (long long c = 0; c < 64; ++c)
+        for (long long o = -3; o <= 3; ++o)
+            for (long long d = -2 * cell - 5; d <= 2 * cell + 5; d += cell / 3 + 1) {
+                const long long a = c * cell + o, b = a + d;
+                if (b < 0) continue;
+                if (sph::lsb_diff(at(a), at(b)) != a - b || sph::lsb_diff(at(b), at(a)) != b - a) return 1;
+                ++n;
+            }
+    std::printf("%lld pairs\n", n);
+    return n > 1000 ? 0 : 2;
+}
+"""
+
+
+def test_integer_positions_wrap_without_overflow(tmp_path):
+    """Separations across a wrap of the integer positions, under the
+    undefined-behaviour sanitizer on the CPU; the kernels form every
+    separation with that one function."""
+    src = tmp_path / "wrap.cpp"
+    src.write_text(WRAP)
+    exe = tmp_path / "wrap"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-fsanitize=undefined", "-fno-sanitize-recover=all",
+                    "-I", str(CSRC), str(src), "-o", str(exe)], check=True)
+    subprocess.run([str(exe)], check=True)
+    code = _code("sph_kernels.hip")
+    assert len(re.findall(r"\(float\)lsb_diff\(", code)) >= 12
+    # no signed difference of positions turned into a float
+    assert not re.findall(r"\(float\)\(\w+\.[xyz] - (?:\w+\.[xyz]\b|__float_as_int)", code)
