@@ -617,6 +617,19 @@ int check_slip_mode(int mode, int btype) {
     return 0;
 }
 
+// The unit of the integer positions and what follows from it.  2D: one cell row
+// holds every particle whatever its y, and the row's side (a caller's; CreaGrid's
+// is near 2h) says nothing about separations.
+void set_lsb(DP& P) {
+    const double side = std::max(P.dim == 2 ? 0.0 : P.dcd[1], std::max(P.dcd[0], P.dcd[2]));
+    P.lsb = side * 0x1p-28;
+    P.inv_lsb = 1.0 / P.lsb;
+    P.f_q = (float)(P.lsb / P.h);
+    P.f_etal = (float)(P.eta * P.inv_lsb);
+    P.f_eta2l = (float)(P.eta2 * P.inv_lsb * P.inv_lsb);
+    P.f_side = (float)side;
+}
+
 // Validates one solve's parameters and fills its constants (placement fields
 // zero).  The reference's values: ReadInput.f90:198-205 (h, 2h, eta, eta2),
 // Gest_Input.f90:266-289 (kernel constants).
@@ -692,12 +705,7 @@ int fill_dp(const sph_params* p, const sph_faces* f, DP& P, bool dry = false) {
     P.pesodt = p->pesodt;
     P.tetap = p->tetap;
     P.tetav = p->tetav;
-    P.lsb = std::max(P.dcd[0], std::max(P.dcd[1], P.dcd[2])) * 0x1p-28;
-    P.inv_lsb = 1.0 / P.lsb;
-    P.f_q = (float)(P.lsb / P.h);
-    P.f_etal = (float)(P.eta * P.inv_lsb);
-    P.f_eta2l = (float)(P.eta2 * P.inv_lsb * P.inv_lsb);
-    for (int d = 0; d < 3; ++d) P.f_dcd[d] = (float)P.dcd[d];
+    set_lsb(P);
     P.f_kin_visc = (float)P.kin_visc;
     P.f_den0 = (float)P.den0;
     P.f_eosk = (float)(P.eps / P.den0);
@@ -1121,6 +1129,7 @@ int sph_ctx_create2d(const sph_params* p, const sph_sides2d* sd, sph_ctx** out) 
     sph_ctx* c = *out;
     DP& P = c->P;
     P.dim = 2;
+    set_lsb(P);
     P.semi = p->semi ? 1 : 0;
     P.nf = sd ? sd->ns : 0;
     P.nopen = P.semi ? nopen : 0;  // open sides (CancelOutgoneParticles_2D)
@@ -1373,8 +1382,13 @@ int sph_segment_upload(sph_ctx* c, int32_t seg, int32_t n, const double* coord, 
     for (int i = 1; i < n && um; ++i) um = mass[i] == mass[0];
     const int umass = um ? 1 : 0;
     const float f_mass = um ? (float)mass[0] : 0.0f;
-    if (umass != P.umass || f_mass != P.f_mass) {
+    // 2D: particles that share y and its velocity share y for good
+    int far_y = 0;
+    for (int i = 1; i < n && P.dim == 2; ++i)
+        if (coord[3 * i + 1] != coord[1] || vel[3 * i + 1] != vel[1]) far_y = 1;
+    if (umass != P.umass || f_mass != P.f_mass || far_y != P.far_y) {
         DP& Q = c->nseg > 1 ? c->segs[seg] : c->P;
+        Q.far_y = far_y;
         Q.umass = umass;
         Q.f_mass = f_mass;
         if (!Q.f32) Q.tcap = umass && !Q.dbsph ? c->tile_cap : 0;  // the FP64 slots hold no mass

@@ -52,11 +52,14 @@ struct DP {
     double ke_coef, kacl_coef, ktdelta, GI;
     double grav[3], prif, den0, eps, celerita, alfamon, kin_visc;
     double cfl, vsc_coeff, pesodt, tetap, tetav;
-    // unit of the integer positions: 2^-28 of the largest cell side
     double inv_h, inv_squareh;  // reciprocals of h and squareh
+    // unit of the integer positions: 2^-28 of the largest cell side (2D: in the plane)
     double lsb, inv_lsb;
+    float f_side;  // that side
+    // 2D: the particles differ in y, where they may lie whole wraps apart
+    int far_y;
     // FP32-mixed pair sums: h, eta and eta2 in units of lsb (f_q = lsb / h)
-    float f_q, f_etal, f_eta2l, f_dcd[3], f_kin_visc;
+    float f_q, f_etal, f_eta2l, f_kin_visc;
     // the density slot of the FP32 velocity records holds rho - den0; the
     // linear EoS p = eps/den0 (rho - den0) + prif gives the pressure from it
     float f_den0, f_eosk, f_prif;

@@ -695,7 +695,9 @@ __device__ int nb_particle_global(DPC& P, int p, const double4* __restrict__ xm,
 // A wavefront takes the cells whose first particle lies in its NBC_SLOTS
 // sorted slots: about one cell, so small solves spread over the chip.
 // Cells with more candidates than the registers hold (denser than 1.35 times
-// water) take one lane per particle from global memory.
+// water) take one lane per particle from global memory, as do 2D solves whose
+// particles differ in y: there two may lie whole wraps of the integer positions
+// apart, so every candidate the FP32 test takes goes to the FP64 test.
 constexpr int NBC_CH = 10;             // chunks of 64 candidates in registers
 constexpr int NBC_MAX = 64 * NBC_CH;
 constexpr int NBC_SLOTS = 16, NBC_SLOTS_L = 64;  // sorted slots per wavefront: small, large solves
@@ -842,8 +844,7 @@ __global__ __launch_bounds__(256, 4) void k_neighbours(Seg S, const double4* __r
     if (vb * 4 * slots - P.base >= n) return;
     const int ni = P.ncd[0], nj = P.ncd[1], nk = P.ncd[2];
     const float sq = (float)(P.square_doubleh * P.inv_lsb * P.inv_lsb);
-    const float dm = fmaxf(P.f_dcd[0], fmaxf(P.f_dcd[1], P.f_dcd[2]));
-    const float band = 4.0e-5f * fmaxf(1.0f, dm * dm / (float)P.square_doubleh);
+    const float band = 4.0e-5f * fmaxf(1.0f, P.f_side * P.f_side / (float)P.square_doubleh);
     const float lo = sq * (1.0f - band), hi = sq * (1.0f + band);
     const int s0 = (vb * 4 + wid) * slots;
     uint32_t* cand = s_cand[wid];
@@ -893,10 +894,11 @@ __global__ __launch_bounds__(256, 4) void k_neighbours(Seg S, const double4* __r
         const int total = __builtin_amdgcn_readlane(incl, 63);
         const int hb = __builtin_amdgcn_readlane(b, 13), hc = __builtin_amdgcn_readlane(cnt, 13);
         wave_lds_sync();
-        if (total > NBC_MAX) {
+        if (total > NBC_MAX || P.far_y) {
             for (int q = lane; q < hc; q += 64) {
                 bool ov;
-                const int k = nb_particle_global(P, hb + q, xm, xq, cell, start, nbr, s_aux[wid], fits, lo, hi, ov);
+                const int k = nb_particle_global(P, hb + q, xm, xq, cell, start, nbr, s_aux[wid], fits,
+                                                 P.far_y ? -1.0f : lo, hi, ov);
                 nnb[hb + q] = k;
                 if (ov) atomicAdd(&iscal[IS_NB_OVERFLOW], 1);
                 atomicAdd(&pairs[(vb % NBC_PAIRS) * NBC_PSTRIDE], (unsigned long long)(k - 1));
