@@ -239,7 +239,8 @@ int sph_free_surface(sph_ctx* ctx, double* pelolib, double* zlft);
  * sum_i (nPartIntorno(i) - 1) (the unit of the pair-interactions/s metric). */
 int sph_pair_counter(sph_ctx* ctx, unsigned long long* total);
 /* Debug: neighbour lists in pg order, entries are pg indices (0-based), in the
- * reference's list order.  stride >= nmaxpartj. */
+ * reference's list order.  stride >= nmaxpartj.  All counts are 0 between a
+ * sort (also the upload's) and the next search. */
 int sph_get_neighbour_lists(sph_ctx* ctx, int32_t* count, int32_t* ids, int32_t stride);
 /* Debug: the SA-SPH boundary table (BoundaryDataTab, ComputeBoundaryDataTab_3D
  * .f90:62-106) in pg order: ncbf[r] close faces of row r; for slot q < ncbf[r]

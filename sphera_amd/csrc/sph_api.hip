@@ -117,6 +117,7 @@ struct sph_ctx {
     int* mon_icont = nullptr;
     double *mon_pts = nullptr, *mon_out = nullptr;
     Phase phase = PH_EMPTY;
+    bool lists_ok = false;  // the neighbour lists are of the present order
     bool timing = false;
     std::vector<Timer> timers;
     std::vector<hipEvent_t> ev;
@@ -209,6 +210,7 @@ int run_sort(sph_ctx* c) {
     const int m = c->nkeys;
     const int cap = c->P.cap;
     const int nsb = nblk(m, SCAN_B);
+    c->lists_ok = false;
     {
         KTime t(c, "sort_count");
         SEGL(k_cell_count, nblk(cap), 256, c->xm[1], c->vel[2], c->key, c->slot, c->cnt, c->idslot, c->rmids,
@@ -236,6 +238,7 @@ int run_sort(sph_ctx* c) {
 
 int run_neighbours(sph_ctx* c) {
     KTime t(c, "neighbours");
+    c->lists_ok = true;
     const int slots = c->P.cap < NBC_LARGE ? NBC_SLOTS : NBC_SLOTS_L;
     SEGL(k_neighbours, nblk(c->P.cap, 4 * slots), 256, c->xm[0], c->xq, c->cell, c->start, c->nbr, c->nnb,
          c->iscal, c->pairs, slots);
@@ -1679,6 +1682,10 @@ int sph_get_neighbour_lists(sph_ctx* c, int32_t* count, int32_t* ids, int32_t st
     HIPC(hipStreamSynchronize(c->stream));
     int n;
     HIPC(hipMemcpy(&n, c->iscal + IS_N, sizeof(int), hipMemcpyDeviceToHost));
+    if (!c->lists_ok) {  // a sort came after the lists, whose slots and indices are of the order before
+        std::fill(count, count + n, 0);
+        return 0;
+    }
     const size_t N = c->P.cap;
     std::vector<int> nn(n);
     std::vector<double4> hv(n);
