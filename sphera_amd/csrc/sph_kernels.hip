@@ -627,14 +627,14 @@ __global__ void k_gather(Seg S, const int* __restrict__ perm, const int* __restr
 // is decided by the reference's FP64 expression on the FP64 positions, so the
 // lists are exactly the reference's.
 // ----------------------------------------------------------------------------
-// One lane per particle, candidates from global memory (cells too dense for
-// the wavefront form below).  aux: per stencil cell in list order what turns
-// a sorted index into its list entry.  Every accepted candidate is counted;
-// the first NMAXPARTJ are stored, as in the reference.
+// One lane per particle, candidates from global memory, every one that FP32
+// finds near decided in FP64 (P.far_y).  aux: per stencil cell in list order
+// what turns a sorted index into its list entry.  Every accepted candidate is
+// counted; the first NMAXPARTJ are stored, as in the reference.  Returns the count.
 __device__ int nb_particle_global(DPC& P, int p, const double4* __restrict__ xm,
                                   const int4* __restrict__ xq, const int* __restrict__ cell,
                                   const int* __restrict__ start, uint32_t* __restrict__ nbr,
-                                  const int* aux, bool fits, float lo, float hi, bool& ov) {
+                                  const int* aux, bool fits, float hi) {
     const int ni = P.ncd[0], nj = P.ncd[1], nk = P.ncd[2];
     const int mj = P.nmaxpartj;
     const size_t N = P.cap;
@@ -654,13 +654,11 @@ __device__ int nb_particle_global(DPC& P, int p, const double4* __restrict__ xm,
                         r2 = (float)lsb_diff(xi.z, xj.z);
             const float rr = __builtin_fmaf(r0, r0, __builtin_fmaf(r1, r1, r2 * r2));
             if (rr > hi) continue;
-            if (!(rr < lo)) {  // guard band: the reference's FP64 test
-                const double4 xj64 = xm[m];
-                const double d0 = xi64.x - xj64.x;
-                const double d1 = xi64.y - xj64.y;
-                const double d2 = xi64.z - xj64.z;
-                if (d0 * d0 + d1 * d1 + d2 * d2 > P.square_doubleh) continue;
-            }
+            const double4 xj64 = xm[m];
+            const double d0 = xi64.x - xj64.x;
+            const double d1 = xi64.y - xj64.y;
+            const double d2 = xi64.z - xj64.z;
+            if (d0 * d0 + d1 * d1 + d2 * d2 > P.square_doubleh) continue;
             if (k < mj) {
                 if (fits) nbr16[nb16_index(N, p, k)] = (uint16_t)((m + aux[t]) << 4);
                 else nbr[nb_index(N, p, k)] = (uint32_t)m | (uint32_t)aux[t];
@@ -668,10 +666,8 @@ __device__ int nb_particle_global(DPC& P, int p, const double4* __restrict__ xm,
             ++k;
         }
     }
-    ov = k > mj;
-    k = min(k, mj);
     if (fits)
-        for (int q = k; q & 7; ++q) nbr16[nb16_index(N, p, q)] = (uint16_t)((p + aux[13]) << 4);
+        for (int q = min(k, mj); q & 7; ++q) nbr16[nb16_index(N, p, q)] = (uint16_t)((p + aux[13]) << 4);
     return k;
 }
 
@@ -694,11 +690,18 @@ __device__ int nb_particle_global(DPC& P, int p, const double4* __restrict__ xm,
 // guard band 4e-5 (2h)^2 (wider for cells larger than 2h) goes to the FP64 test.
 // A wavefront takes the cells whose first particle lies in its NBC_SLOTS
 // sorted slots: about one cell, so small solves spread over the chip.
-// Cells with more candidates than the registers hold (denser than 1.35 times
-// water) take one lane per particle from global memory, as do 2D solves whose
-// particles differ in y: there two may lie whole wraps of the integer positions
-// apart, so every candidate the FP32 test takes goes to the FP64 test.
-constexpr int NBC_CH = 10;             // chunks of 64 candidates in registers
+// More candidates than the registers hold (27 cells of lattice water at h/dx of
+// 1.4 and more, clusters) are taken in equal parts, one after the other, for 64
+// particles of the cell at a time: a particle's count and the entries that do
+// not fill a store yet wait in a register and in LDS for the next part.
+// (One lane per particle over global memory before: 576,000 particles at h/dx of
+// 1.4 831 -> 262 us, at 1.5 1550 -> 350; 72,000 189 -> 67, 216 -> 78; a cluster
+// of twice the density 260 -> 91.)  A part has five to eight chunks: forms of
+// nine and ten beside these spilled and took 163 -> 173 us from the common one.
+// 2D solves whose particles differ in y take one lane per particle from global
+// memory: two of them may lie whole wraps of the integer positions apart, so
+// every candidate the FP32 test takes goes to the FP64 test.
+constexpr int NBC_CH = 9;              // chunks of 64 candidates in registers
 constexpr int NBC_MAX = 64 * NBC_CH;
 constexpr int NBC_SLOTS = 16, NBC_SLOTS_L = 64;  // sorted slots per wavefront: small, large solves
 constexpr int NBC_LARGE = 150000;      // particles from which the chip is full with 64 slots per wavefront
@@ -710,17 +713,24 @@ __device__ __forceinline__ float readlane_f(float v, int l) {
 }
 
 // The cell's particles hb .. hb+hc-1 against its `total` candidates, NCH chunks
-// of 64 (64 (NCH-1) < total <= 64 NCH).  A lane without a hit writes to the
+// of 64 (total <= 64 NCH).  A lane without a hit writes to the
 // slot past the list, so a chunk's append has no branch.  FIT: 16-bit entries
 // (the tile fits LDS).  Returns the sum of the list lengths without the
 // particles themselves; over counts truncated lists.
-template <int NCH, bool FIT>
+// PART: one part of the candidates against the particles from h0 on, 64 at
+// most: mine holds the lengths so far (lane u: particle h0 + u), tail the last
+// length % 8 entries of each; last: the last part.
+constexpr int NBC_VOID = NBC_MAX + 16;  // the slot of a lane without a hit, past the list and what fills it up
+template <int NCH, bool FIT, bool PART = false>
 __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__ xm,
                                              const int4* __restrict__ xq, const uint32_t* cand, const int* aux,
                                              uint32_t* list32, int total, int hb, int hc, float lo, float hi,
-                                             uint32_t* __restrict__ nbr, int* __restrict__ nnb, int& over) {
+                                             uint32_t* __restrict__ nbr, int* __restrict__ nnb, int& over,
+                                             int h0 = 0, bool last = true, uint32_t* tail32 = nullptr,
+                                             int* lengths = nullptr) {
     using E = typename std::conditional<FIT, uint16_t, uint32_t>::type;
     E* list = reinterpret_cast<E*>(list32);
+    E* tail = reinterpret_cast<E*>(tail32);
     const int lane = threadIdx.x & 63;
     const int mj = P.nmaxpartj;
     const size_t N = P.cap;
@@ -745,7 +755,7 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
     }
     const int self = FIT ? aux[13] : 0;
     int pairs = 0;
-    for (int h0 = 0; h0 < hc; h0 += 64) {
+    for (; h0 < hc; h0 += 64) {
         // the lane's own particle of the cell, as it enters the test
         float mx = 0.f, my = 0.f, mz = 0.f, tl = 0.f, th = 0.f;
         if (h0 + lane < hc) {
@@ -760,7 +770,7 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
             th = hi - r2;
         }
         const int hn = min(64, hc - h0);
-        int mine = 0;  // list length of the lane's own particle
+        int mine = PART ? *lengths : 0;  // list length of the lane's own particle
         for (int u = 0; u < hn; ++u) {
             const int p = hb + h0 + u;
             const float ax = readlane_f(mx, u), ay = readlane_f(my, u), az = readlane_f(mz, u);
@@ -769,12 +779,15 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
                 return __builtin_fmaf(ax, cx[q], __builtin_fmaf(ay, cy[q], __builtin_fmaf(az, cz[q], cq[q])));
             };
             unsigned long long guard = 0ull;
-            int k = 0;
+            const int before = PART ? __builtin_amdgcn_readlane(mine, u) : 0;
+            const int base = before & ~7;  // the list's first entry in LDS
+            int k = before & 7;
+            if (PART && lane < 8) list[lane] = tail[8 * u + lane];
             auto append = [&](int q, bool in) {
                 const unsigned long long m = __ballot(in);
                 const int at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, k));
-                list[in ? at : NBC_MAX + 8] = (E)ce[q];
+                list[in ? at : NBC_VOID] = (E)ce[q];
                 k += __popcll(m);
                 return m;
             };
@@ -785,7 +798,7 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
             }
             if (guard) {  // candidates in the guard band (1 particle in 100): the reference's FP64 test
                 const double4 xi = xm[p];
-                k = 0;
+                k = before & 7;
 #pragma unroll
                 for (int q = 0; q < NCH; ++q) {
                     const float r2 = r2of(q);
@@ -800,8 +813,12 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
                     append(q, in);
                 }
             }
-            const int kn = min(k, mj);
-            if (FIT && lane < 8) list[kn + lane] = (E)((uint32_t)(p + self) << 4);  // fills the last group
+            const int room = mj - base;  // entries that the list still takes from `base` on
+            // entries to store; the last group filled with the particle itself, as often as it is formed
+            const int kn = PART ? max(0, min(last ? k : k & ~7, room)) : min(k, mj);
+            const int end = PART ? min(k, room) : kn;
+            if (FIT && lane < 8 && (!PART || ((last || room < k) && room >= 0)))
+                list[end + lane] = (E)((uint32_t)(p + self) << 4);
             wave_lds_sync();
             auto run = [&](int e) {  // 16 bytes of the list, stored as entries of either width
                 uint4 v;
@@ -810,16 +827,25 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
             };
             if constexpr (FIT) {
                 for (int e = 8 * lane; e < kn; e += 512)
-                    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(nbr) + nb16_index(N, p, e)) = run(e);
+                    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(nbr) + nb16_index(N, p, base + e)) = run(e);
             } else {
-                for (int e = 4 * lane; e < kn; e += 256) *reinterpret_cast<uint4*>(nbr + nb_index(N, p, e)) = run(e);
+                for (int e = 4 * lane; e < kn; e += 256)
+                    *reinterpret_cast<uint4*>(nbr + nb_index(N, p, base + e)) = run(e);
             }
+            if (PART && lane < 8) tail[8 * u + lane] = list[(k & ~7) + lane];
             wave_lds_sync();
-            mine = lane == u ? kn : mine;
-            pairs += kn - 1;
-            over += k > mj;
+            const int len = last ? min(base + k, mj) : base + k;
+            mine = lane == u ? len : mine;
+            if (last) {
+                pairs += len - 1;
+                over += base + k > mj;
+            }
         }
-        if (lane < hn) nnb[hb + h0 + lane] = mine;
+        if (last && lane < hn) nnb[hb + h0 + lane] = mine;
+        if (PART) {
+            *lengths = mine;
+            break;
+        }
     }
     return pairs;
 }
@@ -832,10 +858,11 @@ __global__ __launch_bounds__(256, 4) void k_neighbours(Seg S, const double4* __r
                                                     uint32_t* __restrict__ nbr, int* __restrict__ nnb,
                                                     int* iscal, unsigned long long* pairs, int slots) {
     __shared__ uint32_t s_cand[4][NBC_MAX];  // a wave's candidates: sorted index | stencil cell in list order
-    __shared__ __align__(16) uint32_t s_list[4][NBC_MAX + 12];  // the list of its current particle
+    __shared__ __align__(16) uint32_t s_list[4][NBC_VOID + 4];  // the list of its current particle
+    __shared__ uint32_t s_tail[4][64 * 8];  // candidates in parts: entries that wait for the next part
     __shared__ int s_aux[4][28];  // per stencil cell: sorted index to slot, or the stencil code's bits
     __shared__ int s_pairs[4];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int vb = xcd_block(gridDim.x);
     const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * 4 * slots) >> 8]) : 0;
     DPC& P = S.P[sg];
@@ -894,47 +921,78 @@ __global__ __launch_bounds__(256, 4) void k_neighbours(Seg S, const double4* __r
         const int total = __builtin_amdgcn_readlane(incl, 63);
         const int hb = __builtin_amdgcn_readlane(b, 13), hc = __builtin_amdgcn_readlane(cnt, 13);
         wave_lds_sync();
-        if (total > NBC_MAX || P.far_y) {
-            for (int q = lane; q < hc; q += 64) {
-                bool ov;
-                const int k = nb_particle_global(P, hb + q, xm, xq, cell, start, nbr, s_aux[wid], fits,
-                                                 P.far_y ? -1.0f : lo, hi, ov);
-                nnb[hb + q] = k;
-                if (ov) atomicAdd(&iscal[IS_NB_OVERFLOW], 1);
-                atomicAdd(&pairs[(vb % NBC_PAIRS) * NBC_PSTRIDE], (unsigned long long)(k - 1));
+#define NB_LISTS(n, fit) mypairs += nb_cell_lists<n, fit>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over)
+#define NB_PART(n, fit)                                                                                               \
+    mypairs += nb_cell_lists<n, fit, true>(P, xm, xq, cand, s_aux[wid], list, c1 - c0, hb, hc, lo, hi, nbr, nnb, over, \
+                                           h0, c1 == total, s_tail[wid], &lengths)
+        if (__builtin_expect(total > NBC_MAX || P.far_y, 0)) {
+            if (P.far_y) {
+                for (int q = lane; q < hc; q += 64) {
+                    const int found = nb_particle_global(P, hb + q, xm, xq, cell, start, nbr, s_aux[wid], fits, hi);
+                    const int k = min(found, P.nmaxpartj);
+                    nnb[hb + q] = k;
+                    if (found > k) atomicAdd(&iscal[IS_NB_OVERFLOW], 1);
+                    atomicAdd(&pairs[(vb % NBC_PAIRS) * NBC_PSTRIDE], (unsigned long long)(k - 1));
+                }
+                wave_lds_sync();  // s_aux is reused
+                continue;
             }
-            wave_lds_sync();  // s_aux is reused
+            const int chunks = (total + 63) >> 6, parts = (chunks + 7) / 8;
+            const int per = (chunks + parts - 1) / parts;  // chunks of a part: 5 to 8
+            for (int h0 = 0; h0 < hc; h0 += 64) {
+                int lengths = 0;
+                for (int c0 = 0; c0 < total; c0 += 64 * per) {
+                    const int c1 = min(total, c0 + 64 * per);
+                    const int first = incl - cnt;  // the lane's cell: its first candidate
+                    for (int c = max(first, c0); c < min(incl, c1); ++c)
+                        cand[c - c0] = (uint32_t)(b + c - first) | ((uint32_t)lane << NB_SHIFT);
+                    wave_lds_sync();
+                    if (per == 5) {
+                        if (fits) NB_PART(5, true);
+                        else NB_PART(5, false);
+                    } else if (per == 6) {
+                        if (fits) NB_PART(6, true);
+                        else NB_PART(6, false);
+                    } else if (per == 7) {
+                        if (fits) NB_PART(7, true);
+                        else NB_PART(7, false);
+                    } else {
+                        if (fits) NB_PART(8, true);
+                        else NB_PART(8, false);
+                    }
+                }
+            }
             continue;
         }
         for (int u = 0, pre = incl - cnt; u < cnt; ++u) cand[pre + u] = (uint32_t)(b + u) | ((uint32_t)lane << NB_SHIFT);
         wave_lds_sync();
         if (fits) {
             switch ((total + 63) >> 6) {
-                case 1: mypairs += nb_cell_lists<1, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 2: mypairs += nb_cell_lists<2, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 3: mypairs += nb_cell_lists<3, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 4: mypairs += nb_cell_lists<4, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 5: mypairs += nb_cell_lists<5, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 6: mypairs += nb_cell_lists<6, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 7: mypairs += nb_cell_lists<7, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 8: mypairs += nb_cell_lists<8, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 9: mypairs += nb_cell_lists<9, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 10: mypairs += nb_cell_lists<10, true>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 1: NB_LISTS(1, true); break;
+                case 2: NB_LISTS(2, true); break;
+                case 3: NB_LISTS(3, true); break;
+                case 4: NB_LISTS(4, true); break;
+                case 5: NB_LISTS(5, true); break;
+                case 6: NB_LISTS(6, true); break;
+                case 7: NB_LISTS(7, true); break;
+                case 8: NB_LISTS(8, true); break;
+                case 9: NB_LISTS(9, true); break;
             }
         } else {
             switch ((total + 63) >> 6) {
-                case 1: mypairs += nb_cell_lists<1, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 2: mypairs += nb_cell_lists<2, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 3: mypairs += nb_cell_lists<3, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 4: mypairs += nb_cell_lists<4, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 5: mypairs += nb_cell_lists<5, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 6: mypairs += nb_cell_lists<6, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 7: mypairs += nb_cell_lists<7, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 8: mypairs += nb_cell_lists<8, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 9: mypairs += nb_cell_lists<9, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
-                case 10: mypairs += nb_cell_lists<10, false>(P, xm, xq, cand, s_aux[wid], list, total, hb, hc, lo, hi, nbr, nnb, over); break;
+                case 1: NB_LISTS(1, false); break;
+                case 2: NB_LISTS(2, false); break;
+                case 3: NB_LISTS(3, false); break;
+                case 4: NB_LISTS(4, false); break;
+                case 5: NB_LISTS(5, false); break;
+                case 6: NB_LISTS(6, false); break;
+                case 7: NB_LISTS(7, false); break;
+                case 8: NB_LISTS(8, false); break;
+                case 9: NB_LISTS(9, false); break;
             }
         }
+#undef NB_LISTS
+#undef NB_PART
     }
     // pair-interaction counter: sum_i (nPartIntorno(i) - 1), self excluded
     if (lane == 0) {
