@@ -85,7 +85,13 @@ struct sph_ctx {
     int nrep = 1;  // copies of the scan blocks' sums
     int *tlist = nullptr, *ntile = nullptr;  // the tiles that hold particles, their number
     int ntiles = 0;                          // tile ids of all segments (whole 256-blocks)
-    int tile_cap = 0, tile_grid = 8, tile_wg = 64, tile_g = 1;  // slots of the pair passes' LDS form, their launch shape
+    // the pair passes' form: slots of the LDS form (TILE_CAP_0: gathers), launch
+    // shape; in use, and that of choose_tile
+    struct Form {
+        int cap = 0, grid = 8, wg = 64, g = 1;  // g: lanes a particle
+        double home = 0.0, pairs = 0.0;         // particles of a full tile, pairs of a particle
+    } form, lds_form;
+    int ncu = 256;  // CUs
     int *work = nullptr, *nwork = nullptr;  // (particle, face) pairs of the boundary table
     int *idslot = nullptr, *rmids = nullptr;  // id -> slot, ids removed by a sort
     int wg = 256, grid = 1, bt_grid = 1024;  // launch shape of the particle kernels
@@ -285,37 +291,35 @@ using IntC = std::integral_constant<int, V>;
 template <class Launch>
 void tile_dispatch(sph_ctx* c, Launch&& launch) {
     auto form = [&](auto sg) {
-        if (c->tile_cap == TILE_CAP_L) launch(IntC<TILE_CAP_L>{}, sg, IntC<1>{});
-        else if (c->tile_cap == TILE_CAP_M) launch(IntC<TILE_CAP_M>{}, sg, IntC<1>{});
-        else if (c->tile_g == 1) launch(IntC<TILE_CAP_S>{}, sg, IntC<1>{});
-        else launch(IntC<TILE_CAP_S>{}, sg, IntC<2>{});
+        if (c->form.cap == TILE_CAP_L) launch(IntC<TILE_CAP_L>{}, sg, IntC<1>{});
+        else if (c->form.cap == TILE_CAP_M) launch(IntC<TILE_CAP_M>{}, sg, IntC<1>{});
+        else if (c->form.cap == TILE_CAP_S && c->form.g == 1) launch(IntC<TILE_CAP_S>{}, sg, IntC<1>{});
+        else if (c->form.cap == TILE_CAP_S) launch(IntC<TILE_CAP_S>{}, sg, IntC<2>{});
+        else if (c->form.g == 1) launch(IntC<TILE_CAP_0>{}, sg, IntC<1>{});
+        else launch(IntC<TILE_CAP_0>{}, sg, IntC<2>{});
     };
     if (c->nseg > 1) form(std::true_type{});
     else form(std::false_type{});
 }
-// The FP64 passes.  TILE_CAP_0 (lists with stencil codes): no LDS form, lanes
-// by particles.
+// The FP64 passes (no LDS form with eight lanes).
 template <class Launch>
 void tile_dispatch64(sph_ctx* c, Launch&& launch) {
-    if (c->tile_cap == TILE_CAP_0) {
-        if (c->tile_g == 4) launch(IntC<TILE_CAP_0>{}, std::false_type{}, IntC<4>{});
-        else launch(IntC<TILE_CAP_0>{}, std::false_type{}, IntC<8>{});
-        return;
-    }
     auto lanes = [&](auto cap, auto sg) {
-        if (c->tile_g == 1) launch(cap, sg, IntC<1>{});
-        else if (c->tile_g == 2) launch(cap, sg, IntC<2>{});
+        if (c->form.g == 1) launch(cap, sg, IntC<1>{});
+        else if (c->form.g == 2) launch(cap, sg, IntC<2>{});
         else launch(cap, sg, IntC<4>{});
     };
     auto form = [&](auto sg) {
-        if (c->tile_cap == TILE_CAP_L) lanes(IntC<TILE_CAP_L>{}, sg);
-        else lanes(IntC<TILE_CAP_S>{}, sg);
+        if (c->form.cap == TILE_CAP_L) lanes(IntC<TILE_CAP_L>{}, sg);
+        else if (c->form.cap == TILE_CAP_S) lanes(IntC<TILE_CAP_S>{}, sg);
+        else if (c->form.g == 8) launch(IntC<TILE_CAP_0>{}, sg, IntC<8>{});
+        else lanes(IntC<TILE_CAP_0>{}, sg);
     };
     if (c->nseg > 1) form(std::true_type{});
     else form(std::false_type{});
 }
 #define TILE_RUN(...) \
-    <<<c->tile_grid, c->tile_wg, 0, c->stream>>>(c->S, Tiles{c->tlist, c->ntile}, c->start, __VA_ARGS__)
+    <<<c->form.grid, c->form.wg, 0, c->stream>>>(c->S, Tiles{c->tlist, c->ntile}, c->start, __VA_ARGS__)
 
 int run_momentum(sph_ctx* c) {
     KTime t(c, "momentum");
@@ -421,7 +425,7 @@ int run_dbsph_lists(sph_ctx* c, int mode) {
 
 template <class Launch>
 void dbsph_lanes(sph_ctx* c, Launch&& launch) {
-    if (c->tile_g == 4) launch(IntC<4>{});
+    if (c->form.g == 4) launch(IntC<4>{});
     else launch(IntC<8>{});
 }
 
@@ -538,7 +542,7 @@ int sph_ctx::alloc() {
     HIPC(da(&dr, P.f32 ? N : 1));
     for (auto& p : vf) HIPC(da(&p, P.f32 ? N : 1));
     HIPC(da(&tlist, ntiles ? (size_t)ntiles : 1));
-    HIPC(da(&ntile, 1));
+    HIPC(da(&ntile, 2));
     HIPC(da(&dden, N));
     HIPC(da(&vpres, N));
     HIPC(da(&dden2, P.rk1 ? N : 1));
@@ -577,7 +581,7 @@ int sph_ctx::alloc() {
         HIPC(hipMemset(dden2, 0, sizeof(double) * N));
         HIPC(hipMemset(vpres2, 0, sizeof(double) * N));
     }
-    HIPC(hipMemset(ntile, 0, sizeof(int)));
+    HIPC(hipMemset(ntile, 0, 2 * sizeof(int)));
     // every sort leaves its counters cleared for the next
     HIPC(hipMemset(cnt, 0, sizeof(int) * m));
     HIPC(hipMemset(bsum, 0, sizeof(int) * (size_t)nrep * nblk((int)m, SCAN_B)));
@@ -735,8 +739,12 @@ inline int round256(long long v) { return (int)((v + 255) / 256 * 256); }
 // 2x1x1 236, 1x1x1 252, 3x1x1 258; 2D 61,000 7x6 167, 8x8 172, 6x5 183; 20,000
 // 4x4 130, 6x5 142, 3x3 143; 5,000 3x3 115, 2x2 119, 4x4 122.  Lanes: 72,000
 // one 379, two 410; 50,000 (3x3x2) two 327, one 355; 20,000 (3x2x2) two 276,
-// four 306; 2D 20,000 four 130, two 139; 5,000 four 119, two 123.
+// four 306; 2D 20,000 four 130, two 139; 5,000 four 119, two 123; two lanes up to
+// 384 particles a tile, where they leave the SIMDs three half walks instead of
+// two whole ones: a cloud of 16.7 million, 370 a tile, 42.3 -> 37.5 ms; 576,000 at
+// h/dx = 1.5, 323 a tile, 2374 -> 2129.
 void choose_tile(sph_ctx* c) {
+    sph_ctx::Form& F = c->lds_form;
     const int L3[][3] = {{3, 3, 3}, {3, 3, 2}, {3, 2, 2}, {3, 2, 1}, {3, 1, 1}, {2, 1, 1}, {1, 1, 1}};
     const int L2[][3] = {{8, 1, 8}, {7, 1, 6}, {6, 1, 5}, {4, 1, 4}, {3, 1, 3}, {2, 1, 2}, {1, 1, 1}};
     const DP& A = c->segs[0];
@@ -756,16 +764,16 @@ void choose_tile(sph_ctx* c) {
         const int least = !A.f32 ? (flat ? TILE_MIN64_2 : TILE_MIN64) : k == 0 ? TILE_MIN_L : flat ? TILE_MIN2 : TILE_MIN;
         if (need <= TILE_CAP_L && A.cap >= least * home) break;
     }
-    c->tile_cap = need <= TILE_CAP_S ? TILE_CAP_S : need <= TILE_CAP_M ? TILE_CAP_M : TILE_CAP_L;
-    c->tile_g = c->tile_cap != TILE_CAP_S ? 1 : A.cap < TILE_G2 ? 2 : 1;
+    F.cap = need <= TILE_CAP_S ? TILE_CAP_S : need <= TILE_CAP_M ? TILE_CAP_M : TILE_CAP_L;
+    F.g = F.cap != TILE_CAP_S ? 1 : A.cap < TILE_G2 ? 2 : 1;
     if (!A.f32) {
-        c->tile_cap = need <= TILE_CAP_S ? TILE_CAP_S : TILE_CAP_L;
-        c->tile_g = 4 * home <= TILE_WG ? 4 : 2 * home <= 1.25 * TILE_WG ? 2 : 1;
+        F.cap = need <= TILE_CAP_S ? TILE_CAP_S : TILE_CAP_L;
+        F.g = 4 * home <= TILE_WG ? 4 : 2 * home <= 1.5 * TILE_WG ? 2 : 1;
     }
     // threads for the most particles a tile of lattice water holds
-    double most = c->tile_g;
+    double most = F.g;
     for (int d = 0; d < 3; d += flat ? 2 : 1) most *= std::ceil(best[d] * A.dcd[d] / A.dx);
-    c->tile_wg = (int)std::min<double>(TILE_WG, std::max(256.0, 64.0 * std::ceil(most / 64.0)));
+    F.wg = (int)std::min<double>(TILE_WG, std::max(256.0, 64.0 * std::ceil(most / 64.0)));
     long long tiles = 0;
     for (DP& Q : c->segs) {
         long long n = 1;
@@ -779,14 +787,19 @@ void choose_tile(sph_ctx* c) {
         Q.inv_nti = 1.0 / Q.ntile[0];
         Q.inv_ry = 1.0 / (Q.tdim[1] + 2);
         Q.toff = (int)tiles;
-        Q.tcap = Q.f32 ? c->tile_cap : 0;  // FP64: set by the upload
         tiles += (n + 255) / 256 * 256;
     }
     c->ntiles = (int)tiles;
+    F.home = home;
+    F.pairs = flat ? 3.1416 * 4.0 * (A.h / A.dx) * (A.h / A.dx) : 33.51 * std::pow(A.h / A.dx, 3);
     // a workgroup per tile where every tile is full, and as many again for partly filled ones
     const double full = 2.0 * A.cap / home + 64.0;
-    c->tile_grid = (int)(std::min((double)tiles, full) / 8.0 + 1.0) * 8;
+    F.grid = (int)(std::min((double)tiles, full) / 8.0 + 1.0) * 8;
+    c->form = F;
 }
+
+// Passes that gather for every particle: G lanes each
+void gather_form(sph_ctx* c, int g) { c->form = sph_ctx::Form{TILE_CAP_0, nblk(c->P.cap * g), 256, g}; }
 
 // Places nseg solves in one context: slots and keys of segment s follow
 // those of segment s-1 (slots and keys in whole 256-blocks).  One solve keeps
@@ -851,6 +864,7 @@ int setup_launch(sph_ctx* c, const sph_params* p) {
     if (c->nseg > 1)  // the segmented pair passes are built for whole-group walks
         c->chunk = c->chunk_v = c->chunk_c = c->chunk_p = 8;
     c->bt_grid = 4 * ncu;
+    c->ncu = ncu;
     if (p->nb_shape < 0 || p->nb_shape > 4) return fail(2, "nb_shape must be 0 to 4");
     return 0;
 }
@@ -1003,6 +1017,58 @@ int upload_segment_maps(sph_ctx* c) {
     if (!ok) return fail(102, "device allocation/copy of the segment maps failed");
     c->S = Seg{(DPC*)c->d_P, c->d_pblk, c->d_kblk, c->d_tblk, c->nseg};
     return 0;
+}
+
+// The form of the pair passes for the state just sorted: on tiles, or (sums of 4
+// passes, us, tiles against gathers) gathering for every particle
+// - where the tiles of too many particles do not fit, since those gather too, with
+//   the LDS form's few wavefronts: FP64 from an eighth of the particles on, several
+//   masses among them (576,000 particles of two masses 2009, 1373; a cluster of
+//   1.3 times water, a third unfit, 210, 170), FP32-mixed from a quarter on (the
+//   cluster 140, 88; a hundredth unfit, 576,000 particles, 445, 682);
+// - FP32-mixed where a tile is one cell, whose slots are 27 times its particles
+//   (h/dx = 2: 576,000 2488, 1994, 72,000 424, 266; tiles of two cells, 1.9:
+//   576,000 1653, 1961, 72,000 299, 260);
+// - FP64 where the tiles take a few rounds of a workgroup a CU, the last one far
+//   from full: a round's lanes (85 us for a wavefront a SIMD at 75 pairs a
+//   particle) and staging (23) against 2.9e-3 us a gathering particle.  72,000
+//   particles: 240 tiles (h/dx 1.3) 195, 214; 270 (1.2) 259, 175; 396 (1.4) 302,
+//   218; 330 (1.5) 371, 264; 576,000: 1.3 1037, 1380; 1.5 1630, 1807.
+int choose_form(sph_ctx* c) {
+    if (c->P.dbsph) return 0;
+    const sph_ctx::Form before = c->form, &L = c->lds_form;
+    const Tiles T{c->tlist, c->ntile};
+    SEGL(k_tile_unfit, 256, 256, T, c->start, L.cap, c->ntile + 1);
+    int tiles[2] = {0, 0};  // their number, particles in those that do not fit
+    std::vector<int> is((size_t)IS_COUNT * c->nseg);
+    HIPC(hipMemcpyAsync(tiles, c->ntile, sizeof(tiles), hipMemcpyDeviceToHost, c->stream));
+    HIPC(hipMemcpyAsync(is.data(), c->iscal, sizeof(int) * is.size(), hipMemcpyDeviceToHost, c->stream));
+    HIPC(hipStreamSynchronize(c->stream));
+    long long n = 0;
+    for (int s = 0; s < c->nseg; ++s) n += is[(size_t)s * IS_COUNT + IS_N];
+    c->form = L;
+    if (c->P.f32) {
+        const DP& A = c->segs[0];
+        if (4ll * tiles[1] > n || (L.cap == TILE_CAP_L && A.tdim[0] * A.tdim[1] * A.tdim[2] == 1)) gather_form(c, 2);
+    } else {
+        const double rounds = std::ceil((double)tiles[0] / c->ncu);
+        const double waves = std::ceil(std::ceil(L.home * L.g / 64.0) / 4.0) / L.g;  // of a SIMD, for one lane a particle
+        const bool few = L.cap == TILE_CAP_L && rounds > 1.0 &&
+                         rounds * (85.0 * waves * L.pairs / 75.0 + 23.0) > 2.9e-3 * n * L.pairs / 75.0;
+        if (8ll * tiles[1] > n || few) gather_form(c, c->P.cap < TILE_G8 ? 8 : 4);
+    }
+    bool change = c->form.cap != before.cap || c->form.g != before.g;
+    for (int s = 0; s < c->nseg; ++s) {
+        DP& Q = c->nseg > 1 ? c->segs[s] : c->P;
+        // FP64 slots hold no mass
+        const int tcap = c->form.cap != TILE_CAP_0 && (Q.f32 || Q.umass) ? c->form.cap : 0;
+        change = change || tcap != Q.tcap;
+        Q.tcap = tcap;
+    }
+    if (c->nseg > 1) c->P.tcap = c->segs[0].tcap;
+    if (!change) return 0;
+    drop_graphs(c);
+    return upload_constants(c);
 }
 
 int create_ctx(int nseg, const sph_params* p, const sph_faces* const* f, sph_ctx** out) {
@@ -1290,10 +1356,7 @@ int sph_dbsph_walls(sph_ctx* c, const sph_dbsph_walls_t* w) {
     P.muscl_bnd = w->muscl_boundary ? 1 : 0;
     P.tcap = 0;  // the DB-SPH kernels read the lists' stencil codes
     drop_graphs(c);
-    c->tile_cap = TILE_CAP_0;
-    c->tile_g = P.cap < TILE_G8 ? 8 : 4;
-    c->tile_wg = 256;
-    c->tile_grid = nblk((long long)P.cap * c->tile_g);
+    gather_form(c, P.cap < TILE_G8 ? 8 : 4);
     return upload_constants(c);
 }
 
@@ -1394,11 +1457,9 @@ int sph_segment_upload(sph_ctx* c, int32_t seg, int32_t n, const double* coord, 
         Q.far_y = far_y;
         Q.umass = umass;
         Q.f_mass = f_mass;
-        if (!Q.f32) Q.tcap = umass && !Q.dbsph ? c->tile_cap : 0;  // the FP64 slots hold no mass
         if (c->nseg > 1 && seg == 0) {
             c->P.umass = umass;
             c->P.f_mass = f_mass;
-            c->P.tcap = Q.tcap;
         }
         if (int rc = upload_constants(c)) return rc;
         drop_graphs(c);  // they hold the momentum kernel chosen for the old masses
@@ -1425,6 +1486,7 @@ int sph_segment_upload(sph_ctx* c, int32_t seg, int32_t n, const double* coord, 
         if (!c->staged[s]) return 0;  // the other segments come in later calls
     c->staged.clear();
     int rc = run_sort(c);
+    if (!rc) rc = choose_form(c);
     if (rc) return rc;
     // the sort leaves (rho,p) in the buffer the continuity pass reads; the
     // state at rest keeps it in the buffer the momentum pass reads

@@ -247,9 +247,10 @@ constexpr int TILE_CAP_L = 2496, TILE_CAP_M = 1632, TILE_CAP_S = 1216, TILE_CAP_
 constexpr int TILE_WG = 512;   // most threads of a pair pass
 constexpr int TILE_U = 5;      // slots a thread stages at a time (FP64: 3)
 constexpr int TILE_G2 = 40000;  // particles below which two lanes take a particle
-// DB-SPH: particles below which eight lanes take a particle, else four (step
-// times, us: 2,000 particles eight 265, four 292, two 357; 70,000 eight 611,
-// four 582, two 623)
+// FP64 passes that gather: particles below which eight lanes take a particle,
+// else four (DB-SPH steps, us: 2,000 particles eight 265, four 292, two 357;
+// 70,000 eight 611, four 582, two 623; the four passes: 9,000 eight 81, four 88,
+// two 133; 54,000 of twice water's density 331, 317, 327; 576,000 1834, 1375, 1442)
 constexpr int TILE_G8 = 20000;
 // tiles of water a solve is cut into (choose_tile); FP64
 constexpr int TILE_MIN = 300, TILE_MIN2 = 200, TILE_MIN_L = 500;
@@ -324,7 +325,7 @@ __global__ __launch_bounds__(256) void k_cell_count(Seg S, const double4* __rest
     iscal += sg * IS_COUNT;
     rmids += sg * RM_CAP;
     const int n = iscal[IS_N];
-    if (i == 0) *ntile = 0;  // k_scatter counts them
+    if (i == 0) ntile[0] = ntile[1] = 0;  // k_scatter counts the tiles
     bsum += (blockIdx.x % nrep) * nsb;
     for (int b = threadIdx.x; b < HIST_W; b += blockDim.x)
         for (int w = 0; w < 4; ++w) wcnt[w][b] = 0;
@@ -2170,17 +2171,18 @@ __device__ __forceinline__ int tile_find(const int* pre, int rows, int x) {
 // for every slot of a tile that fits, then part(P, segment, sorted index,
 // slot, fits) with G lanes for every home particle, then done(P, segment).  A
 // workgroup takes the tiles of its XCD's contiguous share, so tiles that share
-// halo rows share an L2.  TILED false: G lanes for every particle of one
-// solve, 256 threads a block, nothing staged.
+// halo rows share an L2.  TILED false: G lanes for every particle, 256 threads
+// a block (its slots lie in one segment), nothing staged.
 template <bool SG, int G, int U, bool TILED = true, class Stage, class Part, class Done>
 __device__ __forceinline__ void for_tiles(const Seg& S, const Tiles& T,
                                           const int* __restrict__ start, Stage&& stage, Part&& part,
                                           Done&& done) {
     if constexpr (!TILED) {
-        DPC& P = S.P[0];
-        const int i = (xcd_block(gridDim.x) * 256 + (int)threadIdx.x) / G;
-        if (i < start[P.nmax]) part(P, 0, i, 0, false);
-        done(P, 0);
+        const int vb = xcd_block(gridDim.x), i = (vb * 256 + (int)threadIdx.x) / G;
+        const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[(vb * 256 / G) >> 8]) : 0;
+        DPC& P = S.P[sg];
+        if (i < start[P.koff + P.nmax]) part(P, sg, i, 0, false);
+        done(P, sg);
         return;
     }
     __shared__ TileS ts;
@@ -2232,6 +2234,25 @@ __device__ __forceinline__ void for_tiles(const Seg& S, const Tiles& T,
         done(P, sg);
         __syncthreads();  // the slots and rows are reused
     }
+}
+
+// Particles in tiles that have more than cap slots, or whose solve's records do
+// not fit the LDS form (FP64 with several masses), added to *out: a wavefront a
+// tile.
+template <bool SG>
+__global__ __launch_bounds__(256) void k_tile_unfit(Seg S, Tiles T, const int* __restrict__ start, int cap, int* out) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    int n = 0;
+    for (int t = blockIdx.x * 4 + wid; t < *T.n; t += gridDim.x * 4) {
+        const int id = __builtin_amdgcn_readfirstlane(T.list[t]);
+        DPC& P = S.P[SG ? __builtin_amdgcn_readfirstlane(S.tblk[id >> 8]) : 0];
+        int ti, tj, tk, g0, g1, h0, h1;
+        tile_coords(P, id, ti, tj, tk);
+        tile_row(P, start, ti, tj, tk, lane, g0, g1, h0, h1);
+        const int total = __builtin_amdgcn_readlane(wave_incl_scan(g1 - g0), 63);
+        if (total > (P.f32 || P.umass ? cap : 0)) n += __builtin_amdgcn_readlane(wave_incl_scan(h1 - h0), 63);
+    }
+    if (lane == 0 && n) atomicAdd(out, n);
 }
 
 // 16 bytes at byte offset o of an LDS array
@@ -2940,7 +2961,8 @@ __device__ __forceinline__ double psmooth_end(DPC& P, const DFace* __restrict__ 
 // lanes a particle, 1024 threads) measured the same, reading a neighbour's
 // records ahead of the previous one's arithmetic 1% slower.
 // Tiles that do not fit, solves of several masses, and lists that carry stencil
-// codes (DB-SPH walls) gather from global memory with the same expressions.
+// codes (DB-SPH walls) gather from global memory with the same expressions;
+// choose_form takes such solves off the tiles (CAP TILE_CAP_0).
 // ----------------------------------------------------------------------------
 #define TILE_ARGS Seg S, Tiles T, const int* __restrict__ start
 
@@ -3292,7 +3314,10 @@ __global__ __launch_bounds__(TILE_WG, 2) void k_psmooth64(
 // Pair math on xq's integer positions: a separation is exact to 2^-28 of a
 // cell, in units of P.lsb, whose powers are taken out of the sums.
 // Tiles with more candidates than the LDS holds gather from global memory
-// with the same expressions, so a sum does not depend on the tile.
+// with the same expressions, so a sum does not depend on the tile.  Solves in
+// which most do (choose_form) take no LDS and two lanes a particle, eight
+// neighbours in flight each: a cluster of three times water, 81,000 particles,
+// four passes: on tiles 1199 us (one neighbour in flight) and 582 (four), 270.
 // 576,000 particles: momentum 186 -> 120 us, velocity smoothing 202 -> 87,
 // continuity 185 -> 79, pressure smoothing 101 -> 55; 25,000 particles: 33 ->
 // 28, 24 -> 17, 23 -> 16, 19 -> 13.
@@ -3336,11 +3361,12 @@ __device__ __forceinline__ float4 bits4(int4 x, float w) {
 // momentum pass at 576,000.)
 // fits: 16-bit entries (LDS slot times 16), 16 of them per 32 bytes, filled up
 // with the particle itself to whole eights; lds(sums, byte offset of the
-// neighbour's 16-byte record, place in the list).  Else glob(sums, sorted
-// index).  The next entries are loaded while some are used.
-template <int G, int NS, class Lds, class Glob>
+// neighbour's 16-byte record, place in the list).  Else term(sums, glob(sorted
+// index), place), CH neighbours' records in flight, past the end the particle
+// itself.  The next entries are loaded while some are used.
+template <int G, int CH, int NS, class Lds, class Glob, class Term>
 __device__ __forceinline__ void pair_sums(const uint32_t* __restrict__ nbr, size_t N, int i, int nn, int g,
-                                          bool fits, float (&sum)[NS], Lds&& lds, Glob&& glob) {
+                                          bool fits, float (&sum)[NS], Lds&& lds, Glob&& glob, Term&& term) {
 #pragma unroll
     for (int c = 0; c < NS; ++c) sum[c] = 0.0f;
 #pragma unroll 1
@@ -3359,9 +3385,28 @@ __device__ __forceinline__ void pair_sums(const uint32_t* __restrict__ nbr, size
 #pragma unroll
                 for (int u = 0; u < 8; ++u) lds(a, (u & 1) ? w[u >> 1] >> 16 : w[u >> 1] & 0xFFFFu, k + u);
             }
-        } else {
+        } else if constexpr (CH == 1) {
             for (int k0 = 8 * m; k0 < nn; k0 += 16)
-                for (int k = k0; k < min(nn, k0 + 8); ++k) glob(a, (int)(nbr[nb_index(N, i, k)] & NB_MASK));
+                for (int k = k0; k < min(nn, k0 + 8); ++k) term(a, glob((int)(nbr[nb_index(N, i, k)] & NB_MASK)), k);
+        } else {
+            const uint4* L = reinterpret_cast<const uint4*>(nbr) + 2 * ((size_t)m * N + (size_t)i);
+            uint4 na = L[0], nb = L[1];
+            for (int k0 = 8 * m; k0 < nn; k0 += 16) {
+                const uint32_t w[8] = {na.x, na.y, na.z, na.w, nb.x, nb.y, nb.z, nb.w};
+                L += 4 * N;
+                if (k0 + 16 < nn) {
+                    na = L[0];
+                    nb = L[1];
+                }
+#pragma unroll
+                for (int c = 0; c < 8; c += CH) {
+                    decltype(glob(0)) r[CH];
+#pragma unroll
+                    for (int u = 0; u < CH; ++u) r[u] = glob(k0 + c + u < nn ? (int)(w[c + u] & NB_MASK) : i);
+#pragma unroll
+                    for (int u = 0; u < CH; ++u) term(a, r[u], k0 + c + u);
+                }
+            }
         }
 #pragma unroll
         for (int c = 0; c < NS; ++c) sum[c] += a[c];
@@ -3370,6 +3415,11 @@ __device__ __forceinline__ void pair_sums(const uint32_t* __restrict__ nbr, size
 #pragma unroll
         for (int c = 0; c < NS; ++c) sum[c] += __shfl_xor(sum[c], 1, 64);
 }
+
+struct RecF { int4 x; float4 v; };  // a gathered neighbour
+// neighbours in flight: the LDS form's registers leave room for fewer (the
+// pressure smoothing's for one: four took its seventh wavefront, 56 -> 64 us)
+constexpr int GATHER_CH(int cap) { return cap == TILE_CAP_0 ? 8 : 4; }
 
 // momentum; UM: every particle of the context has its solve's mass
 template <int CAP, bool SG, int G, bool UM>
@@ -3390,7 +3440,7 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_momentum(
     auto rec_b = [](int4 x, float4 v) {
         return make_float4(v.x, v.y, v.z, UM ? v.w : __int_as_float(x.w));
     };
-    for_tiles<SG, G, TILE_U>(S, T, start,
+    for_tiles<SG, G, TILE_U, CAP != TILE_CAP_0>(S, T, start,
         [&](DPC& P, int, int j, int slot) {
             const int4 x = xq[j];
             const float4 v = vf[j];
@@ -3443,13 +3493,10 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_momentum(
                 s[8] = __builtin_fmaf(cv, v2, s[8]);
             };
             float s[9];
-            pair_sums<G>(nbr, (size_t)P.cap, i, nnb[i], threadIdx.x % G, fits, s,
+            pair_sums<G, GATHER_CH(CAP)>(nbr, (size_t)P.cap, i, nnb[i], threadIdx.x % G, fits, s,
                          [&](float* a, uint32_t o, int) { pair(a, lds16(sA, o), lds16(sB, o)); },
-                         [&](float* a, int j) {
-                             const int4 x = xq[j];
-                             const float4 v = vf[j];
-                             pair(a, rec_a(P, x, v), rec_b(x, v));
-                         });
+                         [&](int j) { return RecF{xq[j], vf[j]}; },
+                         [&](float* a, const RecF& r, int) { pair(a, rec_a(P, r.x, r.v), rec_b(r.x, r.v)); });
             if (threadIdx.x % G) return;
             const double m = UM ? (double)P.f_mass : 1.0, ke = P.ke_coef * P.inv_lsb;
             const double sp = 3.0 * P.kacl_coef * m;
@@ -3488,7 +3535,7 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_vsmooth(
         return bits4(x, __int_as_float(x.w) * __builtin_amdgcn_rcpf(P.f_den0 + v.w));
     };
     unsigned long long dtbits = 0x7FF0000000000000ull;
-    for_tiles<SG, G, TILE_U>(S, T, start,
+    for_tiles<SG, G, TILE_U, CAP != TILE_CAP_0>(S, T, start,
         [&](DPC& P, int, int j, int slot) {
             if (!(P.tetav > 1.0e-9)) return;
             const float4 v = vf[j];
@@ -3510,12 +3557,10 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_vsmooth(
                     s[2] = __builtin_fmaf(B.z - vi.z, pes, s[2]);
                 };
                 float s[3];
-                pair_sums<G>(nbr, (size_t)P.cap, i, nnb[i], threadIdx.x % G, fits, s,
+                pair_sums<G, GATHER_CH(CAP)>(nbr, (size_t)P.cap, i, nnb[i], threadIdx.x % G, fits, s,
                              [&](float* a, uint32_t o, int) { pair(a, lds16(sA, o), lds16(sB, o)); },
-                             [&](float* a, int j) {
-                                 const float4 vj = vf[j];
-                                 pair(a, rec_a(P, xq[j], vj), vj);
-                             });
+                             [&](int j) { return RecF{xq[j], vf[j]}; },
+                             [&](float* a, const RecF& r, int) { pair(a, rec_a(P, r.x, r.v), r.v); });
                 v[0] = P.coefke * (double)s[0];
                 v[1] = P.coefke * (double)s[1];
                 v[2] = P.coefke * (double)s[2];
@@ -3548,7 +3593,7 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_continuity(
     auto rec_a = [](DPC& P, int4 x, float4 v) {
         return bits4(x, __int_as_float(x.w) * __builtin_amdgcn_rcpf(P.f_den0 + v.w));
     };
-    for_tiles<SG, G, TILE_U>(S, T, start,
+    for_tiles<SG, G, TILE_U, CAP != TILE_CAP_0>(S, T, start,
         [&](DPC& P, int, int j, int slot) {
             const float4 v = vf[j];
             sA[slot] = rec_a(P, xq[j], v);
@@ -3565,12 +3610,10 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_continuity(
                 s[0] = __builtin_fmaf(k, dv, s[0]);
             };
             float s[1];
-            pair_sums<G>(nbr, (size_t)P.cap, i, nnb[i], threadIdx.x % G, fits, s,
+            pair_sums<G, GATHER_CH(CAP)>(nbr, (size_t)P.cap, i, nnb[i], threadIdx.x % G, fits, s,
                          [&](float* a, uint32_t o, int) { pair(a, lds16(sA, o), lds16(sB, o)); },
-                         [&](float* a, int j) {
-                             const float4 vj = vf[j];
-                             pair(a, rec_a(P, xq[j], vj), vj);
-                         });
+                         [&](int j) { return RecF{xq[j], vf[j]}; },
+                         [&](float* a, const RecF& r, int) { pair(a, rec_a(P, r.x, r.v), r.v); });
             if (threadIdx.x % G) return;
             const double2 rpi = rp[i];
             int* iscal = iscal0 + sg * IS_COUNT;
@@ -3594,7 +3637,7 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_psmooth(
     auto rec_a = [](DPC& P, int4 x, float d) {
         return bits4(x, __int_as_float(x.w) * __builtin_amdgcn_rcpf(P.f_den0 + d));
     };
-    for_tiles<SG, G, TILE_U>(S, T, start,
+    for_tiles<SG, G, TILE_U, CAP != TILE_CAP_0>(S, T, start,
         [&](DPC& P, int, int j, int slot) {
             const float d = dr[j];
             sA[slot] = rec_a(P, xq[j], d);
@@ -3611,12 +3654,14 @@ __global__ __launch_bounds__(TILE_WG, 4) void k_psmooth(
                 s[1] = __builtin_fmaf(dj - di, pes, s[1]);
             };
             float s[2];
-            pair_sums<G>(nbr, (size_t)P.cap, i, nn, threadIdx.x % G, fits, s,
+            struct RecD { int4 x; float d; };
+            pair_sums<G, CAP == TILE_CAP_0 ? 8 : 1>(nbr, (size_t)P.cap, i, nn, threadIdx.x % G, fits, s,
                          [&](float* a, uint32_t o, int k) {
                              const float dj = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(sD) + (o >> 2));
                              pair(a, lds16(sA, o), dj, k < nn);
                          },
-                         [&](float* a, int j) { pair(a, rec_a(P, xq[j], dr[j]), dr[j], true); });
+                         [&](int j) { return RecD{xq[j], dr[j]}; },
+                         [&](float* a, const RecD& r, int k) { pair(a, rec_a(P, r.x, r.d), r.d, k < nn); });
             if (threadIdx.x % G) return;
             const double rho2 = psmooth_end(P, faces, bn, bt, i, nn, rp[i], scal0[sg * SC_COUNT + SC_TP1],
                                             P.eps / P.den0 * P.coefke * (double)s[1], P.coefke * (double)s[0],
