@@ -531,7 +531,10 @@ __global__ __launch_bounds__(256) void k_scatter(Seg S, const int* __restrict__ 
         const unsigned long long m = __ballot(n > 0);
         if (lane == 0) wn[wid] = __popcll(m);
         __syncthreads();
-        if (threadIdx.x == 0) first = atomicAdd(ntile, wn[0] + wn[1] + wn[2] + wn[3]);
+        // (no atomic for 256 empty tiles: of a large grid most are, and the atomics queue)
+        const int some = wn[0] + wn[1] + wn[2] + wn[3];
+        if (some == 0) return;
+        if (threadIdx.x == 0) first = atomicAdd(ntile, some);
         __syncthreads();
         int at = first + __popcll(m & ((1ull << lane) - 1ull));
         for (int w = 0; w < wid; ++w) at += wn[w];
