@@ -1026,6 +1026,11 @@ int upload_segment_maps(sph_ctx* c) {
 //   masses among them (576,000 particles of two masses 2009, 1373; a cluster of
 //   1.3 times water, a third unfit, 210, 170), FP32-mixed from a quarter on (the
 //   cluster 140, 88; a hundredth unfit, 576,000 particles, 445, 682);
+// - where the particles fill less than half of the tiles that hold any (spray, a
+//   thin cloud): a tile costs its workgroup whatever it holds.  Clouds of 500,000
+//   particles, fill 0.02, 0.2, 0.4, 0.6: mixed 2827, 123; 406, 182; 313, 284; 429,
+//   460; FP64 5607, 208; 1014, 443; 895, 674; 1278, 1039; of 8,000, fill 0.5: mixed
+//   87, 40, FP64 92, 51 (dam breaks fill 0.7 to 0.95);
 // - FP32-mixed where a tile is one cell, whose slots are 27 times its particles
 //   (h/dx = 2: 576,000 2488, 1994, 72,000 424, 266; tiles of two cells, 1.9:
 //   576,000 1653, 1961, 72,000 299, 260);
@@ -1047,15 +1052,16 @@ int choose_form(sph_ctx* c) {
     long long n = 0;
     for (int s = 0; s < c->nseg; ++s) n += is[(size_t)s * IS_COUNT + IS_N];
     c->form = L;
+    const bool thin = 2.0 * n < tiles[0] * L.home;
     if (c->P.f32) {
         const DP& A = c->segs[0];
-        if (4ll * tiles[1] > n || (L.cap == TILE_CAP_L && A.tdim[0] * A.tdim[1] * A.tdim[2] == 1)) gather_form(c, 2);
+        if (thin || 4ll * tiles[1] > n || (L.cap == TILE_CAP_L && A.tdim[0] * A.tdim[1] * A.tdim[2] == 1)) gather_form(c, 2);
     } else {
         const double rounds = std::ceil((double)tiles[0] / c->ncu);
         const double waves = std::ceil(std::ceil(L.home * L.g / 64.0) / 4.0) / L.g;  // of a SIMD, for one lane a particle
         const bool few = L.cap == TILE_CAP_L && rounds > 1.0 &&
                          rounds * (85.0 * waves * L.pairs / 75.0 + 23.0) > 2.9e-3 * n * L.pairs / 75.0;
-        if (8ll * tiles[1] > n || few) gather_form(c, c->P.cap < TILE_G8 ? 8 : 4);
+        if (thin || 8ll * tiles[1] > n || few) gather_form(c, c->P.cap < TILE_G8 ? 8 : 4);
     }
     bool change = c->form.cap != before.cap || c->form.g != before.g;
     for (int s = 0; s < c->nseg; ++s) {

@@ -1,6 +1,6 @@
 """Forms of the pair passes: on tiles in LDS, or gathering for every particle
-(clusters whose tiles do not fit, FP64 with several masses, tiles of one cell,
-FP64 tiles that fill their last round badly).  Against the oracle: FP64 equal,
+(clusters whose tiles do not fit, thin clouds, FP64 with several masses, tiles of
+one cell, FP64 tiles that fill their last round badly).  Against the oracle: FP64 equal,
 FP32-mixed within 1e-4 of each field's largest value, the bar of the other
 tests; between contexts that take different forms, lane counts and batches: bit
 for bit; captured steps are not replayed in another form."""
