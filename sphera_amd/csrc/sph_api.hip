@@ -557,8 +557,14 @@ int sph_ctx::alloc() {
     HIPC(da(&nwork, 1));
     HIPC(da(&cnt, m));
     HIPC(da(&start, m + 1));
-    nrep = nblk((int)m, SCAN_B) <= 256 ? 16 : nblk((int)m, SCAN_B) <= 1024 ? 4 : 1;
-    HIPC(da(&bsum, (size_t)nrep * nblk((int)m, SCAN_B)));
+    // copies of the scan blocks' sums: k_cell_count's atomics queue on few, every
+    // block of k_cell_scan adds up all of them (both kernels, us, 500,000 particles
+    // and 20,000, copies 16, 4, 1: 259 blocks 43, 52, 78 and 27, 29, 34; 926: 104, 141,
+    // 282 and 48, 43, 45; 1,782: 136, 140, 239 and 79, 62, 62; 3,906: 293, 201, 240 and
+    // 224, 116, 105)
+    const int nsb = nblk((int)m, SCAN_B);
+    nrep = nsb <= 1024 ? 16 : nsb <= 4096 ? 4 : 1;
+    HIPC(da(&bsum, (size_t)nrep * nsb));
     HIPC(da(&idslot, N));
     HIPC(da(&rmids, RM_CAP * ns));
     HIPC(da(&nbr, N * (size_t)nb_stride(nb_stride_max)));
@@ -584,7 +590,7 @@ int sph_ctx::alloc() {
     HIPC(hipMemset(ntile, 0, 2 * sizeof(int)));
     // every sort leaves its counters cleared for the next
     HIPC(hipMemset(cnt, 0, sizeof(int) * m));
-    HIPC(hipMemset(bsum, 0, sizeof(int) * (size_t)nrep * nblk((int)m, SCAN_B)));
+    HIPC(hipMemset(bsum, 0, sizeof(int) * (size_t)nrep * nsb));
     HIPC(hipMemset(nwork, 0, sizeof(int)));
     HIPC(hipMemset(nnb, 0, sizeof(int) * N));
     HIPC(hipMemset(gone, 0, sizeof(int) * N));

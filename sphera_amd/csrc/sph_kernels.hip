@@ -707,8 +707,11 @@ __device__ int nb_particle_global(DPC& P, int p, const double4* __restrict__ xm,
 // every candidate the FP32 test takes goes to the FP64 test.
 constexpr int NBC_CH = 9;              // chunks of 64 candidates in registers
 constexpr int NBC_MAX = 64 * NBC_CH;
-constexpr int NBC_SLOTS = 16, NBC_SLOTS_L = 64;  // sorted slots per wavefront: small, large solves
-constexpr int NBC_LARGE = 150000;      // particles from which the chip is full with 64 slots per wavefront
+// sorted slots per wavefront: small contexts, those of NBC_LARGE particles and more
+// (us, 16 slots, 64: 72,000 particles 40, 59; 117,000 52, 61; 171,000 66, 72; 262,000
+// 90, 87; 576,000 181, 162)
+constexpr int NBC_SLOTS = 16, NBC_SLOTS_L = 64;
+constexpr int NBC_LARGE = 200000;
 constexpr int NBC_PAIRS = 64;          // pair counters, one 128-byte line each
 constexpr int NBC_PSTRIDE = 16;
 

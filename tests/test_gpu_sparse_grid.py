@@ -7,15 +7,15 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("prec", [0, 1])
-@pytest.mark.parametrize("capacity", [None, 120000])
-def test_scattered_clusters(capacity, prec):
+@pytest.mark.parametrize("side,capacity", [(2.0, None), (2.0, 120000), (4.6, None)])  # 0.5, 5.6 million cells
+def test_scattered_clusters(side, capacity, prec):
     from oracle.pyoracle import Oracle
     from sphera_amd import runtime as rt
     from sphera_amd.case import DamBreak3D, build
-    tb = build(DamBreak3D(tank=(2.0, 2.0, 2.0), column=(0.1, 0.1, 0.1), dx=0.01, name="sparse"), particles=False,
+    tb = build(DamBreak3D(tank=(side, side, side), column=(0.1, 0.1, 0.1), dx=0.01, name="sparse"), particles=False,
                incidence=False)
     rng = np.random.default_rng(6)
-    at = np.concatenate([[[0.05, 0.05, 0.05], [1.95, 1.95, 1.95]], rng.uniform(0.05, 1.95, (30, 3))])
+    at = np.concatenate([[[0.05, 0.05, 0.05], [side - 0.05] * 3], rng.uniform(0.05, side - 0.05, (30, 3))])
     coord = np.concatenate([c + rng.uniform(-0.03, 0.03, (60, 3)) for c in at])
     n = len(coord)
     dens = 1000.0 * (1.0 + rng.uniform(-1e-3, 1e-3, n))
