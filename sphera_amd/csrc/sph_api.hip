@@ -273,7 +273,8 @@ int run_btab(sph_ctx* c, bool again = false) {
     if (c->P.f32)  // eight lanes per pair
         SEGL(k_boundary_int_f32, 4 * c->bt_grid, 256, c->d_faces, c->d_btf, c->bt, c->work, c->nwork);
     else
-        SEGL(k_boundary_int, 2 * c->bt_grid, 256, c->d_faces, c->d_kt, c->d_bit, c->d_btf, c->bt, c->work, c->nwork);
+        SEGL(k_boundary_int, c->nseg > 1 ? c->P.cap / 256 * BT_SPLIT : 2 * c->bt_grid, 256, c->d_faces, c->d_kt, c->d_bit, c->d_btf, c->bt,
+             c->work, c->nwork, c->bn, c->iscal);
     return 0;
 }
 

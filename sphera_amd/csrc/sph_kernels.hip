@@ -477,6 +477,9 @@ __global__ __launch_bounds__(256) void k_cell_scan(Seg S, const int* __restrict_
         before += bsum[(threadIdx.x & (nrep - 1)) * nsb + b];
     constexpr int U = SCAN_B / 256;
     const int k0 = blockIdx.x * SCAN_B + threadIdx.x * U;
+    // the particles of the segments before the workgroup's first are taken off again
+    const int sg0 = SG ? S.kblk[(blockIdx.x * SCAN_B) >> 8] : 0;
+    for (int q = threadIdx.x; q < sg0; q += 256) before -= iscal[q * IS_COUNT + IS_N];
     int v[U], tsum = 0;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -493,7 +496,7 @@ __global__ __launch_bounds__(256) void k_cell_scan(Seg S, const int* __restrict_
     if (SG && k0 < m) {  // a thread's keys lie in one 256-block, hence in one segment
         const int sg = S.kblk[k0 >> 8];
         int earlier = 0;
-        for (int q = 0; q < sg; ++q) earlier += iscal[q * IS_COUNT + IS_N];
+        for (int q = sg0; q < sg; ++q) earlier += iscal[q * IS_COUNT + IS_N];
         run += S.P[sg].base - earlier;
     }
 #pragma unroll
@@ -1189,9 +1192,6 @@ __global__ __launch_bounds__(256) void k_boundary_find(Seg S, const DFace* __res
     }
 }
 
-// Segmented contexts: a workgroup's pairs may belong to several segments, so
-// each lane reads its segment's constants and tables (kernel and direction
-// tables of every segment, consecutive) from global memory.
 // ----------------------------------------------------------------------------
 // 2D form (x-z plane): boundary table over the boundary sides.
 // FindCloseBoundarySides2D.f90:68-170, SelectCloseBoundarySides2D.f90:66-120,
@@ -1557,43 +1557,65 @@ __device__ __forceinline__ int ring_side(const DFace& F, const PIC& c, double c0
 // it moves by rounding only, so a ring is refreshed by its first kept direction
 // or not at all; a pair in which a ring's move is within 1e-9 of 1e-3, and any
 // table whose rings are not of this form, goes through d_volume_integrals.
+// Segmented contexts: BT_SPLIT workgroups take the pairs of a 256-slot block,
+// which share a segment and so these tables.  (From the work list, which holds
+// the segments' pairs mixed, with the tables in global memory, 2 solves of 1,440
+// particles took 186 us, now 60; 256 of them 1760, 402; 16 of 11,000 482, 146.)
+constexpr int BT_SPLIT = 4;
 template <bool SG>
 __global__ __launch_bounds__(256) void k_boundary_int(Seg S, const DFace* __restrict__ faces,
                                                       const double* __restrict__ kt_g,
                                                       const double* __restrict__ bit_g,
                                                       const BtF32* __restrict__ tab, BTab* __restrict__ bt,
-                                                      const int* __restrict__ work, const int* nwork) {
+                                                      const int* __restrict__ work, const int* nwork,
+                                                      const int* __restrict__ bn, const int* iscal) {
     constexpr int ND = BT_RINGS * BT_RDIRS, G = 4;
-    __shared__ double kt_s[SG ? 1 : 41 * 5];
-    __shared__ double2 b_s[SG ? 1 : ND];
-    __shared__ double f_s[SG ? 1 : ND * 12];  // lane l's factors of direction k: [12 k + 3 l, + 3)
-    const int nw = *nwork;
-    if ((int)blockIdx.x * (256 / G) >= nw) return;  // no pair for this workgroup
+    __shared__ double kt_s[41 * 5];
+    __shared__ double2 b_s[ND];
+    __shared__ double f_s[ND * 12];  // lane l's factors of direction k: [12 k + 3 l, + 3)
+    __shared__ uint16_t pair_s[SG ? 256 * SPH_MB : 1];  // slot of the block, table slot << 8
+    __shared__ int wsum[4];
+    const int blk = SG ? blockIdx.x / BT_SPLIT : blockIdx.x, first = SG ? blockIdx.x % BT_SPLIT : blockIdx.x;
+    const int stride = SG ? BT_SPLIT : gridDim.x;
+    const int sg = SG ? __builtin_amdgcn_readfirstlane(S.pblk[blk]) : 0;
+    DPC& P = S.P[sg];
+    int nw;
+    if (SG) {
+        const int i = blk * 256 + threadIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+        const int n = i - P.base < iscal[sg * IS_COUNT + IS_N] ? bn[i] : 0;
+        const int incl = wave_incl_scan(n);
+        if (lane == 63) wsum[wid] = incl;
+        __syncthreads();
+        int at = incl - n;
+        for (int v = 0; v < wid; ++v) at += wsum[v];
+        nw = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+        for (int q = 0; q < n; ++q) pair_s[at + q] = (uint16_t)(threadIdx.x | (q << 8));
+    } else {
+        nw = *nwork;
+    }
+    if (first * (256 / G) >= nw) return;  // no pair for this workgroup
+    const double* ktg = kt_g + (size_t)sg * (41 * 5);
+    const double* bitg = bit_g + (size_t)sg * (ND * 7);
+    const BtF32& T = tab[sg];
     auto factors = [](const double* R, int l, double f[3]) {
         f[0] = l == 0 ? 1.0 : l == 1 ? R[0] : l == 2 ? R[0] * R[0] : R[1] * R[1];
         f[1] = l == 0 ? 1.0 : l == 1 ? R[1] : l == 2 ? R[0] * R[1] : R[1] * R[2];
         f[2] = l == 0 ? R[2] * R[2] : l == 1 ? R[2] : l == 2 ? R[0] * R[2] : R[2] * R[2];
     };
-    if (!SG) {
-        for (int t = threadIdx.x; t < 41 * 5; t += 256) kt_s[t] = kt_g[t];
-        for (int t = threadIdx.x; t < ND; t += 256) {
-            const double* b = &bit_g[t * 7];
-            b_s[t] = make_double2(b[0], b[1]);
-            for (int l = 0; l < G; ++l) factors(b + 4, l, &f_s[12 * t + 3 * l]);
-        }
-        __syncthreads();
+    for (int t = threadIdx.x; t < 41 * 5; t += 256) kt_s[t] = ktg[t];
+    for (int t = threadIdx.x; t < ND; t += 256) {
+        const double* b = &bitg[t * 7];
+        b_s[t] = make_double2(b[0], b[1]);
+        for (int l = 0; l < G; ++l) factors(b + 4, l, &f_s[12 * t + 3 * l]);
     }
+    __syncthreads();
     const int l = threadIdx.x % G;
-    for (int w = (blockIdx.x * 256 + threadIdx.x) / G; w < nw; w += gridDim.x * (256 / G)) {
-        const int e = work[w];
-        const int i = e & (int)NB_MASK, q = (int)((uint32_t)e >> NB_SHIFT);
-        const int sg = SG ? S.pblk[i >> 8] : 0;
-        DPC& P = S.P[sg];
-        const BtF32& T = tab[sg];
-        const double* ktg = kt_g + (size_t)sg * (41 * 5);
-        const double* bitg = bit_g + (size_t)sg * (ND * 7);
-        const double* kt = SG ? ktg : kt_s;
-        auto dir = [&](int k) { return SG ? make_double2(bitg[k * 7], bitg[k * 7 + 1]) : b_s[k]; };
+    for (int w = (first * 256 + threadIdx.x) / G; w < nw; w += stride * (256 / G)) {
+        const int e = SG ? pair_s[w] : work[w];
+        const int i = SG ? blk * 256 + (e & 255) : e & (int)NB_MASK;
+        const int q = SG ? e >> 8 : (int)((uint32_t)e >> NB_SHIFT);
+        const double* kt = kt_s;
+        auto dir = [&](int k) { return b_s[k]; };
         BTab& rec = bt[(size_t)q * P.cap + i];
         const DFace& F = faces[rec.face];
         const double loc[3] = {rec.loc[0], rec.loc[1], rec.loc[2]};
@@ -1657,14 +1679,7 @@ __global__ __launch_bounds__(256) void k_boundary_int(Seg S, const DFace* __rest
 #pragma unroll 4
             for (int k = 0; k < BT_RDIRS; ++k) {
                 const int d = r * BT_RDIRS + k;
-                double f[3];
-                if (SG) {
-                    factors(&bitg[d * 7 + 4], l, f);
-                } else {
-                    f[0] = f_s[12 * d + 3 * l];
-                    f[1] = f_s[12 * d + 3 * l + 1];
-                    f[2] = f_s[12 * d + 3 * l + 2];
-                }
+                const double f[3] = {f_s[12 * d + 3 * l], f_s[12 * d + 3 * l + 1], f_s[12 * d + 3 * l + 2]};
                 const bool on = !part || ((m >> k) & 1u);
                 const double ka = on ? ma : 0.0, kb = on ? mb : 0.0;
                 s[0] = s[0] + f[0] * ka;
