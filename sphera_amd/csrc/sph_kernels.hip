@@ -1555,8 +1555,9 @@ __device__ __forceinline__ int ring_side(const DFace& F, const PIC& c, double c0
 // directions in order, the factors from an LDS table: 32 and 60 us.  The
 // table values are refreshed where rob moves by more than 1e-3: within a ring
 // it moves by rounding only, so a ring is refreshed by its first kept direction
-// or not at all; a pair in which a ring's move is within 1e-9 of 1e-3, and any
-// table whose rings are not of this form, goes through d_volume_integrals.
+// or not at all; a pair in which a ring's move is within 1e-9 of 1e-3 goes through
+// d_volume_integrals, and so does every pair of a table whose rings are not of
+// this form, one lane a pair.
 // Segmented contexts: BT_SPLIT workgroups take the pairs of a 256-slot block,
 // which share a segment and so these tables.  (From the work list, which holds
 // the segments' pairs mixed, with the tables in global memory, 2 solves of 1,440
@@ -1609,14 +1610,28 @@ __global__ __launch_bounds__(256) void k_boundary_int(Seg S, const DFace* __rest
         for (int l = 0; l < G; ++l) factors(b + 4, l, &f_s[12 * t + 3 * l]);
     }
     __syncthreads();
-    const int l = threadIdx.x % G;
-    for (int w = (first * 256 + threadIdx.x) / G; w < nw; w += stride * (256 / G)) {
+    auto record = [&](int w) -> BTab& {
         const int e = SG ? pair_s[w] : work[w];
         const int i = SG ? blk * 256 + (e & 255) : e & (int)NB_MASK;
         const int q = SG ? e >> 8 : (int)((uint32_t)e >> NB_SHIFT);
+        return bt[(size_t)q * P.cap + i];
+    };
+    auto serially = [&](BTab& rec) {
+        const double loc[3] = {rec.loc[0], rec.loc[1], rec.loc[2]};
+        double bi[8], ig[9];
+        d_volume_integrals(P, faces[rec.face], ktg, bitg, loc, bi, ig);
+        for (int t = 0; t < 8; ++t) rec.bi[t] = bi[t];
+        for (int t = 0; t < 9; ++t) rec.ig[t] = ig[t];
+    };
+    if (!T.all_ok) {  // no rings: one lane a pair
+        for (int w = first * 256 + threadIdx.x; w < nw; w += stride * 256) serially(record(w));
+        return;
+    }
+    const int l = threadIdx.x % G;
+    for (int w = (first * 256 + threadIdx.x) / G; w < nw; w += stride * (256 / G)) {
         const double* kt = kt_s;
         auto dir = [&](int k) { return b_s[k]; };
-        BTab& rec = bt[(size_t)q * P.cap + i];
+        BTab& rec = record(w);
         const DFace& F = faces[rec.face];
         const double loc[3] = {rec.loc[0], rec.loc[1], rec.loc[2]};
         const double zpmin = 0.05 * P.h;
@@ -1624,13 +1639,13 @@ __global__ __launch_bounds__(256) void k_boundary_int(Seg S, const DFace* __rest
         const PIC pic = pic_of(F);
         uint32_t mask[2] = {0u, 0u};  // the kept directions of the rings l and l + 4
         double rob[2] = {0.0, 0.0}, J[2][4];
-        bool serial = !T.all_ok;
+        bool serial = false;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             J[u][0] = J[u][1] = J[u][2] = J[u][3] = 0.0;
             const int r = l + 4 * u;
             const double Pj2 = L2 + T.rc[r].bz;
-            if (loc[2] < 0.0 || serial || !(Pj2 <= 0.0)) continue;
+            if (loc[2] < 0.0 || !(Pj2 <= 0.0)) continue;
             const double ts = L2 / (L2 - Pj2);
             auto point = [&](int k, double& X0, double& X1) {
                 const double2 b = dir(r * BT_RDIRS + k);
@@ -1688,12 +1703,7 @@ __global__ __launch_bounds__(256) void k_boundary_int(Seg S, const DFace* __rest
             }
         }
         if (serial) {
-            if (l == 0) {
-                double bi[8], ig[9];
-                d_volume_integrals(P, F, ktg, bitg, loc, bi, ig);
-                for (int t = 0; t < 8; ++t) rec.bi[t] = bi[t];
-                for (int t = 0; t < 9; ++t) rec.ig[t] = ig[t];
-            }
+            if (l == 0) serially(rec);
         } else if (l == 0) {
             rec.bi[0] = 0.0;
             rec.bi[1] = loc[2] >= 0.0 && L2 == zpmin ? (d_point_internal(F, L0, L1) ? 0.5 : 0.0) : s[0];
