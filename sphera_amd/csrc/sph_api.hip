@@ -57,6 +57,7 @@ struct sph_ctx {
     int nkeys = 1;             // cell keys (cells + out-of-grid bucket per segment)
     int nb_stride_max = 1;     // largest NMAXPARTJ of the segments (list capacity)
     std::vector<int> staged;   // segments uploaded since the last commit
+    std::vector<int> seg_n;    // particles of each segment's last upload
     int precision = SPH_FP64;
     hipStream_t stream = nullptr;
     // faces / tables
@@ -1052,12 +1053,9 @@ int choose_form(sph_ctx* c) {
     const Tiles T{c->tlist, c->ntile};
     SEGL(k_tile_unfit, 256, 256, T, c->start, L.cap, c->ntile + 1);
     int tiles[2] = {0, 0};  // their number, particles in those that do not fit
-    std::vector<int> is((size_t)IS_COUNT * c->nseg);
     HIPC(hipMemcpyAsync(tiles, c->ntile, sizeof(tiles), hipMemcpyDeviceToHost, c->stream));
-    HIPC(hipMemcpyAsync(is.data(), c->iscal, sizeof(int) * is.size(), hipMemcpyDeviceToHost, c->stream));
     HIPC(hipStreamSynchronize(c->stream));
-    long long n = 0;
-    for (int s = 0; s < c->nseg; ++s) n += is[(size_t)s * IS_COUNT + IS_N];
+    const long long n = std::accumulate(c->seg_n.begin(), c->seg_n.end(), 0ll);
     c->form = L;
     const bool thin = 2.0 * n < tiles[0] * L.home;
     if (c->P.f32) {
@@ -1495,6 +1493,8 @@ int sph_segment_upload(sph_ctx* c, int32_t seg, int32_t n, const double* coord, 
     // the staging buffers go out of scope: wait for the copies
     HIPC(hipStreamSynchronize(c->stream));
     c->staged[seg] = 1;
+    c->seg_n.resize(c->nseg, 0);
+    c->seg_n[seg] = n;
     for (int s = 0; s < c->nseg; ++s)
         if (!c->staged[s]) return 0;  // the other segments come in later calls
     c->staged.clear();
