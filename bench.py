@@ -35,26 +35,27 @@ sys.path.insert(0, str(ROOT))
 import numpy as np  # noqa: E402
 
 HBM_PEAK_GBS = 8000.0
-# algorithmic bytes per particle of one pair pass: each cell stages its 27
-# neighbour cells once (record size S per particle) plus the per-particle output
-REC_BYTES = {  # pass: (S fp64, out fp64, S fp32, out fp32)
-    "continuity": (68, 8, 36, 4),
-    "pressure_smoothing": (52, 8, 28, 4),
-    "momentum": (84, 24, 44, 12),
-    "velocity_smoothing": (68, 24, 36, 12),
+# bytes a pass cannot do without, per particle: each array it takes read once,
+# each it leaves written once (fp64, fp32); beside them the list, 2 bytes an entry
+# (self included)
+PASS_BYTES = {
+    "momentum": (92 + 68, 92 + 84),
+    "velocity_smoothing": (88 + 64, 104 + 64),
+    "continuity": (88 + 24, 88 + 28),
+    "pressure_smoothing": (56 + 24, 44 + 28),
 }
-# neighbour search: each cell stages the FP32 positions (float4, 16 B) of its 27
-# neighbour cells once; output 4 B per list entry (self included) + 4 B count
-NB_STAGE_BYTES = 16
+# neighbour search: the integer position (16 B) and the cell of each particle,
+# its list and its count
+NB_BYTES = 16 + 4 + 4
 
 
 def alg_bytes(kernel, n, pairs_per_step, fp32=True):
-    """Algorithmic bytes of one launch of `kernel` on n particles."""
-    if kernel in REC_BYTES:
-        S, out = REC_BYTES[kernel][2:] if fp32 else REC_BYTES[kernel][:2]
-        return n * (27 * S + out)
+    """Bytes that one launch of `kernel` on n particles cannot do without."""
+    lists = 2 * (pairs_per_step + n)
+    if kernel in PASS_BYTES:
+        return n * PASS_BYTES[kernel][1 if fp32 else 0] + lists
     if kernel == "neighbours":
-        return n * 27 * NB_STAGE_BYTES + 4 * (pairs_per_step + n) + 4 * n
+        return n * NB_BYTES + lists
     return None
 
 
@@ -215,14 +216,16 @@ def main():
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-ref-cpu", action="store_true",
                     help="time only the oracle's CPU restatement, not the reference's own build")
-    ap.add_argument("--no-autotune", action="store_true")
+    ap.add_argument("--no-autotune", action="store_true",
+                    help="accepted for earlier commands; the kernels choose their launch shapes themselves")
     ap.add_argument("--no-graph", action="store_true",
                     help="launch every kernel of a step instead of replaying the step's HIP graph")
     ap.add_argument("--wg", type=int, default=0,
-                    help="fixed workgroup size of the particle kernels (skips the autotuner)")
-    ap.add_argument("--chunk", type=int, default=0, help="fixed FP32 list-walk chunk (4 or 8)")
+                    help="sph_params.wg_size (checked, without effect)")
+    ap.add_argument("--chunk", type=int, default=0,
+                    help="sph_params.chunk (4 or 8; checked, without effect), with --wg")
     ap.add_argument("--nb-shape", type=int, default=0,
-                    help="fixed neighbour-search launch shape (sph_params.nb_shape), with --wg")
+                    help="sph_params.nb_shape (checked, without effect), with --wg")
     ap.add_argument("--only", choices=("fp32_mixed", "fp64"), default=None,
                     help="time one precision only (profiling runs)")
     ap.add_argument("--ens-requests", type=int, default=512,
@@ -253,10 +256,6 @@ def main():
         if args.only and name != args.only:
             continue
         tune = dict(wg_size=args.wg, chunk=args.chunk, nb_shape=args.nb_shape) if args.wg else None
-        if not args.no_autotune and not args.wg:
-            from sphera_amd.autotune import autotune
-            tune, _ = autotune(tb, coord, prec, log=log)
-            log(f"[bench] {name}: autotuned launch {tune}")
         tunes[name] = tune
         log(f"[bench] running {name}")
         res[name] = run_device(tb, coord, prec, args.steps, args.warmup, tune, graph=not args.no_graph)
@@ -282,7 +281,7 @@ def main():
     dom = max(per_k, key=lambda k: per_k[k]["avg_launch_ms"])
     kern = {k: round(v[0] / v[1], 4) for k, v in main_r["timing"].items()}
     # pair kernels only: the four passes' average launch times, one launch each per step
-    pair_step_s = sum(v[0] / v[1] for k, v in main_r["timing"].items() if k in REC_BYTES and v[1]) / 1e3
+    pair_step_s = sum(v[0] / v[1] for k, v in main_r["timing"].items() if k in PASS_BYTES and v[1]) / 1e3
     fp64 = None
     if "fp64" in res and main_name != "fp64":
         r64 = res["fp64"]
@@ -367,7 +366,9 @@ def main():
         "mixed_over_fp64": value / fp64["value"] if fp64 else None,
         "pair_kernels_only_value": pairs_per_step / pair_step_s if pair_step_s > 0 else None,
         "kernel_ms": kern,
-        "roofline": {"bound": "hbm", "kernel": dom, "achieved": per_k[dom]["achieved_gbs"],
+        # the passes and the search issue more than they move: their bytes take
+        # frac of the launch at the peak
+        "roofline": {"bound": "hbm" if per_k[dom]["frac"] > 0.5 else "issue", "kernel": dom, "achieved": per_k[dom]["achieved_gbs"],
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": per_k[dom]["frac"],
                      "traffic": traffic_bytes(dom, n, fp32),
                      "bytes_alg_per_launch": per_k[dom]["bytes_alg_per_launch"],

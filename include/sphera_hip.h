@@ -46,8 +46,8 @@ typedef struct sph_params {
     double den0, eps, celerita, alfamon, kin_visc; /* Med(1) */
     double cfl, vsc_coeff, pesodt, tetap, tetav;   /* input_any_t */
     int32_t semi;        /* 1: SA-SPH frontiers active (Domain%tipo=="semi") */
-    /* launch tunables of the particle kernels (0 = default; the autotuner in
-     * sphera_amd/autotune.py picks them per case) */
+    /* launch tunables of earlier kernels: values out of their range are refused
+     * (status 2), those in it have no effect */
     int32_t wg_size;     /* 64 (default), 128, 192 or 256: accepted for callers that set it, as are the next */
     int32_t chunk;       /* four, 4 or 8 (default): the pair passes choose their own launch shape */
     int32_t chunk_v, chunk_c, chunk_p;

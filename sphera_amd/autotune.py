@@ -1,9 +1,9 @@
-"""Launch-shape autotuner for the particle kernels.
+"""The launch tunables of a case and its step time with them.
 
-The pair passes choose their workgroups by the solve's size (tiles of cells
-held in LDS), so there is one shape left to time: for one case and precision a
-scratch context runs a few steps, and the ``tune`` dict that ``SphContext`` /
-``sph_params`` accept comes back with its time per step.
+The kernels choose their launch shapes themselves (by capacity, h/dx and the
+uploaded state), and the tunables of ``sph_params`` have no effect: there is
+nothing to search, so ``autotune`` times a few steps of a scratch context and
+returns the one ``tune`` dict, which ``SphContext`` accepts, with that time.
 
 The grid's cell size is not a tunable: it is the reference's (CreaGrid), and
 it fixes the neighbour-list order the device reproduces.
@@ -30,7 +30,7 @@ def _run(tb, coord, precision, tune, steps, warmup):
 
 
 def autotune(tb, coord, precision, steps=4, warmup=2, log=None):
-    """Returns (best tune dict, list of (tune, seconds per step))."""
+    """Returns (the tune dict, [(tune, seconds per step)])."""
     tune = dict(wg_size=64, chunk=8)
     s = _run(tb, coord, precision, tune, steps, warmup)
     if log:

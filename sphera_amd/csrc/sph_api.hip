@@ -95,9 +95,8 @@ struct sph_ctx {
     int ncu = 256;  // CUs
     int *work = nullptr, *nwork = nullptr;  // (particle, face) pairs of the boundary table
     int *idslot = nullptr, *rmids = nullptr;  // id -> slot, ids removed by a sort
-    int wg = 256, grid = 1, bt_grid = 1024;  // launch shape of the particle kernels
-    int chunk = 8;                            // list entries gathered per step of the FP32 walks
-    int chunk_v = 8, chunk_c = 8, chunk_p = 8;  // the same for smoothing, continuity, pressure smoothing
+    int wg = 256, grid = 1, chunk = 8;  // what sph_get_launch reports
+    int bt_grid = 1024;
     std::vector<std::pair<int, hipGraphExec_t>> graphs;  // captured n-step sequences
     uint32_t* nbr = nullptr;
     int* nnb = nullptr;
@@ -297,13 +296,12 @@ void tile_dispatch(sph_ctx* c, Launch&& launch) {
         else if (c->form.cap == TILE_CAP_M) launch(IntC<TILE_CAP_M>{}, sg, IntC<1>{});
         else if (c->form.cap == TILE_CAP_S && c->form.g == 1) launch(IntC<TILE_CAP_S>{}, sg, IntC<1>{});
         else if (c->form.cap == TILE_CAP_S) launch(IntC<TILE_CAP_S>{}, sg, IntC<2>{});
-        else if (c->form.g == 1) launch(IntC<TILE_CAP_0>{}, sg, IntC<1>{});
         else launch(IntC<TILE_CAP_0>{}, sg, IntC<2>{});
     };
     if (c->nseg > 1) form(std::true_type{});
     else form(std::false_type{});
 }
-// The FP64 passes (no LDS form with eight lanes).
+// The FP64 passes.
 template <class Launch>
 void tile_dispatch64(sph_ctx* c, Launch&& launch) {
     auto lanes = [&](auto cap, auto sg) {
@@ -315,7 +313,7 @@ void tile_dispatch64(sph_ctx* c, Launch&& launch) {
         if (c->form.cap == TILE_CAP_L) lanes(IntC<TILE_CAP_L>{}, sg);
         else if (c->form.cap == TILE_CAP_S) lanes(IntC<TILE_CAP_S>{}, sg);
         else if (c->form.g == 8) launch(IntC<TILE_CAP_0>{}, sg, IntC<8>{});
-        else lanes(IntC<TILE_CAP_0>{}, sg);
+        else launch(IntC<TILE_CAP_0>{}, sg, IntC<4>{});
     };
     if (c->nseg > 1) form(std::true_type{});
     else form(std::false_type{});
@@ -852,7 +850,8 @@ int layout_segments(sph_ctx* c, int nseg, const sph_params* p, const sph_faces* 
     return 0;
 }
 
-// Launch shape of the particle kernels and the persistent grids.
+// The stream, the wall kernels' grid, and the launch tunables, which are checked
+// and have no effect.
 int setup_launch(sph_ctx* c, const sph_params* p) {
     if (hipStreamCreate(&c->stream) != hipSuccess) return fail(101, "hipStreamCreate failed");
     int dev = 0, ncu = 256;
@@ -862,15 +861,9 @@ int setup_launch(sph_ctx* c, const sph_params* p) {
     c->wg = p->wg_size > 0 ? p->wg_size : 64;
     if (c->wg < 64 || c->wg > 256 || c->wg % 64) return fail(2, "wg_size must be 64, 128, 192 or 256");
     c->grid = (c->P.cap + c->wg - 1) / c->wg;
-    c->chunk = p->chunk > 0 ? p->chunk : 8;
-    c->chunk_v = p->chunk_v > 0 ? p->chunk_v : c->chunk;
-    c->chunk_c = p->chunk_c > 0 ? p->chunk_c : c->chunk;
-    c->chunk_p = p->chunk_p > 0 ? p->chunk_p : c->chunk;
-    auto bad = [](int v) { return v != 4 && v != 8; };
-    if (bad(c->chunk) || bad(c->chunk_v) || bad(c->chunk_c) || bad(c->chunk_p))
-        return fail(2, "chunk must be 4 or 8");
-    if (c->nseg > 1)  // the segmented pair passes are built for whole-group walks
-        c->chunk = c->chunk_v = c->chunk_c = c->chunk_p = 8;
+    for (int v : {p->chunk, p->chunk_v, p->chunk_c, p->chunk_p})
+        if (v > 0 && v != 4 && v != 8) return fail(2, "chunk must be 4 or 8");
+    c->chunk = p->chunk > 0 && c->nseg == 1 ? p->chunk : 8;
     c->bt_grid = 4 * ncu;
     c->ncu = ncu;
     if (p->nb_shape < 0 || p->nb_shape > 4) return fail(2, "nb_shape must be 0 to 4");

@@ -118,8 +118,10 @@ __device__ __forceinline__ d2 fma2(d2 a, d2 b, d2 c) { return __builtin_elementw
 // sqrt() are, without the scaling steps those take for operands near the ends
 // of the exponent range: Newton's iteration for the reciprocal and Markstein's
 // final correction, q + (a - d q) y with y = 1/d (P. Markstein, "Computation of
-// elementary functions on the IBM RISC System/6000 processor", 1990).  A
-// divisor that several quotients share is inverted once.
+// elementary functions on the IBM RISC System/6000 processor", 1990); for the
+// root Goldschmidt's iteration (R. E. Goldschmidt, "Applications of division by
+// convergence", 1964) and the residual's correction.  A divisor that several
+// quotients share is inverted once.
 __device__ __forceinline__ d2 newton64(d2 d, d2 y) { return fma2(fma2(-d, y, d2(1.0)), y, y); }
 __device__ __forceinline__ d2 inv64(d2 d) {
     return newton64(d, newton64(d, d2{__builtin_amdgcn_rcp(d.x), __builtin_amdgcn_rcp(d.y)}));
@@ -246,8 +248,8 @@ __device__ __forceinline__ bool d_point_internal(const DFace& F, double px0, dou
 constexpr int TILE_CAP_L = 2496, TILE_CAP_M = 1632, TILE_CAP_S = 1216, TILE_CAP_0 = 16;
 constexpr int TILE_WG = 512;   // most threads of a pair pass
 constexpr int TILE_U = 5;      // slots a thread stages at a time (FP64: 3)
-constexpr int TILE_G2 = 40000;  // particles below which two lanes take a particle
-// FP64 passes that gather: particles below which eight lanes take a particle,
+constexpr int TILE_G2 = 40000;  // capacity below which two lanes take a particle
+// FP64 passes that gather: capacity below which eight lanes take a particle,
 // else four (DB-SPH steps, us: 2,000 particles eight 265, four 292, two 357;
 // 70,000 eight 611, four 582, two 623; the four passes: 9,000 eight 81, four 88,
 // two 133; 54,000 of twice water's density 331, 317, 327; 576,000 1834, 1375, 1442)
@@ -301,7 +303,7 @@ __device__ __forceinline__ void tile_coords(DPC& P, int id, int& ti, int& tj, in
 // them in an LDS histogram and issues one global atomic per occupied cell.
 // Inside the window a particle's rank among the workgroup's particles of its
 // cell follows the thread order, so particles that stay in their cell keep
-// their previous (ascending-id) order and k_cell_sort finds its runs sorted.
+// their previous (ascending-id) order, in which k_gather compares few ids.
 // ----------------------------------------------------------------------------
 constexpr int HIST_W = 512;
 constexpr int SCAN_B = 4096;  // keys per scan block (HIST_W < SCAN_B)
@@ -2290,8 +2292,6 @@ __global__ __launch_bounds__(256) void k_tile_unfit(Seg S, Tiles T, const int* _
 __device__ __forceinline__ float4 lds16(const float4* a, uint32_t o) {
     return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a) + o);
 }
-
-constexpr uint32_t NB_NONE = 0xFFFFFFFFu;
 
 // wall_function_for_SASPH.f90:56-80 (no land-cover map), FP64: slip
 // coefficient and mixing-length viscosity of one particle-frontier pair at
