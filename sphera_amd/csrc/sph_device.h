@@ -28,8 +28,11 @@ __host__ __device__ inline size_t nb16_index(size_t N, int p, int k) {
 // where a pair lies across a wrap
 __host__ __device__ inline int lsb_diff(int a, int b) { return (int)((uint32_t)a - (uint32_t)b); }
 
-// list capacity per particle: NMAXPARTJ rounded up to whole groups
-__host__ __device__ inline int nb_stride(int nmaxpartj) { return (nmaxpartj + NB_G - 1) / NB_G * NB_G; }
+// list capacity per particle: NMAXPARTJ rounded up to whole groups, two at least
+// (a gathering FP32 walk reads the first two before it knows the list's length)
+__host__ __device__ inline int nb_stride(int nmaxpartj) {
+    return nmaxpartj <= 2 * NB_G ? 2 * NB_G : (nmaxpartj + NB_G - 1) / NB_G * NB_G;
+}
 
 // indices into the device scalar blocks
 enum { SC_DT = 0, SC_DTPREV, SC_DTAVG, SC_TIME, SC_DTVEL, SC_TV1, SC_TP1, SC_COUNT };

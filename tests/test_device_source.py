@@ -71,3 +71,29 @@ def test_integer_positions_wrap_without_overflow(tmp_path):
     assert len(re.findall(r"\(float\)lsb_diff\(", code)) >= 12
     # no signed difference of positions turned into a float
     assert not re.findall(r"\(float\)\(\w+\.[xyz] - (?:\w+\.[xyz]\b|__float_as_int)", code)
+
+
+WALKS = r"""
+#define __host__
+#define __device__
+#include "sph_device.h"
+int main() {
+    // the FP32 walk of a gathering particle i reads the groups 0 and 1 of its list,
+    // whatever its length, before it looks at the length
+    for (int mj = 1; mj <= 100; ++mj)
+        for (size_t N = 1; N <= 300; N += 23)
+            for (size_t i = 0; i < N; ++i)
+                for (size_t m = 0; m < 2; ++m)
+                    if ((m * N + i + 1) * sph::NB_G > N * (size_t)sph::nb_stride(mj)) return 1;
+    for (int mj = 1; mj <= 1000; ++mj)
+        if (sph::nb_stride(mj) < mj || sph::nb_stride(mj) % sph::NB_G) return 2;
+    return 0;
+}
+"""
+
+
+def test_first_groups_of_a_list_are_in_range(tmp_path):
+    (tmp_path / "walks.cpp").write_text(WALKS)
+    exe = tmp_path / "walks"
+    subprocess.run(["g++", "-std=c++17", f"-I{CSRC}", str(tmp_path / "walks.cpp"), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)]).returncode == 0

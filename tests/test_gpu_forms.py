@@ -136,3 +136,23 @@ def test_form_changes_between_uploads(prec):
         for f in FIELDS:
             assert np.array_equal(s[f], r[f]), f
     d.close()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("kind", ["gathers", "tiles"])
+@pytest.mark.parametrize("cut", [1, 8, 9, 16])
+def test_short_lists(cut, kind, prec):
+    """Lists cut at NMAXPARTJ of less than two groups of entries."""
+    from oracle.pyoracle import Oracle
+    tb, st = _cluster(1, n0=500, n1=300) if kind == "gathers" else _water(column=(0.3, 0.2, 0.2))
+    tb.scalars["nmaxpartj"] = cut
+    print(f"[gpu] cut={cut} {kind} prec={prec}", flush=True)
+    o = Oracle(tb, semi=False, **st)
+    o.preloop()
+    o.step(1)
+    s = _run(tb, st, prec, 1, semi=False)
+    _held(s, o.state(), prec)
+    cnt, ids = o.lists()
+    assert np.array_equal(s["lists"][0], cnt)
+    for i, k in enumerate(cnt):
+        assert np.array_equal(s["lists"][1][i, :k], ids[i, :k]), i
