@@ -794,7 +794,7 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
             const int before = PART ? __builtin_amdgcn_readlane(mine, u) : 0;
             const int base = before & ~7;  // the list's first entry in LDS
             int k = before & 7;
-            if (PART && lane < 8) list[lane] = tail[8 * u + lane];
+            if (PART && lane < k) list[lane] = tail[8 * u + lane];
             auto append = [&](int q, bool in) {
                 const unsigned long long m = __ballot(in);
                 const int at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
@@ -811,6 +811,7 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
             if (guard) {  // candidates in the guard band (1 particle in 100): the reference's FP64 test
                 const double4 xi = xm[p];
                 k = before & 7;
+                wave_lds_sync();  // other lanes write the same places again
 #pragma unroll
                 for (int q = 0; q < NCH; ++q) {
                     const float r2 = r2of(q);
@@ -829,6 +830,7 @@ __device__ __forceinline__ int nb_cell_lists(DPC& P, const double4* __restrict__
             // entries to store; the last group filled with the particle itself, as often as it is formed
             const int kn = PART ? max(0, min(last ? k : k & ~7, room)) : min(k, mj);
             const int end = PART ? min(k, room) : kn;
+            wave_lds_sync();
             if (FIT && lane < 8 && (!PART || ((last || room < k) && room >= 0)))
                 list[end + lane] = (E)((uint32_t)(p + self) << 4);
             wave_lds_sync();
